@@ -37,8 +37,8 @@ extern "C" int astrai_moe_abi_version(void) { return ASTRAI_MOE_ABI_VERSION; }
 
 extern "C" const char* astrai_moe_last_error(void) { return g_last_error; }
 
-// Row-tile policy. The bf16 matrix-core kernels need K % 64 == 0 for both
-// GEMMs (dim and dim_ffn multiples of 64); other shapes and fp32 use 64-row
+// Row-tile policy. The bf16 matrix-core kernels take dim and dim_ffn that are
+// multiples of 8 from 64 on (mfma_k_supported); other shapes and fp32 use 64-row
 // tiles (the fp32 matrix-core kernel's and the general kernel's). Among
 // matrix-core tiles (measured on MI355X, both GEMMs, one process; the 32-,
 // 64- and 128-row tiles sum in the same order and give equal bits):
@@ -62,8 +62,7 @@ extern "C" int astrai_moe_select_block_m(int64_t n_tokens, int n_experts,
     return fail(ASTRAI_MOE_EINVAL, "select_block_m: bad sizes");
   if (dtype != ASTRAI_MOE_BF16 && dtype != ASTRAI_MOE_F32)
     return fail(ASTRAI_MOE_EINVAL, "select_block_m: unsupported dtype %d", dtype);
-  const bool mfma_shapes = dtype == ASTRAI_MOE_BF16 && dim % 64 == 0 && dim_ffn % 64 == 0 &&
-                           dim <= (1ll << 22) && dim_ffn <= (1ll << 22);
+  const bool mfma_shapes = dtype == ASTRAI_MOE_BF16 && mfma_shape_supported(dim, dim_ffn);
   if (!mfma_shapes) return 64;
   if (n_experts == 1 && top_k == 1) {
     if (n_tokens < 96) return kMfmaSmallBM;

@@ -30,6 +30,12 @@ static_assert(!(idle_threshold(true, 0) >= 1), "wave 0 never idles");
 static_assert(idle_threshold(true, 128) >= 128 && !(idle_threshold(true, 128) >= 129),
               "the second half idles exactly on tiles of at most 128 rows");
 constexpr int kRowBytes = kBK * 2;  // 128 bytes per staged row
+
+// K steps of a tile. K needs only to be a multiple of 8 (rows of whole
+// 16-byte chunks): in the last, partial step the chunks past the row's end
+// are staged from zeros in both operands (dma_16_or_zero), so they add
+// nothing whatever lies behind the row.
+__host__ __device__ constexpr int k_steps(int64_t K) { return (int)((K + kBK - 1) / kBK); }
 constexpr int kXcds = 8;
 
 template <typename F, int... Is>
@@ -67,6 +73,15 @@ __device__ __forceinline__ T load_scalar(const T* p) {
 __device__ inline void lds_dma_16(const void* gsrc, void* lds_dst) {
   __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)gsrc,
                                    (__attribute__((address_space(3))) void*)lds_dst, 16, 0, 0);
+}
+
+// Source of staged chunks and K-rows past the end of an operand.
+__device__ __attribute__((aligned(512))) uint4 g_zero_row[32] = {};
+
+// lds_dma_16 of byte `off` of a matrix whose lane's chunk starts at byte `col`
+// of a row of `row_bytes`: zeros past the row's end.
+__device__ inline void dma_16_or_zero(const char* base, uint32_t off, uint32_t col, uint32_t row_bytes, void* lds) {
+  lds_dma_16(col < row_bytes ? base + off : reinterpret_cast<const char*>(g_zero_row), lds);
 }
 
 template <int N>

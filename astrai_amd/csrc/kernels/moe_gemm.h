@@ -34,8 +34,17 @@ struct GemmWorkspace {
 constexpr int64_t kSchedBytes = 65536;
 int64_t gemm_workspace_bytes(bool down);
 
-// Shape constraints of the bf16 kernels: K a multiple of 64, the output
-// columns a multiple of the column tile, 16-byte aligned operands.
+// K of the bf16 kernels: a multiple of 8, at least one 64-K step. (Below it,
+// a tile is mostly padding and the general kernels stay.)
+inline bool mfma_k_supported(int64_t k) { return k >= 64 && k % 8 == 0; }
+// Expert shapes whose bf16 GEMMs, forward and backward, all run on the matrix
+// cores.
+inline bool mfma_shape_supported(int64_t dim, int64_t dim_ffn) {
+  return mfma_k_supported(dim) && mfma_k_supported(dim_ffn) && dim <= (1ll << 22) && dim_ffn <= (1ll << 22);
+}
+
+// Shape constraints of the bf16 kernels: K as above, the output columns a
+// multiple of 8, 16-byte aligned operands.
 bool mfma_gate_up_supported(int64_t dim, int64_t dim_ffn, int block_m,
                             const void* a, const void* c);
 bool mfma_down_supported(int64_t dim_ffn, int64_t dim, int block_m,
@@ -53,6 +62,38 @@ int launch_mfma_down(const void* h, const int32_t* tiles, int64_t capacity,
                      int64_t dim_ffn, int64_t dim, int block_m, bool packed,
                      void* y, hipStream_t s,
                      const GemmWorkspace& ws = {});
+
+// The same for K that is no multiple of 64 (moe_gemm_mfma_ragged.hip,
+// moe_gemm_bwd_ragged.hip), where the functions of these names go by
+// themselves; unpacked weights only.
+namespace ragged {
+int launch_mfma_gate_up(const void* x_perm, const int32_t* tiles,
+                        int64_t capacity, const void* const* w_gate,
+                        const void* const* w_up, int64_t dim, int64_t dim_ffn,
+                        int block_m, bool packed, void* h, hipStream_t s,
+                        const GemmWorkspace& ws);
+int launch_mfma_down(const void* h, const int32_t* tiles, int64_t capacity,
+                     const void* const* w_down, const void* sorted_w,
+                     int64_t dim_ffn, int64_t dim, int block_m, bool packed,
+                     void* y, hipStream_t s, const GemmWorkspace& ws);
+int launch_mfma_gate_up_save(const void* x_perm, const int32_t* tiles,
+                             int64_t capacity, const void* const* w_gate,
+                             const void* const* w_up, int64_t dim,
+                             int64_t dim_ffn, void* h, void* gu,
+                             hipStream_t s, const GemmWorkspace& ws);
+int launch_mfma_down_save(const void* h, const int32_t* tiles,
+                          int64_t capacity, const void* const* w_down,
+                          const void* sorted_w, int64_t dim_ffn, int64_t dim,
+                          void* y, void* y_unweighted, hipStream_t s,
+                          const GemmWorkspace& ws);
+int launch_dgrad_down(const void* dy, const int32_t* tiles, int64_t capacity,
+                      const void* const* w_down, const void* gu, int64_t dim,
+                      int64_t dim_ffn, void* dg, void* du, hipStream_t s);
+int launch_dgrad_in(const void* d, const int32_t* tiles, int64_t capacity,
+                    const void* const* w, int64_t k, int64_t n,
+                    const void* add, void* dx, hipStream_t s,
+                    const GemmWorkspace& ws);
+}  // namespace ragged
 
 // As launch_mfma_gate_up, reading the activation rows as x[sorted_token[r]]
 // (x: [n_tokens, dim]) instead of a copied x_perm.

@@ -231,7 +231,7 @@ extern "C" int astrai_moe_gemm_gate_up_gather(const void* x, const int32_t* sort
                  "gemm_gate_up_gather: x must be under 4 GiB (n_tokens %lld, dim %lld)", (long long)n_tokens,
                  (long long)dim);
   if (n_rows == 0) return ASTRAI_MOE_OK;
-  ASTRAI_REQUIRE(mfma_gate_up_supported(dim, dim_ffn, block_m, x, h),
+  ASTRAI_REQUIRE(dim % 64 == 0 && mfma_gate_up_supported(dim, dim_ffn, block_m, x, h),
                  "gemm_gate_up_gather: unsupported shape (dim %lld, dim_ffn %lld, block_m %d) or alignment",
                  (long long)dim, (long long)dim_ffn, block_m);
   ASTRAI_REQUIRE(sorted_token && w_gate && w_up, "gemm_gate_up_gather: null row list or weight table");
@@ -313,7 +313,7 @@ extern "C" int astrai_moe_gemm_gate_up_packed(const void* x_perm, const int32_t*
   if ((rc = check_workspace("gemm_gate_up_packed", workspace, workspace_bytes))) return rc;
   ASTRAI_REQUIRE(dtype == ASTRAI_MOE_BF16, "gemm_gate_up_packed: packed weights are bf16 only");
   // packed weights come in whole 256-row tiles (128 gate + 128 up rows)
-  ASTRAI_REQUIRE(n_rows == 0 || (dim_ffn % 128 == 0 && mfma_gate_up_supported(dim, dim_ffn, block_m, x_perm, h)),
+  ASTRAI_REQUIRE(n_rows == 0 || (dim_ffn % 128 == 0 && dim % 64 == 0 && mfma_gate_up_supported(dim, dim_ffn, block_m, x_perm, h)),
                  "gemm_gate_up_packed: unsupported shape (dim %lld, dim_ffn %lld, block_m %d) or alignment",
                  (long long)dim, (long long)dim_ffn, block_m);
   if (n_rows == 0) return ASTRAI_MOE_OK;
@@ -334,7 +334,7 @@ extern "C" int astrai_moe_gemm_down_packed(const void* h, const int32_t* tiles, 
   if (rc) return rc;
   if ((rc = check_workspace("gemm_down_packed", workspace, workspace_bytes))) return rc;
   ASTRAI_REQUIRE(dtype == ASTRAI_MOE_BF16, "gemm_down_packed: packed weights are bf16 only");
-  ASTRAI_REQUIRE(n_rows == 0 || (dim % 256 == 0 && mfma_down_supported(dim_ffn, dim, block_m, h, y)),
+  ASTRAI_REQUIRE(n_rows == 0 || (dim % 256 == 0 && dim_ffn % 64 == 0 && mfma_down_supported(dim_ffn, dim, block_m, h, y)),
                  "gemm_down_packed: unsupported shape (dim_ffn %lld, dim %lld, block_m %d) or alignment",
                  (long long)dim_ffn, (long long)dim, block_m);
   if (n_rows == 0) return ASTRAI_MOE_OK;
@@ -348,13 +348,21 @@ extern "C" int astrai_moe_gemm_down_packed(const void* h, const int32_t* tiles, 
 // ---------------------------------------------------------------------------
 // Training forward and backward. bf16 with dim and dim_ffn multiples of 64
 // runs the matrix-core kernels (256-row tile lists; partial last column tiles
-// clamp and mask); every other shape and fp32 runs the general-shape kernels
-// (any tile height).
+// clamp and mask). So do the other shapes with dims multiples of 8
+// (mfma_shape_supported) where the tile list has 256 rows and the buffers are
+// aligned; with another tile height, and for every other shape and fp32, the
+// general-shape kernels run (any tile height and alignment).
 // ---------------------------------------------------------------------------
 
 static bool mfma_train_shape(int dtype, int64_t dim, int64_t dim_ffn) {
   return dtype == ASTRAI_MOE_BF16 && dim > 0 && dim_ffn > 0 && dim % 64 == 0 && dim_ffn % 64 == 0 &&
          dim <= (1ll << 22) && dim_ffn <= (1ll << 22);
+}
+
+template <typename... P>
+static bool mfma_train_ragged(int dtype, int64_t dim, int64_t dim_ffn, int block_m, P... buffers) {
+  return dtype == ASTRAI_MOE_BF16 && mfma_shape_supported(dim, dim_ffn) && block_m == kMfmaBigBM &&
+         (aligned16_ptr(buffers) && ...);
 }
 
 static int check_train(const char* who, int dtype, int64_t dim, int64_t dim_ffn, int block_m) {
@@ -381,7 +389,7 @@ extern "C" int astrai_moe_gemm_gate_up_train(const void* x_perm, const int32_t* 
   ASTRAI_REQUIRE(w_gate && w_up && gu, "gemm_gate_up_train: null weight table or output");
   const int64_t capacity = (tiles_len - ASTRAI_MOE_TILE_HEADER) / ASTRAI_MOE_TILE_STRIDE;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (mfma_train_shape(dtype, dim, dim_ffn)) {
+  if (mfma_train_shape(dtype, dim, dim_ffn) || mfma_train_ragged(dtype, dim, dim_ffn, block_m, x_perm, h, gu)) {
     ASTRAI_REQUIRE(aligned16_ptr(x_perm) && aligned16_ptr(h) && aligned16_ptr(gu),
                    "gemm_gate_up_train: buffers must be 16-byte aligned");
     return launch_mfma_gate_up_save(x_perm, tiles, capacity, w_gate, w_up, dim, dim_ffn, h, gu, s,
@@ -409,7 +417,7 @@ extern "C" int astrai_moe_gemm_down_train(const void* h, const int32_t* tiles, i
   ASTRAI_REQUIRE(w_down && sorted_w && y_unweighted, "gemm_down_train: null weight table, row weights or output");
   const int64_t capacity = (tiles_len - ASTRAI_MOE_TILE_HEADER) / ASTRAI_MOE_TILE_STRIDE;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (mfma_train_shape(dtype, dim, dim_ffn)) {
+  if (mfma_train_shape(dtype, dim, dim_ffn) || mfma_train_ragged(dtype, dim, dim_ffn, block_m, h, y, y_unweighted)) {
     ASTRAI_REQUIRE(aligned16_ptr(h) && aligned16_ptr(y) && aligned16_ptr(y_unweighted),
                    "gemm_down_train: buffers must be 16-byte aligned");
     return launch_mfma_down_save(h, tiles, capacity, w_down, sorted_w, dim_ffn, dim, y, y_unweighted, s,
@@ -454,7 +462,7 @@ extern "C" int astrai_moe_gemm_dgrad_down(const void* dy, const int32_t* tiles, 
   ASTRAI_REQUIRE(w_down && gu && du, "gemm_dgrad_down: null weight table or buffer");
   const int64_t capacity = (tiles_len - ASTRAI_MOE_TILE_HEADER) / ASTRAI_MOE_TILE_STRIDE;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (mfma_train_shape(dtype, dim, dim_ffn)) {
+  if (mfma_train_shape(dtype, dim, dim_ffn) || mfma_train_ragged(dtype, dim, dim_ffn, block_m, dy, gu, dg, du)) {
     ASTRAI_REQUIRE(aligned16_ptr(dy) && aligned16_ptr(gu) && aligned16_ptr(dg) && aligned16_ptr(du),
                    "gemm_dgrad_down: buffers must be 16-byte aligned");
     return launch_dgrad_down(dy, tiles, capacity, w_down, gu, dim, dim_ffn, dg, du, s);
@@ -480,7 +488,7 @@ extern "C" int astrai_moe_gemm_dgrad_gate_up(const void* dg, const void* du, con
   const int64_t capacity = (tiles_len - ASTRAI_MOE_TILE_HEADER) / ASTRAI_MOE_TILE_STRIDE;
   hipStream_t s = static_cast<hipStream_t>(stream);
   // dx_perm = round(dg . W_gate), then dx_perm = round(round(du . W_up) + dx_perm)
-  if (mfma_train_shape(dtype, dim, dim_ffn)) {
+  if (mfma_train_shape(dtype, dim, dim_ffn) || mfma_train_ragged(dtype, dim, dim_ffn, block_m, dg, du, dx_perm)) {
     ASTRAI_REQUIRE(aligned16_ptr(dg) && aligned16_ptr(du) && aligned16_ptr(dx_perm),
                    "gemm_dgrad_gate_up: buffers must be 16-byte aligned");
     const GemmWorkspace ws{workspace, workspace_bytes};

@@ -49,16 +49,25 @@
 
 #include <type_traits>
 
+// Set to 1 by moe_gemm_bwd_ragged.hip, which builds the dgrad kernels a second
+// time for K that is no multiple of 64.
+#ifndef ASTRAI_MOE_RAGGED_K
+#define ASTRAI_MOE_RAGGED_K 0
+#endif
+
 namespace astrai_moe {
 namespace {
+
+constexpr bool kRagged = ASTRAI_MOE_RAGGED_K != 0;
+// K steps of a dgrad tile
+__host__ __device__ inline int dgrad_steps(int K) {
+  return kRagged ? (int)((uint32_t)(K + kBK - 1) / kBK) : K / kBK;
+}
 
 typedef short s16x4_t __attribute__((ext_vector_type(4)));
 typedef short s16x8_t __attribute__((ext_vector_type(8)));
 
 enum class Bwd { kDgradDown, kDgradIn, kDgradInAdd, kWgrad };
-
-// Source of K-rows past an expert's last row in wgrad (zero contribution).
-__device__ __attribute__((aligned(512))) uint4 g_zero_row[32] = {};
 
 struct BwdArgs {
   const bf16_t* a0;          // A: dy / dg / du (dgrad, K-major [rows, K]); wgrad: A [rows, M]
@@ -117,7 +126,7 @@ struct RowTileWalk {
   std::conditional_t<kSplit, SplitWalk<BwdCfg::GM>, TileWalk<BwdCfg::GM>> w;
   const int32_t* tiles;
   int ksteps, G, begin, total;
-  __device__ RowTileWalk(const BwdArgs& p, bool tail) : w(make_walk(p)), tiles(p.tiles), ksteps(p.K / kBK), G(w.G) {
+  __device__ RowTileWalk(const BwdArgs& p, bool tail) : w(make_walk(p)), tiles(p.tiles), ksteps(dgrad_steps(p.K)), G(w.G) {
     if constexpr (kSplit) {
       begin = tail ? w.full : 0;
       total = tail ? w.items() : w.full;
@@ -128,7 +137,7 @@ struct RowTileWalk {
   }
   __device__ static decltype(w) make_walk(const BwdArgs& p) {
     if constexpr (kSplit)
-      return SplitWalk<BwdCfg::GM>(p.tiles, p.capacity, p.n_tiles_n, p.K / kBK, p.part != nullptr, p.grid);
+      return SplitWalk<BwdCfg::GM>(p.tiles, p.capacity, p.n_tiles_n, dgrad_steps(p.K), p.part != nullptr, p.grid);
     else
       return TileWalk<BwdCfg::GM>(p.tiles, p.capacity, p.n_tiles_n);
   }
@@ -273,14 +282,18 @@ struct BwdSrc {
       for (int i = 0; i < BwdCfg::OPS; ++i) {
         const int q = dw * BwdCfg::OPS + i;
         const uint32_t row = (uint32_t)min(q * 8 + dl.row, rows - 1);
-        lds_dma_16(a0 + (row * ((uint32_t)p.K * 2u) + dl.chunk(q)), stage + q * 1024);
+        if (kRagged && (kstep + 1) * kBK > p.K)  // the partial last step
+          dma_16_or_zero(a0, row * ((uint32_t)p.K * 2u) + dl.chunk(q), dl.chunk(q), (uint32_t)p.K * 2u,
+                         stage + q * 1024);
+        else
+          lds_dma_16(a0 + (row * ((uint32_t)p.K * 2u) + dl.chunk(q)), stage + q * 1024);
       }
     }
   }
   // This DMA wave's share of step kstep's B stage (MN-major in every mode;
-  // dgrad's weights have no rows to zero).
+  // dgrad's weights have rows to zero past a ragged K only).
   __device__ void dma_b(const BwdArgs& p, int lane, int kstep, int dw, char* stage) const {
-    const int valid = kMode == Bwd::kWgrad ? rows : 0x7fffffff;
+    const int valid = kMode == Bwd::kWgrad ? rows : kRagged ? p.K : 0x7fffffff;
     dma_mn_step(b0, kstep * kBK, valid, (uint32_t)p.N * 2u, b_col0, (uint32_t)p.N * 2u, b_mn, lane, dw, stage);
   }
 };
@@ -645,7 +658,7 @@ __global__ __launch_bounds__(Cfg::THREADS, 1) void gemm_bwd_kernel(const BwdArgs
   constexpr bool kIdleHalf = kMode == Bwd::kDgradDown;
   // first row tile where padding-only waves idle: every tile with short
   // tiles, else the tiles after the list's whole groups (as in the forward)
-  const int idle_mt0 = kIdleHalf ? __builtin_amdgcn_readfirstlane(p.K / kBK < kIdleMaxSteps ? 0 : p.tiles[3]) : 0;
+  const int idle_mt0 = kIdleHalf ? __builtin_amdgcn_readfirstlane(dgrad_steps(p.K) < kIdleMaxSteps ? 0 : p.tiles[3]) : 0;
   while (true) {
     // dgrad_down: in an expert's last row tile of at most BM / 2 rows the
     // waves of the second half hold only padding rows; they keep the step
@@ -748,7 +761,7 @@ int launch_bwd(BwdArgs p, int64_t total, hipStream_t s, const char* name, const 
   p.grid = (int)grid;
   p.part = nullptr;
   constexpr bool kSplit = kMode == Bwd::kDgradIn || kMode == Bwd::kDgradInAdd;
-  if (kSplit && ws.base != nullptr && p.K / kBK >= kSplitMinTileSteps &&
+  if (kSplit && ws.base != nullptr && dgrad_steps(p.K) >= kSplitMinTileSteps &&
       ws.bytes >= kSchedBytes + grid * (int64_t)sizeof(float) * kSplitUnitFloats)
     p.part = reinterpret_cast<float*>(static_cast<char*>(ws.base) + kSchedBytes);
   hipLaunchKernelGGL((gemm_bwd_kernel<kMode>), dim3((unsigned)grid), dim3(BwdCfg::THREADS), 0, s, p);
@@ -766,6 +779,9 @@ int launch_bwd(BwdArgs p, int64_t total, hipStream_t s, const char* name, const 
 
 }  // namespace
 
+#if ASTRAI_MOE_RAGGED_K
+namespace ragged {
+#else
 int launch_row_grad(const void* dout, const int32_t* sorted_token, const void* sorted_w, const void* y,
                     int64_t n_rows, int64_t dim, void* dy, void* dw_rows, hipStream_t s) {
   if (n_rows == 0) return ASTRAI_MOE_OK;
@@ -775,9 +791,13 @@ int launch_row_grad(const void* dout, const int32_t* sorted_token, const void* s
                      static_cast<bf16_t*>(dw_rows));
   return check_launch("row_grad_kernel");
 }
+#endif  // ASTRAI_MOE_RAGGED_K
 
 int launch_dgrad_down(const void* dy, const int32_t* tiles, int64_t capacity, const void* const* w_down,
                       const void* gu, int64_t dim, int64_t dim_ffn, void* dg, void* du, hipStream_t s) {
+#if !ASTRAI_MOE_RAGGED_K
+  if (dim % kBK != 0) return ragged::launch_dgrad_down(dy, tiles, capacity, w_down, gu, dim, dim_ffn, dg, du, s);
+#endif
   BwdArgs p{};
   p.a0 = static_cast<const bf16_t*>(dy);
   p.w0 = w_down;
@@ -794,6 +814,9 @@ int launch_dgrad_down(const void* dy, const int32_t* tiles, int64_t capacity, co
 
 int launch_dgrad_in(const void* d, const int32_t* tiles, int64_t capacity, const void* const* w, int64_t k,
                     int64_t n, const void* add, void* dx, hipStream_t s, const GemmWorkspace& ws) {
+#if !ASTRAI_MOE_RAGGED_K
+  if (k % kBK != 0) return ragged::launch_dgrad_in(d, tiles, capacity, w, k, n, add, dx, s, ws);
+#endif
   BwdArgs p{};
   p.a0 = static_cast<const bf16_t*>(d);
   p.w0 = w;
@@ -809,6 +832,9 @@ int launch_dgrad_in(const void* d, const int32_t* tiles, int64_t capacity, const
   return launch_bwd<Bwd::kDgradIn>(p, capacity * p.n_tiles_n, s, "gemm_bwd_kernel<dgrad_in>", ws);
 }
 
+#if ASTRAI_MOE_RAGGED_K
+}  // namespace ragged
+#else
 int launch_wgrad(const void* a, const void* b, const int32_t* offsets, int n_experts, int64_t m, int64_t n,
                  void* dw, hipStream_t s) {
   BwdArgs p{};
@@ -823,5 +849,6 @@ int launch_wgrad(const void* a, const void* b, const int32_t* offsets, int n_exp
   p.n_experts = n_experts;
   return launch_bwd<Bwd::kWgrad>(p, (int64_t)n_experts * p.n_tiles_m * p.n_tiles_n, s, "gemm_bwd_kernel<wgrad>");
 }
+#endif  // ASTRAI_MOE_RAGGED_K
 
 }  // namespace astrai_moe

@@ -77,9 +77,16 @@
 
 #include <type_traits>
 
+// Set to 1 by moe_gemm_mfma_ragged.hip, which builds these kernels a second
+// time for K that is no multiple of 64.
+#ifndef ASTRAI_MOE_RAGGED_K
+#define ASTRAI_MOE_RAGGED_K 0
+#endif
 
 namespace astrai_moe {
 namespace {
+
+constexpr bool kRagged = ASTRAI_MOE_RAGGED_K != 0;
 
 // Per-tile global bases: activation rows and the expert's weight rows. With
 // kPacked the expert's weight comes as a packed copy (pack_kernel): the BN
@@ -114,18 +121,25 @@ struct TileSrc {
                         : b_base0;
     }
   }
-  // 8-row group q of the A tile (pad rows past the tile's last row re-read that row)
+  // 8-row group q of the A tile (pad rows past the tile's last row re-read that row).
+  // kTail: the partial last step of a K that is no multiple of 64.
+  template <bool kTail>
   __device__ void dma_a(const DmaLane& dl, int q, uint32_t k2, char* lds) const {
     const uint32_t row = (uint32_t)min(q * 8 + dl.row, rows - 1);
-    lds_dma_16(a_base + (row * k2 + dl.chunk(q)), lds);
+    dma_a_rows<kTail>(dl, row * k2, q, k2, lds);
   }
-  // 8-row group q of the A tile, the lane's row at byte offset row_off of x (gather)
-  __device__ void dma_a_rows(const DmaLane& dl, uint32_t row_off, int q, char* lds) const {
-    lds_dma_16(a_base + (row_off + dl.chunk(q)), lds);
+  // 8-row group q of the A tile, the lane's row at byte offset row_off (of x: gather)
+  template <bool kTail>
+  __device__ void dma_a_rows(const DmaLane& dl, uint32_t row_off, int q, uint32_t k2, char* lds) const {
+    if constexpr (kTail)
+      dma_16_or_zero(a_base, row_off + dl.chunk(q), dl.chunk(q), k2, lds);
+    else
+      lds_dma_16(a_base + (row_off + dl.chunk(q)), lds);
   }
   // 8-row group q of the B tile of K step kstep (up rows follow the gate rows;
   // in a partial last column tile, rows past the matrix re-read its last row,
   // and the epilogue stores none of their columns)
+  template <bool kTail>
   __device__ void dma_b(const DmaLane& dl, int lane, int kstep, int q, uint32_t k2, char* lds) const {
     if constexpr (kPacked) {
       lds_dma_16(b_base0 + ((uint32_t)kstep * (BN * kRowBytes) + (uint32_t)q * 1024 + (uint32_t)lane * 16), lds);
@@ -134,7 +148,11 @@ struct TileSrc {
       const int r0 = q * 8;
       const char* bb = (kGateUp && r0 >= BN / 2) ? b_base1 : b_base0;
       const int rq = (kGateUp && r0 >= BN / 2) ? r0 - BN / 2 : r0;
-      lds_dma_16(bb + ((uint32_t)min(rq + dl.row, b_rows - 1) * k2 + dl.chunk(q)), lds);
+      const uint32_t off = (uint32_t)min(rq + dl.row, b_rows - 1) * k2 + dl.chunk(q);
+      if constexpr (kTail)
+        dma_16_or_zero(bb, off, dl.chunk(q), k2, lds);
+      else
+        lds_dma_16(bb + off, lds);
     }
   }
 };
@@ -473,7 +491,8 @@ __global__ __launch_bounds__(StreamCfg<kGateUp>::THREADS, 1) void gemm_stream_ke
   using Cfg = StreamCfg<kGateUp>;
   __shared__ __attribute__((aligned(1024))) char smem[Cfg::LDS];
 
-  const int KT = K / kBK;  // steps per tile
+  // steps per tile (the rounding in signed arithmetic made this kernel spill 21 registers)
+  const int KT = kRagged ? (int)((uint32_t)(K + kBK - 1) / kBK) : K / kBK;
   // part: partial sums of the split tail tiles (null: the tail runs whole;
   // only the down GEMMs take one); sched: the run-time claims (null: the
   // whole walk is dealt statically)
@@ -504,27 +523,41 @@ __global__ __launch_bounds__(StreamCfg<kGateUp>::THREADS, 1) void gemm_stream_ke
     ca.start(walk, seq, tiles, A, W0, W1, K, N);
     cb.start(walk, seq, tiles, A, W0, W1, K, N);
     load_rows();
-    auto issue_a = [&](int buf) {
+    auto tail_step = [&](int kt) { return kRagged && (kt + 1) * kBK > K; };
+    auto ops_a = [&](auto tail_c, int buf) {
+      constexpr bool kTail = decltype(tail_c)::value;
       const DmaLane dl(lane, ca.kt);
       char* base = smem + Cfg::A_OFF + buf * Cfg::A_BYTES;
 #pragma unroll
       for (int i = 0; i < Cfg::OPS; ++i) {
         const int q = dw * Cfg::OPS + i;
         if constexpr (kGather)
-          ca.src.dma_a_rows(dl, grows.off[i], q, base + q * 1024);
+          ca.src.template dma_a_rows<kTail>(dl, grows.off[i], q, k2, base + q * 1024);
         else
-          ca.src.dma_a(dl, q, k2, base + q * 1024);
+          ca.src.template dma_a<kTail>(dl, q, k2, base + q * 1024);
       }
+    };
+    auto issue_a = [&](int buf) {
+      if (tail_step(ca.kt))
+        ops_a(std::true_type{}, buf);
+      else
+        ops_a(std::false_type{}, buf);
       if (ca.advance(walk, seq, tiles, A, W0, W1, K, N)) load_rows();  // the next item's rows
     };
-    auto issue_b = [&](int buf) {
+    auto ops_b = [&](auto tail_c, int buf) {
       const DmaLane dl(lane, cb.kt);
       char* base = smem + Cfg::B_OFF + buf * Cfg::B_BYTES;
 #pragma unroll
       for (int i = 0; i < Cfg::OPS; ++i) {
         const int q = dw * Cfg::OPS + i;
-        cb.src.dma_b(dl, lane, cb.kt, q, k2, base + q * 1024);
+        cb.src.template dma_b<decltype(tail_c)::value>(dl, lane, cb.kt, q, k2, base + q * 1024);
       }
+    };
+    auto issue_b = [&](int buf) {
+      if (tail_step(cb.kt))
+        ops_b(std::true_type{}, buf);
+      else
+        ops_b(std::false_type{}, buf);
       cb.advance(walk, seq, tiles, A, W0, W1, K, N);
     };
     // prologue in issue order B0, A0, B1, A1, B2 (as far as the steps exist)
@@ -756,7 +789,7 @@ __global__ __launch_bounds__(64) void split_reduce_kernel(const float* __restric
                                                            const bf16_t* __restrict__ row_w, bf16_t* __restrict__ C,
                                                            int N, bf16_t* __restrict__ S0) {
   using Cfg = StreamCfg<kGateUp>;
-  const SplitWalk<Cfg::GM> walk(tiles, capacity, n_tiles_n, K / kBK, true, G);
+  const SplitWalk<Cfg::GM> walk(tiles, capacity, n_tiles_n, kRagged ? k_steps(K) : K / kBK, true, G);
   const int t = blockIdx.x;
   if (walk.S < 2 || t >= walk.total - walk.full) return;
   int mt = 0, nt = 0;
@@ -842,31 +875,38 @@ __global__ __launch_bounds__(Cfg::THREADS, 1) void gemm_mfma_kernel(
   // one stacked allocation) at equal offsets, which measured 11 % slower on
   // the decode gate/up GEMM. The start depends only on the expert, so every
   // tile height sums an output in the same order.
-  const int kt_n = K / kBK;
+  const int kt_n = kRagged ? k_steps(K) : K / kBK;
   int k_start = 0;
   auto setup_tile = [&](int mt_, int nt_) {
     src.setup(tiles, A, W0, W1, K, N, mt_, nt_);
     k_start = (tiles[ASTRAI_MOE_TILE_HEADER + (int64_t)mt_ * ASTRAI_MOE_TILE_STRIDE] * 7) % kt_n;
     if constexpr (kGather) grows.load(row_src, src.row0, src.rows, wave * Cfg::A_PER_WAVE, lane, k2);
   };
-  auto issue_stage = [&](int kstep, int buf) {  // the tile's kstep-th step
+  auto stage_ops = [&](auto tail_c, int ks, int buf) {
+    constexpr bool kTail = decltype(tail_c)::value;
     char* sa = smem + buf * Cfg::STAGE_BYTES;
     char* sb = sa + Cfg::A_BYTES;
-    const int ks = kstep + k_start < kt_n ? kstep + k_start : kstep + k_start - kt_n;  // K step loaded
     const DmaLane dl(lane, ks);
 #pragma unroll
     for (int i = 0; i < Cfg::A_PER_WAVE; ++i) {
       const int q = wave * Cfg::A_PER_WAVE + i;
       if constexpr (kGather)
-        src.dma_a_rows(dl, grows.off[i], q, sa + q * 1024);
+        src.template dma_a_rows<kTail>(dl, grows.off[i], q, k2, sa + q * 1024);
       else
-        src.dma_a(dl, q, k2, sa + q * 1024);
+        src.template dma_a<kTail>(dl, q, k2, sa + q * 1024);
     }
 #pragma unroll
     for (int i = 0; i < Cfg::B_PER_WAVE; ++i) {
       const int q = wave * Cfg::B_PER_WAVE + i;
-      src.dma_b(dl, lane, ks, q, k2, sb + q * 1024);
+      src.template dma_b<kTail>(dl, lane, ks, q, k2, sb + q * 1024);
     }
+  };
+  auto issue_stage = [&](int kstep, int buf) {  // the tile's kstep-th step
+    const int ks = kstep + k_start < kt_n ? kstep + k_start : kstep + k_start - kt_n;  // K step loaded
+    if (kRagged && (ks + 1) * kBK > K)
+      stage_ops(std::true_type{}, ks, buf);
+    else
+      stage_ops(std::false_type{}, ks, buf);
   };
 
   // ---- MFMA fragment reads (16x16x32: lane l holds row l % 16, K 8*(l/16)..+7) ----
@@ -917,7 +957,7 @@ __global__ __launch_bounds__(Cfg::THREADS, 1) void gemm_mfma_kernel(
     __builtin_amdgcn_sched_group_barrier(0x008, MT16 * NT16 - (MT16 + NT16), 0);
   };
 
-  const int KT = K / kBK;
+  const int KT = kt_n;
   setup_tile(mt, nt);
 #pragma unroll
   for (int s = 0; s < S; ++s)
@@ -1009,7 +1049,7 @@ int launch_stream(const void* A, const int32_t* tiles, int64_t capacity, const v
   // run-time claims need the scheduling block and long tiles; the down
   // GEMMs' tail is split when its tiles are long and the partial sums hold a
   // unit per workgroup
-  const int64_t ksteps = K / kBK;
+  const int64_t ksteps = k_steps(K);
   const bool have_ws = ws.base != nullptr && ws.bytes >= kSchedBytes && grid <= kMaxSchedGroups;
   int32_t* sched = (have_ws && ksteps >= kDynamicMinSteps) ? static_cast<int32_t*>(ws.base) : nullptr;
   float* part = (!kGateUp && have_ws && ksteps >= kSplitMinTileSteps &&
@@ -1078,42 +1118,66 @@ int down_dispatch(const void* h, const int32_t* tiles, int64_t capacity, const v
 
 }  // namespace
 
-// K a multiple of the 64-K step; output columns a multiple of 8 (16-byte
+#if !ASTRAI_MOE_RAGGED_K
+// K a multiple of 8 (whole 16-byte chunks; the last 64-K step may be partial)
+// and at least one whole step; output columns a multiple of 8 (16-byte
 // stores; the last column tile may be partial). 32-bit DMA offsets: a tile
 // spans at most 256 rows of K * 2 bytes.
 bool mfma_gate_up_supported(int64_t dim, int64_t dim_ffn, int block_m, const void* a, const void* c) {
   return (block_m == kMfmaBigBM || block_m == kMfmaMid2BM || block_m == kMfmaMidBM || block_m == kMfmaSmallBM) &&
-         dim > 0 && dim_ffn > 0 && dim % kBK == 0 && dim_ffn % 8 == 0 && dim <= (1ll << 22) &&
+         mfma_k_supported(dim) && dim_ffn > 0 && dim_ffn % 8 == 0 && dim <= (1ll << 22) &&
          dim_ffn <= (1ll << 22) && aligned16(a) && aligned16(c);
-}
-
-bool mfma_down_supported(int64_t dim_ffn, int64_t dim, int block_m, const void* a, const void* c) {
-  return (block_m == kMfmaBigBM || block_m == kMfmaMid2BM || block_m == kMfmaMidBM || block_m == kMfmaSmallBM) &&
-         dim > 0 && dim_ffn > 0 && dim_ffn % kBK == 0 && dim % 8 == 0 && dim <= (1ll << 22) &&
-         dim_ffn <= (1ll << 22) && aligned16(a) && aligned16(c);
-}
-
-int launch_mfma_gate_up(const void* x_perm, const int32_t* tiles, int64_t capacity, const void* const* w_gate,
-                        const void* const* w_up, int64_t dim, int64_t dim_ffn, int block_m, bool packed, void* h,
-                        hipStream_t s, const GemmWorkspace& ws) {
-  return packed ? gate_up_dispatch<true>(x_perm, tiles, capacity, w_gate, w_gate, dim, dim_ffn, block_m, h, s, ws)
-                : gate_up_dispatch<false>(x_perm, tiles, capacity, w_gate, w_up, dim, dim_ffn, block_m, h, s, ws);
-}
-
-int launch_mfma_down(const void* h, const int32_t* tiles, int64_t capacity, const void* const* w_down,
-                     const void* sorted_w, int64_t dim_ffn, int64_t dim, int block_m, bool packed, void* y,
-                     hipStream_t s, const GemmWorkspace& ws) {
-  return packed ? down_dispatch<true>(h, tiles, capacity, w_down, sorted_w, dim_ffn, dim, block_m, y, s, ws)
-                : down_dispatch<false>(h, tiles, capacity, w_down, sorted_w, dim_ffn, dim, block_m, y, s, ws);
 }
 
 int64_t gemm_workspace_bytes(bool down) {
   return kSchedBytes + (down ? (int64_t)cu_count() * (int64_t)sizeof(float) * kSplitUnitFloats : 0);
 }
 
+bool mfma_down_supported(int64_t dim_ffn, int64_t dim, int block_m, const void* a, const void* c) {
+  return (block_m == kMfmaBigBM || block_m == kMfmaMid2BM || block_m == kMfmaMidBM || block_m == kMfmaSmallBM) &&
+         mfma_k_supported(dim_ffn) && dim > 0 && dim % 8 == 0 && dim <= (1ll << 22) &&
+         dim_ffn <= (1ll << 22) && aligned16(a) && aligned16(c);
+}
+
+#endif  // !ASTRAI_MOE_RAGGED_K
+
+#if ASTRAI_MOE_RAGGED_K
+namespace ragged {
+#endif
+
+int launch_mfma_gate_up(const void* x_perm, const int32_t* tiles, int64_t capacity, const void* const* w_gate,
+                        const void* const* w_up, int64_t dim, int64_t dim_ffn, int block_m, bool packed, void* h,
+                        hipStream_t s, const GemmWorkspace& ws) {
+#if ASTRAI_MOE_RAGGED_K
+  if (packed) return fail(ASTRAI_MOE_EINVAL, "gemm_gate_up: packed weights need whole K steps");
+#else
+  if (dim % kBK != 0)
+    return ragged::launch_mfma_gate_up(x_perm, tiles, capacity, w_gate, w_up, dim, dim_ffn, block_m, packed, h, s, ws);
+#endif
+  return packed ? gate_up_dispatch<!kRagged>(x_perm, tiles, capacity, w_gate, w_gate, dim, dim_ffn, block_m, h, s, ws)
+                : gate_up_dispatch<false>(x_perm, tiles, capacity, w_gate, w_up, dim, dim_ffn, block_m, h, s, ws);
+}
+
+int launch_mfma_down(const void* h, const int32_t* tiles, int64_t capacity, const void* const* w_down,
+                     const void* sorted_w, int64_t dim_ffn, int64_t dim, int block_m, bool packed, void* y,
+                     hipStream_t s, const GemmWorkspace& ws) {
+#if ASTRAI_MOE_RAGGED_K
+  if (packed) return fail(ASTRAI_MOE_EINVAL, "gemm_down: packed weights need whole K steps");
+#else
+  if (dim_ffn % kBK != 0)
+    return ragged::launch_mfma_down(h, tiles, capacity, w_down, sorted_w, dim_ffn, dim, block_m, packed, y, s, ws);
+#endif
+  return packed ? down_dispatch<!kRagged>(h, tiles, capacity, w_down, sorted_w, dim_ffn, dim, block_m, y, s, ws)
+                : down_dispatch<false>(h, tiles, capacity, w_down, sorted_w, dim_ffn, dim, block_m, y, s, ws);
+}
+
 int launch_mfma_gate_up_save(const void* x_perm, const int32_t* tiles, int64_t capacity, const void* const* w_gate,
                              const void* const* w_up, int64_t dim, int64_t dim_ffn, void* h, void* gu,
                              hipStream_t s, const GemmWorkspace& ws) {
+#if !ASTRAI_MOE_RAGGED_K
+  if (dim % kBK != 0)
+    return ragged::launch_mfma_gate_up_save(x_perm, tiles, capacity, w_gate, w_up, dim, dim_ffn, h, gu, s, ws);
+#endif
   return launch_stream<true, false, true>(x_perm, tiles, capacity, w_gate, w_up, nullptr, dim, dim_ffn, h, s, gu,
                                           nullptr, nullptr, ws);
 }
@@ -1121,9 +1185,17 @@ int launch_mfma_gate_up_save(const void* x_perm, const int32_t* tiles, int64_t c
 int launch_mfma_down_save(const void* h, const int32_t* tiles, int64_t capacity, const void* const* w_down,
                           const void* sorted_w, int64_t dim_ffn, int64_t dim, void* y, void* y_unweighted,
                           hipStream_t s, const GemmWorkspace& ws) {
+#if !ASTRAI_MOE_RAGGED_K
+  if (dim_ffn % kBK != 0)
+    return ragged::launch_mfma_down_save(h, tiles, capacity, w_down, sorted_w, dim_ffn, dim, y, y_unweighted, s, ws);
+#endif
   return launch_stream<false, false, true>(h, tiles, capacity, w_down, nullptr, sorted_w, dim_ffn, dim, y, s,
                                            y_unweighted, nullptr, nullptr, ws);
 }
+
+#if ASTRAI_MOE_RAGGED_K
+}  // namespace ragged
+#else
 
 int launch_mfma_gate_up_gather(const void* x, const int32_t* sorted_token, const int32_t* tiles, int64_t capacity,
                                const void* const* w_gate, const void* const* w_up, int64_t dim, int64_t dim_ffn,
@@ -1155,5 +1227,6 @@ int launch_pack(const void* w0, const void* w1, int64_t rows, int64_t k, bool ga
                        static_cast<const bf16_t*>(w0), n_tiles, (int)k, static_cast<uint4*>(out));
   return check_launch(gate_up ? "pack_kernel<gate_up>" : "pack_kernel<down>");
 }
+#endif  // !ASTRAI_MOE_RAGGED_K
 
 }  // namespace astrai_moe

@@ -295,17 +295,18 @@ def _out_buffer(out: torch.Tensor | None, rows: int, cols: int, like: torch.Tens
 
 
 def matrix_core_supported(dim: int, dim_ffn: int, dtype: torch.dtype) -> bool:
-    """Whether the bf16 forward GEMMs of this expert shape run on the matrix
-    cores (dim and dim_ffn multiples of 64; the last column tile may be
-    partial)."""
-    return (dtype == torch.bfloat16 and dim % 64 == 0 and dim_ffn % 64 == 0 and 0 < dim <= 1 << 22
-            and 0 < dim_ffn <= 1 << 22)
+    """Whether the bf16 GEMMs of this expert shape run on the matrix cores
+    (dim and dim_ffn multiples of 8 from 64 on; the last column tile and the
+    last K step may be partial)."""
+    return (dtype == torch.bfloat16 and dim % 8 == 0 and dim_ffn % 8 == 0 and 64 <= dim <= 1 << 22
+            and 64 <= dim_ffn <= 1 << 22)
 
 
 def gather_supported(n_tokens: int, dim: int, dim_ffn: int, dtype: torch.dtype) -> bool:
     """Whether ``moe_gemm_gate_up_gather`` takes this problem (bf16, the
-    matrix-core shapes, x under 4 GiB)."""
-    return matrix_core_supported(dim, dim_ffn, dtype) and n_tokens * dim * 2 < 1 << 32
+    matrix-core shapes with dims multiples of 64, x under 4 GiB)."""
+    return (matrix_core_supported(dim, dim_ffn, dtype) and dim % 64 == 0 and dim_ffn % 64 == 0
+            and n_tokens * dim * 2 < 1 << 32)
 
 
 def moe_gemm_gate_up_gather(x: torch.Tensor, sorted_token: torch.Tensor, tiles: torch.Tensor, w_gate: torch.Tensor,
@@ -511,7 +512,7 @@ def moe_routed_forward(x: torch.Tensor, logits: torch.Tensor, w_gate: torch.Tens
 
 def backward_on_matrix_cores(dim: int, dim_ffn: int, dtype: torch.dtype) -> bool:
     """Whether training runs the matrix-core kernels for this expert shape
-    (bf16, dim and dim_ffn multiples of 64; 256-row tile lists). Every other
+    (bf16, dim and dim_ffn multiples of 8; 256-row tile lists). Every other
     shape and fp32 runs the general-shape kernels."""
     return matrix_core_supported(dim, dim_ffn, dtype)
 

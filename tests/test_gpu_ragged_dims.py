@@ -1,0 +1,55 @@
+"""bf16 layers whose dims are multiples of 8 but not of 64 on the matrix-core
+kernels: the last K step of every GEMM is partial and staged with zeros behind
+the rows. Remainders of 8, 40 and 56 of a step, one step and several, at row
+counts of every tile height, against the oracle with the tolerances of
+test_gpu_layer.py and test_gpu_backward.py; and what lies behind a row (the
+next row) must not reach its output, NaN included."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from astrai_amd.extension import ops
+from test_gpu_backward import _check_moe, _random_layer
+from test_gpu_layer import check_layer
+
+pytestmark = pytest.mark.gpu
+
+DIMS = [(72, 120), (1000, 424), (184, 1080)]
+
+
+@pytest.mark.parametrize("dim,dim_ffn", DIMS)
+@pytest.mark.parametrize("n_tok", [3, 130, 257, 700])  # 32-, 64-, 128- and 256-row tiles at 4 experts, top-2
+def test_layer(gpu, dim, dim_ffn, n_tok):
+    assert ops.matrix_core_supported(dim, dim_ffn, torch.bfloat16)
+    layer = _random_layer(gpu, dim, dim_ffn, 4, 1, 2, torch.bfloat16, seed=dim + n_tok).requires_grad_(False)
+    x = torch.randn(1, n_tok, dim, device=gpu).to(torch.bfloat16)
+    check_layer(layer, x, f"d{dim}_f{dim_ffn}_t{n_tok}")
+
+
+@pytest.mark.parametrize("dim,dim_ffn", DIMS)
+def test_training(gpu, dim, dim_ffn):
+    layer = _random_layer(gpu, dim, dim_ffn, 4, 1, 2, torch.bfloat16, seed=dim)
+    x = torch.randn(1, 333, dim, device=gpu).to(torch.bfloat16)
+    _check_moe(layer, x, f"d{dim}_f{dim_ffn}")
+
+
+@pytest.mark.parametrize("n_tok", [40, 700])
+def test_rows_do_not_read_past_their_end(gpu, n_tok):
+    layer = _random_layer(gpu, 1000, 424, 1, 0, 1, torch.bfloat16, seed=1).requires_grad_(False)
+    x = torch.randn(1, n_tok, 1000, device=gpu).to(torch.bfloat16)
+    clean = layer(x)
+    x[0, 1::2] = float("nan")  # every even row is followed by NaN
+    got = layer(x)
+    assert torch.equal(got[0, ::2], clean[0, ::2])
+    assert got[0, 1::2].isnan().all()
+
+
+def test_unaligned_rows_still_run(gpu):
+    # 8-byte aligned rows: the general kernels, as before
+    layer = _random_layer(gpu, 1000, 424, 4, 0, 2, torch.bfloat16, seed=2).requires_grad_(False)
+    flat = torch.randn(1 + 4 + 65 * 1000, device=gpu).to(torch.bfloat16)
+    x = flat[4:4 + 65 * 1000].view(1, 65, 1000)
+    assert x.data_ptr() % 16 == 8
+    check_layer(layer, x, "unaligned")
