@@ -28,6 +28,7 @@
 // rows are read and the output written with non-temporal hints (each byte is
 // touched once), which measured faster there and slower at top-6.
 #include "moe_common.h"
+#include "moe_gemm.h"
 
 namespace astrai_moe {
 namespace {
@@ -70,7 +71,7 @@ template <typename T, int VW, int KMAX, int U, bool NT>
 __global__ __launch_bounds__(kCombineThreads) void combine_kernel(
     const T* __restrict__ y, const int32_t* __restrict__ token_pos, const T* __restrict__ row_w,
     const T* __restrict__ shared, int n_shared, float inv_shared,
-    int64_t n_tokens, int top_k, int64_t dim, int64_t seg_units, T* __restrict__ out) {
+    int64_t n_tokens, int top_k, int pos_stride, int64_t dim, int64_t seg_units, T* __restrict__ out) {
   const int lane = threadIdx.x & 63;
   const int64_t nvec = dim / VW;
   const int64_t nseg = (nvec + seg_units - 1) / seg_units;
@@ -79,9 +80,10 @@ __global__ __launch_bounds__(kCombineThreads) void combine_kernel(
   const int64_t seg = gw - t * nseg;
   if (t >= n_tokens) return;
 
+  // (pos_stride > top_k: the slots past top_k are not combined.)
   // Lane k < top_k holds row k; rank rows by position (distinct values, an
   // invalid -1 sorts first and is skipped).
-  const int my_pos = lane < top_k ? token_pos[t * top_k + lane] : 0x7fffffff;
+  const int my_pos = lane < top_k ? token_pos[t * pos_stride + lane] : 0x7fffffff;
   int rank = 0;
   for (int k = 0; k < top_k; ++k) {
     const int o = __shfl(my_pos, k, 64);
@@ -152,32 +154,32 @@ __global__ __launch_bounds__(kCombineThreads) void combine_kernel(
 
 template <typename T, int VW, int KMAX, int U, bool NT>
 void launch_combine_cfg(const void* y, const int32_t* token_pos, const void* row_w, const void* shared, int n_shared,
-                        float inv_shared, int64_t n_tokens, int top_k, int64_t dim, int64_t seg_units, int64_t grid,
+                        float inv_shared, int64_t n_tokens, int top_k, int pos_stride, int64_t dim, int64_t seg_units, int64_t grid,
                         void* out, hipStream_t s) {
   hipLaunchKernelGGL((combine_kernel<T, VW, KMAX, U, NT>), dim3((unsigned)grid), dim3(kCombineThreads), 0, s,
                      static_cast<const T*>(y), token_pos, static_cast<const T*>(row_w), static_cast<const T*>(shared),
                      n_shared, inv_shared,
-                     n_tokens, top_k, dim, seg_units, static_cast<T*>(out));
+                     n_tokens, top_k, pos_stride, dim, seg_units, static_cast<T*>(out));
 }
 
 template <typename T, int VW>
 void dispatch_k(const void* y, const int32_t* token_pos, const void* row_w, const void* shared, int n_shared,
-                float inv_shared, int64_t n_tokens, int top_k, int64_t dim, int64_t seg_units, int64_t grid, void* out,
+                float inv_shared, int64_t n_tokens, int top_k, int pos_stride, int64_t dim, int64_t seg_units, int64_t grid, void* out,
                 hipStream_t s) {
   if (top_k <= 2)
-    launch_combine_cfg<T, VW, 2, 8, true>(y, token_pos, row_w, shared, n_shared, inv_shared, n_tokens, top_k, dim,
+    launch_combine_cfg<T, VW, 2, 8, true>(y, token_pos, row_w, shared, n_shared, inv_shared, n_tokens, top_k, pos_stride, dim,
                                           seg_units, grid, out, s);
   else if (top_k <= 8)
-    launch_combine_cfg<T, VW, 8, 2, false>(y, token_pos, row_w, shared, n_shared, inv_shared, n_tokens, top_k, dim,
+    launch_combine_cfg<T, VW, 8, 2, false>(y, token_pos, row_w, shared, n_shared, inv_shared, n_tokens, top_k, pos_stride, dim,
                                            seg_units, grid, out, s);
   else
     launch_combine_cfg<T, VW, ASTRAI_MOE_MAX_TOPK, 1, false>(y, token_pos, row_w, shared, n_shared, inv_shared,
-                                                            n_tokens, top_k, dim, seg_units, grid, out, s);
+                                                            n_tokens, top_k, pos_stride, dim, seg_units, grid, out, s);
 }
 
 template <typename T>
-int launch_combine(const void* y, const int32_t* token_pos, const void* row_w, const void* shared,
-                   int n_shared, int64_t n_tokens, int top_k, int64_t dim,
+int launch_combine_typed(const void* y, const int32_t* token_pos, const void* row_w, const void* shared,
+                   int n_shared, int64_t n_tokens, int top_k, int pos_stride, int64_t dim,
                    void* out, hipStream_t s) {
   const float inv_shared = n_shared > 0 ? 1.0f / (float)n_shared : 0.0f;
   constexpr int kVW = 16 / sizeof(T);
@@ -194,15 +196,24 @@ int launch_combine(const void* y, const int32_t* token_pos, const void* row_w, c
   const int64_t grid = ceil_div(waves, kWavesPerBlock);
   if (grid >= (1ll << 31)) return fail(ASTRAI_MOE_EINVAL, "combine: too many tokens");
   if (vec)
-    dispatch_k<T, kVW>(y, token_pos, row_w, shared, n_shared, inv_shared, n_tokens, top_k, dim, seg_units, grid, out,
+    dispatch_k<T, kVW>(y, token_pos, row_w, shared, n_shared, inv_shared, n_tokens, top_k, pos_stride, dim, seg_units, grid, out,
                        s);
   else
-    dispatch_k<T, 1>(y, token_pos, row_w, shared, n_shared, inv_shared, n_tokens, top_k, dim, seg_units, grid, out,
+    dispatch_k<T, 1>(y, token_pos, row_w, shared, n_shared, inv_shared, n_tokens, top_k, pos_stride, dim, seg_units, grid, out,
                      s);
   return check_launch("combine_kernel");
 }
 
 }  // namespace
+
+int launch_combine(const void* y, const int32_t* token_pos, const void* row_w, const void* shared, int n_shared,
+                   int dtype, int64_t n_tokens, int top_k, int pos_stride, int64_t dim, void* out, hipStream_t s) {
+  if (dtype == ASTRAI_MOE_BF16)
+    return launch_combine_typed<bf16_t>(y, token_pos, row_w, shared, n_shared, n_tokens, top_k, pos_stride, dim, out,
+                                        s);
+  return launch_combine_typed<float>(y, token_pos, row_w, shared, n_shared, n_tokens, top_k, pos_stride, dim, out, s);
+}
+
 }  // namespace astrai_moe
 
 using namespace astrai_moe;
@@ -221,10 +232,8 @@ extern "C" int astrai_moe_combine(const void* y, const int32_t* token_pos, const
   ASTRAI_REQUIRE(y && token_pos && out, "combine: null buffer");
   ASTRAI_REQUIRE(n_shared >= 0 && (n_shared == 0 || shared),
                  "combine: n_shared must be >= 0 with a buffer when > 0");
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  if (dtype == ASTRAI_MOE_BF16)
-    return launch_combine<bf16_t>(y, token_pos, row_w, shared, n_shared, n_tokens, top_k, dim, out, s);
-  if (dtype == ASTRAI_MOE_F32)
-    return launch_combine<float>(y, token_pos, row_w, shared, n_shared, n_tokens, top_k, dim, out, s);
-  return fail(ASTRAI_MOE_EINVAL, "combine: unsupported dtype %d", dtype);
+  if (dtype != ASTRAI_MOE_BF16 && dtype != ASTRAI_MOE_F32)
+    return fail(ASTRAI_MOE_EINVAL, "combine: unsupported dtype %d", dtype);
+  return launch_combine(y, token_pos, row_w, shared, n_shared, dtype, n_tokens, top_k, top_k, dim, out,
+                        static_cast<hipStream_t>(stream));
 }

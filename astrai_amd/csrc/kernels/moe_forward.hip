@@ -1,0 +1,154 @@
+// The layer's forward behind the router as one call (mlp.py:71-77, :84-100):
+// routing, permutation, the grouped GEMMs and the combine, with the shared
+// experts as experts n_experts .. n_experts + n_shared - 1 of the same
+// permutation and GEMMs. Every token's last n_shared slots are theirs, with
+// weight 1, so their rows of y lie behind the routed ones as [n_shared,
+// n_tokens, dim], which is what the combine takes as the shared outputs.
+//
+// One host call and one workspace in place of nine to twelve wrapped calls and
+// about twenty allocations, and two launches fewer for each shared expert plus
+// one for their tile list: at one token of D 512, F 1024, 8 experts, top-2 and
+// a shared expert the host, not the GPU, set the time (125 us a layer, of
+// which the kernels take 63).
+#include "moe_common.h"
+#include "moe_gemm.h"
+
+namespace astrai_moe {
+namespace {
+
+struct Sizes {
+  int64_t n_tokens;
+  int n_experts, top_k, n_shared;
+  int64_t dim, dim_ffn;
+  int dtype;
+  bool packed;
+};
+
+// Byte offsets of the workspace's parts, 256-byte aligned.
+struct Plan {
+  int experts, slots, block_m;
+  int64_t rows, tiles_len;
+  bool gather;
+  int64_t topk_idx, topk_w, chunk_hist, chunk_base, offsets, sorted_token, sorted_w, token_pos, tiles, x_perm, h, y,
+      gemm_ws, gemm_ws_bytes, bytes;
+};
+
+int check_sizes(const Sizes& z) {
+  ASTRAI_REQUIRE(z.dtype == ASTRAI_MOE_BF16 || z.dtype == ASTRAI_MOE_F32, "forward: unsupported dtype %d", z.dtype);
+  ASTRAI_REQUIRE(z.n_shared >= 0 && z.n_shared <= ASTRAI_MOE_MAX_TOPK, "forward: bad n_shared %d", z.n_shared);
+  ASTRAI_REQUIRE(z.n_experts >= 1 && z.n_experts + z.n_shared <= ASTRAI_MOE_MAX_EXPERTS,
+                 "forward: n_experts + n_shared must be in [1, %d] (got %d + %d)", ASTRAI_MOE_MAX_EXPERTS, z.n_experts,
+                 z.n_shared);
+  ASTRAI_REQUIRE(z.top_k >= 1 && z.top_k <= z.n_experts && z.top_k + z.n_shared <= ASTRAI_MOE_MAX_TOPK,
+                 "forward: top_k must be in [1, n_experts] and top_k + n_shared at most %d (got %d + %d)",
+                 ASTRAI_MOE_MAX_TOPK, z.top_k, z.n_shared);
+  ASTRAI_REQUIRE(z.dim >= 1 && z.dim_ffn >= 1, "forward: dims must be >= 1");
+  ASTRAI_REQUIRE(z.n_tokens >= 0 && z.n_tokens * (int64_t)(z.top_k + z.n_shared) < (1ll << 31),
+                 "forward: n_tokens * (top_k + n_shared) must be in [0, 2^31)");
+  return ASTRAI_MOE_OK;
+}
+
+Plan make_plan(const Sizes& z) {
+  Plan p{};
+  const int64_t size = z.dtype == ASTRAI_MOE_BF16 ? 2 : 4, T = z.n_tokens;
+  p.experts = z.n_experts + z.n_shared;
+  p.slots = z.top_k + z.n_shared;
+  p.rows = T * p.slots;
+  p.block_m = astrai_moe_select_block_m(T, z.n_experts, z.top_k, z.dim, z.dim_ffn, z.dtype);
+  p.tiles_len = astrai_moe_tile_list_len(T, p.experts, p.slots, p.block_m);
+  // the bf16 gate/up GEMM reads the token rows itself where its kernels do
+  // (32-bit row offsets: x under 4 GiB)
+  p.gather = z.dtype == ASTRAI_MOE_BF16 && !z.packed && mfma_shape_supported(z.dim, z.dim_ffn) && z.dim % 64 == 0 &&
+             z.dim_ffn % 64 == 0 && T * z.dim * 2 < (1ll << 32);
+  int64_t at = 0;
+  auto part = [&](int64_t bytes) {
+    const int64_t here = at;
+    at += (bytes + 255) / 256 * 256;
+    return here;
+  };
+  p.topk_idx = part(p.rows * 4);
+  p.topk_w = part(p.rows * size);
+  p.chunk_hist = part(n_chunks(T) * p.experts * 4);
+  p.chunk_base = part(n_chunks(T) * p.experts * 4);
+  p.offsets = part((p.experts + 1) * 4);
+  p.sorted_token = part(p.rows * 4);
+  p.sorted_w = part(p.rows * size);
+  p.token_pos = part(p.rows * 4);
+  p.tiles = part(p.tiles_len * 4);
+  p.x_perm = p.gather ? 0 : part(p.rows * z.dim * size);
+  p.h = part(p.rows * z.dim_ffn * size);
+  p.y = part(p.rows * z.dim * size);
+  // the 256-row GEMMs' scheduling block, and partial sums where the down
+  // GEMM's tiles are long enough to be split
+  if (p.block_m == kMfmaBigBM) p.gemm_ws_bytes = gemm_workspace_bytes(z.dim_ffn >= 64 * 64);
+  p.gemm_ws = part(p.gemm_ws_bytes);
+  p.bytes = at;
+  return p;
+}
+
+}  // namespace
+}  // namespace astrai_moe
+
+using namespace astrai_moe;
+
+extern "C" int64_t astrai_moe_forward_workspace_bytes(int64_t n_tokens, int n_experts, int top_k, int n_shared,
+                                                      int64_t dim, int64_t dim_ffn, int dtype, int packed) {
+  clear_error();
+  const Sizes z{n_tokens, n_experts, top_k, n_shared, dim, dim_ffn, dtype, packed != 0};
+  if (int rc = check_sizes(z)) return rc;
+  return make_plan(z).bytes;
+}
+
+extern "C" int astrai_moe_forward(const void* x, const void* logits, const void* const* w_gate,
+                                  const void* const* w_up, const void* const* w_down, const void* const* packed_gate_up,
+                                  const void* const* packed_down, int dtype, int64_t n_tokens, int n_experts,
+                                  int top_k, int n_shared, int64_t dim, int64_t dim_ffn, void* workspace,
+                                  int64_t workspace_bytes, void* out, void* stream) {
+  clear_error();
+  const Sizes z{n_tokens, n_experts, top_k, n_shared, dim, dim_ffn, dtype, packed_gate_up != nullptr};
+  int rc = check_sizes(z);
+  if (rc) return rc;
+  if (n_tokens == 0) return ASTRAI_MOE_OK;
+  ASTRAI_REQUIRE(x && logits && w_gate && w_up && w_down && workspace && out, "forward: null buffer");
+  ASTRAI_REQUIRE((packed_gate_up == nullptr) == (packed_down == nullptr), "forward: one packed table without the other");
+  ASTRAI_REQUIRE(reinterpret_cast<uintptr_t>(workspace) % 256 == 0, "forward: workspace must be 256-byte aligned");
+  const Plan p = make_plan(z);
+  ASTRAI_REQUIRE(workspace_bytes >= p.bytes, "forward: workspace holds %lld bytes, needs %lld",
+                 (long long)workspace_bytes, (long long)p.bytes);
+  ASTRAI_REQUIRE(!p.gather || reinterpret_cast<uintptr_t>(x) % 16 == 0,
+                 "forward: unsupported alignment (x must start on a 16-byte boundary)");
+  char* const base = static_cast<char*>(workspace);
+  auto i32 = [&](int64_t off) { return reinterpret_cast<int32_t*>(base + off); };
+  int32_t *topk_idx = i32(p.topk_idx), *hist = i32(p.chunk_hist), *sorted_token = i32(p.sorted_token),
+          *token_pos = i32(p.token_pos), *tiles = i32(p.tiles);
+  void *topk_w = base + p.topk_w, *sorted_w = base + p.sorted_w, *h = base + p.h, *y = base + p.y;
+  void* const x_perm = p.gather ? nullptr : base + p.x_perm;
+  void* const gws = p.gemm_ws_bytes > 0 ? base + p.gemm_ws : nullptr;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+
+  if ((rc = launch_route(logits, dtype, n_tokens, n_experts, top_k, n_shared, topk_idx, topk_w, hist, s))) return rc;
+  if ((rc = astrai_moe_permute(topk_idx, topk_w, hist, x, dtype, n_tokens, p.experts, p.slots, dim, p.block_m,
+                               i32(p.offsets), sorted_token, sorted_w, token_pos, x_perm, tiles, p.tiles_len,
+                               i32(p.chunk_base), stream)))
+    return rc;
+  if (p.gather)
+    rc = astrai_moe_gemm_gate_up_gather(x, sorted_token, n_tokens, tiles, p.tiles_len, w_gate, w_up, dtype, p.rows,
+                                        p.experts, dim, dim_ffn, p.block_m, h, gws, p.gemm_ws_bytes, stream);
+  else if (z.packed)
+    rc = astrai_moe_gemm_gate_up_packed(x_perm, tiles, p.tiles_len, packed_gate_up, dtype, p.rows, p.experts, dim,
+                                        dim_ffn, p.block_m, h, gws, p.gemm_ws_bytes, stream);
+  else
+    rc = astrai_moe_gemm_gate_up(x_perm, tiles, p.tiles_len, w_gate, w_up, dtype, p.rows, p.experts, dim, dim_ffn,
+                                 p.block_m, h, gws, p.gemm_ws_bytes, stream);
+  if (rc) return rc;
+  if (z.packed)
+    rc = astrai_moe_gemm_down_packed(h, tiles, p.tiles_len, packed_down, sorted_w, dtype, p.rows, p.experts, dim_ffn,
+                                     dim, p.block_m, y, gws, p.gemm_ws_bytes, stream);
+  else
+    rc = astrai_moe_gemm_down(h, tiles, p.tiles_len, w_down, sorted_w, dtype, p.rows, p.experts, dim_ffn, dim,
+                              p.block_m, y, gws, p.gemm_ws_bytes, stream);
+  if (rc) return rc;
+  const int64_t size = dtype == ASTRAI_MOE_BF16 ? 2 : 4;
+  const void* shared = n_shared > 0 ? static_cast<const char*>(y) + n_tokens * top_k * dim * size : nullptr;
+  return launch_combine(y, token_pos, nullptr, shared, n_shared, dtype, n_tokens, top_k, p.slots, dim, out, s);
+}

@@ -1,5 +1,5 @@
-// Internal interface between the grouped-GEMM entry points (moe_gemm.hip) and
-// the CDNA4 matrix-core kernels (moe_gemm_mfma.hip).
+// Internal interface between the entry points (moe_gemm.hip, moe_forward.hip)
+// and the kernels of the other files.
 #pragma once
 
 #include "moe_common.h"
@@ -157,6 +157,20 @@ int launch_mfma_f32_dgrad_in(const void* d, const int32_t* tiles,
 int launch_mfma_f32_wgrad(const void* a, const void* b, const int32_t* offsets,
                           int n_experts, int64_t m, int64_t n, void* dw,
                           hipStream_t s);
+
+// Routing with n_shared always-chosen experts behind the n_experts routed ones
+// (moe_route.hip): topk_idx, topk_w [n_tokens, top_k + n_shared], chunk_hist
+// [n_chunks, n_experts + n_shared].
+int launch_route(const void* logits, int dtype, int64_t n_tokens,
+                 int n_experts, int top_k, int n_shared, int32_t* topk_idx,
+                 void* topk_w, int32_t* chunk_hist, hipStream_t s);
+
+// astrai_moe_combine with token_pos rows pos_stride >= top_k wide, of which
+// the first top_k are combined (moe_combine.hip).
+int launch_combine(const void* y, const int32_t* token_pos, const void* row_w,
+                   const void* shared, int n_shared, int dtype,
+                   int64_t n_tokens, int top_k, int pos_stride, int64_t dim,
+                   void* out, hipStream_t s);
 
 // Backward (moe_gemm_bwd.hip), bf16, 256-row tile lists:
 // dy = dout[sorted_token] * sorted_w and dw_rows = sum(dout[tok] * y) per row;

@@ -25,7 +25,13 @@
 // Each block handles one chunk of ASTRAI_MOE_CHUNK_TOKENS tokens and also
 // writes that chunk's per-expert routed-token histogram, which the permute
 // step scans into per-expert offsets.
+//
+// n_shared > 0 (the layer's forward): every token also goes to the n_shared
+// shared experts, numbered from n_experts on, with weight 1. They take
+// n_shared more slots per token and as many columns of the histogram, and so
+// become experts of the permutation and the grouped GEMMs like any other.
 #include "moe_common.h"
+#include "moe_gemm.h"
 
 namespace astrai_moe {
 namespace {
@@ -57,7 +63,7 @@ struct KeyOf<float> {  // fp32 bits above a 32-bit inverted column
 
 template <typename T, int WS, int ITER>
 __global__ __launch_bounds__(kRouteThreads) void route_kernel(
-    const T* __restrict__ logits, int64_t n_tokens, int n_experts, int top_k,
+    const T* __restrict__ logits, int64_t n_tokens, int n_experts, int top_k, int n_shared,
     int32_t* __restrict__ topk_idx, T* __restrict__ topk_w,
     int32_t* __restrict__ chunk_hist) {
   __shared__ int hist[ASTRAI_MOE_MAX_EXPERTS];
@@ -70,6 +76,12 @@ __global__ __launch_bounds__(kRouteThreads) void route_kernel(
   const int group = threadIdx.x / WS;
   const int64_t t_begin = chunk * ASTRAI_MOE_CHUNK_TOKENS;
   const int64_t t_end = min(t_begin + (int64_t)ASTRAI_MOE_CHUNK_TOKENS, n_tokens);
+  const int slots = top_k + n_shared;
+  for (int i = threadIdx.x; i < (int)(t_end - t_begin) * n_shared; i += kRouteThreads) {
+    const int64_t at = (t_begin + i / n_shared) * slots + top_k + i % n_shared;
+    topk_idx[at] = n_experts + i % n_shared;
+    topk_w[at] = Elem<T>::from_f32(1.0f);
+  }
   // bw = last_pow2(K): lanes that torch's row reduction uses for K values.
   int bw = 1;
   while (bw * 2 <= top_k) bw *= 2;
@@ -149,36 +161,37 @@ __global__ __launch_bounds__(kRouteThreads) void route_kernel(
     const float denom = Elem<T>::round(__shfl(part, 0, WS));
     if (lane < top_k) {
       const float w = v / denom;
-      topk_idx[t * top_k + lane] = my_i;
-      topk_w[t * top_k + lane] = Elem<T>::from_f32(w);
+      topk_idx[t * slots + lane] = my_i;
+      topk_w[t * slots + lane] = Elem<T>::from_f32(w);
       atomicAdd(&hist[my_i], 1);
     }
   }
   __syncthreads();
-  for (int e = threadIdx.x; e < n_experts; e += kRouteThreads)
-    chunk_hist[chunk * n_experts + e] = hist[e];
+  const int columns = n_experts + n_shared;
+  for (int e = threadIdx.x; e < columns; e += kRouteThreads)
+    chunk_hist[chunk * columns + e] = e < n_experts ? hist[e] : (int)(t_end - t_begin);
 }
 
 template <typename T, int WS, int ITER>
-void launch_route(const void* logits, int64_t n_tokens, int n_experts,
-                  int top_k, int32_t* topk_idx, void* topk_w,
+void launch_route_cfg(const void* logits, int64_t n_tokens, int n_experts,
+                  int top_k, int n_shared, int32_t* topk_idx, void* topk_w,
                   int32_t* chunk_hist, hipStream_t stream) {
   const int64_t grid = n_chunks(n_tokens);
   hipLaunchKernelGGL((route_kernel<T, WS, ITER>), dim3((unsigned)grid),
                      dim3(kRouteThreads), 0, stream,
-                     static_cast<const T*>(logits), n_tokens, n_experts, top_k,
+                     static_cast<const T*>(logits), n_tokens, n_experts, top_k, n_shared,
                      topk_idx, static_cast<T*>(topk_w), chunk_hist);
 }
 
 template <typename T>
 int dispatch_route(const void* logits, int64_t n_tokens, int n_experts,
-                   int top_k, int32_t* topk_idx, void* topk_w,
+                   int top_k, int n_shared, int32_t* topk_idx, void* topk_w,
                    int32_t* chunk_hist, hipStream_t s) {
   int p2 = 1;
   while (p2 < n_experts) p2 *= 2;
 #define ROUTE_CASE(WS, IT)                                                   \
-  launch_route<T, WS, IT>(logits, n_tokens, n_experts, top_k, topk_idx,     \
-                          topk_w, chunk_hist, s);                           \
+  launch_route_cfg<T, WS, IT>(logits, n_tokens, n_experts, top_k, n_shared, \
+                              topk_idx, topk_w, chunk_hist, s);             \
   break;
   switch (p2) {
     case 1: ROUTE_CASE(1, 1)
@@ -200,6 +213,14 @@ int dispatch_route(const void* logits, int64_t n_tokens, int n_experts,
 }
 
 }  // namespace
+
+int launch_route(const void* logits, int dtype, int64_t n_tokens, int n_experts, int top_k, int n_shared,
+                 int32_t* topk_idx, void* topk_w, int32_t* chunk_hist, hipStream_t s) {
+  if (dtype == ASTRAI_MOE_BF16)
+    return dispatch_route<bf16_t>(logits, n_tokens, n_experts, top_k, n_shared, topk_idx, topk_w, chunk_hist, s);
+  return dispatch_route<float>(logits, n_tokens, n_experts, top_k, n_shared, topk_idx, topk_w, chunk_hist, s);
+}
+
 }  // namespace astrai_moe
 
 using namespace astrai_moe;
@@ -220,12 +241,8 @@ extern "C" int astrai_moe_route(const void* logits, int dtype, int64_t n_tokens,
   if (n_tokens == 0) return ASTRAI_MOE_OK;
   ASTRAI_REQUIRE(logits && topk_idx && topk_w && chunk_hist,
                  "route: null buffer");
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  if (dtype == ASTRAI_MOE_BF16)
-    return dispatch_route<bf16_t>(logits, n_tokens, n_experts, top_k, topk_idx,
-                                  topk_w, chunk_hist, s);
-  if (dtype == ASTRAI_MOE_F32)
-    return dispatch_route<float>(logits, n_tokens, n_experts, top_k, topk_idx,
-                                 topk_w, chunk_hist, s);
-  return fail(ASTRAI_MOE_EINVAL, "route: unsupported dtype %d", dtype);
+  if (dtype != ASTRAI_MOE_BF16 && dtype != ASTRAI_MOE_F32)
+    return fail(ASTRAI_MOE_EINVAL, "route: unsupported dtype %d", dtype);
+  return launch_route(logits, dtype, n_tokens, n_experts, top_k, 0, topk_idx, topk_w, chunk_hist,
+                      static_cast<hipStream_t>(stream));
 }

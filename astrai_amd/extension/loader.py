@@ -30,7 +30,7 @@ import torch  # noqa: F401  (loads torch's HIP runtime before the library)
 
 KERNEL_NAMES = ["moe_route", "moe_permute", "moe_gemm_gate_up", "moe_gemm_down", "moe_combine"]
 
-ABI_VERSION = 10
+ABI_VERSION = 11
 LIB_PATH = Path(os.environ.get("ASTRAI_MOE_LIB", Path(__file__).resolve().parent / "libastrai_moe.so"))
 
 _c_i32p = ctypes.POINTER(ctypes.c_int32)
@@ -68,6 +68,9 @@ _SIGNATURES: dict[str, tuple] = {
                                               _vp]),
     "astrai_moe_gemm_down_packed": (_int, [_vp, _vp, _i64, _vp, _vp, _int, _i64, _int, _i64, _i64, _int, _vp, _vp,
                                            _i64, _vp]),
+    "astrai_moe_forward_workspace_bytes": (_i64, [_i64, _int, _int, _int, _i64, _i64, _int, _int]),
+    "astrai_moe_forward": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _int, _i64, _int, _int, _int, _i64, _i64, _vp,
+                                  _i64, _vp, _vp]),
     "astrai_moe_gemm_gate_up_train": (_int, [_vp, _vp, _i64, _vp, _vp, _int, _i64, _int, _i64, _i64, _int, _vp, _vp,
                                              _vp, _i64, _vp]),
     "astrai_moe_gemm_down_train": (_int, [_vp, _vp, _i64, _vp, _vp, _int, _i64, _int, _i64, _i64, _int, _vp, _vp,

@@ -177,6 +177,14 @@ def expert_weight_table(weights: Sequence[torch.Tensor], shape: tuple[int, int])
     return table
 
 
+def weight_table_slice(table: torch.Tensor, first: int, count: int) -> torch.Tensor:
+    """Entries ``first`` to ``first + count - 1`` of a table from
+    ``expert_weight_table`` as a table of their own (the same memory)."""
+    part = table[first:first + count]
+    part._astrai_weights = table._astrai_weights[first:first + count]
+    return part
+
+
 def moe_route(logits: torch.Tensor, top_k: int) -> RouteResult:
     """Softmax, top-k and renormalisation of router logits (mlp.py:84-87)."""
     fn = _kernel("moe_route")
@@ -505,6 +513,44 @@ def moe_routed_forward(x: torch.Tensor, logits: torch.Tensor, w_gate: torch.Tens
         h = moe_gemm_gate_up(perm.x_perm, perm.tiles, w_gate, w_up, n_experts, dim_ffn, block_m, packed=packed)
     y = moe_gemm_down(h, perm.tiles, w_down, perm.sorted_w, n_experts, dim, block_m, packed=packed)
     return moe_combine(y, perm.token_pos, shared)
+
+
+def layer_forward_supported(n_experts: int, n_shared: int, top_k: int) -> bool:
+    """Whether ``moe_layer_forward`` takes these counts (its shared experts
+    are more slots per token and more experts of the permutation)."""
+    return n_experts + n_shared <= MAX_EXPERTS and top_k + n_shared <= MAX_TOPK
+
+
+def moe_layer_forward(x: torch.Tensor, logits: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor,
+                      w_down: torch.Tensor, n_shared: int, dim_ffn: int, top_k: int,
+                      packed: tuple[torch.Tensor, torch.Tensor] | None = None) -> torch.Tensor:
+    """The layer's output for ``x [T, D]`` and its router logits (mlp.py:71-100)
+    in one call of the library. The pointer tables hold the routed experts and
+    then the ``n_shared`` shared ones; ``packed``: tables (gate/up, down) of
+    their packed copies, read in place of the weights."""
+    _require_gpu(x, "x", 2)
+    _require_gpu(logits, "logits", 2)
+    code = _dtype_code(x, "x")
+    n_tokens, dim = x.shape
+    n_experts = logits.shape[1]
+    if logits.shape[0] != n_tokens or logits.dtype != x.dtype or logits.device != x.device:
+        raise ValueError(f"logits must be [{n_tokens}, n_experts] {x.dtype} on {x.device}")
+    if not 1 <= top_k <= n_experts:
+        raise ValueError(f"top_k must be in [1, n_experts = {n_experts}], got {top_k}")
+    tables = (w_gate, w_up, w_down, *(packed or ()))
+    for name, t in zip(("w_gate", "w_up", "w_down", "packed gate/up", "packed down"), tables):
+        _require_table(t, name, n_experts + n_shared, x)
+    lib = loader.library()
+    out = torch.empty_like(x)
+    nbytes = lib.astrai_moe_forward_workspace_bytes(n_tokens, n_experts, top_k, n_shared, dim, dim_ffn, code,
+                                                    packed is not None)
+    _check(0 if nbytes >= 0 else int(nbytes), "moe_layer_forward")
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+    pg, pd = (packed[0].data_ptr(), packed[1].data_ptr()) if packed is not None else (None, None)
+    _check(lib.astrai_moe_forward(x.data_ptr(), logits.data_ptr(), w_gate.data_ptr(), w_up.data_ptr(),
+                                  w_down.data_ptr(), pg, pd, code, n_tokens, n_experts, top_k, n_shared, dim, dim_ffn,
+                                  ws.data_ptr(), nbytes, out.data_ptr(), _stream(x)), "moe_layer_forward")
+    return out
 
 
 # -- training: forward that keeps g, u, y and the backward kernels ------------

@@ -117,14 +117,16 @@ _requires_grad = attrgetter("requires_grad")
 class _ExpertState:
     """A DeepSeekMoE's validated expert weights (routed and shared, each as
     gate, up, down lists), their dtype and device, and the device pointer
-    tables built from them; ``sig`` identifies the modules, parameter objects
-    and storages they were read from."""
+    tables built from them: ``tables`` (routed; each shared expert's), and
+    ``joint``, the tables of all experts, routed then shared, which the former
+    are slices of (None where their shapes differ). ``sig`` identifies the
+    modules, parameter objects and storages they were read from."""
 
-    __slots__ = ("sig", "ptrs", "routed", "shared", "flat", "dtype", "device", "tables")
+    __slots__ = ("sig", "ptrs", "routed", "shared", "flat", "dtype", "device", "tables", "joint")
 
-    def __init__(self, sig, ptrs, routed, shared, flat, dtype, device, tables):
+    def __init__(self, sig, ptrs, routed, shared, flat, dtype, device, tables, joint):
         self.sig, self.ptrs, self.routed, self.shared, self.flat = sig, ptrs, routed, shared, flat
-        self.dtype, self.device, self.tables = dtype, device, tables
+        self.dtype, self.device, self.tables, self.joint = dtype, device, tables, joint
 
 
 @FFNFactory.register("moe")
@@ -158,11 +160,10 @@ class DeepSeekMoE(nn.Module):
         # The experts' validated weights and their device pointer tables
         # (_current; not part of the state_dict).
         self._state: _ExpertState | None = None
-        # Opt-in, inference only: keep a packed copy of the routed experts'
-        # weights in the order the GEMMs stage it (ops.moe_pack_*), rebuilt
-        # when a weight moves or changes (its version counter), for bf16 shapes
-        # the packed GEMMs take. Same results; doubles the routed weights'
-        # memory for about 1 % less GEMM time (3 % on the down GEMM of
+        # Opt-in, inference only: keep a packed copy of the experts' weights
+        # in the order the GEMMs stage it (ops.moe_pack_*), rebuilt when a
+        # weight moves or changes (its version counter), for bf16 shapes the
+        # packed GEMMs take. Same results; doubles the weights' memory for about 1 % less GEMM time (3 % on the down GEMM of
         # decode-sized loads), so it is off by default.
         self.pack_weights = False
         self._packed: tuple | None = None
@@ -214,21 +215,24 @@ class DeepSeekMoE(nn.Module):
                 raise RuntimeError(f"DeepSeekMoE: parameters must be on {device} in {dtype}, found {w.device}/{w.dtype}")
         ptrs = tuple(w.data_ptr() for w in flat_w)
         if st is not None and st.ptrs == ptrs:
-            tables = st.tables
+            tables, joint = st.tables, st.joint
         else:
             shape_in = tuple(routed[0][0].shape)
             shape_out = tuple(routed[2][0].shape)
-            t_routed = (
-                ops.expert_weight_table(routed[0], shape_in),
-                ops.expert_weight_table(routed[1], shape_in),
-                ops.expert_weight_table(routed[2], shape_out),
-            )
-            t_shared = tuple(
-                tuple(ops.expert_weight_table([w], tuple(w.shape)) for w in (shared[0][i], shared[1][i], shared[2][i]))
-                for i in range(len(shared[0]))
-            )
+            shapes = (shape_in, shape_in, shape_out)
+            n_routed, n_shared = len(routed[0]), len(shared[0])
+            joint = None
+            if all(w.shape == shape for ws, shape in zip(shared, shapes) for w in ws):
+                joint = tuple(ops.expert_weight_table(r + s, shape) for r, s, shape in zip(routed, shared, shapes))
+                t_routed = tuple(ops.weight_table_slice(t, 0, n_routed) for t in joint)
+                t_shared = tuple(tuple(ops.weight_table_slice(t, n_routed + i, 1) for t in joint)
+                                 for i in range(n_shared))
+            else:
+                t_routed = tuple(ops.expert_weight_table(r, shape) for r, shape in zip(routed, shapes))
+                t_shared = tuple(tuple(ops.expert_weight_table([ws[i]], tuple(ws[i].shape)) for ws in shared)
+                                 for i in range(n_shared))
             tables = (t_routed, t_shared)
-        self._state = _ExpertState(sig, ptrs, routed, shared, flat_w, dtype, device, tables)
+        self._state = _ExpertState(sig, ptrs, routed, shared, flat_w, dtype, device, tables, joint)
         return self._state
 
     def _weight_tables(self) -> tuple[Tensor, ...]:
@@ -240,12 +244,13 @@ class DeepSeekMoE(nn.Module):
     def _packed_tables(self, dtype: torch.dtype, st: _ExpertState) -> tuple[Tensor, Tensor] | None:
         """Pointer tables of the packed gate/up and down copies, or None when
         this forward reads the live weights. The copies are rebuilt whenever a
-        routed weight's storage or version counter changes; the cache holds a
-        view of each source weight so that its storage (and address) cannot be
+        weight's storage or version counter changes (the shared experts' are
+        packed with the routed ones where both run in one forward call); the
+        cache holds a view of each source weight so that its storage (and address) cannot be
         reused by another tensor while the copy made from it is in use."""
         if not self.uses_packed_weights(dtype):
             return None
-        g, u, d = st.routed
+        g, u, d = map(list.__add__, st.routed, st.shared) if self._joint(st) else st.routed
         srcs = [w for ws in (g, u, d) for w in ws]
         if any(w.is_inference() for w in srcs):  # no version counter to follow
             return None
@@ -265,6 +270,12 @@ class DeepSeekMoE(nn.Module):
         dim_ffn = self.routed_experts[0].up.weight.shape[0]
         return self.pack_weights and ops.packed_supported(self.dim, dim_ffn, dtype)
 
+    def _joint(self, st: _ExpertState) -> bool:
+        """Whether routed and shared experts run in one forward call
+        (``ops.moe_layer_forward``)."""
+        return st.joint is not None and ops.layer_forward_supported(len(st.routed[0]), len(st.shared[0]),
+                                                                    self.n_activated_experts)
+
     # -- forward ----------------------------------------------------------------
     def forward(self, x: Tensor) -> Tensor:
         bsz, seq_len, dim = x.shape
@@ -277,8 +288,12 @@ class DeepSeekMoE(nn.Module):
         if torch.is_grad_enabled() and (x_flat.requires_grad or router_w.requires_grad
                                         or any(map(_requires_grad, st.flat))):
             return self._forward_autograd(x_flat, st).view(bsz, seq_len, dim)
-        shared_out = self._shared_forward(x_flat, st)
-        out = self._routed_forward(x_flat, st, shared_out)
+        if x_flat.shape[0] and self._joint(st):
+            packed = self._packed_tables(x_flat.dtype, st) if self.pack_weights else None
+            out = ops.moe_layer_forward(x_flat, self.router(x_flat), *st.joint, len(st.shared[0]),
+                                        st.routed[1][0].shape[0], self.n_activated_experts, packed)
+        else:
+            out = self._routed_forward(x_flat, st, self._shared_forward(x_flat, st))
         return out.view(bsz, seq_len, dim)
 
     def _shared_forward(self, x: Tensor, st: _ExpertState) -> Tensor | None:

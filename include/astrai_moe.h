@@ -32,7 +32,7 @@
 extern "C" {
 #endif
 
-#define ASTRAI_MOE_ABI_VERSION 10
+#define ASTRAI_MOE_ABI_VERSION 11
 
 /* Element types. */
 #define ASTRAI_MOE_F32 0
@@ -343,6 +343,43 @@ int astrai_moe_gemm_down_packed(const void* h, const int32_t* tiles,
 int astrai_moe_combine(const void* y, const int32_t* token_pos, const void* row_w,
                        const void* shared, int n_shared, int dtype,
                        int64_t n_tokens, int top_k, int64_t dim, void* out,
+                       void* stream);
+
+/*
+ * The layer's forward behind the router in one call: mlp.py:84-100 with the
+ * shared experts of :74-77 and the sum of :71, from the router's logits to the
+ * layer's output. The same kernels as the entry points above, one after the
+ * other on `stream`; the shared experts are experts n_experts .. n_experts +
+ * n_shared - 1 of the same permutation and grouped GEMMs (each token routed to
+ * all of them with weight 1), so the same values as running them by themselves
+ * up to the order of a GEMM's fp32 sums.
+ *
+ *   x        [n_tokens, dim]        dtype
+ *   logits   [n_tokens, n_experts]  dtype
+ *   w_gate, w_up, w_down  device arrays of n_experts + n_shared pointers, the
+ *            routed experts' first ([dim_ffn, dim], [dim_ffn, dim], [dim, dim_ffn])
+ *   packed_gate_up, packed_down  tables of packed copies of the same experts
+ *            (astrai_moe_pack_*), read in place of the weights, or NULL
+ *   workspace  astrai_moe_forward_workspace_bytes(...) bytes for the same
+ *            sizes, 256-byte aligned, nothing to initialise; calls sharing one
+ *            must not overlap
+ *   out      [n_tokens, dim]        dtype
+ *
+ * top_k + n_shared <= ASTRAI_MOE_MAX_TOPK and n_experts + n_shared <=
+ * ASTRAI_MOE_MAX_EXPERTS.
+ */
+int64_t astrai_moe_forward_workspace_bytes(int64_t n_tokens, int n_experts,
+                                           int top_k, int n_shared,
+                                           int64_t dim, int64_t dim_ffn,
+                                           int dtype, int packed);
+int astrai_moe_forward(const void* x, const void* logits,
+                       const void* const* w_gate, const void* const* w_up,
+                       const void* const* w_down,
+                       const void* const* packed_gate_up,
+                       const void* const* packed_down, int dtype,
+                       int64_t n_tokens, int n_experts, int top_k,
+                       int n_shared, int64_t dim, int64_t dim_ffn,
+                       void* workspace, int64_t workspace_bytes, void* out,
                        void* stream);
 
 /*

@@ -1,0 +1,54 @@
+"""The layer's one-call forward (astrai_moe_forward): shared experts as experts
+of the same permutation and GEMMs, against the oracle at every tile height,
+with copied rows (fp32) and gathered ones, and where it does not apply (slots
+or shapes beyond it) the separate calls."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from astrai_amd.extension import loader, ops
+from test_gpu_backward import _random_layer
+from test_gpu_layer import check_layer
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n_exp,n_shared,top_k", [(4, 1, 2), (8, 3, 1), (1, 2, 1), (40, 1, 31), (40, 1, 32)])
+@pytest.mark.parametrize("n_tok", [1, 33, 160, 700])
+def test_shared_experts_in_one_call(gpu, n_tok, n_exp, n_shared, top_k, dtype):
+    layer = _random_layer(gpu, 192, 320, n_exp, n_shared, top_k, dtype, seed=n_tok + n_exp).requires_grad_(False)
+    x = torch.randn(1, n_tok, 192, device=gpu).to(dtype)
+    assert layer._joint(layer._current(dtype, x.device)) == (top_k + n_shared <= 32)
+    check_layer(layer, x, f"e{n_exp}_s{n_shared}_k{top_k}_t{n_tok}")
+
+
+@pytest.mark.gpu
+def test_shared_experts_of_another_width(gpu):
+    layer = _random_layer(gpu, 192, 320, 4, 1, 2, torch.bfloat16, seed=3)
+    layer.shared_experts[0] = _random_layer(gpu, 192, 256, 1, 0, 1, torch.bfloat16, seed=4).routed_experts[0]
+    layer.requires_grad_(False)
+    x = torch.randn(1, 70, 192, device=gpu).to(torch.bfloat16)
+    assert layer._current(x.dtype, x.device).joint is None
+    check_layer(layer, x, "narrow shared expert")
+
+
+def test_arguments_are_checked_on_the_host():
+    lib = loader.library()
+    size = lib.astrai_moe_forward_workspace_bytes
+    assert size(10, 8, 2, 1, 64, 128, 1, 0) > 0
+    for args, word in (((10, 8, 9, 0, 64, 128, 1, 0), "top_k"), ((10, 40, 32, 1, 64, 128, 1, 0), "top_k + n_shared"),
+                       ((10, 1024, 2, 1, 64, 128, 1, 0), "n_experts + n_shared"), ((10, 8, 2, 0, 64, 128, 7, 0), "dtype"),
+                       ((10, 8, 2, 0, 0, 128, 1, 0), "dims"), ((1 << 30, 8, 2, 0, 64, 128, 1, 0), "n_tokens")):
+        assert size(*args) == -1 and word in loader.last_error()
+
+    def call(workspace=256, nbytes=1 << 40, gate=16, tokens=10):
+        return lib.astrai_moe_forward(16, 16, gate, 16, 16, None, None, 1, tokens, 8, 2, 1, 64, 128, workspace, nbytes,
+                                      16, None)
+
+    assert call(tokens=0) == 0
+    assert call(gate=None) == -1 and "null" in loader.last_error()
+    assert call(workspace=16) == -1 and "256-byte aligned" in loader.last_error()
+    assert call(nbytes=100) == -1 and "needs" in loader.last_error()
+    assert not ops.layer_forward_supported(8, 1, 32) and ops.layer_forward_supported(8, 1, 31)
