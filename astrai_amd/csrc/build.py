@@ -61,7 +61,7 @@ register("moe_route")
 register("moe_permute")
 register("moe_gemm", sources=[str(KERNELS_DIR / "moe_gemm.hip"), str(KERNELS_DIR / "moe_gemm_mfma.hip"),
                               str(KERNELS_DIR / "moe_gemm_mfma_f32.hip"), str(KERNELS_DIR / "moe_gemm_mfma_f32_bwd.hip"),
-                              str(KERNELS_DIR / "moe_gemm_bwd.hip"),
+                              str(KERNELS_DIR / "moe_gemm_few.hip"), str(KERNELS_DIR / "moe_gemm_bwd.hip"),
                               str(KERNELS_DIR / "moe_gemm_mfma_ragged.hip"),
                               str(KERNELS_DIR / "moe_gemm_bwd_ragged.hip"),
                               str(KERNELS_DIR / "moe_gemm_generic_bwd.hip")])

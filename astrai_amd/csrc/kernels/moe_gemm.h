@@ -105,6 +105,20 @@ int launch_mfma_gate_up_gather(const void* x, const int32_t* sorted_token,
                                hipStream_t s,
                         const GemmWorkspace& ws = {});
 
+// Few rows (moe_gemm_few.hip), any tile height: whether the kernels there take
+// a GEMM of n_rows rows over n_experts experts with n output columns, and the GEMMs (row_src: the
+// gathered rows' tokens, or null; packed: the tables hold packed copies).
+bool few_rows(int64_t n_rows, int n_experts, int64_t n, bool gate_up);
+int launch_few_gate_up(const void* x, const int32_t* row_src,
+                       const int32_t* tiles, int64_t capacity,
+                       const void* const* w_gate, const void* const* w_up,
+                       int64_t dim, int64_t dim_ffn, bool packed, void* h,
+                       hipStream_t s);
+int launch_few_down(const void* h, const int32_t* tiles, int64_t capacity,
+                    const void* const* w_down, const void* sorted_w,
+                    int64_t dim_ffn, int64_t dim, bool packed, void* y,
+                    hipStream_t s);
+
 // Training forward (256-row tiles): as launch_mfma_gate_up / launch_mfma_down,
 // also storing the bf16 gate and up projections (gu: [rows, 2 dim_ffn],
 // blocks of 4 gate columns then the same 4 up columns) or the unweighted bf16

@@ -202,7 +202,10 @@ extern "C" int astrai_moe_gemm_gate_up(const void* x_perm, const int32_t* tiles,
   const int64_t capacity = (tiles_len - ASTRAI_MOE_TILE_HEADER) / ASTRAI_MOE_TILE_STRIDE;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (dtype == ASTRAI_MOE_BF16) {
-    if (mfma_gate_up_supported(dim, dim_ffn, block_m, x_perm, h))
+    const bool mfma = mfma_gate_up_supported(dim, dim_ffn, block_m, x_perm, h);
+    if (mfma && few_rows(n_rows, n_experts, dim_ffn, true))
+      return launch_few_gate_up(x_perm, nullptr, tiles, capacity, w_gate, w_up, dim, dim_ffn, false, h, s);
+    if (mfma)
       return launch_mfma_gate_up(x_perm, tiles, capacity, w_gate, w_up, dim,
                                  dim_ffn, block_m, false, h, s,
                                  GemmWorkspace{workspace, workspace_bytes});
@@ -236,6 +239,9 @@ extern "C" int astrai_moe_gemm_gate_up_gather(const void* x, const int32_t* sort
                  (long long)dim, (long long)dim_ffn, block_m);
   ASTRAI_REQUIRE(sorted_token && w_gate && w_up, "gemm_gate_up_gather: null row list or weight table");
   const int64_t capacity = (tiles_len - ASTRAI_MOE_TILE_HEADER) / ASTRAI_MOE_TILE_STRIDE;
+  if (few_rows(n_rows, n_experts, dim_ffn, true))
+    return launch_few_gate_up(x, sorted_token, tiles, capacity, w_gate, w_up, dim, dim_ffn, false, h,
+                              static_cast<hipStream_t>(stream));
   return launch_mfma_gate_up_gather(x, sorted_token, tiles, capacity, w_gate, w_up, dim, dim_ffn, block_m, h,
                                     static_cast<hipStream_t>(stream), GemmWorkspace{workspace, workspace_bytes});
 }
@@ -258,7 +264,10 @@ extern "C" int astrai_moe_gemm_down(const void* h, const int32_t* tiles,
   const int64_t capacity = (tiles_len - ASTRAI_MOE_TILE_HEADER) / ASTRAI_MOE_TILE_STRIDE;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (dtype == ASTRAI_MOE_BF16) {
-    if (mfma_down_supported(dim_ffn, dim, block_m, h, y))
+    const bool mfma = mfma_down_supported(dim_ffn, dim, block_m, h, y);
+    if (mfma && few_rows(n_rows, n_experts, dim, false))
+      return launch_few_down(h, tiles, capacity, w_down, sorted_w, dim_ffn, dim, false, y, s);
+    if (mfma)
       return launch_mfma_down(h, tiles, capacity, w_down, sorted_w, dim_ffn,
                               dim, block_m, false, y, s,
                               GemmWorkspace{workspace, workspace_bytes});
@@ -319,6 +328,9 @@ extern "C" int astrai_moe_gemm_gate_up_packed(const void* x_perm, const int32_t*
   if (n_rows == 0) return ASTRAI_MOE_OK;
   ASTRAI_REQUIRE(w_packed, "gemm_gate_up_packed: null weight table");
   const int64_t capacity = (tiles_len - ASTRAI_MOE_TILE_HEADER) / ASTRAI_MOE_TILE_STRIDE;
+  if (few_rows(n_rows, n_experts, dim_ffn, true))
+    return launch_few_gate_up(x_perm, nullptr, tiles, capacity, w_packed, w_packed, dim, dim_ffn, true, h,
+                              static_cast<hipStream_t>(stream));
   return launch_mfma_gate_up(x_perm, tiles, capacity, w_packed, w_packed, dim, dim_ffn, block_m, true, h,
                              static_cast<hipStream_t>(stream), GemmWorkspace{workspace, workspace_bytes});
 }
@@ -340,6 +352,9 @@ extern "C" int astrai_moe_gemm_down_packed(const void* h, const int32_t* tiles, 
   if (n_rows == 0) return ASTRAI_MOE_OK;
   ASTRAI_REQUIRE(w_packed, "gemm_down_packed: null weight table");
   const int64_t capacity = (tiles_len - ASTRAI_MOE_TILE_HEADER) / ASTRAI_MOE_TILE_STRIDE;
+  if (few_rows(n_rows, n_experts, dim, false))
+    return launch_few_down(h, tiles, capacity, w_packed, sorted_w, dim_ffn, dim, true, y,
+                           static_cast<hipStream_t>(stream));
   return launch_mfma_down(h, tiles, capacity, w_packed, sorted_w, dim_ffn, dim, block_m, true, y,
                           static_cast<hipStream_t>(stream),
                           GemmWorkspace{workspace, workspace_bytes});

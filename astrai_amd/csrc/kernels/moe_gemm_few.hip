@@ -1,0 +1,319 @@
+// bf16 grouped expert GEMMs for few rows (single-sequence and small-batch
+// decode) on CDNA4 matrix cores (gfx950): same contracts as the kernels of
+// moe_gemm_mfma.hip.
+//
+// Bound by reading each live expert's weights once, which needs every compute
+// unit to hold reads in flight. The 256-column tiles of gemm_mfma_kernel give
+// a down GEMM of D 4096 only 16 workgroups per row tile: one MLP of D 4096,
+// F 14336 over 24 rows streamed its 117 MB at 0.8 TB/s (150 us), two experts
+// of one token at 1.6 TB/s (145 us). Here a column tile is 32 weight rows
+// (down) or 16 gate and 16 up rows, eight times as many workgroups, and the
+// four waves of a workgroup share a tile by taking every fourth 64-K step of
+// it: each wave streams its steps through an LDS ring of its own (four stages
+// of 32 activation and 32 weight rows by 128 bytes, DMA'd and swizzled as in
+// moe_gemm_mfma.hip), with no barrier in the K loop and across tile ends.
+// Then the waves' fp32 sums meet in LDS, summed in wave order, one barrier per
+// tile (the LDS they meet in alternates between two halves).
+//
+// Persistent, workgroup b taking tiles b, b + G, ...: consecutive workgroups
+// read consecutive weight rows of one expert. The steps of a tile start at a
+// place that depends on its expert and columns (see gemm_mfma_kernel), never
+// on the row tile's height, and each tile is walked in runs of 32 rows, so
+// results are the same for every block_m and for packed and gathered operands.
+//
+// Measured: an MLP of D 4096, F 14336 over 24 rows 205 -> 100 us (352 MB of
+// weights, 3.5 TB/s), two experts of one token 240 -> 141 us (705 MB, 5.0
+// TB/s; its down GEMM 145 -> 45 us); more at few_rows below.
+#include <cmath>
+
+#include "mfma_tile.h"
+
+namespace astrai_moe {
+namespace {
+
+struct FewCfg {
+  static constexpr int BM = 32, BN = 32, WAVES = 4, STAGES = 4;
+  static constexpr int A_BYTES = BM * kRowBytes, B_BYTES = BN * kRowBytes, STAGE = A_BYTES + B_BYTES;
+  static constexpr int OPS = STAGE / 1024;                     // DMA ops per wave and step
+  static constexpr int RED_WAVE = BM * BN * 4;                 // one wave's fp32 sums
+  static constexpr int RED_OFF = WAVES * STAGES * STAGE;       // 128 KB of rings
+  static constexpr int LDS = RED_OFF + 2 * WAVES * RED_WAVE;   // 160 KB
+  static_assert(LDS <= 160 * 1024, "LDS");
+  static_assert(OPS * (STAGES - 1) <= 63, "vmcnt range");
+};
+
+// Position of a wave in its sequence of K steps: run `sub` of 32 rows of tile
+// `unit`, the wave's step j of n.
+template <bool kGateUp, bool kGather, bool kPacked>
+struct FewCursor {
+  using Cfg = FewCfg;
+  int unit, mt, nt, row0, rows, sub, j, n, rot;
+  bool live;
+  const char *a, *b0, *b1;
+  uint32_t off[Cfg::BM / 8];  // byte offsets of the rows a lane loads of the activation tile
+  int b_rows;
+
+  // tile and weights of `unit` (< total)
+  __device__ void enter(const int32_t* tiles, const void* const* W0, const void* const* W1, int K, int N, int n_cols) {
+    constexpr int kCols = kGateUp ? Cfg::BN / 2 : Cfg::BN;
+    mt = unit / n_cols;
+    nt = unit - mt * n_cols;
+    const int32_t* ti = tiles + ASTRAI_MOE_TILE_HEADER + (int64_t)mt * ASTRAI_MOE_TILE_STRIDE;
+    const int e = load_scalar(ti);
+    row0 = load_scalar(ti + 1);
+    rows = min(load_scalar(tiles + 1), load_scalar(ti + 2) - row0);
+    const int KT = k_steps(K);
+    b_rows = min(kCols, N - nt * kCols);
+    const char* w0 = static_cast<const char*>(load_scalar(W0 + e));
+    if constexpr (kPacked) {
+      // rows of the packed 256-row tile (128 gate and 128 up rows) that holds these columns
+      constexpr int kTile = kGateUp ? 128 : 256;
+      const int t = nt * kCols / kTile, r = nt * kCols - t * kTile;
+      b0 = w0 + ((int64_t)t * KT * 256 + r) * kRowBytes;
+      b1 = b0 + 128 * kRowBytes;
+    } else {
+      b0 = w0 + (int64_t)nt * kCols * K * 2;
+      b1 = kGateUp ? static_cast<const char*>(load_scalar(W1 + e)) + (int64_t)nt * kCols * K * 2 : b0;
+    }
+    rot = n > 0 ? (7 * e + 3 * nt) % n : 0;
+    sub = 0;
+  }
+  __device__ void enter_rows(const bf16_t* A, const int32_t* row_src, int K, int lane) {
+    j = 0;
+    const uint32_t k2 = (uint32_t)K * 2u;
+    a = reinterpret_cast<const char*>(kGather ? A : A + (int64_t)(row0 + sub * Cfg::BM) * K);
+    const int last = rows - sub * Cfg::BM - 1;  // pad rows re-read the last row
+#pragma unroll
+    for (int q = 0; q < Cfg::BM / 8; ++q) {
+      const int r = min(q * 8 + (lane >> 3), last);
+      off[q] = kGather ? (uint32_t)row_src[row0 + sub * Cfg::BM + r] * k2 : (uint32_t)r * k2;
+    }
+  }
+  __device__ void advance(int total, int G, const int32_t* tiles, const bf16_t* A, const void* const* W0,
+                          const void* const* W1, const int32_t* row_src, int K, int N, int n_cols, int lane) {
+    if (++j < n) return;
+    const int old_mt = mt, old_sub = sub;
+    if ((sub + 1) * Cfg::BM < rows) {
+      ++sub;
+    } else {
+      unit += G;
+      live = unit < total;
+      if (!live) return;
+      enter(tiles, W0, W1, K, N, n_cols);
+    }
+    // (the same rows: only the step restarts; their list is read again only where it changes)
+    if (mt == old_mt && sub == old_sub)
+      j = 0;
+    else
+      enter_rows(A, row_src, K, lane);
+  }
+  // the wave's next step into LDS at `lds`
+  __device__ void issue(int wave, int lane, int K, char* lds) const {
+    int jr = j + rot;
+    if (jr >= n) jr -= n;
+    const int ks = wave + Cfg::WAVES * jr;
+    const uint32_t k2 = (uint32_t)K * 2u;
+    const DmaLane dl(lane, ks);
+    const bool tail = (ks + 1) * kBK > K;
+#pragma unroll
+    for (int q = 0; q < Cfg::BM / 8; ++q) {
+      if (tail)
+        dma_16_or_zero(a, off[q] + dl.chunk(q), dl.chunk(q), k2, lds + q * 1024);
+      else
+        lds_dma_16(a + (off[q] + dl.chunk(q)), lds + q * 1024);
+    }
+    lds += Cfg::A_BYTES;
+#pragma unroll
+    for (int q = 0; q < Cfg::BN / 8; ++q) {
+      constexpr int kHalf = Cfg::BN / 16;  // gate/up: ops of the gate rows, then of the up rows
+      const bool up = kGateUp && q >= kHalf;
+      const int q_in = kGateUp ? q % kHalf : q;
+      const char* b = up ? b1 : b0;
+      if constexpr (kPacked) {
+        lds_dma_16(b + ((uint32_t)ks * (256u * kRowBytes) + (uint32_t)q_in * 1024u + (uint32_t)lane * 16u), lds + q * 1024);
+      } else {
+        const uint32_t o = (uint32_t)min(q_in * 8 + dl.row, b_rows - 1) * k2 + dl.chunk(q);
+        if (tail)
+          dma_16_or_zero(b, o, dl.chunk(q), k2, lds + q * 1024);
+        else
+          lds_dma_16(b + o, lds + q * 1024);
+      }
+    }
+  }
+};
+
+template <bool kGateUp, bool kGather, bool kPacked>
+__global__ __launch_bounds__(FewCfg::WAVES * 64, 1) void gemm_few_kernel(
+    const bf16_t* __restrict__ A, const int32_t* __restrict__ tiles, const void* const* __restrict__ W0,
+    const void* const* __restrict__ W1, const bf16_t* __restrict__ row_w, int K, int N, int n_cols, int capacity,
+    bf16_t* __restrict__ C, const int32_t* __restrict__ row_src) {
+  using Cfg = FewCfg;
+  __shared__ __attribute__((aligned(1024))) char smem[Cfg::LDS];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int G = gridDim.x;
+  const int total = min(load_scalar(tiles), min(load_scalar(tiles + 2), capacity)) * n_cols;
+  if ((int)blockIdx.x >= total) return;
+  char* const ring = smem + wave * (Cfg::STAGES * Cfg::STAGE);
+
+  FewCursor<kGateUp, kGather, kPacked> ld;  // the next step to load
+  const int KT = k_steps(K);
+  const int n_steps = KT > wave ? (KT - wave + Cfg::WAVES - 1) / Cfg::WAVES : 0;
+  ld.n = n_steps;
+  ld.unit = blockIdx.x;
+  ld.enter(tiles, W0, W1, K, N, n_cols);
+  ld.enter_rows(A, row_src, K, lane);
+  ld.live = n_steps > 0;
+  int issued = 0, used = 0;  // steps loaded and consumed so far; step i sits in stage i % STAGES
+  auto issue = [&]() {
+    ld.issue(wave, lane, K, ring + (issued % Cfg::STAGES) * Cfg::STAGE);
+    ++issued;
+    ld.advance(total, G, tiles, A, W0, W1, row_src, K, N, n_cols, lane);
+  };
+#pragma unroll 1
+  for (int i = 0; i < Cfg::STAGES; ++i)
+    if (ld.live) issue();
+
+  const int frag_row = lane & 15, fq = lane >> 4, fsw = (frag_row >> 1) & 7;
+  int parity = 0;
+  for (int unit = blockIdx.x; unit < total; unit += G) {
+    const int mt = unit / n_cols, nt = unit - mt * n_cols;
+    const int32_t* ti = tiles + ASTRAI_MOE_TILE_HEADER + (int64_t)mt * ASTRAI_MOE_TILE_STRIDE;
+    const int row0 = load_scalar(ti + 1);
+    const int rows = min(load_scalar(tiles + 1), load_scalar(ti + 2) - row0);
+    for (int r0 = 0; r0 < rows; r0 += Cfg::BM) {
+      f32x4_t acc[2][2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) acc[i][c] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+      for (int step = 0; step < n_steps; ++step) {
+        wait_groups<Cfg::OPS, Cfg::STAGES - 1>(issued - used - 1);  // this step has landed
+        const char* sa = ring + (used % Cfg::STAGES) * Cfg::STAGE + frag_row * kRowBytes;
+        bf16x8_t fa[2][2], fb[2][2];
+#pragma unroll
+        for (int kh = 0; kh < 2; ++kh) {
+          const int chunk = ((kh * 4 + fq) ^ fsw) << 4;
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            fa[kh][i] = *reinterpret_cast<const bf16x8_t*>(sa + i * 16 * kRowBytes + chunk);
+            fb[kh][i] = *reinterpret_cast<const bf16x8_t*>(sa + Cfg::A_BYTES + i * 16 * kRowBytes + chunk);
+          }
+        }
+        wait_lds();  // the stage has been read: it may be loaded again
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("" ::: "memory");
+        ++used;
+        if (ld.live) issue();
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int kh = 0; kh < 2; ++kh)
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int c = 0; c < 2; ++c)
+              acc[i][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[kh][c], fa[kh][i], acc[i][c], 0, 0, 0);
+      }
+      // the waves' sums meet: row r's 16-byte piece c at piece c ^ (r & 7)
+      char* const red = smem + Cfg::RED_OFF + parity * (Cfg::WAVES * Cfg::RED_WAVE);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+          const int r = i * 16 + frag_row;
+          *reinterpret_cast<f32x4_t*>(red + wave * Cfg::RED_WAVE + r * 128 + (((c * 4 + fq) ^ (r & 7)) << 4)) = acc[i][c];
+        }
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      auto sum = [&](int r, int piece) {
+        f32x4_t v = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int w = 0; w < Cfg::WAVES; ++w)
+          v += *reinterpret_cast<const f32x4_t*>(red + w * Cfg::RED_WAVE + r * 128 + ((piece ^ (r & 7)) << 4));
+        return v;
+      };
+      if constexpr (kGateUp) {
+        const int r = threadIdx.x >> 2, p = threadIdx.x & 3, n = nt * 16 + p * 4;
+        if (r < Cfg::BM && r0 + r < rows && n < N) {
+          const f32x4_t g4 = sum(r, p), u4 = sum(r, 4 + p);
+          bf16x4_t o;
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const float g = (float)(__bf16)g4[q], u = (float)(__bf16)u4[q];
+            const float ex = __builtin_amdgcn_exp2f(g * -1.4426950408889634f);
+            o[q] = (__bf16)(u * (float)(__bf16)(g * __builtin_amdgcn_rcpf(1.0f + ex)));
+          }
+          *reinterpret_cast<bf16x4_t*>(C + (int64_t)(row0 + r0 + r) * N + n) = o;
+        }
+      } else {
+        const int r = threadIdx.x >> 3, p = threadIdx.x & 7, n = nt * 32 + p * 4;
+        if (r0 + r < rows && n < N) {
+          const int64_t row = row0 + r0 + r;
+          const f32x4_t y4 = sum(r, p);
+          const float w = row_w != nullptr ? bf16_bits_to_f32(row_w[row]) : 1.0f;
+          bf16x4_t o;
+#pragma unroll
+          for (int q = 0; q < 4; ++q) o[q] = (__bf16)((float)(__bf16)y4[q] * w);
+          *reinterpret_cast<bf16x4_t*>(C + row * N + n) = o;
+        }
+      }
+      parity ^= 1;
+    }
+  }
+}
+
+template <bool kGateUp, bool kGather, bool kPacked>
+int launch_few(const void* A, const int32_t* tiles, int64_t capacity, const void* const* W0, const void* const* W1,
+               const void* row_w, int64_t K, int64_t N, void* C, hipStream_t s, const int32_t* row_src) {
+  if (capacity == 0) return ASTRAI_MOE_OK;
+  const int64_t n_cols = ceil_div(N, kGateUp ? FewCfg::BN / 2 : FewCfg::BN);  // the last may be partial
+  int64_t grid = 0;
+  if (int rc = persistent_grid(capacity, n_cols, &grid)) return rc;
+  hipLaunchKernelGGL((gemm_few_kernel<kGateUp, kGather, kPacked>), dim3((unsigned)grid), dim3(FewCfg::WAVES * 64), 0,
+                     s, static_cast<const bf16_t*>(A), tiles, W0, W1, static_cast<const bf16_t*>(row_w), (int)K,
+                     (int)N, (int)n_cols, (int)capacity, static_cast<bf16_t*>(C), row_src);
+  return check_launch(kGateUp ? "gemm_few_kernel<gate_up>" : "gemm_few_kernel<down>");
+}
+
+}  // namespace
+
+// Where these kernels replace the 256-column tiles of moe_gemm_mfma.hip: up to
+// kFewRowsPerExpert rows per expert (above, experts of more than 32 rows read
+// their weights in two runs), or kFewDenseRows of one expert, whose rows are
+// known; and where the other kernel's last round of tiles would leave more
+// than a tenth of its compute-unit time idle. Not by block_m, so that every
+// tile height gives the same bits. Measured, us per layer or MLP without and
+// with (replayed from a graph, three sets of weights in turn):
+// - 8 experts, top-2, D 4096, F 14336: 1 token 264 / 165, 2 368 / 286, 8 532 /
+//   495, 64 593 / 552, 96 (24 rows per expert) 602 / 590, 128 608 / 716;
+// - 64 experts, top-6, D 2048, F 1408: 1 token 74 / 60, 8 158 / 144, 32 226 /
+//   224, 64 (rounds of 0.92 and 1.0, past the line) 232 / 233;
+// - MLP, D 4096, F 14336: 1 token 201 / 92, 24 217 / 100, 96 223 / 197, 128
+//   234 / 228, 160 256 / 289; D 2048, F 5632: 24 66 / 29, 128 72 / 56.
+constexpr int kFewRowsPerExpert = 24, kFewDenseRows = 128;
+constexpr double kFewMaxFill = 0.9;
+
+bool few_rows(int64_t n_rows, int n_experts, int64_t n, bool gate_up) {
+  if (n_rows > (n_experts == 1 ? (int64_t)kFewDenseRows : (int64_t)kFewRowsPerExpert * n_experts)) return false;
+  // experts that meet a row, expected under even routing
+  const double live = n_experts * (1.0 - std::pow(1.0 - 1.0 / n_experts, (double)n_rows));
+  const double rounds = live * (double)ceil_div(n, gate_up ? 128 : 256) / cu_count();
+  return rounds < kFewMaxFill * std::ceil(rounds);
+}
+
+int launch_few_gate_up(const void* x, const int32_t* row_src, const int32_t* tiles, int64_t capacity,
+                       const void* const* w_gate, const void* const* w_up, int64_t dim, int64_t dim_ffn, bool packed,
+                       void* h, hipStream_t s) {
+  if (packed) return launch_few<true, false, true>(x, tiles, capacity, w_gate, w_gate, nullptr, dim, dim_ffn, h, s, nullptr);
+  if (row_src != nullptr)
+    return launch_few<true, true, false>(x, tiles, capacity, w_gate, w_up, nullptr, dim, dim_ffn, h, s, row_src);
+  return launch_few<true, false, false>(x, tiles, capacity, w_gate, w_up, nullptr, dim, dim_ffn, h, s, nullptr);
+}
+
+int launch_few_down(const void* h, const int32_t* tiles, int64_t capacity, const void* const* w_down,
+                    const void* sorted_w, int64_t dim_ffn, int64_t dim, bool packed, void* y, hipStream_t s) {
+  if (packed)
+    return launch_few<false, false, true>(h, tiles, capacity, w_down, w_down, sorted_w, dim_ffn, dim, y, s, nullptr);
+  return launch_few<false, false, false>(h, tiles, capacity, w_down, w_down, sorted_w, dim_ffn, dim, y, s, nullptr);
+}
+
+}  // namespace astrai_moe

@@ -1,0 +1,41 @@
+"""The GEMMs for few rows (gemm_few_kernel): fewer K steps than the workgroup
+has waves, partial last steps and column tiles, one run of 32 rows and several,
+one token over many experts; MLP and layer against the oracle."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from astrai_amd.model.components.mlp import MLP
+from oracle import moe_ref as R
+from test_gpu_backward import _random_layer
+from test_gpu_layer import check_layer
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dim,dim_ffn", [(64, 64), (72, 328), (512, 1408), (1096, 200)])
+@pytest.mark.parametrize("n_tok", [1, 16, 32, 33, 95, 128])
+def test_mlp(gpu, n_tok, dim, dim_ffn):
+    torch.manual_seed(n_tok + dim)
+    mlp = MLP(dim, dim_ffn)
+    for m in (mlp.up, mlp.gate, mlp.down):
+        m.reset_parameters()
+    mlp = mlp.to(device=gpu, dtype=torch.bfloat16).requires_grad_(False)
+    x = torch.randn(n_tok, dim, device=gpu).to(torch.bfloat16)
+    got = mlp(x)
+    want = R.expert_mlp(x, R.ExpertWeights(mlp.gate.weight, mlp.up.weight, mlp.down.weight))
+    # h and y are each rounded to bf16 (8 bits) at the same points; sums in another order
+    torch.testing.assert_close(got, want, rtol=2e-2, atol=2e-3)
+
+
+@pytest.mark.parametrize("n_tok,n_exp,top_k,n_shared", [(1, 64, 6, 1), (5, 8, 2, 2), (47, 8, 2, 0), (12, 128, 8, 0)])
+def test_layer(gpu, n_tok, n_exp, top_k, n_shared):
+    layer = _random_layer(gpu, 512, 640, n_exp, n_shared, top_k, torch.bfloat16, seed=n_exp).requires_grad_(False)
+    x = torch.randn(1, n_tok, 512, device=gpu).to(torch.bfloat16)
+    check_layer(layer, x, f"t{n_tok}_e{n_exp}_k{top_k}_s{n_shared}")
+    live = layer(x)
+    layer.pack_weights = True
+    assert layer.uses_packed_weights(x.dtype)
+    assert torch.equal(layer(x), live)  # packed copies: the same bits
