@@ -67,6 +67,7 @@ register("moe_gemm", sources=[str(KERNELS_DIR / "moe_gemm.hip"), str(KERNELS_DIR
                               str(KERNELS_DIR / "moe_gemm_generic_bwd.hip")])
 register("moe_combine")
 register("moe_forward")
+register("moe_route_grad")
 register("capi")
 
 # The kernel names the Python loader binds (entry point astrai_<name>).

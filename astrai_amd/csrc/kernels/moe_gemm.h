@@ -105,10 +105,11 @@ int launch_mfma_gate_up_gather(const void* x, const int32_t* sorted_token,
                                hipStream_t s,
                         const GemmWorkspace& ws = {});
 
-// Few rows (moe_gemm_few.hip), any tile height: whether the kernels there take
-// a GEMM of n_rows rows over n_experts experts with n output columns, and the GEMMs (row_src: the
+// Few rows (moe_gemm_few.hip), tiles below 256 rows: whether the kernels there
+// take a GEMM of n_rows rows over n_experts experts with n output columns, and the GEMMs (row_src: the
 // gathered rows' tokens, or null; packed: the tables hold packed copies).
-bool few_rows(int64_t n_rows, int n_experts, int64_t n, bool gate_up);
+bool few_rows(int64_t n_rows, int n_experts, int block_m, int64_t n,
+              bool gate_up);
 int launch_few_gate_up(const void* x, const int32_t* row_src,
                        const int32_t* tiles, int64_t capacity,
                        const void* const* w_gate, const void* const* w_up,

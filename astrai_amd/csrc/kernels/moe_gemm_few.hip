@@ -19,7 +19,7 @@
 // read consecutive weight rows of one expert. The steps of a tile start at a
 // place that depends on its expert and columns (see gemm_mfma_kernel), never
 // on the row tile's height, and each tile is walked in runs of 32 rows, so
-// results are the same for every block_m and for packed and gathered operands.
+// results are the same for every height and for packed and gathered operands.
 //
 // Measured: an MLP of D 4096, F 14336 over 24 rows 205 -> 100 us (352 MB of
 // weights, 3.5 TB/s), two experts of one token 240 -> 141 us (705 MB, 5.0
@@ -280,8 +280,9 @@ int launch_few(const void* A, const int32_t* tiles, int64_t capacity, const void
 // kFewRowsPerExpert rows per expert (above, experts of more than 32 rows read
 // their weights in two runs), or kFewDenseRows of one expert, whose rows are
 // known; and where the other kernel's last round of tiles would leave more
-// than a tenth of its compute-unit time idle. Not by block_m, so that every
-// tile height gives the same bits. Measured, us per layer or MLP without and
+// than a tenth of its compute-unit time idle. The same for tiles of 32, 64 and
+// 128 rows, so that these give the same bits; lists of 256-row tiles keep their
+// kernels, whose bits the training forward shares. Measured, us per layer or MLP without and
 // with (replayed from a graph, three sets of weights in turn):
 // - 8 experts, top-2, D 4096, F 14336: 1 token 264 / 165, 2 368 / 286, 8 532 /
 //   495, 64 593 / 552, 96 (24 rows per expert) 602 / 590, 128 608 / 716;
@@ -292,7 +293,8 @@ int launch_few(const void* A, const int32_t* tiles, int64_t capacity, const void
 constexpr int kFewRowsPerExpert = 24, kFewDenseRows = 128;
 constexpr double kFewMaxFill = 0.9;
 
-bool few_rows(int64_t n_rows, int n_experts, int64_t n, bool gate_up) {
+bool few_rows(int64_t n_rows, int n_experts, int block_m, int64_t n, bool gate_up) {
+  if (block_m == kMfmaBigBM) return false;
   if (n_rows > (n_experts == 1 ? (int64_t)kFewDenseRows : (int64_t)kFewRowsPerExpert * n_experts)) return false;
   // experts that meet a row, expected under even routing
   const double live = n_experts * (1.0 - std::pow(1.0 - 1.0 / n_experts, (double)n_rows));

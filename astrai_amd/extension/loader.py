@@ -75,6 +75,7 @@ _SIGNATURES: dict[str, tuple] = {
                                              _vp, _i64, _vp]),
     "astrai_moe_gemm_down_train": (_int, [_vp, _vp, _i64, _vp, _vp, _int, _i64, _int, _i64, _i64, _int, _vp, _vp,
                                           _vp, _i64, _vp]),
+    "astrai_moe_route_grad": (_int, [_vp, _vp, _vp, _int, _i64, _int, _int, _vp, _vp]),
     "astrai_moe_row_grad": (_int, [_vp, _vp, _vp, _vp, _int, _i64, _i64, _vp, _vp, _vp]),
     "astrai_moe_gemm_dgrad_down": (_int, [_vp, _vp, _i64, _vp, _vp, _int, _i64, _int, _i64, _i64, _int, _vp, _vp,
                                           _vp]),

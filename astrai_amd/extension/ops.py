@@ -631,6 +631,24 @@ def moe_gemm_down_train(h: torch.Tensor, tiles: torch.Tensor, w_down: torch.Tens
     return y, y_unw
 
 
+def moe_route_grad(logits: torch.Tensor, topk_idx: torch.Tensor, dw: torch.Tensor) -> torch.Tensor:
+    """The logits' gradient from that of ``moe_route``'s weights
+    (``dw [T, K]``), mlp.py:84-87 differentiated at the chosen experts."""
+    _require_gpu(logits, "logits", 2)
+    _require_gpu(topk_idx, "topk_idx", 2)
+    _require_gpu(dw, "dw", 2)
+    code = _dtype_code(logits, "logits")
+    n_tokens, n_experts = logits.shape
+    if topk_idx.shape[0] != n_tokens or topk_idx.dtype != torch.int32 or dw.shape != topk_idx.shape:
+        raise ValueError("topk_idx must be int32 [n_tokens, top_k] and dw of its shape")
+    if dw.dtype != logits.dtype:
+        raise ValueError("dw must have the logits' dtype")
+    dlogits = torch.empty_like(logits)
+    _lib_call("astrai_moe_route_grad", logits.data_ptr(), topk_idx.data_ptr(), dw.data_ptr(), code, n_tokens,
+              n_experts, topk_idx.shape[1], dlogits.data_ptr(), _stream(logits))
+    return dlogits
+
+
 def moe_row_grad(dout: torch.Tensor, sorted_token: torch.Tensor, sorted_w: torch.Tensor,
                  y_unweighted: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     """Per permuted row: ``dy = dout[token] * w`` and ``dw = sum(dout[token] * y)``

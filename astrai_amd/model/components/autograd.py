@@ -100,7 +100,7 @@ class RoutedExperts(torch.autograd.Function):
         if ctx.needs_input_grad[0]:
             dx_perm = ops.moe_gemm_dgrad_gate_up(dg, du, tiles, tg, tu, n_experts, dim)
             dx = ops.moe_combine(dx_perm, token_pos)
-        dw = dw_rows[token_pos.long()] if ctx.needs_input_grad[1] else None
+        dw = dw_rows.index_select(0, token_pos.view(-1)).view(token_pos.shape) if ctx.needs_input_grad[1] else None
         none = [None] * n_experts
         g_gate, g_up, g_down = list(none), list(none), list(none)
         if any(ctx.needs_input_grad[6:]):
@@ -118,6 +118,24 @@ class RoutedExperts(torch.autograd.Function):
                 if offs[e + 1] > offs[e]:
                     g_gate[e], g_up[e], g_down[e] = v_gate[e], v_up[e], v_down[e]
         return (dx, dw, None, None, None, None, *g_gate, *g_up, *g_down)
+
+
+class RouteWeights(torch.autograd.Function):
+    """Routing (mlp.py:84-87) with the weights' gradient back to the logits:
+    ``forward(logits [T, E], top_k)`` gives ``(topk_w, topk_idx, chunk_hist)``
+    of ``ops.moe_route``, differentiable in ``logits`` through ``topk_w``."""
+
+    @staticmethod
+    def forward(ctx, logits, top_k):
+        route = ops.moe_route(logits, top_k)
+        ctx.save_for_backward(logits, route.topk_idx)
+        ctx.mark_non_differentiable(route.topk_idx, route.chunk_hist)
+        return route.topk_w, route.topk_idx, route.chunk_hist
+
+    @staticmethod
+    def backward(ctx, dw, *_):
+        logits, topk_idx = ctx.saved_tensors
+        return ops.moe_route_grad(logits, topk_idx, dw.contiguous()), None
 
 
 class DenseExpert(torch.autograd.Function):
@@ -163,8 +181,9 @@ class DenseExpert(torch.autograd.Function):
 
 def routing_weights(logits: Tensor, topk_idx: Tensor, dtype: torch.dtype) -> Tensor:
     """The renormalised top-k weights as differentiable torch ops
-    (mlp.py:84-87), evaluated at the route kernel's indices: the same values
-    the kernel produces, with autograd's path back to the logits."""
+    (mlp.py:84-87) in ``dtype``, evaluated at the route kernel's indices, with
+    autograd's path back to the logits: for logits of another dtype than the
+    activations (autocast), where ``RouteWeights``' weights would have theirs."""
     probs = torch.softmax(logits.float(), dim=-1).to(dtype)
     w = probs.gather(1, topk_idx.long())
     return w / w.sum(dim=-1, keepdim=True)

@@ -39,7 +39,8 @@ from torch import Tensor
 
 from astrai_amd.extension import ops
 from astrai_amd.factory import BaseFactory
-from astrai_amd.model.components.autograd import DenseExpert, EmptyBatch, RoutedExperts, routing_weights
+from astrai_amd.model.components.autograd import (DenseExpert, EmptyBatch, RoutedExperts, RouteWeights,
+                                                     routing_weights)
 from astrai_amd.model.components.linear import Linear
 
 
@@ -326,9 +327,7 @@ class DeepSeekMoE(nn.Module):
 
     def _forward_autograd(self, x: Tensor, st: _ExpertState) -> Tensor:
         """mlp.py:64-100 with autograd: HIP kernels forward and backward.
-        Routing indices come from the route kernel; the weights are rebuilt
-        from the logits with torch ops (same values) so their gradient reaches
-        the router."""
+        The route kernel's weights carry their gradient back to the router."""
         n_tokens = x.shape[0]
         if n_tokens == 0:
             # the reference's routed output is a graph-less zeros here; only
@@ -340,15 +339,18 @@ class DeepSeekMoE(nn.Module):
         routed_w = st.routed
         dim_ffn = routed_w[0][0].shape[0]
         logits = self.router(x)
-        route = ops.moe_route(logits.detach(), self.n_activated_experts)
-        topk_w = routing_weights(logits, route.topk_idx, x.dtype)
-        routed = RoutedExperts.apply(x, topk_w, route.topk_idx, route.chunk_hist, t_routed, dim_ffn,
+        if logits.dtype == x.dtype:
+            topk_w, topk_idx, chunk_hist = RouteWeights.apply(logits, self.n_activated_experts)
+        else:
+            topk_idx, _, chunk_hist = ops.moe_route(logits.detach(), self.n_activated_experts)
+            topk_w = routing_weights(logits, topk_idx, x.dtype)
+        routed = RoutedExperts.apply(x, topk_w, topk_idx, chunk_hist, t_routed, dim_ffn,
                                      *routed_w[0], *routed_w[1], *routed_w[2])
         if self.n_shared_experts == 0:
             return routed
         shared_w = st.shared
-        shared = sum(
-            DenseExpert.apply(x, t_shared[i], dim_ffn, shared_w[0][i], shared_w[1][i], shared_w[2][i])
-            for i in range(self.n_shared_experts)
-        ) / self.n_shared_experts
+        outs = [DenseExpert.apply(x, t_shared[i], dim_ffn, shared_w[0][i], shared_w[1][i], shared_w[2][i])
+                for i in range(self.n_shared_experts)]
+        # the mean (mlp.py:77); of one expert it is that expert's output
+        shared = outs[0] if len(outs) == 1 else sum(outs) / self.n_shared_experts
         return shared + routed

@@ -425,6 +425,19 @@ int astrai_moe_gemm_down_train(const void* h, const int32_t* tiles,
                                void* stream);
 
 /*
+ * Gradient of the logits from that of the renormalised top-k weights: the
+ * derivative of mlp.py:84-87 (astrai_moe_route) at the chosen experts, in
+ * float with one rounding to dtype.
+ *   logits, dlogits  [n_tokens, n_experts]  dtype
+ *   topk_idx         [n_tokens, top_k]      int32, from astrai_moe_route
+ *   dw               [n_tokens, top_k]      dtype, gradient of topk_w
+ */
+int astrai_moe_route_grad(const void* logits, const int32_t* topk_idx,
+                          const void* dw, int dtype, int64_t n_tokens,
+                          int n_experts, int top_k, void* dlogits,
+                          void* stream);
+
+/*
  * Per permuted row r (token sorted_token[r], weight sorted_w[r]):
  *   dy[r]      = dout[token] * w, rounded per element     [n_rows, dim] dtype
  *   dw_rows[r] = sum_d round(dout[token, d] * y[r, d])    [n_rows] dtype

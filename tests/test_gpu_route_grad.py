@@ -1,0 +1,52 @@
+"""The logits' gradient kernel at every width (logits per lane) and slot count
+against autograd through float64 torch operators, and a layer under autocast,
+whose logits have another dtype than its activations."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from astrai_amd.extension import loader, ops
+from test_gpu_backward import _random_layer
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n_tok,n_exp,top_k", [(1, 1, 1), (5, 2, 2), (130, 64, 6), (33, 65, 32), (64, 128, 8),
+                                               (7, 200, 3), (9, 257, 4), (12, 1024, 32)])
+def test_logits_gradient(gpu, n_tok, n_exp, top_k, dtype):
+    g = torch.Generator(device=gpu).manual_seed(n_exp)
+    logits = torch.randn(n_tok, n_exp, generator=g, device=gpu).to(dtype)
+    dw = torch.randn(n_tok, top_k, generator=g, device=gpu).to(dtype)
+    route = ops.moe_route(logits, top_k)
+    got = ops.moe_route_grad(logits, route.topk_idx, dw)
+    l64 = logits.double().requires_grad_(True)
+    w = torch.softmax(l64, -1).gather(1, route.topk_idx.long())
+    (w / w.sum(-1, keepdim=True)).backward(dw.double())
+    # against exact probabilities: the chosen ones are rounded to dtype (half
+    # a unit, twice over v and S) and the result once; scaled by the largest
+    # gradient of the row, since its terms cancel
+    unit = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -24
+    scale = dw.double().abs().amax(-1, keepdim=True)
+    err = (got.double() - l64.grad).abs() / scale
+    assert err.max().item() <= (4 + top_k) * unit * (1 if dtype == torch.bfloat16 else 8)
+
+
+@pytest.mark.gpu
+def test_layer_under_autocast_still_trains(gpu):
+    layer = _random_layer(gpu, 64, 96, 4, 1, 2, torch.float32, seed=1)
+    x = torch.randn(1, 40, 64, device=gpu, requires_grad=True)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        out = layer(x)
+    out.sum().backward()
+    assert out.dtype == torch.float32 and torch.isfinite(x.grad).all()
+    assert layer.router.weight.grad is not None and torch.isfinite(layer.router.weight.grad).all()
+
+
+def test_arguments_are_checked_on_the_host():
+    lib = loader.library()
+    for args, word in (((16, 16, 16, 1, 10, 0, 1, 16, None), "n_experts"), ((16, 16, 16, 1, 10, 8, 9, 16, None), "top_k"),
+                       ((16, 16, 16, 5, 10, 8, 2, 16, None), "dtype"), ((16, None, 16, 1, 10, 8, 2, 16, None), "null")):
+        assert lib.astrai_moe_route_grad(*args) == -1 and word in loader.last_error()
+    assert lib.astrai_moe_route_grad(None, None, None, 1, 0, 8, 2, None, None) == 0
