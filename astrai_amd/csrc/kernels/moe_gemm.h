@@ -113,12 +113,12 @@ bool few_rows(int64_t n_rows, int n_experts, int block_m, int64_t n,
 int launch_few_gate_up(const void* x, const int32_t* row_src,
                        const int32_t* tiles, int64_t capacity,
                        const void* const* w_gate, const void* const* w_up,
-                       int64_t dim, int64_t dim_ffn, bool packed, void* h,
-                       hipStream_t s);
+                       int64_t n_rows, int n_experts, int64_t dim,
+                       int64_t dim_ffn, bool packed, void* h, hipStream_t s);
 int launch_few_down(const void* h, const int32_t* tiles, int64_t capacity,
                     const void* const* w_down, const void* sorted_w,
-                    int64_t dim_ffn, int64_t dim, bool packed, void* y,
-                    hipStream_t s);
+                    int64_t n_rows, int n_experts, int64_t dim_ffn,
+                    int64_t dim, bool packed, void* y, hipStream_t s);
 
 // Training forward (256-row tiles): as launch_mfma_gate_up / launch_mfma_down,
 // also storing the bf16 gate and up projections (gu: [rows, 2 dim_ffn],

@@ -204,7 +204,7 @@ extern "C" int astrai_moe_gemm_gate_up(const void* x_perm, const int32_t* tiles,
   if (dtype == ASTRAI_MOE_BF16) {
     const bool mfma = mfma_gate_up_supported(dim, dim_ffn, block_m, x_perm, h);
     if (mfma && few_rows(n_rows, n_experts, block_m, dim_ffn, true))
-      return launch_few_gate_up(x_perm, nullptr, tiles, capacity, w_gate, w_up, dim, dim_ffn, false, h, s);
+      return launch_few_gate_up(x_perm, nullptr, tiles, capacity, w_gate, w_up, n_rows, n_experts, dim, dim_ffn, false, h, s);
     if (mfma)
       return launch_mfma_gate_up(x_perm, tiles, capacity, w_gate, w_up, dim,
                                  dim_ffn, block_m, false, h, s,
@@ -240,7 +240,7 @@ extern "C" int astrai_moe_gemm_gate_up_gather(const void* x, const int32_t* sort
   ASTRAI_REQUIRE(sorted_token && w_gate && w_up, "gemm_gate_up_gather: null row list or weight table");
   const int64_t capacity = (tiles_len - ASTRAI_MOE_TILE_HEADER) / ASTRAI_MOE_TILE_STRIDE;
   if (few_rows(n_rows, n_experts, block_m, dim_ffn, true))
-    return launch_few_gate_up(x, sorted_token, tiles, capacity, w_gate, w_up, dim, dim_ffn, false, h,
+    return launch_few_gate_up(x, sorted_token, tiles, capacity, w_gate, w_up, n_rows, n_experts, dim, dim_ffn, false, h,
                               static_cast<hipStream_t>(stream));
   return launch_mfma_gate_up_gather(x, sorted_token, tiles, capacity, w_gate, w_up, dim, dim_ffn, block_m, h,
                                     static_cast<hipStream_t>(stream), GemmWorkspace{workspace, workspace_bytes});
@@ -266,7 +266,7 @@ extern "C" int astrai_moe_gemm_down(const void* h, const int32_t* tiles,
   if (dtype == ASTRAI_MOE_BF16) {
     const bool mfma = mfma_down_supported(dim_ffn, dim, block_m, h, y);
     if (mfma && few_rows(n_rows, n_experts, block_m, dim, false))
-      return launch_few_down(h, tiles, capacity, w_down, sorted_w, dim_ffn, dim, false, y, s);
+      return launch_few_down(h, tiles, capacity, w_down, sorted_w, n_rows, n_experts, dim_ffn, dim, false, y, s);
     if (mfma)
       return launch_mfma_down(h, tiles, capacity, w_down, sorted_w, dim_ffn,
                               dim, block_m, false, y, s,
@@ -329,7 +329,7 @@ extern "C" int astrai_moe_gemm_gate_up_packed(const void* x_perm, const int32_t*
   ASTRAI_REQUIRE(w_packed, "gemm_gate_up_packed: null weight table");
   const int64_t capacity = (tiles_len - ASTRAI_MOE_TILE_HEADER) / ASTRAI_MOE_TILE_STRIDE;
   if (few_rows(n_rows, n_experts, block_m, dim_ffn, true))
-    return launch_few_gate_up(x_perm, nullptr, tiles, capacity, w_packed, w_packed, dim, dim_ffn, true, h,
+    return launch_few_gate_up(x_perm, nullptr, tiles, capacity, w_packed, w_packed, n_rows, n_experts, dim, dim_ffn, true, h,
                               static_cast<hipStream_t>(stream));
   return launch_mfma_gate_up(x_perm, tiles, capacity, w_packed, w_packed, dim, dim_ffn, block_m, true, h,
                              static_cast<hipStream_t>(stream), GemmWorkspace{workspace, workspace_bytes});
@@ -353,7 +353,7 @@ extern "C" int astrai_moe_gemm_down_packed(const void* h, const int32_t* tiles, 
   ASTRAI_REQUIRE(w_packed, "gemm_down_packed: null weight table");
   const int64_t capacity = (tiles_len - ASTRAI_MOE_TILE_HEADER) / ASTRAI_MOE_TILE_STRIDE;
   if (few_rows(n_rows, n_experts, block_m, dim, false))
-    return launch_few_down(h, tiles, capacity, w_packed, sorted_w, dim_ffn, dim, true, y,
+    return launch_few_down(h, tiles, capacity, w_packed, sorted_w, n_rows, n_experts, dim_ffn, dim, true, y,
                            static_cast<hipStream_t>(stream));
   return launch_mfma_down(h, tiles, capacity, w_packed, sorted_w, dim_ffn, dim, block_m, true, y,
                           static_cast<hipStream_t>(stream),

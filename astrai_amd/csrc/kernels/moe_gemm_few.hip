@@ -31,12 +31,14 @@
 namespace astrai_moe {
 namespace {
 
+template <int BN_>
 struct FewCfg {
-  static constexpr int BM = 32, BN = 32, WAVES = 4, STAGES = 4;
+  static constexpr int BM = 32, BN = BN_, WAVES = 4, STAGES = BN == 32 ? 4 : 6;
+  static constexpr int NC = BN / 16;  // 16-column blocks
   static constexpr int A_BYTES = BM * kRowBytes, B_BYTES = BN * kRowBytes, STAGE = A_BYTES + B_BYTES;
   static constexpr int OPS = STAGE / 1024;                     // DMA ops per wave and step
   static constexpr int RED_WAVE = BM * BN * 4;                 // one wave's fp32 sums
-  static constexpr int RED_OFF = WAVES * STAGES * STAGE;       // 128 KB of rings
+  static constexpr int RED_OFF = WAVES * STAGES * STAGE;       // 128 or 144 KB of rings
   static constexpr int LDS = RED_OFF + 2 * WAVES * RED_WAVE;   // 160 KB
   static_assert(LDS <= 160 * 1024, "LDS");
   static_assert(OPS * (STAGES - 1) <= 63, "vmcnt range");
@@ -44,9 +46,8 @@ struct FewCfg {
 
 // Position of a wave in its sequence of K steps: run `sub` of 32 rows of tile
 // `unit`, the wave's step j of n.
-template <bool kGateUp, bool kGather, bool kPacked>
+template <typename Cfg, bool kGateUp, bool kGather, bool kPacked>
 struct FewCursor {
-  using Cfg = FewCfg;
   int unit, mt, nt, row0, rows, sub, j, n, rot;
   bool live;
   const char *a, *b0, *b1;
@@ -130,7 +131,11 @@ struct FewCursor {
       const int q_in = kGateUp ? q % kHalf : q;
       const char* b = up ? b1 : b0;
       if constexpr (kPacked) {
-        lds_dma_16(b + ((uint32_t)ks * (256u * kRowBytes) + (uint32_t)q_in * 1024u + (uint32_t)lane * 16u), lds + q * 1024);
+        // the copy's chunks are swizzled by its own rows: 8 gate or up rows
+        // may lie at the other parity of 8 than their place in the stage
+        const uint32_t flip = (kGateUp && Cfg::BN == 16) ? 64u * (uint32_t)((nt ^ q) & 1) : 0u;
+        const uint32_t at = (uint32_t)ks * (256u * kRowBytes) + (uint32_t)q_in * 1024u + ((uint32_t)lane * 16u ^ flip);
+        lds_dma_16(b + at, lds + q * 1024);
       } else {
         const uint32_t o = (uint32_t)min(q_in * 8 + dl.row, b_rows - 1) * k2 + dl.chunk(q);
         if (tail)
@@ -142,12 +147,12 @@ struct FewCursor {
   }
 };
 
-template <bool kGateUp, bool kGather, bool kPacked>
-__global__ __launch_bounds__(FewCfg::WAVES * 64, 1) void gemm_few_kernel(
+template <typename Cfg, bool kGateUp, bool kGather, bool kPacked>
+__global__ __launch_bounds__(Cfg::WAVES * 64, 1) void gemm_few_kernel(
     const bf16_t* __restrict__ A, const int32_t* __restrict__ tiles, const void* const* __restrict__ W0,
     const void* const* __restrict__ W1, const bf16_t* __restrict__ row_w, int K, int N, int n_cols, int capacity,
     bf16_t* __restrict__ C, const int32_t* __restrict__ row_src) {
-  using Cfg = FewCfg;
+  constexpr int NC = Cfg::NC;
   __shared__ __attribute__((aligned(1024))) char smem[Cfg::LDS];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -156,7 +161,7 @@ __global__ __launch_bounds__(FewCfg::WAVES * 64, 1) void gemm_few_kernel(
   if ((int)blockIdx.x >= total) return;
   char* const ring = smem + wave * (Cfg::STAGES * Cfg::STAGE);
 
-  FewCursor<kGateUp, kGather, kPacked> ld;  // the next step to load
+  FewCursor<Cfg, kGateUp, kGather, kPacked> ld;  // the next step to load
   const int KT = k_steps(K);
   const int n_steps = KT > wave ? (KT - wave + Cfg::WAVES - 1) / Cfg::WAVES : 0;
   ld.n = n_steps;
@@ -182,23 +187,24 @@ __global__ __launch_bounds__(FewCfg::WAVES * 64, 1) void gemm_few_kernel(
     const int row0 = load_scalar(ti + 1);
     const int rows = min(load_scalar(tiles + 1), load_scalar(ti + 2) - row0);
     for (int r0 = 0; r0 < rows; r0 += Cfg::BM) {
-      f32x4_t acc[2][2];
+      f32x4_t acc[2][NC];
 #pragma unroll
       for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int c = 0; c < 2; ++c) acc[i][c] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int c = 0; c < NC; ++c) acc[i][c] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
       for (int step = 0; step < n_steps; ++step) {
         wait_groups<Cfg::OPS, Cfg::STAGES - 1>(issued - used - 1);  // this step has landed
         const char* sa = ring + (used % Cfg::STAGES) * Cfg::STAGE + frag_row * kRowBytes;
-        bf16x8_t fa[2][2], fb[2][2];
+        bf16x8_t fa[2][2], fb[2][NC];
 #pragma unroll
         for (int kh = 0; kh < 2; ++kh) {
           const int chunk = ((kh * 4 + fq) ^ fsw) << 4;
 #pragma unroll
-          for (int i = 0; i < 2; ++i) {
+          for (int i = 0; i < 2; ++i)
             fa[kh][i] = *reinterpret_cast<const bf16x8_t*>(sa + i * 16 * kRowBytes + chunk);
-            fb[kh][i] = *reinterpret_cast<const bf16x8_t*>(sa + Cfg::A_BYTES + i * 16 * kRowBytes + chunk);
-          }
+#pragma unroll
+          for (int c = 0; c < NC; ++c)
+            fb[kh][c] = *reinterpret_cast<const bf16x8_t*>(sa + Cfg::A_BYTES + c * 16 * kRowBytes + chunk);
         }
         wait_lds();  // the stage has been read: it may be loaded again
         __builtin_amdgcn_sched_barrier(0);
@@ -211,30 +217,33 @@ __global__ __launch_bounds__(FewCfg::WAVES * 64, 1) void gemm_few_kernel(
 #pragma unroll
           for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int c = 0; c < 2; ++c)
+            for (int c = 0; c < NC; ++c)
               acc[i][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[kh][c], fa[kh][i], acc[i][c], 0, 0, 0);
       }
-      // the waves' sums meet: row r's 16-byte piece c at piece c ^ (r & 7)
+      // the waves' sums meet: row r's 16-byte piece c at piece c ^ (r % pieces)
+      constexpr int PIECES = Cfg::BN / 4, ROW = Cfg::BN * 4;
       char* const red = smem + Cfg::RED_OFF + parity * (Cfg::WAVES * Cfg::RED_WAVE);
 #pragma unroll
       for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int c = 0; c < 2; ++c) {
+        for (int c = 0; c < NC; ++c) {
           const int r = i * 16 + frag_row;
-          *reinterpret_cast<f32x4_t*>(red + wave * Cfg::RED_WAVE + r * 128 + (((c * 4 + fq) ^ (r & 7)) << 4)) = acc[i][c];
+          *reinterpret_cast<f32x4_t*>(red + wave * Cfg::RED_WAVE + r * ROW +
+                                      (((c * 4 + fq) ^ (r & (PIECES - 1))) << 4)) = acc[i][c];
         }
       asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
       auto sum = [&](int r, int piece) {
         f32x4_t v = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int w = 0; w < Cfg::WAVES; ++w)
-          v += *reinterpret_cast<const f32x4_t*>(red + w * Cfg::RED_WAVE + r * 128 + ((piece ^ (r & 7)) << 4));
+          v += *reinterpret_cast<const f32x4_t*>(red + w * Cfg::RED_WAVE + r * ROW + ((piece ^ (r & (PIECES - 1))) << 4));
         return v;
       };
       if constexpr (kGateUp) {
-        const int r = threadIdx.x >> 2, p = threadIdx.x & 3, n = nt * 16 + p * 4;
+        constexpr int HP = PIECES / 2;  // pieces of the gate columns, then of the up columns
+        const int r = threadIdx.x / HP, p = threadIdx.x % HP, n = nt * (Cfg::BN / 2) + p * 4;
         if (r < Cfg::BM && r0 + r < rows && n < N) {
-          const f32x4_t g4 = sum(r, p), u4 = sum(r, 4 + p);
+          const f32x4_t g4 = sum(r, p), u4 = sum(r, HP + p);
           bf16x4_t o;
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
@@ -245,8 +254,8 @@ __global__ __launch_bounds__(FewCfg::WAVES * 64, 1) void gemm_few_kernel(
           *reinterpret_cast<bf16x4_t*>(C + (int64_t)(row0 + r0 + r) * N + n) = o;
         }
       } else {
-        const int r = threadIdx.x >> 3, p = threadIdx.x & 7, n = nt * 32 + p * 4;
-        if (r0 + r < rows && n < N) {
+        const int r = threadIdx.x / PIECES, p = threadIdx.x % PIECES, n = nt * Cfg::BN + p * 4;
+        if (r < Cfg::BM && r0 + r < rows && n < N) {
           const int64_t row = row0 + r0 + r;
           const f32x4_t y4 = sum(r, p);
           const float w = row_w != nullptr ? bf16_bits_to_f32(row_w[row]) : 1.0f;
@@ -261,17 +270,46 @@ __global__ __launch_bounds__(FewCfg::WAVES * 64, 1) void gemm_few_kernel(
   }
 }
 
-template <bool kGateUp, bool kGather, bool kPacked>
-int launch_few(const void* A, const int32_t* tiles, int64_t capacity, const void* const* W0, const void* const* W1,
+template <typename Cfg, bool kGateUp, bool kGather, bool kPacked>
+int launch_few_cfg(const void* A, const int32_t* tiles, int64_t capacity, const void* const* W0, const void* const* W1,
                const void* row_w, int64_t K, int64_t N, void* C, hipStream_t s, const int32_t* row_src) {
   if (capacity == 0) return ASTRAI_MOE_OK;
-  const int64_t n_cols = ceil_div(N, kGateUp ? FewCfg::BN / 2 : FewCfg::BN);  // the last may be partial
+  const int64_t n_cols = ceil_div(N, kGateUp ? Cfg::BN / 2 : Cfg::BN);  // the last may be partial
   int64_t grid = 0;
   if (int rc = persistent_grid(capacity, n_cols, &grid)) return rc;
-  hipLaunchKernelGGL((gemm_few_kernel<kGateUp, kGather, kPacked>), dim3((unsigned)grid), dim3(FewCfg::WAVES * 64), 0,
-                     s, static_cast<const bf16_t*>(A), tiles, W0, W1, static_cast<const bf16_t*>(row_w), (int)K,
+  hipLaunchKernelGGL((gemm_few_kernel<Cfg, kGateUp, kGather, kPacked>), dim3((unsigned)grid), dim3(Cfg::WAVES * 64),
+                     0, s, static_cast<const bf16_t*>(A), tiles, W0, W1, static_cast<const bf16_t*>(row_w), (int)K,
                      (int)N, (int)n_cols, (int)capacity, static_cast<bf16_t*>(C), row_src);
   return check_launch(kGateUp ? "gemm_few_kernel<gate_up>" : "gemm_few_kernel<down>");
+}
+
+// Experts that meet one of n_rows rows, expected under even routing.
+double live_experts(int64_t n_rows, int n_experts) {
+  return n_experts * (1.0 - std::pow(1.0 - 1.0 / n_experts, (double)n_rows));
+}
+
+// Share of the compute-unit time that `tiles` equal tiles fill, a partial last
+// round included.
+double fill(double tiles) {
+  const double rounds = tiles / cu_count();
+  return rounds / std::ceil(rounds);
+}
+
+// One expert's single run of 32 rows (an MLP decoding) takes tiles of 16 weight
+// rows where those fill the rounds of tiles better: D 4096, F 14336, 24 rows,
+// gate/up 3.5 rounds of 32-row tiles or 7 of 16, down half a round or one, 100
+// -> 89 us; D 1536, F 4096 20.5 -> 19.6. A 16-row tile reads as many
+// activation bytes as one of 32, which costs more elsewhere: more runs (48
+// rows 131 -> 163 us) and routed rows (8 experts of that size, 24 tokens 541
+// -> 560; 64 of D 2048, F 1408, 8 tokens 144 -> 188).
+template <bool kGateUp, bool kGather, bool kPacked>
+int launch_few(const void* A, const int32_t* tiles, int64_t capacity, const void* const* W0, const void* const* W1,
+               const void* row_w, int64_t n_rows, int n_experts, int64_t K, int64_t N, void* C, hipStream_t s,
+               const int32_t* row_src) {
+  if (n_experts == 1 && n_rows <= FewCfg<16>::BM &&
+      fill((double)ceil_div(N, kGateUp ? 8 : 16)) > 1.05 * fill((double)ceil_div(N, kGateUp ? 16 : 32)))
+    return launch_few_cfg<FewCfg<16>, kGateUp, kGather, kPacked>(A, tiles, capacity, W0, W1, row_w, K, N, C, s, row_src);
+  return launch_few_cfg<FewCfg<32>, kGateUp, kGather, kPacked>(A, tiles, capacity, W0, W1, row_w, K, N, C, s, row_src);
 }
 
 }  // namespace
@@ -296,26 +334,24 @@ constexpr double kFewMaxFill = 0.9;
 bool few_rows(int64_t n_rows, int n_experts, int block_m, int64_t n, bool gate_up) {
   if (block_m == kMfmaBigBM) return false;
   if (n_rows > (n_experts == 1 ? (int64_t)kFewDenseRows : (int64_t)kFewRowsPerExpert * n_experts)) return false;
-  // experts that meet a row, expected under even routing
-  const double live = n_experts * (1.0 - std::pow(1.0 - 1.0 / n_experts, (double)n_rows));
-  const double rounds = live * (double)ceil_div(n, gate_up ? 128 : 256) / cu_count();
-  return rounds < kFewMaxFill * std::ceil(rounds);
+  return fill(live_experts(n_rows, n_experts) * (double)ceil_div(n, gate_up ? 128 : 256)) < kFewMaxFill;
 }
 
 int launch_few_gate_up(const void* x, const int32_t* row_src, const int32_t* tiles, int64_t capacity,
-                       const void* const* w_gate, const void* const* w_up, int64_t dim, int64_t dim_ffn, bool packed,
-                       void* h, hipStream_t s) {
-  if (packed) return launch_few<true, false, true>(x, tiles, capacity, w_gate, w_gate, nullptr, dim, dim_ffn, h, s, nullptr);
+                       const void* const* w_gate, const void* const* w_up, int64_t n_rows, int n_experts, int64_t dim,
+                       int64_t dim_ffn, bool packed, void* h, hipStream_t s) {
+  if (packed) return launch_few<true, false, true>(x, tiles, capacity, w_gate, w_gate, nullptr, n_rows, n_experts, dim, dim_ffn, h, s, nullptr);
   if (row_src != nullptr)
-    return launch_few<true, true, false>(x, tiles, capacity, w_gate, w_up, nullptr, dim, dim_ffn, h, s, row_src);
-  return launch_few<true, false, false>(x, tiles, capacity, w_gate, w_up, nullptr, dim, dim_ffn, h, s, nullptr);
+    return launch_few<true, true, false>(x, tiles, capacity, w_gate, w_up, nullptr, n_rows, n_experts, dim, dim_ffn, h, s, row_src);
+  return launch_few<true, false, false>(x, tiles, capacity, w_gate, w_up, nullptr, n_rows, n_experts, dim, dim_ffn, h, s, nullptr);
 }
 
 int launch_few_down(const void* h, const int32_t* tiles, int64_t capacity, const void* const* w_down,
-                    const void* sorted_w, int64_t dim_ffn, int64_t dim, bool packed, void* y, hipStream_t s) {
+                    const void* sorted_w, int64_t n_rows, int n_experts, int64_t dim_ffn, int64_t dim, bool packed,
+                    void* y, hipStream_t s) {
   if (packed)
-    return launch_few<false, false, true>(h, tiles, capacity, w_down, w_down, sorted_w, dim_ffn, dim, y, s, nullptr);
-  return launch_few<false, false, false>(h, tiles, capacity, w_down, w_down, sorted_w, dim_ffn, dim, y, s, nullptr);
+    return launch_few<false, false, true>(h, tiles, capacity, w_down, w_down, sorted_w, n_rows, n_experts, dim_ffn, dim, y, s, nullptr);
+  return launch_few<false, false, false>(h, tiles, capacity, w_down, w_down, sorted_w, n_rows, n_experts, dim_ffn, dim, y, s, nullptr);
 }
 
 }  // namespace astrai_moe
