@@ -106,9 +106,10 @@ int launch_mfma_gate_up_gather(const void* x, const int32_t* sorted_token,
                         const GemmWorkspace& ws = {});
 
 // Few rows (moe_gemm_few.hip), tiles below 256 rows: whether the kernels there
-// take a GEMM of n_rows rows over n_experts experts with n output columns, and the GEMMs (row_src: the
+// take a GEMM of n_rows rows over n_experts experts with k inputs
+// and n output columns, and the GEMMs (row_src: the
 // gathered rows' tokens, or null; packed: the tables hold packed copies).
-bool few_rows(int64_t n_rows, int n_experts, int block_m, int64_t n,
+bool few_rows(int64_t n_rows, int n_experts, int block_m, int64_t k, int64_t n,
               bool gate_up);
 int launch_few_gate_up(const void* x, const int32_t* row_src,
                        const int32_t* tiles, int64_t capacity,

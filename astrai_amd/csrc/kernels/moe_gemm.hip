@@ -203,7 +203,7 @@ extern "C" int astrai_moe_gemm_gate_up(const void* x_perm, const int32_t* tiles,
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (dtype == ASTRAI_MOE_BF16) {
     const bool mfma = mfma_gate_up_supported(dim, dim_ffn, block_m, x_perm, h);
-    if (mfma && few_rows(n_rows, n_experts, block_m, dim_ffn, true))
+    if (mfma && few_rows(n_rows, n_experts, block_m, dim, dim_ffn, true))
       return launch_few_gate_up(x_perm, nullptr, tiles, capacity, w_gate, w_up, n_rows, n_experts, dim, dim_ffn, false, h, s);
     if (mfma)
       return launch_mfma_gate_up(x_perm, tiles, capacity, w_gate, w_up, dim,
@@ -239,7 +239,7 @@ extern "C" int astrai_moe_gemm_gate_up_gather(const void* x, const int32_t* sort
                  (long long)dim, (long long)dim_ffn, block_m);
   ASTRAI_REQUIRE(sorted_token && w_gate && w_up, "gemm_gate_up_gather: null row list or weight table");
   const int64_t capacity = (tiles_len - ASTRAI_MOE_TILE_HEADER) / ASTRAI_MOE_TILE_STRIDE;
-  if (few_rows(n_rows, n_experts, block_m, dim_ffn, true))
+  if (few_rows(n_rows, n_experts, block_m, dim, dim_ffn, true))
     return launch_few_gate_up(x, sorted_token, tiles, capacity, w_gate, w_up, n_rows, n_experts, dim, dim_ffn, false, h,
                               static_cast<hipStream_t>(stream));
   return launch_mfma_gate_up_gather(x, sorted_token, tiles, capacity, w_gate, w_up, dim, dim_ffn, block_m, h,
@@ -265,7 +265,7 @@ extern "C" int astrai_moe_gemm_down(const void* h, const int32_t* tiles,
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (dtype == ASTRAI_MOE_BF16) {
     const bool mfma = mfma_down_supported(dim_ffn, dim, block_m, h, y);
-    if (mfma && few_rows(n_rows, n_experts, block_m, dim, false))
+    if (mfma && few_rows(n_rows, n_experts, block_m, dim_ffn, dim, false))
       return launch_few_down(h, tiles, capacity, w_down, sorted_w, n_rows, n_experts, dim_ffn, dim, false, y, s);
     if (mfma)
       return launch_mfma_down(h, tiles, capacity, w_down, sorted_w, dim_ffn,
@@ -328,7 +328,7 @@ extern "C" int astrai_moe_gemm_gate_up_packed(const void* x_perm, const int32_t*
   if (n_rows == 0) return ASTRAI_MOE_OK;
   ASTRAI_REQUIRE(w_packed, "gemm_gate_up_packed: null weight table");
   const int64_t capacity = (tiles_len - ASTRAI_MOE_TILE_HEADER) / ASTRAI_MOE_TILE_STRIDE;
-  if (few_rows(n_rows, n_experts, block_m, dim_ffn, true))
+  if (few_rows(n_rows, n_experts, block_m, dim, dim_ffn, true))
     return launch_few_gate_up(x_perm, nullptr, tiles, capacity, w_packed, w_packed, n_rows, n_experts, dim, dim_ffn, true, h,
                               static_cast<hipStream_t>(stream));
   return launch_mfma_gate_up(x_perm, tiles, capacity, w_packed, w_packed, dim, dim_ffn, block_m, true, h,
@@ -352,7 +352,7 @@ extern "C" int astrai_moe_gemm_down_packed(const void* h, const int32_t* tiles, 
   if (n_rows == 0) return ASTRAI_MOE_OK;
   ASTRAI_REQUIRE(w_packed, "gemm_down_packed: null weight table");
   const int64_t capacity = (tiles_len - ASTRAI_MOE_TILE_HEADER) / ASTRAI_MOE_TILE_STRIDE;
-  if (few_rows(n_rows, n_experts, block_m, dim, false))
+  if (few_rows(n_rows, n_experts, block_m, dim_ffn, dim, false))
     return launch_few_down(h, tiles, capacity, w_packed, sorted_w, n_rows, n_experts, dim_ffn, dim, true, y,
                            static_cast<hipStream_t>(stream));
   return launch_mfma_down(h, tiles, capacity, w_packed, sorted_w, dim_ffn, dim, block_m, true, y,

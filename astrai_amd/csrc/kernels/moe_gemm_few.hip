@@ -31,15 +31,17 @@
 namespace astrai_moe {
 namespace {
 
-template <int BN_>
+template <int BM_, int BN_>
 struct FewCfg {
-  static constexpr int BM = 32, BN = BN_, WAVES = 4, STAGES = BN == 32 ? 4 : 6;
-  static constexpr int NC = BN / 16;  // 16-column blocks
+  static constexpr int BM = BM_, BN = BN_, WAVES = 4, STAGES = BM == 64 ? 3 : BN == 32 ? 4 : 6;
+  static constexpr int NR = BM / 16, NC = BN / 16;  // 16-row and 16-column blocks
   static constexpr int A_BYTES = BM * kRowBytes, B_BYTES = BN * kRowBytes, STAGE = A_BYTES + B_BYTES;
   static constexpr int OPS = STAGE / 1024;                     // DMA ops per wave and step
-  static constexpr int RED_WAVE = BM * BN * 4;                 // one wave's fp32 sums
+  static constexpr int RED_ROWS = 32;                          // rows whose sums meet at a time
+  static constexpr int RED_WAVE = RED_ROWS * BN * 4;           // one wave's fp32 sums of these
   static constexpr int RED_OFF = WAVES * STAGES * STAGE;       // 128 or 144 KB of rings
-  static constexpr int LDS = RED_OFF + 2 * WAVES * RED_WAVE;   // 160 KB
+  static constexpr int RED_BUFS = BM == 64 ? 1 : 2;            // places they meet in
+  static constexpr int LDS = RED_OFF + RED_BUFS * WAVES * RED_WAVE;  // 160 KB
   static_assert(LDS <= 160 * 1024, "LDS");
   static_assert(OPS * (STAGES - 1) <= 63, "vmcnt range");
 };
@@ -152,7 +154,7 @@ __global__ __launch_bounds__(Cfg::WAVES * 64, 1) void gemm_few_kernel(
     const bf16_t* __restrict__ A, const int32_t* __restrict__ tiles, const void* const* __restrict__ W0,
     const void* const* __restrict__ W1, const bf16_t* __restrict__ row_w, int K, int N, int n_cols, int capacity,
     bf16_t* __restrict__ C, const int32_t* __restrict__ row_src) {
-  constexpr int NC = Cfg::NC;
+  constexpr int NR = Cfg::NR, NC = Cfg::NC;
   __shared__ __attribute__((aligned(1024))) char smem[Cfg::LDS];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -187,20 +189,20 @@ __global__ __launch_bounds__(Cfg::WAVES * 64, 1) void gemm_few_kernel(
     const int row0 = load_scalar(ti + 1);
     const int rows = min(load_scalar(tiles + 1), load_scalar(ti + 2) - row0);
     for (int r0 = 0; r0 < rows; r0 += Cfg::BM) {
-      f32x4_t acc[2][NC];
+      f32x4_t acc[NR][NC];
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+      for (int i = 0; i < NR; ++i)
 #pragma unroll
         for (int c = 0; c < NC; ++c) acc[i][c] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
       for (int step = 0; step < n_steps; ++step) {
         wait_groups<Cfg::OPS, Cfg::STAGES - 1>(issued - used - 1);  // this step has landed
         const char* sa = ring + (used % Cfg::STAGES) * Cfg::STAGE + frag_row * kRowBytes;
-        bf16x8_t fa[2][2], fb[2][NC];
+        bf16x8_t fa[2][NR], fb[2][NC];
 #pragma unroll
         for (int kh = 0; kh < 2; ++kh) {
           const int chunk = ((kh * 4 + fq) ^ fsw) << 4;
 #pragma unroll
-          for (int i = 0; i < 2; ++i)
+          for (int i = 0; i < NR; ++i)
             fa[kh][i] = *reinterpret_cast<const bf16x8_t*>(sa + i * 16 * kRowBytes + chunk);
 #pragma unroll
           for (int c = 0; c < NC; ++c)
@@ -215,12 +217,17 @@ __global__ __launch_bounds__(Cfg::WAVES * 64, 1) void gemm_few_kernel(
 #pragma unroll
         for (int kh = 0; kh < 2; ++kh)
 #pragma unroll
-          for (int i = 0; i < 2; ++i)
+          for (int i = 0; i < NR; ++i)
 #pragma unroll
             for (int c = 0; c < NC; ++c)
               acc[i][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[kh][c], fa[kh][i], acc[i][c], 0, 0, 0);
       }
-      // the waves' sums meet: row r's 16-byte piece c at piece c ^ (r % pieces)
+      // the waves' sums meet, 32 rows at a time: row r's 16-byte piece c at piece
+      // c ^ (r % pieces)
+      static_for<Cfg::BM / Cfg::RED_ROWS>([&](auto half) {
+      constexpr int i0 = decltype(half)::value * 2;  // the first of these rows' two 16-row blocks
+      const int rh = r0 + i0 * 16;
+      if (rh >= rows) return;
       constexpr int PIECES = Cfg::BN / 4, ROW = Cfg::BN * 4;
       char* const red = smem + Cfg::RED_OFF + parity * (Cfg::WAVES * Cfg::RED_WAVE);
 #pragma unroll
@@ -229,7 +236,7 @@ __global__ __launch_bounds__(Cfg::WAVES * 64, 1) void gemm_few_kernel(
         for (int c = 0; c < NC; ++c) {
           const int r = i * 16 + frag_row;
           *reinterpret_cast<f32x4_t*>(red + wave * Cfg::RED_WAVE + r * ROW +
-                                      (((c * 4 + fq) ^ (r & (PIECES - 1))) << 4)) = acc[i][c];
+                                      (((c * 4 + fq) ^ (r & (PIECES - 1))) << 4)) = acc[i0 + i][c];
         }
       asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
       auto sum = [&](int r, int piece) {
@@ -242,7 +249,7 @@ __global__ __launch_bounds__(Cfg::WAVES * 64, 1) void gemm_few_kernel(
       if constexpr (kGateUp) {
         constexpr int HP = PIECES / 2;  // pieces of the gate columns, then of the up columns
         const int r = threadIdx.x / HP, p = threadIdx.x % HP, n = nt * (Cfg::BN / 2) + p * 4;
-        if (r < Cfg::BM && r0 + r < rows && n < N) {
+        if (r < Cfg::RED_ROWS && rh + r < rows && n < N) {
           const f32x4_t g4 = sum(r, p), u4 = sum(r, HP + p);
           bf16x4_t o;
 #pragma unroll
@@ -251,12 +258,12 @@ __global__ __launch_bounds__(Cfg::WAVES * 64, 1) void gemm_few_kernel(
             const float ex = __builtin_amdgcn_exp2f(g * -1.4426950408889634f);
             o[q] = (__bf16)(u * (float)(__bf16)(g * __builtin_amdgcn_rcpf(1.0f + ex)));
           }
-          *reinterpret_cast<bf16x4_t*>(C + (int64_t)(row0 + r0 + r) * N + n) = o;
+          *reinterpret_cast<bf16x4_t*>(C + (int64_t)(row0 + rh + r) * N + n) = o;
         }
       } else {
         const int r = threadIdx.x / PIECES, p = threadIdx.x % PIECES, n = nt * Cfg::BN + p * 4;
-        if (r < Cfg::BM && r0 + r < rows && n < N) {
-          const int64_t row = row0 + r0 + r;
+        if (r < Cfg::RED_ROWS && rh + r < rows && n < N) {
+          const int64_t row = row0 + rh + r;
           const f32x4_t y4 = sum(r, p);
           const float w = row_w != nullptr ? bf16_bits_to_f32(row_w[row]) : 1.0f;
           bf16x4_t o;
@@ -265,7 +272,11 @@ __global__ __launch_bounds__(Cfg::WAVES * 64, 1) void gemm_few_kernel(
           *reinterpret_cast<bf16x4_t*>(C + row * N + n) = o;
         }
       }
-      parity ^= 1;
+      if constexpr (Cfg::RED_BUFS == 2)
+        parity ^= 1;
+      else  // the next sums go to the same place
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      });
     }
   }
 }
@@ -295,6 +306,14 @@ double fill(double tiles) {
   return rounds / std::ceil(rounds);
 }
 
+// Limits of few_rows (below), which has the figures.
+constexpr int kFewRowsPerExpert = 24, kFewDenseRows = 128, kFewLongSteps = 12;
+constexpr double kFewMaxFill = 0.9;
+
+// Tiles of 64 activation rows where most experts, or more than two runs of 32
+// of one expert, have more than 32 rows (MLP of D 4096, F 14336: 96 rows 197 ->
+// 149 us, 64 rows 133 -> 138).
+//
 // One expert's single run of 32 rows (an MLP decoding) takes tiles of 16 weight
 // rows where those fill the rounds of tiles better: D 4096, F 14336, 24 rows,
 // gate/up 3.5 rounds of 32-row tiles or 7 of 16, down half a round or one, 100
@@ -306,35 +325,45 @@ template <bool kGateUp, bool kGather, bool kPacked>
 int launch_few(const void* A, const int32_t* tiles, int64_t capacity, const void* const* W0, const void* const* W1,
                const void* row_w, int64_t n_rows, int n_experts, int64_t K, int64_t N, void* C, hipStream_t s,
                const int32_t* row_src) {
-  if (n_experts == 1 && n_rows <= FewCfg<16>::BM &&
+  if (n_rows > (n_experts == 1 ? 2 * FewCfg<32, 32>::BM : (int64_t)kFewRowsPerExpert * n_experts))
+    return launch_few_cfg<FewCfg<64, 32>, kGateUp, kGather, kPacked>(A, tiles, capacity, W0, W1, row_w, K, N, C, s,
+                                                                     row_src);
+  if (n_experts == 1 && n_rows <= FewCfg<32, 16>::BM &&
       fill((double)ceil_div(N, kGateUp ? 8 : 16)) > 1.05 * fill((double)ceil_div(N, kGateUp ? 16 : 32)))
-    return launch_few_cfg<FewCfg<16>, kGateUp, kGather, kPacked>(A, tiles, capacity, W0, W1, row_w, K, N, C, s, row_src);
-  return launch_few_cfg<FewCfg<32>, kGateUp, kGather, kPacked>(A, tiles, capacity, W0, W1, row_w, K, N, C, s, row_src);
+    return launch_few_cfg<FewCfg<32, 16>, kGateUp, kGather, kPacked>(A, tiles, capacity, W0, W1, row_w, K, N, C, s, row_src);
+  return launch_few_cfg<FewCfg<32, 32>, kGateUp, kGather, kPacked>(A, tiles, capacity, W0, W1, row_w, K, N, C, s, row_src);
 }
 
 }  // namespace
 
-// Where these kernels replace the 256-column tiles of moe_gemm_mfma.hip: up to
-// kFewRowsPerExpert rows per expert (above, experts of more than 32 rows read
-// their weights in two runs), or kFewDenseRows of one expert, whose rows are
-// known; and where the other kernel's last round of tiles would leave more
-// than a tenth of its compute-unit time idle. The same for tiles of 32, 64 and
-// 128 rows, so that these give the same bits; lists of 256-row tiles keep their
-// kernels, whose bits the training forward shares. Measured, us per layer or MLP without and
-// with (replayed from a graph, three sets of weights in turn):
+// Where these kernels replace the 256-column tiles of moe_gemm_mfma.hip:
+// - up to kFewRowsPerExpert rows per expert (above, experts of more than 32 rows
+//   read their weights in two runs), or kFewDenseRows of one expert, whose rows
+//   are known, where the other kernel's last round of tiles would leave more
+//   than a tenth of its compute-unit time idle;
+// - up to twice as many where its tiles occupy at most half the compute units
+//   and are long, kFewLongSteps K steps or more (16 experts, top-4 and a shared
+//   one, D 704, F 576, 9 and 11 steps, 160 tokens: 47.9 / 49.8).
+// The same for tiles of 32, 64 and 128 rows, so that these give the same bits;
+// lists of 256-row tiles keep their kernels, whose bits the training forward
+// shares. Measured, us per layer or MLP without and with (replayed from a
+// graph, three sets of weights in turn):
 // - 8 experts, top-2, D 4096, F 14336: 1 token 264 / 165, 2 368 / 286, 8 532 /
 //   495, 64 593 / 552, 96 (24 rows per expert) 602 / 590, 128 608 / 716;
 // - 64 experts, top-6, D 2048, F 1408: 1 token 74 / 60, 8 158 / 144, 32 226 /
 //   224, 64 (rounds of 0.92 and 1.0, past the line) 232 / 233;
-// - MLP, D 4096, F 14336: 1 token 201 / 92, 24 217 / 100, 96 223 / 197, 128
-//   234 / 228, 160 256 / 289; D 2048, F 5632: 24 66 / 29, 128 72 / 56.
-constexpr int kFewRowsPerExpert = 24, kFewDenseRows = 128;
-constexpr double kFewMaxFill = 0.9;
-
-bool few_rows(int64_t n_rows, int n_experts, int block_m, int64_t n, bool gate_up) {
+// - 8 experts, top-2 and a shared one, D 1000, F 2664, 96 tokens (32 rows per
+//   expert; the down GEMM has 36 tiles) 120 / 97, 160 127 / 109;
+// - MLP, D 4096, F 14336: 1 token 201 / 81, 24 217 / 90, 64 214 / 133, 128 235 /
+//   156, 256 (the down GEMM; its gate/up GEMM has 448 tiles) 255 / 191; D 2048, F
+//   5632: 24 66 / 28, 128 72 / 43, 256 73 / 44.
+bool few_rows(int64_t n_rows, int n_experts, int block_m, int64_t k, int64_t n, bool gate_up) {
   if (block_m == kMfmaBigBM) return false;
-  if (n_rows > (n_experts == 1 ? (int64_t)kFewDenseRows : (int64_t)kFewRowsPerExpert * n_experts)) return false;
-  return fill(live_experts(n_rows, n_experts) * (double)ceil_div(n, gate_up ? 128 : 256)) < kFewMaxFill;
+  const int64_t most = n_experts == 1 ? kFewDenseRows : (int64_t)kFewRowsPerExpert * n_experts;
+  const double cols = (double)ceil_div(n, gate_up ? 128 : 256);
+  if (n_rows <= most) return fill(live_experts(n_rows, n_experts) * cols) < kFewMaxFill;
+  const double row_tiles = n_experts == 1 ? (double)ceil_div(n_rows, kMfmaMidBM) : (double)n_experts;
+  return n_rows <= 2 * most && k_steps(k) >= kFewLongSteps && 2 * row_tiles * cols <= cu_count();
 }
 
 int launch_few_gate_up(const void* x, const int32_t* row_src, const int32_t* tiles, int64_t capacity,

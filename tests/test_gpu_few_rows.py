@@ -16,7 +16,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("dim,dim_ffn", [(64, 64), (72, 328), (512, 1408), (1096, 200)])
-@pytest.mark.parametrize("n_tok", [1, 16, 32, 33, 95, 128])
+@pytest.mark.parametrize("n_tok", [1, 16, 32, 33, 95, 128, 160, 256])
 def test_mlp(gpu, n_tok, dim, dim_ffn):
     torch.manual_seed(n_tok + dim)
     mlp = MLP(dim, dim_ffn)
@@ -30,7 +30,7 @@ def test_mlp(gpu, n_tok, dim, dim_ffn):
     torch.testing.assert_close(got, want, rtol=2e-2, atol=2e-3)
 
 
-@pytest.mark.parametrize("n_tok,n_exp,top_k,n_shared", [(1, 64, 6, 1), (5, 8, 2, 2), (47, 8, 2, 0), (12, 128, 8, 0)])
+@pytest.mark.parametrize("n_tok,n_exp,top_k,n_shared", [(1, 64, 6, 1), (5, 8, 2, 2), (47, 8, 2, 0), (12, 128, 8, 0), (150, 8, 2, 1)])
 def test_layer(gpu, n_tok, n_exp, top_k, n_shared):
     layer = _random_layer(gpu, 512, 640, n_exp, n_shared, top_k, torch.bfloat16, seed=n_exp).requires_grad_(False)
     x = torch.randn(1, n_tok, 512, device=gpu).to(torch.bfloat16)
