@@ -137,18 +137,19 @@ int launch_mfma_down_save(const void* h, const int32_t* tiles,
                           void* y, void* y_unweighted, hipStream_t s,
                           const GemmWorkspace& ws = {});
 
-// fp32 on the matrix cores (moe_gemm_mfma_f32.hip), 64-row tile lists, K a
-// multiple of 32, output columns a multiple of 32 (gate/up) or 64 (down),
-// 16-byte aligned operands. A non-null gu / y_unweighted selects the training
+// fp32 on the matrix cores (moe_gemm_mfma_f32.hip), 64-row tile lists, K and
+// the output columns multiples of 32, 16-byte aligned operands. A non-null gu / y_unweighted selects the training
 // forward, which also stores the gate and up projections (blocked layout of
-// gu_index) or the output before the routing weight.
+// gu_index) or the output before the routing weight. row_src (inference only):
+// x_perm is x and row r is x[row_src[r]] (x under 4 GiB).
 bool mfma_f32_supported(int64_t k, int64_t n, bool gate_up, int block_m,
                         const void* a, const void* c, const void* s0);
 int launch_mfma_f32_gate_up(const void* x_perm, const int32_t* tiles,
                             int64_t capacity, const void* const* w_gate,
                             const void* const* w_up, int64_t n_rows,
                             int n_experts, int64_t dim, int64_t dim_ffn,
-                            void* h, void* gu, hipStream_t s);
+                            void* h, void* gu, hipStream_t s,
+                            const int32_t* row_src = nullptr);
 int launch_mfma_f32_down(const void* h, const int32_t* tiles, int64_t capacity,
                          const void* const* w_down, const void* sorted_w,
                          int64_t n_rows, int n_experts, int64_t dim_ffn,

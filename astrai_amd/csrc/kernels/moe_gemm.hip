@@ -19,7 +19,7 @@
 //   * gemm_mfma_* (moe_gemm_mfma.hip): bf16 on CDNA4 matrix cores, used when
 //     the shapes meet its tiling constraints.
 //   * gemm_f32_mfma_kernel (moe_gemm_mfma_f32.hip): fp32 on CDNA4 matrix
-//     cores (v_mfma_f32_16x16x4_f32), 64-row tiles, K a multiple of 32.
+//     cores (v_mfma_f32_16x16x4_f32), 64-row tiles, dims multiples of 32.
 //   * gemm_generic_kernel (here): any shape, fp32 or bf16, fp32 FMA; 64x64
 //     output tiles walked over the row tile in 64-row steps. Used for the
 //     shapes neither matrix-core kernel tiles.

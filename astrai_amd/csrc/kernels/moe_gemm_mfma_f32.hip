@@ -21,8 +21,14 @@
 // BN = 64 weight rows per column tile (gate/up: 32 gate rows then the same 32
 // up rows), 4 waves of 32 x 32, three 16 KB stages in flight, so a compute
 // unit holds three workgroups and a wave waiting at its barrier leaves the
-// matrix core to the other two. The down GEMM takes BN = 32 when 64-wide
-// column tiles would leave most of those workgroup slots empty. The launch is
+// matrix core to the other two. The down GEMM takes BN = 32, four workgroups
+// per compute unit (us with 64 / 32 columns at D 512, F 1024, 8 experts, top-2:
+// 64 tokens 21.6 / 14.2, 1024 37.8 / 31.7, 2048 56.5 / 51.1; D 1024, F 2048,
+// 2048 tokens 182 / 175), and the gate/up GEMM (16 gate rows and 16 up rows)
+// where 64-wide column tiles would leave most workgroup slots empty (D 512, 64
+// tokens with a shared expert 21.4 / 18.1; with more tiles than that it is the
+// slower one, 2048 tokens 130 / 136). Bound by the matrix cores: busy for 79 %
+// of 2.15 GHz at D 1024, F 2048, 2048 tokens (107 of 157 TFLOP/s). The launch is
 // persistent, round r of workgroup b taking logical tile r * G + b: with
 // several workgroups per compute unit, the XCD-contiguous order of the bf16
 // kernels would put a partial last round on the first XCDs only, where this
@@ -42,9 +48,9 @@ namespace {
 constexpr int kF32BK = kRowBytes / 4;  // 32 floats per staged row piece
 constexpr int kF32BM = 64;
 
-template <int BN_>
+template <int BN_, int WGM_ = 2>
 struct F32Cfg {
-  static constexpr int BM = kF32BM, BN = BN_, STAGES = 3, WGM = 2, WGN = 2;
+  static constexpr int BM = kF32BM, BN = BN_, STAGES = 3, WGM = WGM_, WGN = 4 / WGM_;
   static constexpr int WAVES = WGM * WGN;
   static constexpr int THREADS = WAVES * 64;
   static constexpr int WM = BM / WGM;
@@ -64,12 +70,12 @@ struct F32Cfg {
   static_assert(DMA_PER_WAVE * (STAGES - 1) <= 63, "vmcnt range");
 };
 
-template <int BN, bool kGateUp, bool kSave>
+template <int BN, bool kGateUp, bool kSave, bool kGather>
 __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(
     const float* __restrict__ A, const int32_t* __restrict__ tiles, const void* const* __restrict__ W0,
     const void* const* __restrict__ W1, const float* __restrict__ row_w, int K, int N, int n_tiles_n, int capacity,
-    float* __restrict__ C, float* __restrict__ S0) {
-  using Cfg = F32Cfg<BN>;
+    float* __restrict__ C, float* __restrict__ S0, const int32_t* __restrict__ row_src) {
+  using Cfg = F32Cfg<BN, (kGateUp && BN == 32) ? 4 : 2>;
   static_assert(!kGateUp || Cfg::WN % 32 == 0, "gate/up halves of 16 columns");
   constexpr int S = Cfg::STAGES;
   constexpr int DPW = Cfg::DMA_PER_WAVE;
@@ -92,12 +98,18 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(
   const char* b_base0 = nullptr;
   const char* b_base1 = nullptr;
   int row0 = 0, rows = 0;
+  uint32_t a_off[Cfg::A_PER_WAVE];  // kGather: byte offsets in x of the rows the lane loads
   auto setup_tile = [&](int mt_, int nt_) {
     const int32_t* ti = tiles + ASTRAI_MOE_TILE_HEADER + (int64_t)mt_ * ASTRAI_MOE_TILE_STRIDE;
     const int e = ti[0];
     row0 = ti[1];
     rows = min(Cfg::BM, ti[2] - row0);
-    a_base = reinterpret_cast<const char*>(A + (int64_t)row0 * K);
+    a_base = reinterpret_cast<const char*>(kGather ? A : A + (int64_t)row0 * K);
+    if constexpr (kGather) {
+#pragma unroll
+      for (int i = 0; i < Cfg::A_PER_WAVE; ++i)
+        a_off[i] = (uint32_t)row_src[row0 + min((wave * Cfg::A_PER_WAVE + i) * 8 + (lane >> 3), rows - 1)] * k4;
+    }
     b_base0 = reinterpret_cast<const char*>(static_cast<const float*>(W0[e]) +
                                             (int64_t)nt_ * (kGateUp ? BN / 2 : BN) * K);
     b_base1 = kGateUp ? reinterpret_cast<const char*>(static_cast<const float*>(W1[e]) + (int64_t)nt_ * (BN / 2) * K)
@@ -111,8 +123,8 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(
 #pragma unroll
     for (int i = 0; i < Cfg::A_PER_WAVE; ++i) {
       const int q = wave * Cfg::A_PER_WAVE + i;
-      const uint32_t row = (uint32_t)min(q * 8 + dl.row, rows - 1);
-      lds_dma_16(a_base + (row * k4 + dl.chunk(q)), sa + q * 1024);
+      const uint32_t off = kGather ? a_off[i] : (uint32_t)min(q * 8 + dl.row, rows - 1) * k4;
+      lds_dma_16(a_base + (off + dl.chunk(q)), sa + q * 1024);
     }
 #pragma unroll
     for (int i = 0; i < Cfg::B_PER_WAVE; ++i) {
@@ -130,9 +142,9 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(
   const int frag_row = lane & 15;
   const int fq = lane >> 4;
   const int fsw = (frag_row >> 1) & 7;  // row bases are multiples of 16
-  int a_off[MT16];
+  int fa_off[MT16];
 #pragma unroll
-  for (int i = 0; i < MT16; ++i) a_off[i] = (wm * Cfg::WM + i * 16 + frag_row) * kRowBytes;
+  for (int i = 0; i < MT16; ++i) fa_off[i] = (wm * Cfg::WM + i * 16 + frag_row) * kRowBytes;
   int b_off[NT16];
 #pragma unroll
   for (int j = 0; j < NT16; ++j) {
@@ -151,7 +163,7 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(
     const char* sb = sa + Cfg::A_BYTES;
     const int sw = ((kh * 4 + fq) ^ fsw) << 4;
 #pragma unroll
-    for (int i = 0; i < MT16; ++i) fa[slot][i] = *reinterpret_cast<const f32x4_t*>(sa + a_off[i] + sw);
+    for (int i = 0; i < MT16; ++i) fa[slot][i] = *reinterpret_cast<const f32x4_t*>(sa + fa_off[i] + sw);
 #pragma unroll
     for (int j = 0; j < NT16; ++j) fb[slot][j] = *reinterpret_cast<const f32x4_t*>(sb + b_off[j] + sw);
   };
@@ -183,23 +195,26 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(
     lds_barrier();
     read_frags(0, 0, 0);
     int buf = 0;
-    for (int kt = 0; kt < KT; ++kt) {
+    // (the last step stands behind the loop: with it inside, the compiler waited
+    // for the next step's fragment reads before each step's second half)
+    for (int kt = 0; kt + 1 < KT; ++kt) {
       read_frags(buf, 1, 1);
       mfmas(0);
       const int nbuf = (buf + 1 == S) ? 0 : buf + 1;
-      if (kt + 1 < KT) {
-        wait_groups<DPW, S - 2>(min(S - 2, KT - 2 - kt));
-        __builtin_amdgcn_sched_barrier(0);
-        lds_barrier();  // step kt + 1 landed; every wave is done reading buffer `buf`
-        __builtin_amdgcn_sched_barrier(0);
-        read_frags(nbuf, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        if (kt + S < KT) issue_stage(kt + S, buf);
-        __builtin_amdgcn_sched_barrier(0);
-      }
+      wait_groups<DPW, S - 2>(min(S - 2, KT - 2 - kt));
+      __builtin_amdgcn_sched_barrier(0);
+      lds_barrier();  // step kt + 1 landed; every wave is done reading buffer `buf`
+      __builtin_amdgcn_sched_barrier(0);
+      read_frags(nbuf, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      if (kt + S < KT) issue_stage(kt + S, buf);
+      __builtin_amdgcn_sched_barrier(0);
       mfmas(1);
       buf = nbuf;
     }
+    read_frags(buf, 1, 1);
+    mfmas(0);
+    mfmas(1);
 
     // ---- epilogue: 16 contiguous bytes per lane and tile ----
 #pragma unroll
@@ -243,54 +258,63 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(
   }
 }
 
-template <int BN, bool kGateUp, bool kSave>
+template <int BN, bool kGateUp, bool kSave, bool kGather = false>
 int launch_f32_bn(const void* A, const int32_t* tiles, int64_t capacity, const void* const* W0,
                   const void* const* W1, const void* row_w, int64_t K, int64_t N, void* C, void* S0,
-                  hipStream_t s) {
+                  hipStream_t s, const int32_t* row_src = nullptr) {
   using Cfg = F32Cfg<BN>;
   const int64_t n_tiles_n = kGateUp ? N / (BN / 2) : N / BN;
   const int64_t total = capacity * n_tiles_n;
   if (total >= (1ll << 31))
     return fail(ASTRAI_MOE_EINVAL, "gemm: %lld tiles exceed the tile-index range", (long long)total);
   const int64_t grid = std::min<int64_t>(total, (int64_t)cu_count() * Cfg::PER_CU);
-  hipLaunchKernelGGL((gemm_f32_mfma_kernel<BN, kGateUp, kSave>), dim3((unsigned)grid), dim3(Cfg::THREADS), 0, s,
+  hipLaunchKernelGGL((gemm_f32_mfma_kernel<BN, kGateUp, kSave, kGather>), dim3((unsigned)grid), dim3(Cfg::THREADS), 0, s,
                      static_cast<const float*>(A), tiles, W0, W1, static_cast<const float*>(row_w), (int)K, (int)N,
-                     (int)n_tiles_n, (int)capacity, static_cast<float*>(C), static_cast<float*>(S0));
+                     (int)n_tiles_n, (int)capacity, static_cast<float*>(C), static_cast<float*>(S0), row_src);
   return check_launch(kGateUp ? "gemm_f32_mfma_kernel<gate_up>" : "gemm_f32_mfma_kernel<down>");
 }
 
 template <bool kGateUp, bool kSave>
 int launch_f32(const void* A, const int32_t* tiles, int64_t capacity, const void* const* W0, const void* const* W1,
                const void* row_w, int64_t n_rows, int n_experts, int64_t K, int64_t N, void* C, void* S0,
-               hipStream_t s) {
+               hipStream_t s, const int32_t* row_src = nullptr) {
   if (capacity == 0) return ASTRAI_MOE_OK;
   if constexpr (!kGateUp) {
-    // 32-wide down tiles when the 64-wide ones, estimated from the rows and
-    // the experts' partial last tiles, would not give every compute unit two
+    (void)n_rows, (void)n_experts, (void)row_src;
+    return launch_f32_bn<32, false, kSave>(A, tiles, capacity, W0, W1, row_w, K, N, C, S0, s);
+  } else {
+    // 32 weight rows (16 gate, 16 up) when 64-row tiles, estimated from the
+    // rows and the experts' partial last tiles, would not give every compute
+    // unit two
     const int64_t row_tiles = ceil_div(n_rows, kF32BM) + n_experts / 2;
-    if (row_tiles * (N / 64) < 2ll * cu_count())
-      return launch_f32_bn<32, false, kSave>(A, tiles, capacity, W0, W1, row_w, K, N, C, S0, s);
+    const bool narrow = row_tiles * (N / 32) < 2ll * cu_count();
+    if (row_src != nullptr) {
+      if constexpr (!kSave)
+        return narrow ? launch_f32_bn<32, true, false, true>(A, tiles, capacity, W0, W1, row_w, K, N, C, S0, s, row_src)
+                      : launch_f32_bn<64, true, false, true>(A, tiles, capacity, W0, W1, row_w, K, N, C, S0, s, row_src);
+    }
+    if (narrow) return launch_f32_bn<32, true, kSave>(A, tiles, capacity, W0, W1, row_w, K, N, C, S0, s);
+    return launch_f32_bn<64, true, kSave>(A, tiles, capacity, W0, W1, row_w, K, N, C, S0, s);
   }
-  return launch_f32_bn<64, kGateUp, kSave>(A, tiles, capacity, W0, W1, row_w, K, N, C, S0, s);
 }
 
 }  // namespace
 
 bool mfma_f32_supported(int64_t k, int64_t n, bool gate_up, int block_m, const void* a, const void* c,
                         const void* s0) {
-  const int64_t min_cols = gate_up ? 32 : 64;  // output columns of a column tile
-  return block_m == kF32BM && k > 0 && n > 0 && k % kF32BK == 0 && n % min_cols == 0 && k <= (1ll << 22) &&
+  (void)gate_up;
+  return block_m == kF32BM && k > 0 && n > 0 && k % kF32BK == 0 && n % 32 == 0 && k <= (1ll << 22) &&
          n <= (1ll << 22) && aligned16(a) && aligned16(c) && (s0 == nullptr || aligned16(s0));
 }
 
 int launch_mfma_f32_gate_up(const void* x_perm, const int32_t* tiles, int64_t capacity, const void* const* w_gate,
                             const void* const* w_up, int64_t n_rows, int n_experts, int64_t dim, int64_t dim_ffn,
-                            void* h, void* gu, hipStream_t s) {
+                            void* h, void* gu, hipStream_t s, const int32_t* row_src) {
   if (gu != nullptr)
     return launch_f32<true, true>(x_perm, tiles, capacity, w_gate, w_up, nullptr, n_rows, n_experts, dim, dim_ffn,
                                   h, gu, s);
   return launch_f32<true, false>(x_perm, tiles, capacity, w_gate, w_up, nullptr, n_rows, n_experts, dim, dim_ffn, h,
-                                 nullptr, s);
+                                 nullptr, s, row_src);
 }
 
 int launch_mfma_f32_down(const void* h, const int32_t* tiles, int64_t capacity, const void* const* w_down,

@@ -152,23 +152,26 @@ __global__ __launch_bounds__(256) void gemm_f32_dgrad_kernel(const float* __rest
     lds_barrier();
     read_frags(0, 0, 0);
     int buf = 0;
-    for (int kt = 0; kt < KT; ++kt) {
+    // (the last step stands behind the loop: with it inside, the compiler waited
+    // for the next step's fragment reads before each step's second half)
+    for (int kt = 0; kt + 1 < KT; ++kt) {
       read_frags(buf, 1, 1);
       mfmas(0);
       const int nbuf = (buf + 1 == S) ? 0 : buf + 1;
-      if (kt + 1 < KT) {
-        wait_groups<DPW, S - 2>(min(S - 2, KT - 2 - kt));
-        __builtin_amdgcn_sched_barrier(0);
-        lds_barrier();  // step kt + 1 landed; every wave is done reading buffer `buf`
-        __builtin_amdgcn_sched_barrier(0);
-        read_frags(nbuf, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        if (kt + S < KT) issue_stage(kt + S, buf);
-        __builtin_amdgcn_sched_barrier(0);
-      }
+      wait_groups<DPW, S - 2>(min(S - 2, KT - 2 - kt));
+      __builtin_amdgcn_sched_barrier(0);
+      lds_barrier();  // step kt + 1 landed; every wave is done reading buffer `buf`
+      __builtin_amdgcn_sched_barrier(0);
+      read_frags(nbuf, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      if (kt + S < KT) issue_stage(kt + S, buf);
+      __builtin_amdgcn_sched_barrier(0);
       mfmas(1);
       buf = nbuf;
     }
+    read_frags(buf, 1, 1);
+    mfmas(0);
+    mfmas(1);
 
     // ---- epilogue: row wave * 16 + c, columns 16 g + 4 r .. + 3 ----
     const int rr = wave * 16 + c;
@@ -211,19 +214,32 @@ __global__ __launch_bounds__(256) void gemm_f32_dgrad_kernel(const float* __rest
 
 // ---------------------------------------------------------------------------
 // wgrad: dw[e] [M, N] = a[rows_e]^T . b[rows_e] for every expert with rows,
-// 128 x 128 tiles, 4 waves of 64 x 64, K = the expert's rows in steps of 32
-// (rows past the expert's last read zeros); three 32 KB stages, one
-// workgroup per CU, persistent over (expert, M tile, N tile).
+// 64 x 64 tiles, 4 waves of 32 x 32, K = the expert's rows in steps of 32 (rows
+// past the expert's last read zeros); three 16 KB stages, three workgroups per
+// CU, persistent over (expert, M tile, N tile).
+//
+// Operand reads: for MFMA step s of a 16-K half, lane (g = l / 16, c = l % 16)
+// reads K-row 4 g + s, columns 2 c and 2 c + 1 of its wave's 32 (8 bytes; a
+// 16-lane group covers 128 contiguous bytes). Value q feeds the MFMAs of block
+// q, whose local column c is column 2 c + q. Output (b as the first operand):
+// element r of blocks (qa, qb) is row 2 c + qa, column 2 (4 g + r) + qb, so a
+// lane holds 8 consecutive columns per row.
+//
+// Bound by the matrix cores once enough tiles are in flight: 128 x 128 tiles
+// with one 4-wave workgroup per CU left them waiting on every barrier, and gave
+// one shared expert of D 512, F 1024 32 workgroups. 1024 tokens over 8 experts
+// of that size, top-2: 74 -> 28 us a GEMM, the shared expert's 29 -> 23.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void gemm_f32_wgrad_kernel(const float* __restrict__ a,
                                                             const float* __restrict__ b,
                                                             const int32_t* __restrict__ offsets, int n_experts,
                                                             int M, int N, int n_tiles_m, int n_tiles_n,
                                                             float* __restrict__ dw) {
-  constexpr int OP_BYTES = kF32K * 512;  // 32 K-rows x 128 columns, per operand
+  typedef float f32x2_t __attribute__((ext_vector_type(2)));
+  constexpr int OP_BYTES = kF32K * 256;  // 32 K-rows x 64 columns, per operand
   constexpr int STAGE = 2 * OP_BYTES;
   constexpr int S = kF32Stages;
-  constexpr int DPW = 8;  // 4 ops per operand and wave
+  constexpr int DPW = 4;  // 2 ops per operand and wave
   __shared__ __attribute__((aligned(1024))) char smem[S * STAGE];
 
   const int per_e = n_tiles_m * n_tiles_n;
@@ -235,8 +251,8 @@ __global__ __launch_bounds__(256) void gemm_f32_wgrad_kernel(const float* __rest
 
   const int c = lane & 15;
   const int g = lane >> 4;
-  f32x4_t fa[2][4], fb[2][4];
-  f32x4_t acc[4][4];
+  f32x2_t fa[2][4], fb[2][4];
+  f32x4_t acc[2][2];
 
   for (int logical = (int)blockIdx.x; logical < total; logical += (int)gridDim.x) {
     const int e = logical / per_e;
@@ -248,16 +264,16 @@ __global__ __launch_bounds__(256) void gemm_f32_wgrad_kernel(const float* __rest
     const int KT = (rows + kF32K - 1) / kF32K;
     const char* a_base = reinterpret_cast<const char*>(a + (int64_t)r0 * M);
     const char* b_base = reinterpret_cast<const char*>(b + (int64_t)r0 * N);
-    const uint32_t acol0 = (uint32_t)mt * 512u, bcol0 = (uint32_t)nt * 512u;
+    const uint32_t acol0 = (uint32_t)mt * 256u, bcol0 = (uint32_t)nt * 256u;
 
     auto issue_stage = [&](int kstep, int buf) {
       char* sa = smem + buf * STAGE;
       char* sb = sa + OP_BYTES;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int o = wave * 4 + i;
-        dma_mn_f32<128>(a_base, kstep * kF32K, rows, m4, acol0, m4, lane, o, sa + o * 1024);
-        dma_mn_f32<128>(b_base, kstep * kF32K, rows, n4, bcol0, n4, lane, o, sb + o * 1024);
+      for (int i = 0; i < 2; ++i) {
+        const int o = wave * 2 + i;
+        dma_mn_f32<64>(a_base, kstep * kF32K, rows, m4, acol0, m4, lane, o, sa + o * 1024);
+        dma_mn_f32<64>(b_base, kstep * kF32K, rows, n4, bcol0, n4, lane, o, sb + o * 1024);
       }
     };
     auto read_frags = [&](int buf, int kh, int slot) {
@@ -266,17 +282,17 @@ __global__ __launch_bounds__(256) void gemm_f32_wgrad_kernel(const float* __rest
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
         const int krow = kh * 16 + 4 * g + s;
-        fa[slot][s] = *reinterpret_cast<const f32x4_t*>(sa + krow * 512 + wm * 256 + c * 16);
-        fb[slot][s] = *reinterpret_cast<const f32x4_t*>(sb + krow * 512 + wn * 256 + c * 16);
+        fa[slot][s] = *reinterpret_cast<const f32x2_t*>(sa + krow * 256 + wm * 128 + c * 8);
+        fb[slot][s] = *reinterpret_cast<const f32x2_t*>(sb + krow * 256 + wn * 128 + c * 8);
       }
     };
     auto mfmas = [&](int slot) {
 #pragma unroll
       for (int s = 0; s < 4; ++s)
 #pragma unroll
-        for (int qa = 0; qa < 4; ++qa)
+        for (int qa = 0; qa < 2; ++qa)
 #pragma unroll
-          for (int qb = 0; qb < 4; ++qb)
+          for (int qb = 0; qb < 2; ++qb)
             acc[qa][qb] =
                 __builtin_amdgcn_mfma_f32_16x16x4f32(fb[slot][s][qb], fa[slot][s][qa], acc[qa][qb], 0, 0, 0);
     };
@@ -285,42 +301,44 @@ __global__ __launch_bounds__(256) void gemm_f32_wgrad_kernel(const float* __rest
     for (int s = 0; s < S; ++s)
       if (s < KT) issue_stage(s, s);
 #pragma unroll
-    for (int qa = 0; qa < 4; ++qa)
+    for (int qa = 0; qa < 2; ++qa)
 #pragma unroll
-      for (int qb = 0; qb < 4; ++qb) acc[qa][qb] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+      for (int qb = 0; qb < 2; ++qb) acc[qa][qb] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
     wait_groups<DPW, S - 1>(min(S - 1, KT - 1));  // step 0 landed
     lds_barrier();
     read_frags(0, 0, 0);
     int buf = 0;
-    for (int kt = 0; kt < KT; ++kt) {
+    for (int kt = 0; kt + 1 < KT; ++kt) {
       read_frags(buf, 1, 1);
       mfmas(0);
       const int nbuf = (buf + 1 == S) ? 0 : buf + 1;
-      if (kt + 1 < KT) {
-        wait_groups<DPW, S - 2>(min(S - 2, KT - 2 - kt));
-        __builtin_amdgcn_sched_barrier(0);
-        lds_barrier();
-        __builtin_amdgcn_sched_barrier(0);
-        read_frags(nbuf, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        if (kt + S < KT) issue_stage(kt + S, buf);
-        __builtin_amdgcn_sched_barrier(0);
-      }
+      wait_groups<DPW, S - 2>(min(S - 2, KT - 2 - kt));
+      __builtin_amdgcn_sched_barrier(0);
+      lds_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      read_frags(nbuf, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      if (kt + S < KT) issue_stage(kt + S, buf);
+      __builtin_amdgcn_sched_barrier(0);
       mfmas(1);
       buf = nbuf;
     }
+    read_frags(buf, 1, 1);
+    mfmas(0);
+    mfmas(1);
 
-    // ---- epilogue: rows m = 4 c + qa, columns 16 g + 4 r .. + 3 of the wave's 64 x 64 ----
+    // ---- epilogue: rows 2 c + qa, columns 8 g .. + 7 of the wave's 32 x 32 ----
 #pragma unroll
-    for (int qa = 0; qa < 4; ++qa) {
-      const int m = mt * 128 + wm * 64 + 4 * c + qa;
+    for (int qa = 0; qa < 2; ++qa) {
+      const int m = mt * 64 + wm * 32 + 2 * c + qa;
       if (m >= M) continue;
       float* out = dw + ((int64_t)e * M + m) * N;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int n = nt * 128 + wn * 64 + 16 * g + 4 * r;
+      for (int h = 0; h < 2; ++h) {
+        const int n = nt * 64 + wn * 32 + 8 * g + 4 * h;
         if (n < N)  // N % 4 == 0
-          *reinterpret_cast<f32x4_t*>(out + n) = f32x4_t{acc[qa][0][r], acc[qa][1][r], acc[qa][2][r], acc[qa][3][r]};
+          *reinterpret_cast<f32x4_t*>(out + n) = f32x4_t{acc[qa][0][2 * h], acc[qa][1][2 * h], acc[qa][0][2 * h + 1],
+                                                         acc[qa][1][2 * h + 1]};
       }
     }
     lds_barrier();  // every wave is done with the stage buffers before the next tile's DMA
@@ -373,11 +391,11 @@ int launch_mfma_f32_dgrad_in(const void* d, const int32_t* tiles, int64_t capaci
 
 int launch_mfma_f32_wgrad(const void* a, const void* b, const int32_t* offsets, int n_experts, int64_t m, int64_t n,
                           void* dw, hipStream_t s) {
-  const int64_t n_tiles_m = ceil_div(m, 128), n_tiles_n = ceil_div(n, 128);
+  const int64_t n_tiles_m = ceil_div(m, 64), n_tiles_n = ceil_div(n, 64);
   const int64_t total = (int64_t)n_experts * n_tiles_m * n_tiles_n;
   if (total >= (1ll << 31))
     return fail(ASTRAI_MOE_EINVAL, "gemm_wgrad: %lld tiles exceed the tile-index range", (long long)total);
-  const int64_t grid = std::min<int64_t>(total, cu_count());  // one 96 KB workgroup per CU
+  const int64_t grid = std::min<int64_t>(total, 3ll * cu_count());  // three 48 KB workgroups per CU
   hipLaunchKernelGGL(gemm_f32_wgrad_kernel, dim3((unsigned)grid), dim3(256), 0, s, static_cast<const float*>(a),
                      static_cast<const float*>(b), offsets, n_experts, (int)m, (int)n, (int)n_tiles_m,
                      (int)n_tiles_n, static_cast<float*>(dw));

@@ -383,9 +383,9 @@ def moe_gemm_down(h: torch.Tensor, tiles: torch.Tensor, w_down: torch.Tensor, so
 
 def f32_matrix_cores(dim: int, dim_ffn: int, block_m: int, dtype: torch.dtype) -> bool:
     """Whether both fp32 GEMMs of this shape run on the matrix cores
-    (``gemm_f32_mfma_kernel``: 64-row tiles, dim and dim_ffn multiples of 32,
-    dim a multiple of 64 for the down GEMM's column tiles)."""
-    return (dtype == torch.float32 and block_m == 64 and dim % 64 == 0 and dim_ffn % 32 == 0
+    (``gemm_f32_mfma_kernel``: 64-row tiles, dim and dim_ffn multiples of
+    32)."""
+    return (dtype == torch.float32 and block_m == 64 and dim % 32 == 0 and dim_ffn % 32 == 0
             and 0 < dim <= 1 << 22 and 0 < dim_ffn <= 1 << 22)
 
 

@@ -201,7 +201,7 @@ int astrai_moe_dense_tiles(int64_t n_rows, int block_m, int32_t* tiles,
  * 8 (a partial last column tile clamps its weight rows and stores only the
  * columns inside the matrix);
  * fp32 runs on the matrix cores (v_mfma_f32_16x16x4_f32) with block_m = 64,
- * K a multiple of 32 and dim_ffn % 32 == 0 (gate/up) or dim % 64 == 0 (down);
+ * K a multiple of 32 and dim_ffn % 32 == 0 (gate/up) or dim % 32 == 0 (down);
  * every other case on a general fp32-FMA kernel. Weights whose rows are a
  * multiple of 16 bytes must start on a 16-byte boundary.
  */
