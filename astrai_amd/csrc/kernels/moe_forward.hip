@@ -130,11 +130,20 @@ extern "C" int astrai_moe_forward(const void* x, const void* logits, const void*
   void* const gws = p.gemm_ws_bytes > 0 ? base + p.gemm_ws : nullptr;
   hipStream_t s = static_cast<hipStream_t>(stream);
 
-  if ((rc = launch_route(logits, dtype, n_tokens, n_experts, top_k, n_shared, topk_idx, topk_w, hist, s))) return rc;
-  if ((rc = astrai_moe_permute(topk_idx, topk_w, hist, x, dtype, n_tokens, p.experts, p.slots, dim, p.block_m,
-                               i32(p.offsets), sorted_token, sorted_w, token_pos, x_perm, tiles, p.tiles_len,
-                               i32(p.chunk_base), stream)))
-    return rc;
+  // One chunk of tokens whose rows the GEMM reads itself: routing and
+  // permutation in one workgroup. (Rows to copy want the permutation's grid, more
+  // tokens its many workgroups.)
+  if (n_tokens <= ASTRAI_MOE_CHUNK_TOKENS && x_perm == nullptr) {
+    const RouteList list{sorted_token, sorted_w, token_pos, tiles,
+                         (p.tiles_len - ASTRAI_MOE_TILE_HEADER) / ASTRAI_MOE_TILE_STRIDE, p.block_m,
+                         dim >= kGroupTilesMinDim};
+    rc = launch_route_list(logits, dtype, n_tokens, n_experts, top_k, n_shared, list, s);
+  } else if ((rc = launch_route(logits, dtype, n_tokens, n_experts, top_k, n_shared, topk_idx, topk_w, hist, s)) == 0) {
+    rc = astrai_moe_permute(topk_idx, topk_w, hist, x, dtype, n_tokens, p.experts, p.slots, dim, p.block_m,
+                            i32(p.offsets), sorted_token, sorted_w, token_pos, x_perm, tiles, p.tiles_len,
+                            i32(p.chunk_base), stream);
+  }
+  if (rc) return rc;
   if (p.gather)
     rc = astrai_moe_gemm_gate_up_gather(x, sorted_token, n_tokens, tiles, p.tiles_len, w_gate, w_up, dtype, p.rows,
                                         p.experts, dim, dim_ffn, p.block_m, h, gws, p.gemm_ws_bytes, stream);

@@ -182,6 +182,22 @@ int launch_route(const void* logits, int dtype, int64_t n_tokens,
                  int n_experts, int top_k, int n_shared, int32_t* topk_idx,
                  void* topk_w, int32_t* chunk_hist, hipStream_t s);
 
+// The same for at most ASTRAI_MOE_CHUNK_TOKENS tokens, straight to what
+// astrai_moe_permute writes of the decisions (tiles of block_m >= 32 rows, the
+// grouped order's header where `group`); neither x_perm nor expert offsets.
+struct RouteList {
+  int32_t* sorted_token;
+  void* sorted_w;
+  int32_t* token_pos;
+  int32_t* tiles;
+  int64_t tile_capacity;
+  int block_m;
+  bool group;
+};
+int launch_route_list(const void* logits, int dtype, int64_t n_tokens,
+                      int n_experts, int top_k, int n_shared,
+                      const RouteList& list, hipStream_t s);
+
 // astrai_moe_combine with token_pos rows pos_stride >= top_k wide, of which
 // the first top_k are combined (moe_combine.hip).
 int launch_combine(const void* y, const int32_t* token_pos, const void* row_w,

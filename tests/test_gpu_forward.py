@@ -52,3 +52,18 @@ def test_arguments_are_checked_on_the_host():
     assert call(workspace=16) == -1 and "256-byte aligned" in loader.last_error()
     assert call(nbytes=100) == -1 and "needs" in loader.last_error()
     assert not ops.layer_forward_supported(8, 1, 32) and ops.layer_forward_supported(8, 1, 31)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n_exp,top_k", [(1, 1), (3, 2), (64, 6), (130, 32), (1000, 8)])
+@pytest.mark.parametrize("n_tok", [1, 31, 32, 33])
+def test_one_chunk_is_routed_and_listed_by_one_kernel(gpu, n_tok, n_exp, top_k, dtype):
+    # up to 32 tokens: the same bits as the separate route and permute kernels
+    # (zero rows among the tokens: every probability tied)
+    layer = _random_layer(gpu, 64, 64, n_exp, 0, top_k, dtype, seed=n_tok + n_exp).requires_grad_(False)
+    x = torch.randn(1, n_tok, 64, device=gpu).to(dtype)
+    x[0, ::5] = 0
+    st = layer._current(dtype, x.device)
+    for _ in range(2):
+        assert torch.equal(layer(x)[0], layer._routed_forward(x[0], st))
