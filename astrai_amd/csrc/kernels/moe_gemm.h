@@ -54,12 +54,13 @@ bool mfma_down_supported(int64_t dim_ffn, int64_t dim, int block_m,
 // (bf16, 256-row tiles of K / 64 contiguous 32 KB blocks in staged order).
 int launch_mfma_gate_up(const void* x_perm, const int32_t* tiles,
                         int64_t capacity, const void* const* w_gate,
-                        const void* const* w_up, int64_t dim, int64_t dim_ffn,
-                        int block_m, bool packed, void* h, hipStream_t s,
+                        const void* const* w_up, int64_t n_rows, int n_experts,
+                        int64_t dim, int64_t dim_ffn, int block_m, bool packed, void* h, hipStream_t s,
                         const GemmWorkspace& ws = {});
 int launch_mfma_down(const void* h, const int32_t* tiles, int64_t capacity,
                      const void* const* w_down, const void* sorted_w,
-                     int64_t dim_ffn, int64_t dim, int block_m, bool packed,
+                     int64_t n_rows, int n_experts, int64_t dim_ffn,
+                     int64_t dim, int block_m, bool packed,
                      void* y, hipStream_t s,
                      const GemmWorkspace& ws = {});
 
@@ -69,12 +70,13 @@ int launch_mfma_down(const void* h, const int32_t* tiles, int64_t capacity,
 namespace ragged {
 int launch_mfma_gate_up(const void* x_perm, const int32_t* tiles,
                         int64_t capacity, const void* const* w_gate,
-                        const void* const* w_up, int64_t dim, int64_t dim_ffn,
-                        int block_m, bool packed, void* h, hipStream_t s,
+                        const void* const* w_up, int64_t n_rows, int n_experts,
+                        int64_t dim, int64_t dim_ffn, int block_m, bool packed, void* h, hipStream_t s,
                         const GemmWorkspace& ws);
 int launch_mfma_down(const void* h, const int32_t* tiles, int64_t capacity,
                      const void* const* w_down, const void* sorted_w,
-                     int64_t dim_ffn, int64_t dim, int block_m, bool packed,
+                     int64_t n_rows, int n_experts, int64_t dim_ffn,
+                     int64_t dim, int block_m, bool packed,
                      void* y, hipStream_t s, const GemmWorkspace& ws);
 int launch_mfma_gate_up_save(const void* x_perm, const int32_t* tiles,
                              int64_t capacity, const void* const* w_gate,
@@ -100,10 +102,10 @@ int launch_dgrad_in(const void* d, const int32_t* tiles, int64_t capacity,
 int launch_mfma_gate_up_gather(const void* x, const int32_t* sorted_token,
                                const int32_t* tiles, int64_t capacity,
                                const void* const* w_gate,
-                               const void* const* w_up, int64_t dim,
-                               int64_t dim_ffn, int block_m, void* h,
-                               hipStream_t s,
-                        const GemmWorkspace& ws = {});
+                               const void* const* w_up, int64_t n_rows,
+                               int n_experts, int64_t dim, int64_t dim_ffn,
+                               int block_m, void* h, hipStream_t s,
+                               const GemmWorkspace& ws = {});
 
 // Few rows (moe_gemm_few.hip), tiles below 256 rows: whether the kernels there
 // take a GEMM of n_rows rows over n_experts experts with k inputs

@@ -206,7 +206,7 @@ extern "C" int astrai_moe_gemm_gate_up(const void* x_perm, const int32_t* tiles,
     if (mfma && few_rows(n_rows, n_experts, block_m, dim, dim_ffn, true))
       return launch_few_gate_up(x_perm, nullptr, tiles, capacity, w_gate, w_up, n_rows, n_experts, dim, dim_ffn, false, h, s);
     if (mfma)
-      return launch_mfma_gate_up(x_perm, tiles, capacity, w_gate, w_up, dim,
+      return launch_mfma_gate_up(x_perm, tiles, capacity, w_gate, w_up, n_rows, n_experts, dim,
                                  dim_ffn, block_m, false, h, s,
                                  GemmWorkspace{workspace, workspace_bytes});
     return launch_generic<bf16_t, true>(x_perm, tiles, capacity, w_gate, w_up,
@@ -242,7 +242,7 @@ extern "C" int astrai_moe_gemm_gate_up_gather(const void* x, const int32_t* sort
   if (few_rows(n_rows, n_experts, block_m, dim, dim_ffn, true))
     return launch_few_gate_up(x, sorted_token, tiles, capacity, w_gate, w_up, n_rows, n_experts, dim, dim_ffn, false, h,
                               static_cast<hipStream_t>(stream));
-  return launch_mfma_gate_up_gather(x, sorted_token, tiles, capacity, w_gate, w_up, dim, dim_ffn, block_m, h,
+  return launch_mfma_gate_up_gather(x, sorted_token, tiles, capacity, w_gate, w_up, n_rows, n_experts, dim, dim_ffn, block_m, h,
                                     static_cast<hipStream_t>(stream), GemmWorkspace{workspace, workspace_bytes});
 }
 
@@ -268,7 +268,7 @@ extern "C" int astrai_moe_gemm_down(const void* h, const int32_t* tiles,
     if (mfma && few_rows(n_rows, n_experts, block_m, dim_ffn, dim, false))
       return launch_few_down(h, tiles, capacity, w_down, sorted_w, n_rows, n_experts, dim_ffn, dim, false, y, s);
     if (mfma)
-      return launch_mfma_down(h, tiles, capacity, w_down, sorted_w, dim_ffn,
+      return launch_mfma_down(h, tiles, capacity, w_down, sorted_w, n_rows, n_experts, dim_ffn,
                               dim, block_m, false, y, s,
                               GemmWorkspace{workspace, workspace_bytes});
     return launch_generic<bf16_t, false>(h, tiles, capacity, w_down, nullptr,
@@ -331,7 +331,7 @@ extern "C" int astrai_moe_gemm_gate_up_packed(const void* x_perm, const int32_t*
   if (few_rows(n_rows, n_experts, block_m, dim, dim_ffn, true))
     return launch_few_gate_up(x_perm, nullptr, tiles, capacity, w_packed, w_packed, n_rows, n_experts, dim, dim_ffn, true, h,
                               static_cast<hipStream_t>(stream));
-  return launch_mfma_gate_up(x_perm, tiles, capacity, w_packed, w_packed, dim, dim_ffn, block_m, true, h,
+  return launch_mfma_gate_up(x_perm, tiles, capacity, w_packed, w_packed, n_rows, n_experts, dim, dim_ffn, block_m, true, h,
                              static_cast<hipStream_t>(stream), GemmWorkspace{workspace, workspace_bytes});
 }
 
@@ -355,7 +355,7 @@ extern "C" int astrai_moe_gemm_down_packed(const void* h, const int32_t* tiles, 
   if (few_rows(n_rows, n_experts, block_m, dim_ffn, dim, false))
     return launch_few_down(h, tiles, capacity, w_packed, sorted_w, n_rows, n_experts, dim_ffn, dim, true, y,
                            static_cast<hipStream_t>(stream));
-  return launch_mfma_down(h, tiles, capacity, w_packed, sorted_w, dim_ffn, dim, block_m, true, y,
+  return launch_mfma_down(h, tiles, capacity, w_packed, sorted_w, n_rows, n_experts, dim_ffn, dim, block_m, true, y,
                           static_cast<hipStream_t>(stream),
                           GemmWorkspace{workspace, workspace_bytes});
 }

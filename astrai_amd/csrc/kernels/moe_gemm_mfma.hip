@@ -73,6 +73,9 @@
 //
 // Accumulator layout (16x16x32 with operands (W, A)): lane l, element r of
 // tile (i, j) is output row 16 i + l % 16, column 16 j + 4 (l / 16) + r.
+#include <algorithm>
+#include <cmath>
+
 #include "mfma_tile.h"
 
 #include <type_traits>
@@ -102,11 +105,12 @@ struct TileSrc {
   const char* b_base1 = nullptr;
   int row0 = 0, rows = 0;
   int b_rows = 0;  // weight rows of this column tile inside the matrix (per operand for gate/up)
+  // row_off: first row within the list's tile (the second half of a 256-row tile)
   __device__ void setup(const int32_t* tiles, const bf16_t* A, const void* const* W0, const void* const* W1, int K,
-                        int N, int mt, int nt) {
+                        int N, int mt, int nt, int row_off = 0) {
     const int32_t* ti = tiles + ASTRAI_MOE_TILE_HEADER + (int64_t)mt * ASTRAI_MOE_TILE_STRIDE;
     const int e = ti[0];
-    row0 = ti[1];
+    row0 = ti[1] + row_off;
     rows = min(BM, ti[2] - row0);
     constexpr int kTileRows = kGateUp ? BN / 2 : BN;
     b_rows = min(kTileRows, N - nt * kTileRows);
@@ -840,7 +844,10 @@ struct TileCfg {
   static_assert(DMA_PER_WAVE * (STAGES - 1) <= 63, "vmcnt range");
 };
 
-template <typename Cfg, bool kGateUp, bool kPacked, bool kGather = false>
+// kHalves: the list holds 256-row tiles, each walked as two of 128 rows, the
+// halves of a tile as neighbouring column tiles of the walk. K then starts at
+// step 0, as in the streaming kernel, for the same bits.
+template <typename Cfg, bool kGateUp, bool kPacked, bool kGather = false, bool kHalves = false>
 __global__ __launch_bounds__(Cfg::THREADS, 1) void gemm_mfma_kernel(
     const bf16_t* __restrict__ A, const int32_t* __restrict__ tiles, const void* const* __restrict__ W0,
     const void* const* __restrict__ W1, const bf16_t* __restrict__ row_w, int K, int N, int n_tiles_n,
@@ -852,9 +859,23 @@ __global__ __launch_bounds__(Cfg::THREADS, 1) void gemm_mfma_kernel(
   static_assert(STAGE_AREA + Cfg::WAVES * 16 * OROW <= 160 * 1024, "LDS");
   __shared__ __attribute__((aligned(1024))) char smem[STAGE_AREA + Cfg::WAVES * 16 * OROW];
 
-  const TileWalk<Cfg::GM> walk(tiles, capacity, n_tiles_n);
+  static_assert(!kHalves || (Cfg::BM == 128 && !kPacked), "halves of 256-row tiles");
+  const TileWalk<Cfg::GM> walk(tiles, capacity, kHalves ? 2 * n_tiles_n : n_tiles_n);
   int mt = 0, nt = 0;
-  int logical = walk.seek(walk.first_slot(), mt, nt);
+  // the workgroup's first tile from `logical` on that has rows (a tile of at
+  // most 128 rows has no second half)
+  auto seek = [&](int logical_, int& mt_, int& nt_) {
+    int at = walk.seek(logical_, mt_, nt_);
+    if constexpr (kHalves) {
+      while (at < walk.total && (nt_ & 1) != 0) {
+        const int32_t* ti = tiles + ASTRAI_MOE_TILE_HEADER + (int64_t)mt_ * ASTRAI_MOE_TILE_STRIDE;
+        if (ti[1] + 128 < ti[2]) break;
+        at = walk.seek(at + walk.G, mt_, nt_);
+      }
+    }
+    return at;
+  };
+  int logical = seek(walk.first_slot(), mt, nt);
   if (logical >= walk.total) return;
 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -878,8 +899,12 @@ __global__ __launch_bounds__(Cfg::THREADS, 1) void gemm_mfma_kernel(
   const int kt_n = kRagged ? k_steps(K) : K / kBK;
   int k_start = 0;
   auto setup_tile = [&](int mt_, int nt_) {
-    src.setup(tiles, A, W0, W1, K, N, mt_, nt_);
-    k_start = (tiles[ASTRAI_MOE_TILE_HEADER + (int64_t)mt_ * ASTRAI_MOE_TILE_STRIDE] * 7) % kt_n;
+    if constexpr (kHalves) {
+      src.setup(tiles, A, W0, W1, K, N, mt_, nt_ >> 1, (nt_ & 1) * 128);
+    } else {
+      src.setup(tiles, A, W0, W1, K, N, mt_, nt_);
+      k_start = (tiles[ASTRAI_MOE_TILE_HEADER + (int64_t)mt_ * ASTRAI_MOE_TILE_STRIDE] * 7) % kt_n;
+    }
     if constexpr (kGather) grows.load(row_src, src.row0, src.rows, wave * Cfg::A_PER_WAVE, lane, k2);
   };
   auto stage_ops = [&](auto tail_c, int ks, int buf) {
@@ -995,9 +1020,9 @@ __global__ __launch_bounds__(Cfg::THREADS, 1) void gemm_mfma_kernel(
 
     // ---- next tile's first stages, then this tile's epilogue ----
     int nmt = 0, nnt = 0;
-    const int nlogical = walk.seek(logical + walk.G, nmt, nnt);
+    const int nlogical = seek(logical + walk.G, nmt, nnt);
     const bool has_next = nlogical < walk.total;
-    const int t_row0 = src.row0, t_rows = src.rows, t_nt = nt;
+    const int t_row0 = src.row0, t_rows = src.rows, t_nt = kHalves ? nt >> 1 : nt;
     __builtin_amdgcn_sched_barrier(0);
     lds_barrier();  // every wave is done reading the stage buffers
     __builtin_amdgcn_sched_barrier(0);
@@ -1028,6 +1053,10 @@ using MidCfg = TileCfg<kMfmaMidBM, 256, 3, 2, 4, 8>;
 // the down epilogue's per-wave 16-row slices stay small), three 48 KB stages
 // in flight: 144 KB of stages + 10 KB of epilogue slices.
 using Mid2Cfg = TileCfg<kMfmaMid2BM, 256, 3, 1, 8, 8>;
+// Few tiles: 128 x 128 outputs, 8 waves of 64 x 32, four 32 KB stages. LDS
+// bandwidth bounds a step (96 KB of fragments read and 32 KB written for 0.21 us
+// of MFMA), but twice as many compute units work on a GEMM as with 256 columns.
+using NarrowCfg = TileCfg<kMfmaMid2BM, 128, 4, 2, 4, 8>;
 static_assert(StreamCfg<true>::BM == kMfmaBigBM && StreamCfg<false>::BM == kMfmaBigBM, "prefill tile height");
 
 // Clears the run-time claim counter of a streaming launch's scheduling
@@ -1075,23 +1104,90 @@ int launch_stream(const void* A, const int32_t* tiles, int64_t capacity, const v
   return check_launch("split_reduce_kernel");
 }
 
-template <typename Cfg, bool kGateUp, bool kPacked, bool kGather = false>
+template <typename Cfg, bool kGateUp, bool kPacked, bool kGather = false, bool kHalves = false>
 int launch(const void* A, const int32_t* tiles, int64_t capacity, const void* const* W0, const void* const* W1,
            const void* row_w, int64_t K, int64_t N, void* C, hipStream_t s, const int32_t* row_src = nullptr) {
   if (capacity == 0) return ASTRAI_MOE_OK;
   const int64_t n_tiles_n = ceil_div(N, kGateUp ? Cfg::BN / 2 : Cfg::BN);  // the last may be partial
   int64_t grid = 0;
-  if (int rc = persistent_grid(capacity, n_tiles_n, &grid)) return rc;
-  hipLaunchKernelGGL((gemm_mfma_kernel<Cfg, kGateUp, kPacked, kGather>), dim3((unsigned)grid), dim3(Cfg::THREADS),
+  if (int rc = persistent_grid(capacity, kHalves ? 2 * n_tiles_n : n_tiles_n, &grid)) return rc;
+  hipLaunchKernelGGL((gemm_mfma_kernel<Cfg, kGateUp, kPacked, kGather, kHalves>), dim3((unsigned)grid), dim3(Cfg::THREADS),
                      0, s, static_cast<const bf16_t*>(A), tiles, W0, W1, static_cast<const bf16_t*>(row_w), (int)K,
                      (int)N, (int)n_tiles_n, (int)capacity, static_cast<bf16_t*>(C), row_src);
   return check_launch(kGateUp ? "gemm_mfma_kernel<gate_up>" : "gemm_mfma_kernel<down>");
 }
 
+// Row tiles of `bm` rows that n_rows rows over n_experts experts make, expected
+// under even routing (an expert's rows about normal, with their mean as
+// variance); exact for one expert.
+double expected_row_tiles(int64_t n_rows, int n_experts, int bm) {
+  if (n_experts == 1) return (double)ceil_div(n_rows, bm);
+  const double r = (double)n_rows / n_experts, sd = std::sqrt(std::max(r, 1.0));
+  double tiles = 0.0;
+  for (int64_t j = 0; j * bm < r + 8.0 * sd; ++j) tiles += 0.5 * std::erfc(((double)(j * bm) - r) / (sd * 1.41421356));
+  return n_experts * tiles;
+}
+
+// Which tiles a GEMM takes on a list of 128- or 256-row tiles: the list's own
+// with 256 columns (gate/up: 128 of each), or, where those leave compute units
+// idle, 128 rows by 128 columns, and on a 256-row list also 128 by 256.
+enum class Tiles { kList, kHalves, kNarrow, kNarrowHalves };
+
+// A GEMM of few tiles takes rounds of its compute units times a tile's K steps,
+// however few the tiles of the last round: 1.4 us a step of a 256 x 256 tile,
+// 1.07 of 128 x 256, 0.71 of 128 x 128 (measured; the small tiles pay more per
+// flop, and lose once two tiles of theirs share a compute unit). Taken where
+// this promises a tenth; only within kFewRounds rounds of the list's own tiles,
+// past which the shares are even and the memory system decides. 256-row tiles of
+// kSplitMinTileSteps steps keep their kernel, which splits its last round.
+// Measured, us, a down GEMM of the list's tiles / the ones taken:
+// - 8 experts, top-2, D 1000, F 2664, 130 to 375 rows an expert 50 / 31 to 58 /
+//   33, and 9 of 500 rows 59 / 50 (halves); D 512, F 1024, 130 to 768 rows 23 / 14
+//   to 26 / 15 (gate/up 17 / 13 to 19 / 14.5); D 4096, F 14336, 64 rows (128-row
+//   list) 241 / 191;
+// - 16 experts, top-4, D 704, F 576, 64 to 512 rows 12 / 10 to 21 / 17 (gate/up
+//   21 / 17.5 at 130 to 256); D 2048, F 1408, 64 rows 27 / 20, 130 37 / 29 (halves),
+//   256 (a third more row tiles than places in a round) 42 / 44 if taken;
+// - one expert, D 4096, F 14336, 512 rows 180 / 127, 1024 191 / 141; D 2048, F 5632,
+//   1500 rows 81 / 55.
+constexpr double kFewRounds = 2.0;
+Tiles pick_tiles(int64_t n_rows, int n_experts, int block_m, int64_t k, int64_t n, bool gate_up) {
+  if (block_m != kMfmaMid2BM && (block_m != kMfmaBigBM || k_steps(k) >= kSplitMinTileSteps)) return Tiles::kList;
+  const double cu = cu_count();
+  const double wide = (double)ceil_div(n, gate_up ? 128 : 256), narrow = (double)ceil_div(n, gate_up ? 64 : 128);
+  if ((double)n_rows / block_m * wide > kFewRounds * cu) return Tiles::kList;  // (bounds the sum below)
+  const double own = expected_row_tiles(n_rows, n_experts, block_m) * wide;
+  if (own > kFewRounds * cu) return Tiles::kList;
+  // (a tile without a second half still takes its place in the walk)
+  const double rows128 = (block_m == kMfmaBigBM ? 2.0 : 1.0) * expected_row_tiles(n_rows, n_experts, block_m);
+  const double t_own = std::ceil(own / cu) * (block_m == kMfmaBigBM ? 1.4 : 1.07);
+  const double t_wide = block_m == kMfmaBigBM ? std::ceil(rows128 * wide / cu) * 1.07 : t_own;
+  const double t_narrow = std::ceil(rows128 * narrow / cu) * 0.71;
+  if (t_narrow <= t_wide && t_narrow < 0.9 * t_own)
+    return block_m == kMfmaBigBM ? Tiles::kNarrowHalves : Tiles::kNarrow;
+  return t_wide < 0.9 * t_own ? Tiles::kHalves : Tiles::kList;
+}
+
+template <bool kGateUp, bool kGather = false>
+int launch_picked(Tiles pick, const void* A, const int32_t* tiles, int64_t capacity, const void* const* W0,
+                  const void* const* W1, const void* row_w, int64_t K, int64_t N, void* C, hipStream_t s,
+                  const int32_t* row_src = nullptr) {
+  if (pick == Tiles::kHalves)
+    return launch<Mid2Cfg, kGateUp, false, kGather, true>(A, tiles, capacity, W0, W1, row_w, K, N, C, s, row_src);
+  if (pick == Tiles::kNarrow)
+    return launch<NarrowCfg, kGateUp, false, kGather>(A, tiles, capacity, W0, W1, row_w, K, N, C, s, row_src);
+  return launch<NarrowCfg, kGateUp, false, kGather, true>(A, tiles, capacity, W0, W1, row_w, K, N, C, s, row_src);
+}
+
 template <bool kPacked>
 int gate_up_dispatch(const void* x_perm, const int32_t* tiles, int64_t capacity, const void* const* w_gate,
-                     const void* const* w_up, int64_t dim, int64_t dim_ffn, int block_m, void* h, hipStream_t s,
-                     const GemmWorkspace& ws) {
+                     const void* const* w_up, int64_t n_rows, int n_experts, int64_t dim, int64_t dim_ffn,
+                     int block_m, void* h, hipStream_t s, const GemmWorkspace& ws) {
+  if constexpr (!kPacked) {
+    const Tiles pick = pick_tiles(n_rows, n_experts, block_m, dim, dim_ffn, true);
+    if (pick != Tiles::kList)
+      return launch_picked<true>(pick, x_perm, tiles, capacity, w_gate, w_up, nullptr, dim, dim_ffn, h, s);
+  }
   if (block_m == kMfmaBigBM)
     return launch_stream<true, kPacked>(x_perm, tiles, capacity, w_gate, w_up, nullptr, dim, dim_ffn, h, s, nullptr,
                                         nullptr, nullptr, ws);
@@ -1104,8 +1200,13 @@ int gate_up_dispatch(const void* x_perm, const int32_t* tiles, int64_t capacity,
 
 template <bool kPacked>
 int down_dispatch(const void* h, const int32_t* tiles, int64_t capacity, const void* const* w_down,
-                  const void* sorted_w, int64_t dim_ffn, int64_t dim, int block_m, void* y, hipStream_t s,
-                  const GemmWorkspace& ws) {
+                  const void* sorted_w, int64_t n_rows, int n_experts, int64_t dim_ffn, int64_t dim, int block_m,
+                  void* y, hipStream_t s, const GemmWorkspace& ws) {
+  if constexpr (!kPacked) {
+    const Tiles pick = pick_tiles(n_rows, n_experts, block_m, dim_ffn, dim, false);
+    if (pick != Tiles::kList)
+      return launch_picked<false>(pick, h, tiles, capacity, w_down, nullptr, sorted_w, dim_ffn, dim, y, s);
+  }
   if (block_m == kMfmaBigBM)
     return launch_stream<false, kPacked>(h, tiles, capacity, w_down, nullptr, sorted_w, dim_ffn, dim, y, s, nullptr,
                                          nullptr, nullptr, ws);
@@ -1146,29 +1247,30 @@ namespace ragged {
 #endif
 
 int launch_mfma_gate_up(const void* x_perm, const int32_t* tiles, int64_t capacity, const void* const* w_gate,
-                        const void* const* w_up, int64_t dim, int64_t dim_ffn, int block_m, bool packed, void* h,
-                        hipStream_t s, const GemmWorkspace& ws) {
+                        const void* const* w_up, int64_t n_rows, int n_experts, int64_t dim, int64_t dim_ffn, int block_m,
+                        bool packed, void* h, hipStream_t s, const GemmWorkspace& ws) {
 #if ASTRAI_MOE_RAGGED_K
   if (packed) return fail(ASTRAI_MOE_EINVAL, "gemm_gate_up: packed weights need whole K steps");
 #else
   if (dim % kBK != 0)
-    return ragged::launch_mfma_gate_up(x_perm, tiles, capacity, w_gate, w_up, dim, dim_ffn, block_m, packed, h, s, ws);
+    return ragged::launch_mfma_gate_up(x_perm, tiles, capacity, w_gate, w_up, n_rows, n_experts, dim, dim_ffn, block_m, packed,
+                                       h, s, ws);
 #endif
-  return packed ? gate_up_dispatch<!kRagged>(x_perm, tiles, capacity, w_gate, w_gate, dim, dim_ffn, block_m, h, s, ws)
-                : gate_up_dispatch<false>(x_perm, tiles, capacity, w_gate, w_up, dim, dim_ffn, block_m, h, s, ws);
+  return packed ? gate_up_dispatch<!kRagged>(x_perm, tiles, capacity, w_gate, w_gate, n_rows, n_experts, dim, dim_ffn, block_m, h, s, ws)
+                : gate_up_dispatch<false>(x_perm, tiles, capacity, w_gate, w_up, n_rows, n_experts, dim, dim_ffn, block_m, h, s, ws);
 }
 
 int launch_mfma_down(const void* h, const int32_t* tiles, int64_t capacity, const void* const* w_down,
-                     const void* sorted_w, int64_t dim_ffn, int64_t dim, int block_m, bool packed, void* y,
-                     hipStream_t s, const GemmWorkspace& ws) {
+                     const void* sorted_w, int64_t n_rows, int n_experts, int64_t dim_ffn, int64_t dim, int block_m,
+                     bool packed, void* y, hipStream_t s, const GemmWorkspace& ws) {
 #if ASTRAI_MOE_RAGGED_K
   if (packed) return fail(ASTRAI_MOE_EINVAL, "gemm_down: packed weights need whole K steps");
 #else
   if (dim_ffn % kBK != 0)
-    return ragged::launch_mfma_down(h, tiles, capacity, w_down, sorted_w, dim_ffn, dim, block_m, packed, y, s, ws);
+    return ragged::launch_mfma_down(h, tiles, capacity, w_down, sorted_w, n_rows, n_experts, dim_ffn, dim, block_m, packed, y, s, ws);
 #endif
-  return packed ? down_dispatch<!kRagged>(h, tiles, capacity, w_down, sorted_w, dim_ffn, dim, block_m, y, s, ws)
-                : down_dispatch<false>(h, tiles, capacity, w_down, sorted_w, dim_ffn, dim, block_m, y, s, ws);
+  return packed ? down_dispatch<!kRagged>(h, tiles, capacity, w_down, sorted_w, n_rows, n_experts, dim_ffn, dim, block_m, y, s, ws)
+                : down_dispatch<false>(h, tiles, capacity, w_down, sorted_w, n_rows, n_experts, dim_ffn, dim, block_m, y, s, ws);
 }
 
 int launch_mfma_gate_up_save(const void* x_perm, const int32_t* tiles, int64_t capacity, const void* const* w_gate,
@@ -1198,8 +1300,12 @@ int launch_mfma_down_save(const void* h, const int32_t* tiles, int64_t capacity,
 #else
 
 int launch_mfma_gate_up_gather(const void* x, const int32_t* sorted_token, const int32_t* tiles, int64_t capacity,
-                               const void* const* w_gate, const void* const* w_up, int64_t dim, int64_t dim_ffn,
-                               int block_m, void* h, hipStream_t s, const GemmWorkspace& ws) {
+                               const void* const* w_gate, const void* const* w_up, int64_t n_rows, int n_experts,
+                               int64_t dim, int64_t dim_ffn, int block_m, void* h, hipStream_t s,
+                               const GemmWorkspace& ws) {
+  const Tiles pick = pick_tiles(n_rows, n_experts, block_m, dim, dim_ffn, true);
+  if (pick != Tiles::kList)
+    return launch_picked<true, true>(pick, x, tiles, capacity, w_gate, w_up, nullptr, dim, dim_ffn, h, s, sorted_token);
   if (block_m == kMfmaBigBM)
     return launch_stream<true, false, false, true>(x, tiles, capacity, w_gate, w_up, nullptr, dim, dim_ffn, h, s,
                                                    nullptr, nullptr, sorted_token, ws);
