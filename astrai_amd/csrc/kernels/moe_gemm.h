@@ -122,6 +122,12 @@ int launch_few_down(const void* h, const int32_t* tiles, int64_t capacity,
                     const void* const* w_down, const void* sorted_w,
                     int64_t n_rows, int n_experts, int64_t dim_ffn,
                     int64_t dim, bool packed, void* y, hipStream_t s);
+// Both GEMMs of one dense expert whose GEMMs few_rows both takes, without a
+// tile list.
+int launch_few_dense(const void* x, const void* const* w_gate,
+                     const void* const* w_up, const void* const* w_down,
+                     int64_t n_rows, int64_t dim, int64_t dim_ffn, int block_m,
+                     void* h, void* out, hipStream_t s);
 
 // Training forward (256-row tiles): as launch_mfma_gate_up / launch_mfma_down,
 // also storing the bf16 gate and up projections (gu: [rows, 2 dim_ffn],

@@ -46,6 +46,30 @@ struct FewCfg {
   static_assert(OPS * (STAGES - 1) <= 63, "vmcnt range");
 };
 
+// The row tiles a launch walks: those of the list, or (kDense) one expert's
+// n_rows rows in tiles of block_m, with no list to write and wait for.
+template <bool kDense>
+struct RowTiles {
+  const int32_t* tiles;
+  int n_rows, block_m;
+  __device__ int live(int capacity) const {
+    if constexpr (kDense) return capacity;
+    return min(load_scalar(tiles), min(load_scalar(tiles + 2), capacity));
+  }
+  __device__ void get(int mt, int& e, int& row0, int& rows) const {
+    if constexpr (kDense) {
+      e = 0;
+      row0 = mt * block_m;
+      rows = min(block_m, n_rows - row0);
+    } else {
+      const int32_t* ti = tiles + ASTRAI_MOE_TILE_HEADER + (int64_t)mt * ASTRAI_MOE_TILE_STRIDE;
+      e = load_scalar(ti);
+      row0 = load_scalar(ti + 1);
+      rows = min(load_scalar(tiles + 1), load_scalar(ti + 2) - row0);
+    }
+  }
+};
+
 // Position of a wave in its sequence of K steps: run `sub` of 32 rows of tile
 // `unit`, the wave's step j of n.
 template <typename Cfg, bool kGateUp, bool kGather, bool kPacked>
@@ -57,14 +81,13 @@ struct FewCursor {
   int b_rows;
 
   // tile and weights of `unit` (< total)
-  __device__ void enter(const int32_t* tiles, const void* const* W0, const void* const* W1, int K, int N, int n_cols) {
+  template <bool kDense>
+  __device__ void enter(const RowTiles<kDense>& tiles, const void* const* W0, const void* const* W1, int K, int N, int n_cols) {
     constexpr int kCols = kGateUp ? Cfg::BN / 2 : Cfg::BN;
     mt = unit / n_cols;
     nt = unit - mt * n_cols;
-    const int32_t* ti = tiles + ASTRAI_MOE_TILE_HEADER + (int64_t)mt * ASTRAI_MOE_TILE_STRIDE;
-    const int e = load_scalar(ti);
-    row0 = load_scalar(ti + 1);
-    rows = min(load_scalar(tiles + 1), load_scalar(ti + 2) - row0);
+    int e;
+    tiles.get(mt, e, row0, rows);
     const int KT = k_steps(K);
     b_rows = min(kCols, N - nt * kCols);
     const char* w0 = static_cast<const char*>(load_scalar(W0 + e));
@@ -92,7 +115,8 @@ struct FewCursor {
       off[q] = kGather ? (uint32_t)row_src[row0 + sub * Cfg::BM + r] * k2 : (uint32_t)r * k2;
     }
   }
-  __device__ void advance(int total, int G, const int32_t* tiles, const bf16_t* A, const void* const* W0,
+  template <bool kDense>
+  __device__ void advance(int total, int G, const RowTiles<kDense>& tiles, const bf16_t* A, const void* const* W0,
                           const void* const* W1, const int32_t* row_src, int K, int N, int n_cols, int lane) {
     if (++j < n) return;
     const int old_mt = mt, old_sub = sub;
@@ -149,9 +173,9 @@ struct FewCursor {
   }
 };
 
-template <typename Cfg, bool kGateUp, bool kGather, bool kPacked>
+template <typename Cfg, bool kGateUp, bool kGather, bool kPacked, bool kDense>
 __global__ __launch_bounds__(Cfg::WAVES * 64, 1) void gemm_few_kernel(
-    const bf16_t* __restrict__ A, const int32_t* __restrict__ tiles, const void* const* __restrict__ W0,
+    const bf16_t* __restrict__ A, const RowTiles<kDense> tiles, const void* const* __restrict__ W0,
     const void* const* __restrict__ W1, const bf16_t* __restrict__ row_w, int K, int N, int n_cols, int capacity,
     bf16_t* __restrict__ C, const int32_t* __restrict__ row_src) {
   constexpr int NR = Cfg::NR, NC = Cfg::NC;
@@ -159,7 +183,7 @@ __global__ __launch_bounds__(Cfg::WAVES * 64, 1) void gemm_few_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   const int G = gridDim.x;
-  const int total = min(load_scalar(tiles), min(load_scalar(tiles + 2), capacity)) * n_cols;
+  const int total = tiles.live(capacity) * n_cols;
   if ((int)blockIdx.x >= total) return;
   char* const ring = smem + wave * (Cfg::STAGES * Cfg::STAGE);
 
@@ -185,9 +209,8 @@ __global__ __launch_bounds__(Cfg::WAVES * 64, 1) void gemm_few_kernel(
   int parity = 0;
   for (int unit = blockIdx.x; unit < total; unit += G) {
     const int mt = unit / n_cols, nt = unit - mt * n_cols;
-    const int32_t* ti = tiles + ASTRAI_MOE_TILE_HEADER + (int64_t)mt * ASTRAI_MOE_TILE_STRIDE;
-    const int row0 = load_scalar(ti + 1);
-    const int rows = min(load_scalar(tiles + 1), load_scalar(ti + 2) - row0);
+    int e, row0, rows;
+    tiles.get(mt, e, row0, rows);
     for (int r0 = 0; r0 < rows; r0 += Cfg::BM) {
       f32x4_t acc[NR][NC];
 #pragma unroll
@@ -281,14 +304,14 @@ __global__ __launch_bounds__(Cfg::WAVES * 64, 1) void gemm_few_kernel(
   }
 }
 
-template <typename Cfg, bool kGateUp, bool kGather, bool kPacked>
-int launch_few_cfg(const void* A, const int32_t* tiles, int64_t capacity, const void* const* W0, const void* const* W1,
+template <typename Cfg, bool kGateUp, bool kGather, bool kPacked, bool kDense>
+int launch_few_cfg(const void* A, const RowTiles<kDense>& tiles, int64_t capacity, const void* const* W0, const void* const* W1,
                const void* row_w, int64_t K, int64_t N, void* C, hipStream_t s, const int32_t* row_src) {
   if (capacity == 0) return ASTRAI_MOE_OK;
   const int64_t n_cols = ceil_div(N, kGateUp ? Cfg::BN / 2 : Cfg::BN);  // the last may be partial
   int64_t grid = 0;
   if (int rc = persistent_grid(capacity, n_cols, &grid)) return rc;
-  hipLaunchKernelGGL((gemm_few_kernel<Cfg, kGateUp, kGather, kPacked>), dim3((unsigned)grid), dim3(Cfg::WAVES * 64),
+  hipLaunchKernelGGL((gemm_few_kernel<Cfg, kGateUp, kGather, kPacked, kDense>), dim3((unsigned)grid), dim3(Cfg::WAVES * 64),
                      0, s, static_cast<const bf16_t*>(A), tiles, W0, W1, static_cast<const bf16_t*>(row_w), (int)K,
                      (int)N, (int)n_cols, (int)capacity, static_cast<bf16_t*>(C), row_src);
   return check_launch(kGateUp ? "gemm_few_kernel<gate_up>" : "gemm_few_kernel<down>");
@@ -321,17 +344,25 @@ constexpr double kFewMaxFill = 0.9;
 // activation bytes as one of 32, which costs more elsewhere: more runs (48
 // rows 131 -> 163 us) and routed rows (8 experts of that size, 24 tokens 541
 // -> 560; 64 of D 2048, F 1408, 8 tokens 144 -> 188).
+template <bool kGateUp, bool kGather, bool kPacked, bool kDense>
+int launch_few_tiles(const void* A, const RowTiles<kDense>& tiles, int64_t capacity, const void* const* W0, const void* const* W1,
+               const void* row_w, int64_t n_rows, int n_experts, int64_t K, int64_t N, void* C, hipStream_t s,
+               const int32_t* row_src) {
+  if (n_rows > (n_experts == 1 ? 2 * FewCfg<32, 32>::BM : (int64_t)kFewRowsPerExpert * n_experts))
+    return launch_few_cfg<FewCfg<64, 32>, kGateUp, kGather, kPacked, kDense>(A, tiles, capacity, W0, W1, row_w, K, N, C, s,
+                                                                     row_src);
+  if (n_experts == 1 && n_rows <= FewCfg<32, 16>::BM &&
+      fill((double)ceil_div(N, kGateUp ? 8 : 16)) > 1.05 * fill((double)ceil_div(N, kGateUp ? 16 : 32)))
+    return launch_few_cfg<FewCfg<32, 16>, kGateUp, kGather, kPacked, kDense>(A, tiles, capacity, W0, W1, row_w, K, N, C, s, row_src);
+  return launch_few_cfg<FewCfg<32, 32>, kGateUp, kGather, kPacked, kDense>(A, tiles, capacity, W0, W1, row_w, K, N, C, s, row_src);
+}
+
 template <bool kGateUp, bool kGather, bool kPacked>
 int launch_few(const void* A, const int32_t* tiles, int64_t capacity, const void* const* W0, const void* const* W1,
                const void* row_w, int64_t n_rows, int n_experts, int64_t K, int64_t N, void* C, hipStream_t s,
                const int32_t* row_src) {
-  if (n_rows > (n_experts == 1 ? 2 * FewCfg<32, 32>::BM : (int64_t)kFewRowsPerExpert * n_experts))
-    return launch_few_cfg<FewCfg<64, 32>, kGateUp, kGather, kPacked>(A, tiles, capacity, W0, W1, row_w, K, N, C, s,
-                                                                     row_src);
-  if (n_experts == 1 && n_rows <= FewCfg<32, 16>::BM &&
-      fill((double)ceil_div(N, kGateUp ? 8 : 16)) > 1.05 * fill((double)ceil_div(N, kGateUp ? 16 : 32)))
-    return launch_few_cfg<FewCfg<32, 16>, kGateUp, kGather, kPacked>(A, tiles, capacity, W0, W1, row_w, K, N, C, s, row_src);
-  return launch_few_cfg<FewCfg<32, 32>, kGateUp, kGather, kPacked>(A, tiles, capacity, W0, W1, row_w, K, N, C, s, row_src);
+  return launch_few_tiles<kGateUp, kGather, kPacked>(A, RowTiles<false>{tiles, 0, 0}, capacity, W0, W1, row_w, n_rows,
+                                                     n_experts, K, N, C, s, row_src);
 }
 
 }  // namespace
@@ -381,6 +412,17 @@ int launch_few_down(const void* h, const int32_t* tiles, int64_t capacity, const
   if (packed)
     return launch_few<false, false, true>(h, tiles, capacity, w_down, w_down, sorted_w, n_rows, n_experts, dim_ffn, dim, y, s, nullptr);
   return launch_few<false, false, false>(h, tiles, capacity, w_down, w_down, sorted_w, n_rows, n_experts, dim_ffn, dim, y, s, nullptr);
+}
+
+int launch_few_dense(const void* x, const void* const* w_gate, const void* const* w_up, const void* const* w_down,
+                     int64_t n_rows, int64_t dim, int64_t dim_ffn, int block_m, void* h, void* out, hipStream_t s) {
+  const RowTiles<true> rows{nullptr, (int)n_rows, block_m};
+  const int64_t n_tiles = ceil_div(n_rows, block_m);
+  if (int rc = launch_few_tiles<true, false, false>(x, rows, n_tiles, w_gate, w_up, nullptr, n_rows, 1, dim, dim_ffn, h,
+                                                    s, nullptr))
+    return rc;
+  return launch_few_tiles<false, false, false>(h, rows, n_tiles, w_down, nullptr, nullptr, n_rows, 1, dim_ffn, dim, out,
+                                               s, nullptr);
 }
 
 }  // namespace astrai_moe

@@ -71,6 +71,8 @@ _SIGNATURES: dict[str, tuple] = {
     "astrai_moe_forward_workspace_bytes": (_i64, [_i64, _int, _int, _int, _i64, _i64, _int, _int]),
     "astrai_moe_forward": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _int, _i64, _int, _int, _int, _i64, _i64, _vp,
                                   _i64, _vp, _vp]),
+    "astrai_moe_dense_forward_workspace_bytes": (_i64, [_i64, _i64, _i64, _int]),
+    "astrai_moe_dense_forward": (_int, [_vp, _vp, _vp, _vp, _int, _i64, _i64, _i64, _vp, _i64, _vp, _vp]),
     "astrai_moe_gemm_gate_up_train": (_int, [_vp, _vp, _i64, _vp, _vp, _int, _i64, _int, _i64, _i64, _int, _vp, _vp,
                                              _vp, _i64, _vp]),
     "astrai_moe_gemm_down_train": (_int, [_vp, _vp, _i64, _vp, _vp, _int, _i64, _int, _i64, _i64, _int, _vp, _vp,

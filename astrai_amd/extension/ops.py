@@ -477,12 +477,24 @@ def moe_dense_mlp(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, w_d
                   dim_ffn: int, out: torch.Tensor | None = None, tiles: torch.Tensor | None = None) -> torch.Tensor:
     """One expert ``down(up(x) * silu(gate(x)))`` over all rows of x (mlp.py:22-25),
     on the grouped-GEMM kernels with one-entry weight tables. ``tiles``: a list
-    from ``dense_tiles`` for these rows at ``dense_block_m``'s height (built here
-    when None), so several experts over the same rows can share one."""
+    from ``dense_tiles`` for these rows at ``dense_block_m``'s height, so several
+    experts over the same rows can share one (None: one call of the library)."""
     n_tokens, dim = x.shape
-    block_m = dense_block_m(n_tokens, dim, dim_ffn, x.dtype)
     if tiles is None:
-        tiles = dense_tiles(n_tokens, block_m, x.device)
+        _require_gpu(x, "x", 2)
+        code = _dtype_code(x, "x")
+        for name, t in (("w_gate", w_gate), ("w_up", w_up), ("w_down", w_down)):
+            _require_table(t, name, 1, x)
+        lib = loader.library()
+        out = _out_buffer(out, n_tokens, dim, x)
+        nbytes = lib.astrai_moe_dense_forward_workspace_bytes(n_tokens, dim, dim_ffn, code)
+        _check(0 if nbytes >= 0 else int(nbytes), "moe_dense_mlp")
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+        _check(lib.astrai_moe_dense_forward(x.data_ptr(), w_gate.data_ptr(), w_up.data_ptr(), w_down.data_ptr(), code,
+                                            n_tokens, dim, dim_ffn, ws.data_ptr(), nbytes, out.data_ptr(), _stream(x)),
+               "moe_dense_mlp")
+        return out
+    block_m = dense_block_m(n_tokens, dim, dim_ffn, x.dtype)
     h = moe_gemm_gate_up(x, tiles, w_gate, w_up, 1, dim_ffn, block_m)
     return moe_gemm_down(h, tiles, w_down, None, 1, dim, block_m, out=out)
 

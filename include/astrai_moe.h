@@ -383,6 +383,24 @@ int astrai_moe_forward(const void* x, const void* logits,
                        void* stream);
 
 /*
+ * One dense expert over n_rows rows in one call (MLP.forward, mlp.py:22-25):
+ * astrai_moe_dense_tiles and the grouped GEMMs with one-entry weight tables,
+ * the same values; few rows without the list.
+ *   x, out     [n_rows, dim] dtype
+ *   workspace  astrai_moe_dense_forward_workspace_bytes(...) bytes for the
+ *              same sizes, 256-byte aligned, nothing to initialise; calls
+ *              sharing one must not overlap
+ */
+int64_t astrai_moe_dense_forward_workspace_bytes(int64_t n_rows, int64_t dim,
+                                                 int64_t dim_ffn, int dtype);
+int astrai_moe_dense_forward(const void* x, const void* const* w_gate,
+                             const void* const* w_up,
+                             const void* const* w_down, int dtype,
+                             int64_t n_rows, int64_t dim, int64_t dim_ffn,
+                             void* workspace, int64_t workspace_bytes,
+                             void* out, void* stream);
+
+/*
  * Training: forward that keeps what the backward needs, and the backward.
  * The reference gets its gradients from torch autograd over mlp.py:22-25
  * and :89-98; these entry points compute the same quantities with grouped

@@ -7,6 +7,7 @@ from __future__ import annotations
 import pytest
 import torch
 
+from astrai_amd.extension import ops
 from astrai_amd.model.components.mlp import MLP
 from oracle import moe_ref as R
 from test_gpu_backward import _random_layer
@@ -39,3 +40,19 @@ def test_layer(gpu, n_tok, n_exp, top_k, n_shared):
     layer.pack_weights = True
     assert layer.uses_packed_weights(x.dtype)
     assert torch.equal(layer(x), live)  # packed copies: the same bits
+
+
+@pytest.mark.parametrize("dim,dim_ffn", [(64, 64), (72, 328), (512, 1408), (1536, 4096)])
+@pytest.mark.parametrize("n_tok", [0, 1, 32, 33, 64, 65, 95, 96, 128, 129, 256, 257])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_one_call_is_the_listed_calls(gpu, n_tok, dim, dim_ffn, dtype):
+    # one dense expert without a tile list (few rows) and with one: the same bits
+    torch.manual_seed(n_tok)
+    ws = [(torch.randn(*s, device=gpu) * 0.05).to(dtype) for s in ((dim_ffn, dim), (dim_ffn, dim), (dim, dim_ffn))]
+    tables = [ops.expert_weight_table([w], tuple(w.shape)) for w in ws]
+    x = torch.randn(n_tok, dim, device=gpu).to(dtype)
+    tiles = ops.dense_tiles(n_tok, ops.dense_block_m(n_tok, dim, dim_ffn, dtype), x.device)
+    listed = ops.moe_dense_mlp(x, *tables, dim_ffn, tiles=tiles)
+    out = torch.full_like(x, torch.nan)
+    assert ops.moe_dense_mlp(x, *tables, dim_ffn, out=out) is out
+    assert torch.equal(out, listed) and torch.equal(ops.moe_dense_mlp(x, *tables, dim_ffn), listed)
