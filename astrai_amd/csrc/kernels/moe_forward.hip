@@ -171,13 +171,16 @@ extern "C" int astrai_moe_forward(const void* x, const void* logits, const void*
 
 // One dense expert (MLP.forward, mlp.py:22-25) in one call. A decoding batch
 // needs neither the tile list (5 us to write and wait for, of 82 us at 24 rows
-// of D 4096, F 14336) nor its allocations.
+// of D 4096, F 14336) nor its allocations (8 rows of D 2048, F 5632, bound by the
+// host with the separate calls, 28 -> 23 us; D 704, F 576, 800 rows 27 -> 18). More
+// rows have a list for each GEMM, of the height it runs fastest on.
 namespace astrai_moe {
 namespace {
 
 struct DensePlan {
-  int block_m;
-  int64_t tiles_len, tiles, h, gemm_ws, gemm_ws_bytes, bytes;
+  int block_m, block_m_down;
+  bool few;  // (x and out allowing) both GEMMs on the few-row kernels
+  int64_t len, len_down, tiles, tiles_down, h, gemm_ws, gemm_ws_bytes, bytes;
 };
 
 int check_dense(int64_t n_rows, int64_t dim, int64_t dim_ffn, int dtype) {
@@ -189,16 +192,28 @@ int check_dense(int64_t n_rows, int64_t dim, int64_t dim_ffn, int dtype) {
 
 DensePlan dense_plan(int64_t n_rows, int64_t dim, int64_t dim_ffn, int dtype) {
   DensePlan p{};
-  p.block_m = astrai_moe_select_block_m(n_rows, 1, 1, dim, dim_ffn, dtype);
-  p.tiles_len = astrai_moe_tile_list_len(n_rows, 1, 1, p.block_m);
+  p.block_m = p.block_m_down = astrai_moe_select_block_m(n_rows, 1, 1, dim, dim_ffn, dtype);
+  if (dtype == ASTRAI_MOE_BF16 && mfma_shape_supported(dim, dim_ffn)) {
+    const bool few_up = few_rows(n_rows, 1, p.block_m, dim, dim_ffn, true);
+    const bool few_down = few_rows(n_rows, 1, p.block_m, dim_ffn, dim, false);
+    p.few = few_up && few_down;
+    if (p.block_m > kMfmaSmallBM) {
+      if (!few_up) p.block_m = dense_gemm_block_m(n_rows, dim, dim_ffn, true);
+      if (!few_down) p.block_m_down = dense_gemm_block_m(n_rows, dim_ffn, dim, false);
+    }
+  }
+  p.len = astrai_moe_tile_list_len(n_rows, 1, 1, p.block_m);
+  p.len_down = p.block_m_down == p.block_m ? 0 : astrai_moe_tile_list_len(n_rows, 1, 1, p.block_m_down);
   auto part = [&](int64_t bytes) {
     const int64_t here = p.bytes;
     p.bytes += (bytes + 255) / 256 * 256;
     return here;
   };
-  p.tiles = part(p.tiles_len * 4);
+  p.tiles = part(p.len * 4);
+  p.tiles_down = p.len_down > 0 ? part(p.len_down * 4) : p.tiles;
   p.h = part(n_rows * dim_ffn * (dtype == ASTRAI_MOE_BF16 ? 2 : 4));
-  if (p.block_m == kMfmaBigBM) p.gemm_ws_bytes = gemm_workspace_bytes(dim_ffn >= 64 * 64);
+  if (p.block_m == kMfmaBigBM || p.block_m_down == kMfmaBigBM)
+    p.gemm_ws_bytes = gemm_workspace_bytes(p.block_m_down == kMfmaBigBM && dim_ffn >= 64 * 64);
   p.gemm_ws = part(p.gemm_ws_bytes);
   return p;
 }
@@ -228,17 +243,20 @@ extern "C" int astrai_moe_dense_forward(const void* x, const void* const* w_gate
                  (long long)workspace_bytes, (long long)p.bytes);
   char* const base = static_cast<char*>(workspace);
   int32_t* const tiles = reinterpret_cast<int32_t*>(base + p.tiles);
+  int32_t* const tiles_down = reinterpret_cast<int32_t*>(base + p.tiles_down);
   void* const h = base + p.h;
   void* const gws = p.gemm_ws_bytes > 0 ? base + p.gemm_ws : nullptr;
-  if (dtype == ASTRAI_MOE_BF16 && mfma_gate_up_supported(dim, dim_ffn, p.block_m, x, h) &&
-      mfma_down_supported(dim_ffn, dim, p.block_m, h, out) && few_rows(n_rows, 1, p.block_m, dim, dim_ffn, true) &&
-      few_rows(n_rows, 1, p.block_m, dim_ffn, dim, false))
+  if (p.few && mfma_gate_up_supported(dim, dim_ffn, p.block_m, x, h) &&
+      mfma_down_supported(dim_ffn, dim, p.block_m, h, out))
     return launch_few_dense(x, w_gate, w_up, w_down, n_rows, dim, dim_ffn, p.block_m, h, out,
                             static_cast<hipStream_t>(stream));
-  if ((rc = astrai_moe_dense_tiles(n_rows, p.block_m, tiles, p.tiles_len, nullptr, stream))) return rc;
-  if ((rc = astrai_moe_gemm_gate_up(x, tiles, p.tiles_len, w_gate, w_up, dtype, n_rows, 1, dim, dim_ffn, p.block_m, h,
-                                    gws, p.gemm_ws_bytes, stream)))
+  const int64_t len_down = p.len_down > 0 ? p.len_down : p.len;
+  if ((rc = launch_dense_tiles(n_rows, p.block_m, p.len, tiles, p.block_m_down, p.len_down, tiles_down,
+                               static_cast<hipStream_t>(stream))))
     return rc;
-  return astrai_moe_gemm_down(h, tiles, p.tiles_len, w_down, nullptr, dtype, n_rows, 1, dim_ffn, dim, p.block_m, out,
-                              gws, p.gemm_ws_bytes, stream);
+  if ((rc = astrai_moe_gemm_gate_up(x, tiles, p.len, w_gate, w_up, dtype, n_rows, 1, dim, dim_ffn, p.block_m, h, gws,
+                                    p.gemm_ws_bytes, stream)))
+    return rc;
+  return astrai_moe_gemm_down(h, tiles_down, len_down, w_down, nullptr, dtype, n_rows, 1, dim_ffn, dim, p.block_m_down,
+                              out, gws, p.gemm_ws_bytes, stream);
 }

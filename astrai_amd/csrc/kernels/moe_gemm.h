@@ -50,6 +50,9 @@ bool mfma_gate_up_supported(int64_t dim, int64_t dim_ffn, int block_m,
 bool mfma_down_supported(int64_t dim_ffn, int64_t dim, int block_m,
                          const void* a, const void* c);
 
+// Row-tile height of the list for one GEMM of a dense expert (96 rows or more).
+int dense_gemm_block_m(int64_t n_rows, int64_t k, int64_t n, bool gate_up);
+
 // `packed`: the weight tables point at packed copies written by launch_pack
 // (bf16, 256-row tiles of K / 64 contiguous 32 KB blocks in staged order).
 int launch_mfma_gate_up(const void* x_perm, const int32_t* tiles,
@@ -128,6 +131,12 @@ int launch_few_dense(const void* x, const void* const* w_gate,
                      const void* const* w_up, const void* const* w_down,
                      int64_t n_rows, int64_t dim, int64_t dim_ffn, int block_m,
                      void* h, void* out, hipStream_t s);
+
+// The tile lists of one dense expert for two GEMMs (moe_permute.hip); the second
+// only where len_down > 0.
+int launch_dense_tiles(int64_t n_rows, int block_m, int64_t len, int32_t* tiles,
+                       int block_m_down, int64_t len_down, int32_t* tiles_down,
+                       hipStream_t s);
 
 // Training forward (256-row tiles): as launch_mfma_gate_up / launch_mfma_down,
 // also storing the bf16 gate and up projections (gu: [rows, 2 dim_ffn],

@@ -1057,6 +1057,8 @@ using Mid2Cfg = TileCfg<kMfmaMid2BM, 256, 3, 1, 8, 8>;
 // bandwidth bounds a step (96 KB of fragments read and 32 KB written for 0.21 us
 // of MFMA), but twice as many compute units work on a GEMM as with 256 columns.
 using NarrowCfg = TileCfg<kMfmaMid2BM, 128, 4, 2, 4, 8>;
+// The same of 64-row lists: 64 x 128 outputs, 4 waves of 64 x 32, three stages.
+using NarrowMidCfg = TileCfg<kMfmaMidBM, 128, 3, 1, 4, 8>;
 static_assert(StreamCfg<true>::BM == kMfmaBigBM && StreamCfg<false>::BM == kMfmaBigBM, "prefill tile height");
 
 // Clears the run-time claim counter of a streaming launch's scheduling
@@ -1131,12 +1133,13 @@ double expected_row_tiles(int64_t n_rows, int n_experts, int bm) {
 // Which tiles a GEMM takes on a list of 128- or 256-row tiles: the list's own
 // with 256 columns (gate/up: 128 of each), or, where those leave compute units
 // idle, 128 rows by 128 columns, and on a 256-row list also 128 by 256.
-enum class Tiles { kList, kHalves, kNarrow, kNarrowHalves };
+// (64-row lists: 64 by 128.)
+enum class Tiles { kList, kHalves, kNarrow, kNarrowHalves, kNarrowMid };
 
 // A GEMM of few tiles takes rounds of its compute units times a tile's K steps,
 // however few the tiles of the last round: 1.4 us a step of a 256 x 256 tile,
-// 1.07 of 128 x 256, 0.71 of 128 x 128 (measured; the small tiles pay more per
-// flop, and lose once two tiles of theirs share a compute unit). Taken where
+// 1.07 of 128 x 256, 0.83 of 64 x 256, 0.71 of 128 x 128, 0.55 of 64 x 128
+// (measured; the small tiles pay more per flop). Taken where
 // this promises a tenth; only within kFewRounds rounds of the list's own tiles,
 // past which the shares are even and the memory system decides. 256-row tiles of
 // kSplitMinTileSteps steps keep their kernel, which splits its last round.
@@ -1149,23 +1152,32 @@ enum class Tiles { kList, kHalves, kNarrow, kNarrowHalves };
 //   21 / 17.5 at 130 to 256); D 2048, F 1408, 64 rows 27 / 20, 130 37 / 29 (halves),
 //   256 (a third more row tiles than places in a round) 42 / 44 if taken;
 // - one expert, D 4096, F 14336, 512 rows 180 / 127, 1024 191 / 141; D 2048, F 5632,
-//   1500 rows 81 / 55.
+//   1500 rows 81 / 55, 300 rows (64-row list) 73 / 35.
 constexpr double kFewRounds = 2.0;
-Tiles pick_tiles(int64_t n_rows, int n_experts, int block_m, int64_t k, int64_t n, bool gate_up) {
-  if (block_m != kMfmaMid2BM && (block_m != kMfmaBigBM || k_steps(k) >= kSplitMinTileSteps)) return Tiles::kList;
-  const double cu = cu_count();
+struct Pick {
+  Tiles tiles;
+  double us_per_step;  // rounds times a step's time
+};
+Pick pick_tiles(int64_t n_rows, int n_experts, int block_m, int64_t k, int64_t n, bool gate_up) {
+  const double cu = cu_count(), step = block_m == kMfmaBigBM ? 1.4 : block_m == kMfmaMid2BM ? 1.07 : 0.83;
   const double wide = (double)ceil_div(n, gate_up ? 128 : 256), narrow = (double)ceil_div(n, gate_up ? 64 : 128);
-  if ((double)n_rows / block_m * wide > kFewRounds * cu) return Tiles::kList;  // (bounds the sum below)
-  const double own = expected_row_tiles(n_rows, n_experts, block_m) * wide;
-  if (own > kFewRounds * cu) return Tiles::kList;
-  // (a tile without a second half still takes its place in the walk)
-  const double rows128 = (block_m == kMfmaBigBM ? 2.0 : 1.0) * expected_row_tiles(n_rows, n_experts, block_m);
-  const double t_own = std::ceil(own / cu) * (block_m == kMfmaBigBM ? 1.4 : 1.07);
-  const double t_wide = block_m == kMfmaBigBM ? std::ceil(rows128 * wide / cu) * 1.07 : t_own;
-  const double t_narrow = std::ceil(rows128 * narrow / cu) * 0.71;
-  if (t_narrow <= t_wide && t_narrow < 0.9 * t_own)
-    return block_m == kMfmaBigBM ? Tiles::kNarrowHalves : Tiles::kNarrow;
-  return t_wide < 0.9 * t_own ? Tiles::kHalves : Tiles::kList;
+  const double least = (double)n_rows / block_m * wide;  // (bounds the sum below)
+  if (block_m < kMfmaMidBM || least > kFewRounds * cu) return {Tiles::kList, std::ceil(least / cu) * step};
+  const double row_tiles = expected_row_tiles(n_rows, n_experts, block_m), rounds = std::ceil(row_tiles * wide / cu);
+  const Pick own{Tiles::kList, rounds * step};
+  if (row_tiles * wide > kFewRounds * cu || (block_m == kMfmaBigBM && k_steps(k) >= kSplitMinTileSteps)) return own;
+  // 128-row halves of a 256-row tile: one without a second half still takes its
+  // place in the walk
+  const double halves = block_m == kMfmaBigBM ? 2.0 * row_tiles : row_tiles;
+  const double t_wide = block_m == kMfmaBigBM ? std::ceil(halves * wide / cu) * 1.07 : own.us_per_step;
+  const double t_narrow = std::ceil(halves * narrow / cu) * (block_m == kMfmaMidBM ? 0.55 : 0.71);
+  if (t_narrow <= t_wide && t_narrow < 0.9 * own.us_per_step)
+    return {block_m == kMfmaBigBM    ? Tiles::kNarrowHalves
+            : block_m == kMfmaMid2BM ? Tiles::kNarrow
+                                     : Tiles::kNarrowMid,
+            t_narrow};
+  if (t_wide < 0.9 * own.us_per_step) return {Tiles::kHalves, t_wide};
+  return own;
 }
 
 template <bool kGateUp, bool kGather = false>
@@ -1174,6 +1186,8 @@ int launch_picked(Tiles pick, const void* A, const int32_t* tiles, int64_t capac
                   const int32_t* row_src = nullptr) {
   if (pick == Tiles::kHalves)
     return launch<Mid2Cfg, kGateUp, false, kGather, true>(A, tiles, capacity, W0, W1, row_w, K, N, C, s, row_src);
+  if (pick == Tiles::kNarrowMid)
+    return launch<NarrowMidCfg, kGateUp, false, kGather>(A, tiles, capacity, W0, W1, row_w, K, N, C, s, row_src);
   if (pick == Tiles::kNarrow)
     return launch<NarrowCfg, kGateUp, false, kGather>(A, tiles, capacity, W0, W1, row_w, K, N, C, s, row_src);
   return launch<NarrowCfg, kGateUp, false, kGather, true>(A, tiles, capacity, W0, W1, row_w, K, N, C, s, row_src);
@@ -1184,7 +1198,7 @@ int gate_up_dispatch(const void* x_perm, const int32_t* tiles, int64_t capacity,
                      const void* const* w_up, int64_t n_rows, int n_experts, int64_t dim, int64_t dim_ffn,
                      int block_m, void* h, hipStream_t s, const GemmWorkspace& ws) {
   if constexpr (!kPacked) {
-    const Tiles pick = pick_tiles(n_rows, n_experts, block_m, dim, dim_ffn, true);
+    const Tiles pick = pick_tiles(n_rows, n_experts, block_m, dim, dim_ffn, true).tiles;
     if (pick != Tiles::kList)
       return launch_picked<true>(pick, x_perm, tiles, capacity, w_gate, w_up, nullptr, dim, dim_ffn, h, s);
   }
@@ -1203,7 +1217,7 @@ int down_dispatch(const void* h, const int32_t* tiles, int64_t capacity, const v
                   const void* sorted_w, int64_t n_rows, int n_experts, int64_t dim_ffn, int64_t dim, int block_m,
                   void* y, hipStream_t s, const GemmWorkspace& ws) {
   if constexpr (!kPacked) {
-    const Tiles pick = pick_tiles(n_rows, n_experts, block_m, dim_ffn, dim, false);
+    const Tiles pick = pick_tiles(n_rows, n_experts, block_m, dim_ffn, dim, false).tiles;
     if (pick != Tiles::kList)
       return launch_picked<false>(pick, h, tiles, capacity, w_down, nullptr, sorted_w, dim_ffn, dim, y, s);
   }
@@ -1228,6 +1242,21 @@ bool mfma_gate_up_supported(int64_t dim, int64_t dim_ffn, int block_m, const voi
   return (block_m == kMfmaBigBM || block_m == kMfmaMid2BM || block_m == kMfmaMidBM || block_m == kMfmaSmallBM) &&
          mfma_k_supported(dim) && dim_ffn > 0 && dim_ffn % 8 == 0 && dim <= (1ll << 22) &&
          dim_ffn <= (1ll << 22) && aligned16(a) && aligned16(c);
+}
+
+// The list height of one expert's GEMM of at least 96 rows: the least time by
+// pick_tiles' measure, a shorter tile only for a twentieth less. The two GEMMs of
+// an MLP want different ones (us on lists of 64, 128, 256 rows): D 2048, F 5632,
+// 800 rows gate/up 59, 61, 43, down 36, 43, 90; D 4096, F 14336, 1024 rows 273,
+// 238, 185 and 131, 120, 219; D 1536, F 4096, 1280 rows 48, 51, 34 and 28, 33, 71.
+int dense_gemm_block_m(int64_t n_rows, int64_t k, int64_t n, bool gate_up) {
+  int best = kMfmaBigBM;
+  double least = pick_tiles(n_rows, 1, best, k, n, gate_up).us_per_step;
+  for (int bm : {kMfmaMid2BM, kMfmaMidBM}) {
+    const double t = pick_tiles(n_rows, 1, bm, k, n, gate_up).us_per_step;
+    if (t < 0.95 * least) best = bm, least = t;
+  }
+  return best;
 }
 
 int64_t gemm_workspace_bytes(bool down) {
@@ -1303,7 +1332,7 @@ int launch_mfma_gate_up_gather(const void* x, const int32_t* sorted_token, const
                                const void* const* w_gate, const void* const* w_up, int64_t n_rows, int n_experts,
                                int64_t dim, int64_t dim_ffn, int block_m, void* h, hipStream_t s,
                                const GemmWorkspace& ws) {
-  const Tiles pick = pick_tiles(n_rows, n_experts, block_m, dim, dim_ffn, true);
+  const Tiles pick = pick_tiles(n_rows, n_experts, block_m, dim, dim_ffn, true).tiles;
   if (pick != Tiles::kList)
     return launch_picked<true, true>(pick, x, tiles, capacity, w_gate, w_up, nullptr, dim, dim_ffn, h, s, sorted_token);
   if (block_m == kMfmaBigBM)

@@ -48,9 +48,11 @@
 //                   top_k destinations with 16-byte vector accesses. Column
 //                   splits keep enough workgroups in flight when there are
 //                   few tokens (decode).
+#include <algorithm>
 #include <mutex>
 
 #include "moe_common.h"
+#include "moe_gemm.h"
 
 namespace astrai_moe {
 namespace {
@@ -563,11 +565,19 @@ __global__ __launch_bounds__(kScatterThreads) void scatter_kernel(
 // Tile list of one dense expert over n_rows rows (expert 0 owns every row),
 // for running the shared experts and the standalone MLP on the grouped GEMMs;
 // optionally the matching expert offsets {0, n_rows}. Built on the device so
-// that a captured graph owns it like any other output of the forward.
-__global__ __launch_bounds__(256) void dense_tiles_kernel(
-    int64_t n_rows, int block_m, int64_t tile_capacity,
-    int32_t* __restrict__ tiles, int32_t* __restrict__ offsets) {
-  const int64_t n_tiles = ceil_div(n_rows, block_m);
+// that a captured graph owns it like any other output of the forward. A grid
+// with blockIdx.y = 1 also writes the list `down` of another height.
+struct DenseList {
+  int32_t* tiles;
+  int64_t capacity;
+  int block_m;
+};
+__global__ __launch_bounds__(256) void dense_tiles_kernel(int64_t n_rows, DenseList up, DenseList down,
+                                                          int32_t* __restrict__ offsets) {
+  const DenseList list = blockIdx.y == 0 ? up : down;
+  int32_t* const tiles = list.tiles;
+  const int block_m = list.block_m;
+  const int64_t tile_capacity = list.capacity, n_tiles = ceil_div(n_rows, block_m);
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i == 0) {
     tiles[0] = (int32_t)n_tiles;
@@ -817,6 +827,8 @@ extern "C" int astrai_moe_permute_noalloc(
                       x_perm, tiles, tiles_len, nullptr, true, stream);
 }
 
+static int64_t tile_capacity(int64_t len) { return (len - ASTRAI_MOE_TILE_HEADER) / ASTRAI_MOE_TILE_STRIDE; }
+
 extern "C" int astrai_moe_dense_tiles(int64_t n_rows, int block_m,
                                       int32_t* tiles, int64_t tiles_len,
                                       int32_t* expert_offsets, void* stream) {
@@ -830,12 +842,21 @@ extern "C" int astrai_moe_dense_tiles(int64_t n_rows, int block_m,
                  "dense_tiles: tile list holds %lld int32, needs %lld",
                  (long long)tiles_len, (long long)need);
   ASTRAI_REQUIRE(tiles != nullptr, "dense_tiles: null tile list");
-  const int64_t capacity =
-      (tiles_len - ASTRAI_MOE_TILE_HEADER) / ASTRAI_MOE_TILE_STRIDE;
+  const DenseList list{tiles, tile_capacity(tiles_len), block_m};
   const int64_t n_tiles = ceil_div(n_rows, block_m);
   const int64_t grid = n_tiles > 0 ? ceil_div(n_tiles, 256) : 1;
   hipLaunchKernelGGL(dense_tiles_kernel, dim3((unsigned)grid), dim3(256), 0,
-                     static_cast<hipStream_t>(stream), n_rows, block_m,
-                     capacity, tiles, expert_offsets);
+                     static_cast<hipStream_t>(stream), n_rows, list, list, expert_offsets);
   return check_launch("dense_tiles_kernel");
 }
+
+namespace astrai_moe {
+int launch_dense_tiles(int64_t n_rows, int block_m, int64_t len, int32_t* tiles, int block_m_down, int64_t len_down,
+                       int32_t* tiles_down, hipStream_t s) {
+  const DenseList up{tiles, tile_capacity(len), block_m}, down{tiles_down, tile_capacity(len_down), block_m_down};
+  const int64_t grid = ceil_div(ceil_div(n_rows, std::min(block_m, block_m_down)), 256);
+  hipLaunchKernelGGL(dense_tiles_kernel, dim3((unsigned)grid, len_down > 0 ? 2 : 1), dim3(256), 0, s, n_rows, up, down,
+                     static_cast<int32_t*>(nullptr));
+  return check_launch("dense_tiles_kernel");
+}
+}  // namespace astrai_moe

@@ -43,10 +43,12 @@ def test_layer(gpu, n_tok, n_exp, top_k, n_shared):
 
 
 @pytest.mark.parametrize("dim,dim_ffn", [(64, 64), (72, 328), (512, 1408), (1536, 4096)])
-@pytest.mark.parametrize("n_tok", [0, 1, 32, 33, 64, 65, 95, 96, 128, 129, 256, 257])
+@pytest.mark.parametrize("n_tok", [0, 1, 32, 33, 64, 65, 95, 96, 128, 129, 256, 257, 900])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_one_call_is_the_listed_calls(gpu, n_tok, dim, dim_ffn, dtype):
-    # one dense expert without a tile list (few rows) and with one: the same bits
+    # one dense expert without a tile list (few rows), or with one of each
+    # GEMM's own height (900 rows of 1536, 4096: 256 and 64), and with one list:
+    # the same bits
     torch.manual_seed(n_tok)
     ws = [(torch.randn(*s, device=gpu) * 0.05).to(dtype) for s in ((dim_ffn, dim), (dim_ffn, dim), (dim, dim_ffn))]
     tables = [ops.expert_weight_table([w], tuple(w.shape)) for w in ws]
