@@ -405,7 +405,7 @@ int astrai_moe_dense_forward(const void* x, const void* const* w_gate,
  * The reference gets its gradients from torch autograd over mlp.py:22-25
  * and :89-98; these entry points compute the same quantities with grouped
  * kernels, at autograd's rounding points (identities in fp32): on the matrix
- * cores for bf16 with dim and dim_ffn multiples of 64 (tile lists built with
+ * cores for bf16 with dim and dim_ffn multiples of 8 from 64 on (tile lists built with
  * block_m = 256); for fp32 on the fp32 matrix cores with block_m = 64 where
  * the GEMM's K is a multiple of 32 and its output columns of 4 (the forward
  * GEMMs as astrai_moe_gemm_gate_up / _down choose them); on the general-shape
