@@ -28,7 +28,7 @@ struct Sizes {
 struct Plan {
   int experts, slots, block_m;
   int64_t rows, tiles_len;
-  bool gather, gather_f32;
+  bool gather, gather_ragged, gather_f32;
   int64_t topk_idx, topk_w, chunk_hist, chunk_base, offsets, sorted_token, sorted_w, token_pos, tiles, x_perm, h, y,
       gemm_ws, gemm_ws_bytes, bytes;
 };
@@ -60,6 +60,10 @@ Plan make_plan(const Sizes& z) {
   // (32-bit row offsets: x under 4 GiB)
   p.gather = z.dtype == ASTRAI_MOE_BF16 && !z.packed && mfma_shape_supported(z.dim, z.dim_ffn) && z.dim % 64 == 0 &&
              z.dim_ffn % 64 == 0 && T * z.dim * 2 < (1ll << 32);
+  // (other dims: where x is aligned, below; 1500 tokens of D 1000, F 2664 with a
+  // shared expert 162 us a layer with copied rows, 149 without)
+  p.gather_ragged = z.dtype == ASTRAI_MOE_BF16 && !z.packed && mfma_shape_supported(z.dim, z.dim_ffn) && !p.gather &&
+                    T * z.dim * 2 < (1ll << 32);
   p.gather_f32 = z.dtype == ASTRAI_MOE_F32 && T * z.dim * 4 < (1ll << 32) &&
                  mfma_f32_supported(z.dim, z.dim_ffn, true, p.block_m, nullptr, nullptr, nullptr);
   int64_t at = 0;
@@ -77,7 +81,8 @@ Plan make_plan(const Sizes& z) {
   p.sorted_w = part(p.rows * size);
   p.token_pos = part(p.rows * 4);
   p.tiles = part(p.tiles_len * 4);
-  // (an fp32 x off the 16-byte grid is copied after all: it needs the place)
+  // (such an x, or an fp32 one, off the 16-byte grid is copied after all: it
+  // needs the place)
   p.x_perm = p.gather ? 0 : part(p.rows * z.dim * size);
   p.h = part(p.rows * z.dim_ffn * size);
   p.y = part(p.rows * z.dim * size);
@@ -125,8 +130,9 @@ extern "C" int astrai_moe_forward(const void* x, const void* logits, const void*
   int32_t *topk_idx = i32(p.topk_idx), *hist = i32(p.chunk_hist), *sorted_token = i32(p.sorted_token),
           *token_pos = i32(p.token_pos), *tiles = i32(p.tiles);
   void *topk_w = base + p.topk_w, *sorted_w = base + p.sorted_w, *h = base + p.h, *y = base + p.y;
-  const bool gather_f32 = p.gather_f32 && reinterpret_cast<uintptr_t>(x) % 16 == 0;
-  void* const x_perm = p.gather || gather_f32 ? nullptr : base + p.x_perm;
+  const bool x_aligned = reinterpret_cast<uintptr_t>(x) % 16 == 0;
+  const bool gather = p.gather || (p.gather_ragged && x_aligned), gather_f32 = p.gather_f32 && x_aligned;
+  void* const x_perm = gather || gather_f32 ? nullptr : base + p.x_perm;
   void* const gws = p.gemm_ws_bytes > 0 ? base + p.gemm_ws : nullptr;
   hipStream_t s = static_cast<hipStream_t>(stream);
 
@@ -144,9 +150,9 @@ extern "C" int astrai_moe_forward(const void* x, const void* logits, const void*
                             i32(p.chunk_base), stream);
   }
   if (rc) return rc;
-  if (p.gather)
-    rc = astrai_moe_gemm_gate_up_gather(x, sorted_token, n_tokens, tiles, p.tiles_len, w_gate, w_up, dtype, p.rows,
-                                        p.experts, dim, dim_ffn, p.block_m, h, gws, p.gemm_ws_bytes, stream);
+  if (gather)
+    rc = launch_gate_up_gather(x, sorted_token, tiles, p.tiles_len, w_gate, w_up, p.rows, p.experts, dim, dim_ffn,
+                               p.block_m, h, GemmWorkspace{gws, p.gemm_ws_bytes}, s);
   else if (gather_f32)
     rc = launch_mfma_f32_gate_up(x, tiles, (p.tiles_len - ASTRAI_MOE_TILE_HEADER) / ASTRAI_MOE_TILE_STRIDE, w_gate, w_up,
                                  p.rows, p.experts, dim, dim_ffn, h, nullptr, s, sorted_token);

@@ -81,6 +81,13 @@ int launch_mfma_down(const void* h, const int32_t* tiles, int64_t capacity,
                      int64_t n_rows, int n_experts, int64_t dim_ffn,
                      int64_t dim, int block_m, bool packed,
                      void* y, hipStream_t s, const GemmWorkspace& ws);
+int launch_mfma_gate_up_gather(const void* x, const int32_t* sorted_token,
+                               const int32_t* tiles, int64_t capacity,
+                               const void* const* w_gate,
+                               const void* const* w_up, int64_t n_rows,
+                               int n_experts, int64_t dim, int64_t dim_ffn,
+                               int block_m, void* h, hipStream_t s,
+                               const GemmWorkspace& ws);
 int launch_mfma_gate_up_save(const void* x_perm, const int32_t* tiles,
                              int64_t capacity, const void* const* w_gate,
                              const void* const* w_up, int64_t dim,
@@ -109,6 +116,15 @@ int launch_mfma_gate_up_gather(const void* x, const int32_t* sorted_token,
                                int n_experts, int64_t dim, int64_t dim_ffn,
                                int block_m, void* h, hipStream_t s,
                                const GemmWorkspace& ws = {});
+
+// The gathering gate/up GEMM on the kernel its sizes take (few rows or the
+// above); x and h aligned to 16 bytes, x under 4 GiB.
+int launch_gate_up_gather(const void* x, const int32_t* sorted_token,
+                          const int32_t* tiles, int64_t tiles_len,
+                          const void* const* w_gate, const void* const* w_up,
+                          int64_t n_rows, int n_experts, int64_t dim,
+                          int64_t dim_ffn, int block_m, void* h,
+                          const GemmWorkspace& ws, hipStream_t s);
 
 // Few rows (moe_gemm_few.hip), tiles below 256 rows: whether the kernels there
 // take a GEMM of n_rows rows over n_experts experts with k inputs

@@ -219,6 +219,18 @@ extern "C" int astrai_moe_gemm_gate_up(const void* x_perm, const int32_t* tiles,
                                      nullptr, dim, dim_ffn, h, s);
 }
 
+int astrai_moe::launch_gate_up_gather(const void* x, const int32_t* sorted_token, const int32_t* tiles,
+                                      int64_t tiles_len, const void* const* w_gate, const void* const* w_up,
+                                      int64_t n_rows, int n_experts, int64_t dim, int64_t dim_ffn, int block_m, void* h,
+                                      const GemmWorkspace& ws, hipStream_t s) {
+  const int64_t capacity = (tiles_len - ASTRAI_MOE_TILE_HEADER) / ASTRAI_MOE_TILE_STRIDE;
+  if (few_rows(n_rows, n_experts, block_m, dim, dim_ffn, true))
+    return launch_few_gate_up(x, sorted_token, tiles, capacity, w_gate, w_up, n_rows, n_experts, dim, dim_ffn, false, h,
+                              s);
+  return launch_mfma_gate_up_gather(x, sorted_token, tiles, capacity, w_gate, w_up, n_rows, n_experts, dim, dim_ffn,
+                                    block_m, h, s, ws);
+}
+
 extern "C" int astrai_moe_gemm_gate_up_gather(const void* x, const int32_t* sorted_token, int64_t n_tokens,
                                               const int32_t* tiles, int64_t tiles_len, const void* const* w_gate,
                                               const void* const* w_up, int dtype, int64_t n_rows, int n_experts,
@@ -238,12 +250,8 @@ extern "C" int astrai_moe_gemm_gate_up_gather(const void* x, const int32_t* sort
                  "gemm_gate_up_gather: unsupported shape (dim %lld, dim_ffn %lld, block_m %d) or alignment",
                  (long long)dim, (long long)dim_ffn, block_m);
   ASTRAI_REQUIRE(sorted_token && w_gate && w_up, "gemm_gate_up_gather: null row list or weight table");
-  const int64_t capacity = (tiles_len - ASTRAI_MOE_TILE_HEADER) / ASTRAI_MOE_TILE_STRIDE;
-  if (few_rows(n_rows, n_experts, block_m, dim, dim_ffn, true))
-    return launch_few_gate_up(x, sorted_token, tiles, capacity, w_gate, w_up, n_rows, n_experts, dim, dim_ffn, false, h,
-                              static_cast<hipStream_t>(stream));
-  return launch_mfma_gate_up_gather(x, sorted_token, tiles, capacity, w_gate, w_up, n_rows, n_experts, dim, dim_ffn, block_m, h,
-                                    static_cast<hipStream_t>(stream), GemmWorkspace{workspace, workspace_bytes});
+  return launch_gate_up_gather(x, sorted_token, tiles, tiles_len, w_gate, w_up, n_rows, n_experts, dim, dim_ffn, block_m, h,
+                               GemmWorkspace{workspace, workspace_bytes}, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int astrai_moe_gemm_down(const void* h, const int32_t* tiles,

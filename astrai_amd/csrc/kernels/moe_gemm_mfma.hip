@@ -1324,14 +1324,15 @@ int launch_mfma_down_save(const void* h, const int32_t* tiles, int64_t capacity,
                                            y_unweighted, nullptr, nullptr, ws);
 }
 
-#if ASTRAI_MOE_RAGGED_K
-}  // namespace ragged
-#else
-
 int launch_mfma_gate_up_gather(const void* x, const int32_t* sorted_token, const int32_t* tiles, int64_t capacity,
                                const void* const* w_gate, const void* const* w_up, int64_t n_rows, int n_experts,
                                int64_t dim, int64_t dim_ffn, int block_m, void* h, hipStream_t s,
                                const GemmWorkspace& ws) {
+#if !ASTRAI_MOE_RAGGED_K
+  if (dim % kBK != 0)
+    return ragged::launch_mfma_gate_up_gather(x, sorted_token, tiles, capacity, w_gate, w_up, n_rows, n_experts, dim,
+                                              dim_ffn, block_m, h, s, ws);
+#endif
   const Tiles pick = pick_tiles(n_rows, n_experts, block_m, dim, dim_ffn, true).tiles;
   if (pick != Tiles::kList)
     return launch_picked<true, true>(pick, x, tiles, capacity, w_gate, w_up, nullptr, dim, dim_ffn, h, s, sorted_token);
@@ -1347,6 +1348,10 @@ int launch_mfma_gate_up_gather(const void* x, const int32_t* sorted_token, const
   return launch<SmallCfg, true, false, true>(x, tiles, capacity, w_gate, w_up, nullptr, dim, dim_ffn, h, s,
                                              sorted_token);
 }
+
+#if ASTRAI_MOE_RAGGED_K
+}  // namespace ragged
+#else
 
 int launch_pack(const void* w0, const void* w1, int64_t rows, int64_t k, bool gate_up, void* out, hipStream_t s) {
   // rows: output rows of the projection (dim_ffn for gate/up, each; dim for down)

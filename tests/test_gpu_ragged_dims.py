@@ -53,3 +53,13 @@ def test_unaligned_rows_still_run(gpu):
     x = flat[4:4 + 65 * 1000].view(1, 65, 1000)
     assert x.data_ptr() % 16 == 8
     check_layer(layer, x, "unaligned")
+
+
+@pytest.mark.parametrize("dim,dim_ffn", [(72, 328), (1000, 424), (2056, 136)])
+@pytest.mark.parametrize("n_tok", [1, 32, 33, 300, 1400])
+def test_gathered_rows_are_the_copied_ones(gpu, n_tok, dim, dim_ffn):
+    # the one-call forward reads the token rows itself, the separate calls copy them
+    layer = _random_layer(gpu, dim, dim_ffn, 4, 0, 2, torch.bfloat16, seed=n_tok).requires_grad_(False)
+    x = torch.randn(1, n_tok, dim, device=gpu).to(torch.bfloat16)
+    assert not ops.gather_supported(n_tok, dim, dim_ffn, x.dtype)
+    assert torch.equal(layer(x)[0], layer._routed_forward(x[0], layer._current(x.dtype, x.device)))
