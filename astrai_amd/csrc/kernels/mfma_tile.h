@@ -185,10 +185,6 @@ struct TileWalk {
 // like tiles: item i < full is logical tile i, item full + u is unit u (tile
 // full + u / S, slice u % S).
 constexpr int kSplitMinSteps = 8;
-// Tiles of fewer K steps are never split: the reduce launch and the partial
-// sums' traffic (~15 us at 16 tiles) cost about what splitting a short tile
-// saves (the fine-grained shape's 22-step down tiles take ~31 us).
-constexpr int kSplitMinTileSteps = 64;
 constexpr int kSplitUnitFloats = kMfmaBigBM * 256;  // fp32 accumulators of one 256 x 256 tile
 
 template <int GM>

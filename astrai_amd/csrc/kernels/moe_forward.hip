@@ -88,7 +88,7 @@ Plan make_plan(const Sizes& z) {
   p.y = part(p.rows * z.dim * size);
   // the 256-row GEMMs' scheduling block, and partial sums where the down
   // GEMM's tiles are long enough to be split
-  if (p.block_m == kMfmaBigBM) p.gemm_ws_bytes = gemm_workspace_bytes(z.dim_ffn >= 64 * 64);
+  if (p.block_m == kMfmaBigBM) p.gemm_ws_bytes = gemm_workspace_bytes(splits_tail(z.dim_ffn));
   p.gemm_ws = part(p.gemm_ws_bytes);
   p.bytes = at;
   return p;
@@ -219,7 +219,7 @@ DensePlan dense_plan(int64_t n_rows, int64_t dim, int64_t dim_ffn, int dtype) {
   p.tiles_down = p.len_down > 0 ? part(p.len_down * 4) : p.tiles;
   p.h = part(n_rows * dim_ffn * (dtype == ASTRAI_MOE_BF16 ? 2 : 4));
   if (p.block_m == kMfmaBigBM || p.block_m_down == kMfmaBigBM)
-    p.gemm_ws_bytes = gemm_workspace_bytes(p.block_m_down == kMfmaBigBM && dim_ffn >= 64 * 64);
+    p.gemm_ws_bytes = gemm_workspace_bytes(p.block_m_down == kMfmaBigBM && splits_tail(dim_ffn));
   p.gemm_ws = part(p.gemm_ws_bytes);
   return p;
 }

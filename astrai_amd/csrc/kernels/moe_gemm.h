@@ -32,6 +32,14 @@ struct GemmWorkspace {
   int64_t bytes = 0;
 };
 constexpr int64_t kSchedBytes = 65536;
+// Tiles of fewer K steps (of 64) are never split: the reduce launch and the
+// partial sums' traffic (~15 us at 16 tiles) cost about what splitting a short
+// tile saves (the fine-grained shape's 22-step down tiles take ~31 us).
+constexpr int kSplitMinTileSteps = 64;
+// Whether a 256-row GEMM over k inputs splits its last round of tiles along K.
+// The one test of the kernels' launches, of what sizes their workspace and of
+// the choice of tiles; a partial last step counts as one.
+inline bool splits_tail(int64_t k) { return ceil_div(k, 64) >= kSplitMinTileSteps; }
 int64_t gemm_workspace_bytes(bool down);
 
 // K of the bf16 kernels: a multiple of 8, at least one 64-K step. (Below it,

@@ -761,7 +761,7 @@ int launch_bwd(BwdArgs p, int64_t total, hipStream_t s, const char* name, const 
   p.grid = (int)grid;
   p.part = nullptr;
   constexpr bool kSplit = kMode == Bwd::kDgradIn || kMode == Bwd::kDgradInAdd;
-  if (kSplit && ws.base != nullptr && dgrad_steps(p.K) >= kSplitMinTileSteps &&
+  if (kSplit && ws.base != nullptr && splits_tail(p.K) &&
       ws.bytes >= kSchedBytes + grid * (int64_t)sizeof(float) * kSplitUnitFloats)
     p.part = reinterpret_cast<float*>(static_cast<char*>(ws.base) + kSchedBytes);
   hipLaunchKernelGGL((gemm_bwd_kernel<kMode>), dim3((unsigned)grid), dim3(BwdCfg::THREADS), 0, s, p);

@@ -1083,7 +1083,7 @@ int launch_stream(const void* A, const int32_t* tiles, int64_t capacity, const v
   const int64_t ksteps = k_steps(K);
   const bool have_ws = ws.base != nullptr && ws.bytes >= kSchedBytes && grid <= kMaxSchedGroups;
   int32_t* sched = (have_ws && ksteps >= kDynamicMinSteps) ? static_cast<int32_t*>(ws.base) : nullptr;
-  float* part = (!kGateUp && have_ws && ksteps >= kSplitMinTileSteps &&
+  float* part = (!kGateUp && have_ws && splits_tail(K) &&
                  ws.bytes >= kSchedBytes + grid * (int64_t)sizeof(float) * kSplitUnitFloats)
                     ? reinterpret_cast<float*>(static_cast<char*>(ws.base) + kSchedBytes)
                     : nullptr;
@@ -1165,7 +1165,7 @@ Pick pick_tiles(int64_t n_rows, int n_experts, int block_m, int64_t k, int64_t n
   if (block_m < kMfmaMidBM || least > kFewRounds * cu) return {Tiles::kList, std::ceil(least / cu) * step};
   const double row_tiles = expected_row_tiles(n_rows, n_experts, block_m), rounds = std::ceil(row_tiles * wide / cu);
   const Pick own{Tiles::kList, rounds * step};
-  if (row_tiles * wide > kFewRounds * cu || (block_m == kMfmaBigBM && k_steps(k) >= kSplitMinTileSteps)) return own;
+  if (row_tiles * wide > kFewRounds * cu || (block_m == kMfmaBigBM && splits_tail(k))) return own;
   // 128-row halves of a 256-row tile: one without a second half still takes its
   // place in the walk
   const double halves = block_m == kMfmaBigBM ? 2.0 * row_tiles : row_tiles;

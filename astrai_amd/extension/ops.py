@@ -34,7 +34,7 @@ MAX_TOPK = 32
 TILE_HEADER = 4
 TILE_STRIDE = 3
 # K steps (of 64) per tile from which the 256-row down-sized GEMMs split a
-# partial last round along K (kSplitMinTileSteps in mfma_tile.h)
+# partial last round along K (splits_tail in moe_gemm.h)
 SPLIT_MIN_STEPS = 64
 
 _DTYPE_CODES = {torch.float32: 0, torch.bfloat16: 1}
@@ -253,7 +253,7 @@ def _workspace(a: torch.Tensor, dim: int, dim_ffn: int, block_m: int, down: bool
         return None, 0
     # the partial sums serve only tiles of SPLIT_MIN_STEPS K steps or more
     # (K = dim_ffn for the down-sized users): below that, the scheduling part
-    split = down and dim_ffn // 64 >= SPLIT_MIN_STEPS
+    split = down and -(-dim_ffn // 64) >= SPLIT_MIN_STEPS
     nbytes = int(loader.library().astrai_moe_gemm_workspace_bytes(1 if split else 0))
     return torch.empty(nbytes, dtype=torch.uint8, device=a.device), nbytes
 
