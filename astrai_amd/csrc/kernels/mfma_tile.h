@@ -185,6 +185,7 @@ struct TileWalk {
 // like tiles: item i < full is logical tile i, item full + u is unit u (tile
 // full + u / S, slice u % S).
 constexpr int kSplitMinSteps = 8;
+constexpr double kSplitReduceUs = 15.0;  // the reduce launch and the partial sums' traffic
 constexpr int kSplitUnitFloats = kMfmaBigBM * 256;  // fp32 accumulators of one 256 x 256 tile
 
 template <int GM>

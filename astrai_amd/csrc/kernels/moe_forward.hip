@@ -121,6 +121,10 @@ extern "C" int astrai_moe_forward(const void* x, const void* logits, const void*
   ASTRAI_REQUIRE((packed_gate_up == nullptr) == (packed_down == nullptr), "forward: one packed table without the other");
   ASTRAI_REQUIRE(reinterpret_cast<uintptr_t>(workspace) % 256 == 0, "forward: workspace must be 256-byte aligned");
   const Plan p = make_plan(z);
+  ASTRAI_REQUIRE(!z.packed || (dtype == ASTRAI_MOE_BF16 && dim % 256 == 0 && dim_ffn % 128 == 0 &&
+                               mfma_shape_supported(dim, dim_ffn)),
+                 "forward: unsupported shape for packed weights (dim %lld, dim_ffn %lld) or dtype", (long long)dim,
+                 (long long)dim_ffn);
   ASTRAI_REQUIRE(workspace_bytes >= p.bytes, "forward: workspace holds %lld bytes, needs %lld",
                  (long long)workspace_bytes, (long long)p.bytes);
   ASTRAI_REQUIRE(!p.gather || reinterpret_cast<uintptr_t>(x) % 16 == 0,
@@ -150,25 +154,20 @@ extern "C" int astrai_moe_forward(const void* x, const void* logits, const void*
                             i32(p.chunk_base), stream);
   }
   if (rc) return rc;
+  const RowCounts rows(n_tokens * top_k, n_experts, n_shared, n_tokens);
+  const GemmWorkspace ws{gws, p.gemm_ws_bytes};
   if (gather)
-    rc = launch_gate_up_gather(x, sorted_token, tiles, p.tiles_len, w_gate, w_up, p.rows, p.experts, dim, dim_ffn,
-                               p.block_m, h, GemmWorkspace{gws, p.gemm_ws_bytes}, s);
+    rc = launch_gate_up_gather(x, sorted_token, tiles, p.tiles_len, w_gate, w_up, rows, dim, dim_ffn, p.block_m, h, ws,
+                               s);
   else if (gather_f32)
     rc = launch_mfma_f32_gate_up(x, tiles, (p.tiles_len - ASTRAI_MOE_TILE_HEADER) / ASTRAI_MOE_TILE_STRIDE, w_gate, w_up,
                                  p.rows, p.experts, dim, dim_ffn, h, nullptr, s, sorted_token);
-  else if (z.packed)
-    rc = astrai_moe_gemm_gate_up_packed(x_perm, tiles, p.tiles_len, packed_gate_up, dtype, p.rows, p.experts, dim,
-                                        dim_ffn, p.block_m, h, gws, p.gemm_ws_bytes, stream);
   else
-    rc = astrai_moe_gemm_gate_up(x_perm, tiles, p.tiles_len, w_gate, w_up, dtype, p.rows, p.experts, dim, dim_ffn,
-                                 p.block_m, h, gws, p.gemm_ws_bytes, stream);
+    rc = launch_gate_up(x_perm, tiles, p.tiles_len, z.packed ? packed_gate_up : w_gate, z.packed ? packed_gate_up : w_up,
+                        dtype, rows, dim, dim_ffn, p.block_m, z.packed, h, ws, s);
   if (rc) return rc;
-  if (z.packed)
-    rc = astrai_moe_gemm_down_packed(h, tiles, p.tiles_len, packed_down, sorted_w, dtype, p.rows, p.experts, dim_ffn,
-                                     dim, p.block_m, y, gws, p.gemm_ws_bytes, stream);
-  else
-    rc = astrai_moe_gemm_down(h, tiles, p.tiles_len, w_down, sorted_w, dtype, p.rows, p.experts, dim_ffn, dim,
-                              p.block_m, y, gws, p.gemm_ws_bytes, stream);
+  rc = launch_down(h, tiles, p.tiles_len, z.packed ? packed_down : w_down, sorted_w, dtype, rows, dim_ffn, dim, p.block_m,
+                   z.packed, y, ws, s);
   if (rc) return rc;
   const int64_t size = dtype == ASTRAI_MOE_BF16 ? 2 : 4;
   const void* shared = n_shared > 0 ? static_cast<const char*>(y) + n_tokens * top_k * dim * size : nullptr;
@@ -200,8 +199,8 @@ DensePlan dense_plan(int64_t n_rows, int64_t dim, int64_t dim_ffn, int dtype) {
   DensePlan p{};
   p.block_m = p.block_m_down = astrai_moe_select_block_m(n_rows, 1, 1, dim, dim_ffn, dtype);
   if (dtype == ASTRAI_MOE_BF16 && mfma_shape_supported(dim, dim_ffn)) {
-    const bool few_up = few_rows(n_rows, 1, p.block_m, dim, dim_ffn, true);
-    const bool few_down = few_rows(n_rows, 1, p.block_m, dim_ffn, dim, false);
+    const bool few_up = few_rows({n_rows, 1}, p.block_m, dim, dim_ffn, true);
+    const bool few_down = few_rows({n_rows, 1}, p.block_m, dim_ffn, dim, false);
     p.few = few_up && few_down;
     if (p.block_m > kMfmaSmallBM) {
       if (!few_up) p.block_m = dense_gemm_block_m(n_rows, dim, dim_ffn, true);

@@ -61,16 +61,37 @@ bool mfma_down_supported(int64_t dim_ffn, int64_t dim, int block_m,
 // Row-tile height of the list for one GEMM of a dense expert (96 rows or more).
 int dense_gemm_block_m(int64_t n_rows, int64_t k, int64_t n, bool gate_up);
 
+// Rows of a grouped GEMM as far as the host knows them: `rows` over `experts`
+// experts, divided by the router, and `exact` experts (shared ones, a dense
+// expert) of exactly `exact_rows` rows each. The rules that choose kernels and
+// tiles by the load take it; results depend on it only through those.
+struct RowCounts {
+  int64_t rows;
+  int experts;
+  int exact = 0;
+  int64_t exact_rows = 0;
+  RowCounts(int64_t rows_, int experts_, int exact_ = 0, int64_t exact_rows_ = 0)
+      : rows(rows_), experts(experts_), exact(exact_), exact_rows(exact_rows_) {
+    if (experts == 1 && (exact == 0 || exact_rows == rows)) {  // the only routed expert has every row
+      exact_rows = rows;
+      ++exact;
+      rows = experts = 0;
+    }
+  }
+  int64_t total() const { return rows + exact * exact_rows; }
+  bool dense() const { return experts == 0 && exact == 1; }
+};
+
 // `packed`: the weight tables point at packed copies written by launch_pack
 // (bf16, 256-row tiles of K / 64 contiguous 32 KB blocks in staged order).
 int launch_mfma_gate_up(const void* x_perm, const int32_t* tiles,
                         int64_t capacity, const void* const* w_gate,
-                        const void* const* w_up, int64_t n_rows, int n_experts,
+                        const void* const* w_up, const RowCounts& rows,
                         int64_t dim, int64_t dim_ffn, int block_m, bool packed, void* h, hipStream_t s,
                         const GemmWorkspace& ws = {});
 int launch_mfma_down(const void* h, const int32_t* tiles, int64_t capacity,
                      const void* const* w_down, const void* sorted_w,
-                     int64_t n_rows, int n_experts, int64_t dim_ffn,
+                     const RowCounts& rows, int64_t dim_ffn,
                      int64_t dim, int block_m, bool packed,
                      void* y, hipStream_t s,
                      const GemmWorkspace& ws = {});
@@ -81,20 +102,20 @@ int launch_mfma_down(const void* h, const int32_t* tiles, int64_t capacity,
 namespace ragged {
 int launch_mfma_gate_up(const void* x_perm, const int32_t* tiles,
                         int64_t capacity, const void* const* w_gate,
-                        const void* const* w_up, int64_t n_rows, int n_experts,
+                        const void* const* w_up, const RowCounts& rows,
                         int64_t dim, int64_t dim_ffn, int block_m, bool packed, void* h, hipStream_t s,
                         const GemmWorkspace& ws);
 int launch_mfma_down(const void* h, const int32_t* tiles, int64_t capacity,
                      const void* const* w_down, const void* sorted_w,
-                     int64_t n_rows, int n_experts, int64_t dim_ffn,
+                     const RowCounts& rows, int64_t dim_ffn,
                      int64_t dim, int block_m, bool packed,
                      void* y, hipStream_t s, const GemmWorkspace& ws);
 int launch_mfma_gate_up_gather(const void* x, const int32_t* sorted_token,
                                const int32_t* tiles, int64_t capacity,
                                const void* const* w_gate,
-                               const void* const* w_up, int64_t n_rows,
-                               int n_experts, int64_t dim, int64_t dim_ffn,
-                               int block_m, void* h, hipStream_t s,
+                               const void* const* w_up, const RowCounts& rows,
+                               int64_t dim, int64_t dim_ffn, int block_m, void* h,
+                               hipStream_t s,
                                const GemmWorkspace& ws);
 int launch_mfma_gate_up_save(const void* x_perm, const int32_t* tiles,
                              int64_t capacity, const void* const* w_gate,
@@ -120,35 +141,45 @@ int launch_dgrad_in(const void* d, const int32_t* tiles, int64_t capacity,
 int launch_mfma_gate_up_gather(const void* x, const int32_t* sorted_token,
                                const int32_t* tiles, int64_t capacity,
                                const void* const* w_gate,
-                               const void* const* w_up, int64_t n_rows,
-                               int n_experts, int64_t dim, int64_t dim_ffn,
-                               int block_m, void* h, hipStream_t s,
+                               const void* const* w_up, const RowCounts& rows,
+                               int64_t dim, int64_t dim_ffn, int block_m, void* h,
+                               hipStream_t s,
                                const GemmWorkspace& ws = {});
 
-// The gathering gate/up GEMM on the kernel its sizes take (few rows or the
-// above); x and h aligned to 16 bytes, x under 4 GiB.
+// The GEMMs on the kernels their sizes take (moe_gemm.hip). packed: the tables
+// hold packed copies.
+int launch_gate_up(const void* x_perm, const int32_t* tiles, int64_t tiles_len,
+                   const void* const* w_gate, const void* const* w_up,
+                   int dtype, const RowCounts& rows, int64_t dim,
+                   int64_t dim_ffn, int block_m, bool packed, void* h,
+                   const GemmWorkspace& ws, hipStream_t s);
+int launch_down(const void* h, const int32_t* tiles, int64_t tiles_len,
+                const void* const* w_down, const void* sorted_w, int dtype,
+                const RowCounts& rows, int64_t dim_ffn, int64_t dim,
+                int block_m, bool packed, void* y, const GemmWorkspace& ws,
+                hipStream_t s);
+// gathering (bf16); x and h aligned to 16 bytes, x under 4 GiB
 int launch_gate_up_gather(const void* x, const int32_t* sorted_token,
                           const int32_t* tiles, int64_t tiles_len,
                           const void* const* w_gate, const void* const* w_up,
-                          int64_t n_rows, int n_experts, int64_t dim,
+                          const RowCounts& rows, int64_t dim,
                           int64_t dim_ffn, int block_m, void* h,
                           const GemmWorkspace& ws, hipStream_t s);
 
 // Few rows (moe_gemm_few.hip), tiles below 256 rows: whether the kernels there
-// take a GEMM of n_rows rows over n_experts experts with k inputs
-// and n output columns, and the GEMMs (row_src: the
+// take a GEMM with k inputs and n output columns, and the GEMMs (row_src: the
 // gathered rows' tokens, or null; packed: the tables hold packed copies).
-bool few_rows(int64_t n_rows, int n_experts, int block_m, int64_t k, int64_t n,
+bool few_rows(const RowCounts& rows, int block_m, int64_t k, int64_t n,
               bool gate_up);
 int launch_few_gate_up(const void* x, const int32_t* row_src,
                        const int32_t* tiles, int64_t capacity,
                        const void* const* w_gate, const void* const* w_up,
-                       int64_t n_rows, int n_experts, int64_t dim,
-                       int64_t dim_ffn, bool packed, void* h, hipStream_t s);
+                       const RowCounts& rows, int64_t dim, int64_t dim_ffn,
+                       bool packed, void* h, hipStream_t s);
 int launch_few_down(const void* h, const int32_t* tiles, int64_t capacity,
                     const void* const* w_down, const void* sorted_w,
-                    int64_t n_rows, int n_experts, int64_t dim_ffn,
-                    int64_t dim, bool packed, void* y, hipStream_t s);
+                    const RowCounts& rows, int64_t dim_ffn, int64_t dim,
+                    bool packed, void* y, hipStream_t s);
 // Both GEMMs of one dense expert whose GEMMs few_rows both takes, without a
 // tile list.
 int launch_few_dense(const void* x, const void* const* w_gate,

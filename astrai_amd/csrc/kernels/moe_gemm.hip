@@ -182,6 +182,58 @@ int check_workspace(const char* who, const void* workspace, int64_t workspace_by
 }  // namespace
 }  // namespace astrai_moe
 
+namespace astrai_moe {
+
+static int64_t tile_capacity(int64_t len) { return (len - ASTRAI_MOE_TILE_HEADER) / ASTRAI_MOE_TILE_STRIDE; }
+
+int launch_gate_up(const void* x_perm, const int32_t* tiles, int64_t tiles_len, const void* const* w_gate,
+                   const void* const* w_up, int dtype, const RowCounts& rows, int64_t dim, int64_t dim_ffn,
+                   int block_m, bool packed, void* h, const GemmWorkspace& ws, hipStream_t s) {
+  const int64_t capacity = tile_capacity(tiles_len);
+  if (dtype == ASTRAI_MOE_BF16) {
+    const bool mfma = mfma_gate_up_supported(dim, dim_ffn, block_m, x_perm, h);
+    if (mfma && few_rows(rows, block_m, dim, dim_ffn, true))
+      return launch_few_gate_up(x_perm, nullptr, tiles, capacity, w_gate, w_up, rows, dim, dim_ffn, packed, h, s);
+    if (mfma)
+      return launch_mfma_gate_up(x_perm, tiles, capacity, w_gate, w_up, rows, dim, dim_ffn, block_m, packed, h, s, ws);
+    return launch_generic<bf16_t, true>(x_perm, tiles, capacity, w_gate, w_up, nullptr, dim, dim_ffn, h, s);
+  }
+  if (mfma_f32_supported(dim, dim_ffn, true, block_m, x_perm, h, nullptr))
+    return launch_mfma_f32_gate_up(x_perm, tiles, capacity, w_gate, w_up, rows.total(), rows.experts + rows.exact, dim,
+                                   dim_ffn, h, nullptr, s);
+  return launch_generic<float, true>(x_perm, tiles, capacity, w_gate, w_up, nullptr, dim, dim_ffn, h, s);
+}
+
+int launch_down(const void* h, const int32_t* tiles, int64_t tiles_len, const void* const* w_down,
+                const void* sorted_w, int dtype, const RowCounts& rows, int64_t dim_ffn, int64_t dim, int block_m,
+                bool packed, void* y, const GemmWorkspace& ws, hipStream_t s) {
+  const int64_t capacity = tile_capacity(tiles_len);
+  if (dtype == ASTRAI_MOE_BF16) {
+    const bool mfma = mfma_down_supported(dim_ffn, dim, block_m, h, y);
+    if (mfma && few_rows(rows, block_m, dim_ffn, dim, false))
+      return launch_few_down(h, tiles, capacity, w_down, sorted_w, rows, dim_ffn, dim, packed, y, s);
+    if (mfma)
+      return launch_mfma_down(h, tiles, capacity, w_down, sorted_w, rows, dim_ffn, dim, block_m, packed, y, s, ws);
+    return launch_generic<bf16_t, false>(h, tiles, capacity, w_down, nullptr, sorted_w, dim_ffn, dim, y, s);
+  }
+  if (mfma_f32_supported(dim_ffn, dim, false, block_m, h, y, nullptr))
+    return launch_mfma_f32_down(h, tiles, capacity, w_down, sorted_w, rows.total(), rows.experts + rows.exact, dim_ffn,
+                                dim, y, nullptr, s);
+  return launch_generic<float, false>(h, tiles, capacity, w_down, nullptr, sorted_w, dim_ffn, dim, y, s);
+}
+
+int launch_gate_up_gather(const void* x, const int32_t* sorted_token, const int32_t* tiles, int64_t tiles_len,
+                          const void* const* w_gate, const void* const* w_up, const RowCounts& rows, int64_t dim,
+                          int64_t dim_ffn, int block_m, void* h, const GemmWorkspace& ws, hipStream_t s) {
+  const int64_t capacity = tile_capacity(tiles_len);
+  if (few_rows(rows, block_m, dim, dim_ffn, true))
+    return launch_few_gate_up(x, sorted_token, tiles, capacity, w_gate, w_up, rows, dim, dim_ffn, false, h, s);
+  return launch_mfma_gate_up_gather(x, sorted_token, tiles, capacity, w_gate, w_up, rows, dim, dim_ffn, block_m, h, s,
+                                    ws);
+}
+
+}  // namespace astrai_moe
+
 using namespace astrai_moe;
 
 extern "C" int astrai_moe_gemm_gate_up(const void* x_perm, const int32_t* tiles,
@@ -199,36 +251,8 @@ extern "C" int astrai_moe_gemm_gate_up(const void* x_perm, const int32_t* tiles,
   if ((rc = check_workspace("gemm_gate_up", workspace, workspace_bytes))) return rc;
   if (n_rows == 0) return ASTRAI_MOE_OK;
   ASTRAI_REQUIRE(w_gate && w_up, "gemm_gate_up: null weight table");
-  const int64_t capacity = (tiles_len - ASTRAI_MOE_TILE_HEADER) / ASTRAI_MOE_TILE_STRIDE;
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  if (dtype == ASTRAI_MOE_BF16) {
-    const bool mfma = mfma_gate_up_supported(dim, dim_ffn, block_m, x_perm, h);
-    if (mfma && few_rows(n_rows, n_experts, block_m, dim, dim_ffn, true))
-      return launch_few_gate_up(x_perm, nullptr, tiles, capacity, w_gate, w_up, n_rows, n_experts, dim, dim_ffn, false, h, s);
-    if (mfma)
-      return launch_mfma_gate_up(x_perm, tiles, capacity, w_gate, w_up, n_rows, n_experts, dim,
-                                 dim_ffn, block_m, false, h, s,
-                                 GemmWorkspace{workspace, workspace_bytes});
-    return launch_generic<bf16_t, true>(x_perm, tiles, capacity, w_gate, w_up,
-                                        nullptr, dim, dim_ffn, h, s);
-  }
-  if (mfma_f32_supported(dim, dim_ffn, true, block_m, x_perm, h, nullptr))
-    return launch_mfma_f32_gate_up(x_perm, tiles, capacity, w_gate, w_up, n_rows, n_experts, dim, dim_ffn, h,
-                                   nullptr, s);
-  return launch_generic<float, true>(x_perm, tiles, capacity, w_gate, w_up,
-                                     nullptr, dim, dim_ffn, h, s);
-}
-
-int astrai_moe::launch_gate_up_gather(const void* x, const int32_t* sorted_token, const int32_t* tiles,
-                                      int64_t tiles_len, const void* const* w_gate, const void* const* w_up,
-                                      int64_t n_rows, int n_experts, int64_t dim, int64_t dim_ffn, int block_m, void* h,
-                                      const GemmWorkspace& ws, hipStream_t s) {
-  const int64_t capacity = (tiles_len - ASTRAI_MOE_TILE_HEADER) / ASTRAI_MOE_TILE_STRIDE;
-  if (few_rows(n_rows, n_experts, block_m, dim, dim_ffn, true))
-    return launch_few_gate_up(x, sorted_token, tiles, capacity, w_gate, w_up, n_rows, n_experts, dim, dim_ffn, false, h,
-                              s);
-  return launch_mfma_gate_up_gather(x, sorted_token, tiles, capacity, w_gate, w_up, n_rows, n_experts, dim, dim_ffn,
-                                    block_m, h, s, ws);
+  return launch_gate_up(x_perm, tiles, tiles_len, w_gate, w_up, dtype, {n_rows, n_experts}, dim, dim_ffn, block_m,
+                        false, h, GemmWorkspace{workspace, workspace_bytes}, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int astrai_moe_gemm_gate_up_gather(const void* x, const int32_t* sorted_token, int64_t n_tokens,
@@ -250,8 +274,8 @@ extern "C" int astrai_moe_gemm_gate_up_gather(const void* x, const int32_t* sort
                  "gemm_gate_up_gather: unsupported shape (dim %lld, dim_ffn %lld, block_m %d) or alignment",
                  (long long)dim, (long long)dim_ffn, block_m);
   ASTRAI_REQUIRE(sorted_token && w_gate && w_up, "gemm_gate_up_gather: null row list or weight table");
-  return launch_gate_up_gather(x, sorted_token, tiles, tiles_len, w_gate, w_up, n_rows, n_experts, dim, dim_ffn, block_m, h,
-                               GemmWorkspace{workspace, workspace_bytes}, static_cast<hipStream_t>(stream));
+  return launch_gate_up_gather(x, sorted_token, tiles, tiles_len, w_gate, w_up, {n_rows, n_experts}, dim, dim_ffn,
+                               block_m, h, GemmWorkspace{workspace, workspace_bytes}, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int astrai_moe_gemm_down(const void* h, const int32_t* tiles,
@@ -269,24 +293,8 @@ extern "C" int astrai_moe_gemm_down(const void* h, const int32_t* tiles,
   if ((rc = check_workspace("gemm_down", workspace, workspace_bytes))) return rc;
   if (n_rows == 0) return ASTRAI_MOE_OK;
   ASTRAI_REQUIRE(w_down, "gemm_down: null weight table");
-  const int64_t capacity = (tiles_len - ASTRAI_MOE_TILE_HEADER) / ASTRAI_MOE_TILE_STRIDE;
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  if (dtype == ASTRAI_MOE_BF16) {
-    const bool mfma = mfma_down_supported(dim_ffn, dim, block_m, h, y);
-    if (mfma && few_rows(n_rows, n_experts, block_m, dim_ffn, dim, false))
-      return launch_few_down(h, tiles, capacity, w_down, sorted_w, n_rows, n_experts, dim_ffn, dim, false, y, s);
-    if (mfma)
-      return launch_mfma_down(h, tiles, capacity, w_down, sorted_w, n_rows, n_experts, dim_ffn,
-                              dim, block_m, false, y, s,
-                              GemmWorkspace{workspace, workspace_bytes});
-    return launch_generic<bf16_t, false>(h, tiles, capacity, w_down, nullptr,
-                                         sorted_w, dim_ffn, dim, y, s);
-  }
-  if (mfma_f32_supported(dim_ffn, dim, false, block_m, h, y, nullptr))
-    return launch_mfma_f32_down(h, tiles, capacity, w_down, sorted_w, n_rows, n_experts, dim_ffn, dim, y, nullptr,
-                                s);
-  return launch_generic<float, false>(h, tiles, capacity, w_down, nullptr,
-                                      sorted_w, dim_ffn, dim, y, s);
+  return launch_down(h, tiles, tiles_len, w_down, sorted_w, dtype, {n_rows, n_experts}, dim_ffn, dim, block_m, false, y,
+                     GemmWorkspace{workspace, workspace_bytes}, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int64_t astrai_moe_gemm_workspace_bytes(int down) { return gemm_workspace_bytes(down != 0); }
@@ -335,12 +343,8 @@ extern "C" int astrai_moe_gemm_gate_up_packed(const void* x_perm, const int32_t*
                  (long long)dim, (long long)dim_ffn, block_m);
   if (n_rows == 0) return ASTRAI_MOE_OK;
   ASTRAI_REQUIRE(w_packed, "gemm_gate_up_packed: null weight table");
-  const int64_t capacity = (tiles_len - ASTRAI_MOE_TILE_HEADER) / ASTRAI_MOE_TILE_STRIDE;
-  if (few_rows(n_rows, n_experts, block_m, dim, dim_ffn, true))
-    return launch_few_gate_up(x_perm, nullptr, tiles, capacity, w_packed, w_packed, n_rows, n_experts, dim, dim_ffn, true, h,
-                              static_cast<hipStream_t>(stream));
-  return launch_mfma_gate_up(x_perm, tiles, capacity, w_packed, w_packed, n_rows, n_experts, dim, dim_ffn, block_m, true, h,
-                             static_cast<hipStream_t>(stream), GemmWorkspace{workspace, workspace_bytes});
+  return launch_gate_up(x_perm, tiles, tiles_len, w_packed, w_packed, dtype, {n_rows, n_experts}, dim, dim_ffn, block_m,
+                        true, h, GemmWorkspace{workspace, workspace_bytes}, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int astrai_moe_gemm_down_packed(const void* h, const int32_t* tiles, int64_t tiles_len,
@@ -359,13 +363,8 @@ extern "C" int astrai_moe_gemm_down_packed(const void* h, const int32_t* tiles, 
                  (long long)dim_ffn, (long long)dim, block_m);
   if (n_rows == 0) return ASTRAI_MOE_OK;
   ASTRAI_REQUIRE(w_packed, "gemm_down_packed: null weight table");
-  const int64_t capacity = (tiles_len - ASTRAI_MOE_TILE_HEADER) / ASTRAI_MOE_TILE_STRIDE;
-  if (few_rows(n_rows, n_experts, block_m, dim_ffn, dim, false))
-    return launch_few_down(h, tiles, capacity, w_packed, sorted_w, n_rows, n_experts, dim_ffn, dim, true, y,
-                           static_cast<hipStream_t>(stream));
-  return launch_mfma_down(h, tiles, capacity, w_packed, sorted_w, n_rows, n_experts, dim_ffn, dim, block_m, true, y,
-                          static_cast<hipStream_t>(stream),
-                          GemmWorkspace{workspace, workspace_bytes});
+  return launch_down(h, tiles, tiles_len, w_packed, sorted_w, dtype, {n_rows, n_experts}, dim_ffn, dim, block_m, true, y,
+                     GemmWorkspace{workspace, workspace_bytes}, static_cast<hipStream_t>(stream));
 }
 
 // ---------------------------------------------------------------------------
@@ -410,7 +409,7 @@ extern "C" int astrai_moe_gemm_gate_up_train(const void* x_perm, const int32_t* 
   if ((rc = check_train("gemm_gate_up_train", dtype, dim, dim_ffn, block_m))) return rc;
   if (n_rows == 0) return ASTRAI_MOE_OK;
   ASTRAI_REQUIRE(w_gate && w_up && gu, "gemm_gate_up_train: null weight table or output");
-  const int64_t capacity = (tiles_len - ASTRAI_MOE_TILE_HEADER) / ASTRAI_MOE_TILE_STRIDE;
+  const int64_t capacity = tile_capacity(tiles_len);
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (mfma_train_shape(dtype, dim, dim_ffn) || mfma_train_ragged(dtype, dim, dim_ffn, block_m, x_perm, h, gu)) {
     ASTRAI_REQUIRE(aligned16_ptr(x_perm) && aligned16_ptr(h) && aligned16_ptr(gu),
@@ -438,7 +437,7 @@ extern "C" int astrai_moe_gemm_down_train(const void* h, const int32_t* tiles, i
   if ((rc = check_train("gemm_down_train", dtype, dim, dim_ffn, block_m))) return rc;
   if (n_rows == 0) return ASTRAI_MOE_OK;
   ASTRAI_REQUIRE(w_down && sorted_w && y_unweighted, "gemm_down_train: null weight table, row weights or output");
-  const int64_t capacity = (tiles_len - ASTRAI_MOE_TILE_HEADER) / ASTRAI_MOE_TILE_STRIDE;
+  const int64_t capacity = tile_capacity(tiles_len);
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (mfma_train_shape(dtype, dim, dim_ffn) || mfma_train_ragged(dtype, dim, dim_ffn, block_m, h, y, y_unweighted)) {
     ASTRAI_REQUIRE(aligned16_ptr(h) && aligned16_ptr(y) && aligned16_ptr(y_unweighted),
@@ -483,7 +482,7 @@ extern "C" int astrai_moe_gemm_dgrad_down(const void* dy, const int32_t* tiles, 
   if ((rc = check_train("gemm_dgrad_down", dtype, dim, dim_ffn, block_m))) return rc;
   if (n_rows == 0) return ASTRAI_MOE_OK;
   ASTRAI_REQUIRE(w_down && gu && du, "gemm_dgrad_down: null weight table or buffer");
-  const int64_t capacity = (tiles_len - ASTRAI_MOE_TILE_HEADER) / ASTRAI_MOE_TILE_STRIDE;
+  const int64_t capacity = tile_capacity(tiles_len);
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (mfma_train_shape(dtype, dim, dim_ffn) || mfma_train_ragged(dtype, dim, dim_ffn, block_m, dy, gu, dg, du)) {
     ASTRAI_REQUIRE(aligned16_ptr(dy) && aligned16_ptr(gu) && aligned16_ptr(dg) && aligned16_ptr(du),
@@ -508,7 +507,7 @@ extern "C" int astrai_moe_gemm_dgrad_gate_up(const void* dg, const void* du, con
   if ((rc = check_train("gemm_dgrad_gate_up", dtype, dim, dim_ffn, block_m))) return rc;
   if (n_rows == 0) return ASTRAI_MOE_OK;
   ASTRAI_REQUIRE(du && w_gate && w_up, "gemm_dgrad_gate_up: null weight table or buffer");
-  const int64_t capacity = (tiles_len - ASTRAI_MOE_TILE_HEADER) / ASTRAI_MOE_TILE_STRIDE;
+  const int64_t capacity = tile_capacity(tiles_len);
   hipStream_t s = static_cast<hipStream_t>(stream);
   // dx_perm = round(dg . W_gate), then dx_perm = round(round(du . W_up) + dx_perm)
   if (mfma_train_shape(dtype, dim, dim_ffn) || mfma_train_ragged(dtype, dim, dim_ffn, block_m, dg, du, dx_perm)) {

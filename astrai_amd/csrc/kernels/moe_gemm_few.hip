@@ -346,12 +346,12 @@ constexpr double kFewMaxFill = 0.9;
 // -> 560; 64 of D 2048, F 1408, 8 tokens 144 -> 188).
 template <bool kGateUp, bool kGather, bool kPacked, bool kDense>
 int launch_few_tiles(const void* A, const RowTiles<kDense>& tiles, int64_t capacity, const void* const* W0, const void* const* W1,
-               const void* row_w, int64_t n_rows, int n_experts, int64_t K, int64_t N, void* C, hipStream_t s,
+               const void* row_w, const RowCounts& load, int64_t K, int64_t N, void* C, hipStream_t s,
                const int32_t* row_src) {
-  if (n_rows > (n_experts == 1 ? 2 * FewCfg<32, 32>::BM : (int64_t)kFewRowsPerExpert * n_experts))
+  if (load.total() > (load.dense() ? 2 * FewCfg<32, 32>::BM : (int64_t)kFewRowsPerExpert * (load.experts + load.exact)))
     return launch_few_cfg<FewCfg<64, 32>, kGateUp, kGather, kPacked, kDense>(A, tiles, capacity, W0, W1, row_w, K, N, C, s,
                                                                      row_src);
-  if (n_experts == 1 && n_rows <= FewCfg<32, 16>::BM &&
+  if (load.dense() && load.total() <= FewCfg<32, 16>::BM &&
       fill((double)ceil_div(N, kGateUp ? 8 : 16)) > 1.05 * fill((double)ceil_div(N, kGateUp ? 16 : 32)))
     return launch_few_cfg<FewCfg<32, 16>, kGateUp, kGather, kPacked, kDense>(A, tiles, capacity, W0, W1, row_w, K, N, C, s, row_src);
   return launch_few_cfg<FewCfg<32, 32>, kGateUp, kGather, kPacked, kDense>(A, tiles, capacity, W0, W1, row_w, K, N, C, s, row_src);
@@ -359,10 +359,10 @@ int launch_few_tiles(const void* A, const RowTiles<kDense>& tiles, int64_t capac
 
 template <bool kGateUp, bool kGather, bool kPacked>
 int launch_few(const void* A, const int32_t* tiles, int64_t capacity, const void* const* W0, const void* const* W1,
-               const void* row_w, int64_t n_rows, int n_experts, int64_t K, int64_t N, void* C, hipStream_t s,
+               const void* row_w, const RowCounts& load, int64_t K, int64_t N, void* C, hipStream_t s,
                const int32_t* row_src) {
-  return launch_few_tiles<kGateUp, kGather, kPacked>(A, RowTiles<false>{tiles, 0, 0}, capacity, W0, W1, row_w, n_rows,
-                                                     n_experts, K, N, C, s, row_src);
+  return launch_few_tiles<kGateUp, kGather, kPacked>(A, RowTiles<false>{tiles, 0, 0}, capacity, W0, W1, row_w, load, K,
+                                                     N, C, s, row_src);
 }
 
 }  // namespace
@@ -388,40 +388,42 @@ int launch_few(const void* A, const int32_t* tiles, int64_t capacity, const void
 // - MLP, D 4096, F 14336: 1 token 201 / 81, 24 217 / 90, 64 214 / 133, 128 235 /
 //   156, 256 (the down GEMM; its gate/up GEMM has 448 tiles) 255 / 191; D 2048, F
 //   5632: 24 66 / 28, 128 72 / 43, 256 73 / 44.
-bool few_rows(int64_t n_rows, int n_experts, int block_m, int64_t k, int64_t n, bool gate_up) {
+bool few_rows(const RowCounts& rows, int block_m, int64_t k, int64_t n, bool gate_up) {
   if (block_m == kMfmaBigBM) return false;
-  const int64_t most = n_experts == 1 ? kFewDenseRows : (int64_t)kFewRowsPerExpert * n_experts;
+  const int experts = rows.experts + rows.exact;
+  const int64_t n_rows = rows.total(), most = rows.dense() ? kFewDenseRows : (int64_t)kFewRowsPerExpert * experts;
   const double cols = (double)ceil_div(n, gate_up ? 128 : 256);
-  if (n_rows <= most) return fill(live_experts(n_rows, n_experts) * cols) < kFewMaxFill;
-  const double row_tiles = n_experts == 1 ? (double)ceil_div(n_rows, kMfmaMidBM) : (double)n_experts;
+  if (n_rows <= most) return fill(live_experts(n_rows, experts) * cols) < kFewMaxFill;
+  const double row_tiles = rows.dense() ? (double)ceil_div(n_rows, kMfmaMidBM) : (double)experts;
   return n_rows <= 2 * most && k_steps(k) >= kFewLongSteps && 2 * row_tiles * cols <= cu_count();
 }
 
 int launch_few_gate_up(const void* x, const int32_t* row_src, const int32_t* tiles, int64_t capacity,
-                       const void* const* w_gate, const void* const* w_up, int64_t n_rows, int n_experts, int64_t dim,
+                       const void* const* w_gate, const void* const* w_up, const RowCounts& rows, int64_t dim,
                        int64_t dim_ffn, bool packed, void* h, hipStream_t s) {
-  if (packed) return launch_few<true, false, true>(x, tiles, capacity, w_gate, w_gate, nullptr, n_rows, n_experts, dim, dim_ffn, h, s, nullptr);
+  if (packed) return launch_few<true, false, true>(x, tiles, capacity, w_gate, w_gate, nullptr, rows, dim, dim_ffn, h, s, nullptr);
   if (row_src != nullptr)
-    return launch_few<true, true, false>(x, tiles, capacity, w_gate, w_up, nullptr, n_rows, n_experts, dim, dim_ffn, h, s, row_src);
-  return launch_few<true, false, false>(x, tiles, capacity, w_gate, w_up, nullptr, n_rows, n_experts, dim, dim_ffn, h, s, nullptr);
+    return launch_few<true, true, false>(x, tiles, capacity, w_gate, w_up, nullptr, rows, dim, dim_ffn, h, s, row_src);
+  return launch_few<true, false, false>(x, tiles, capacity, w_gate, w_up, nullptr, rows, dim, dim_ffn, h, s, nullptr);
 }
 
 int launch_few_down(const void* h, const int32_t* tiles, int64_t capacity, const void* const* w_down,
-                    const void* sorted_w, int64_t n_rows, int n_experts, int64_t dim_ffn, int64_t dim, bool packed,
+                    const void* sorted_w, const RowCounts& rows, int64_t dim_ffn, int64_t dim, bool packed,
                     void* y, hipStream_t s) {
   if (packed)
-    return launch_few<false, false, true>(h, tiles, capacity, w_down, w_down, sorted_w, n_rows, n_experts, dim_ffn, dim, y, s, nullptr);
-  return launch_few<false, false, false>(h, tiles, capacity, w_down, w_down, sorted_w, n_rows, n_experts, dim_ffn, dim, y, s, nullptr);
+    return launch_few<false, false, true>(h, tiles, capacity, w_down, w_down, sorted_w, rows, dim_ffn, dim, y, s, nullptr);
+  return launch_few<false, false, false>(h, tiles, capacity, w_down, w_down, sorted_w, rows, dim_ffn, dim, y, s, nullptr);
 }
 
 int launch_few_dense(const void* x, const void* const* w_gate, const void* const* w_up, const void* const* w_down,
                      int64_t n_rows, int64_t dim, int64_t dim_ffn, int block_m, void* h, void* out, hipStream_t s) {
   const RowTiles<true> rows{nullptr, (int)n_rows, block_m};
+  const RowCounts load(n_rows, 1);
   const int64_t n_tiles = ceil_div(n_rows, block_m);
-  if (int rc = launch_few_tiles<true, false, false>(x, rows, n_tiles, w_gate, w_up, nullptr, n_rows, 1, dim, dim_ffn, h,
+  if (int rc = launch_few_tiles<true, false, false>(x, rows, n_tiles, w_gate, w_up, nullptr, load, dim, dim_ffn, h,
                                                     s, nullptr))
     return rc;
-  return launch_few_tiles<false, false, false>(h, rows, n_tiles, w_down, nullptr, nullptr, n_rows, 1, dim_ffn, dim, out,
+  return launch_few_tiles<false, false, false>(h, rows, n_tiles, w_down, nullptr, nullptr, load, dim_ffn, dim, out,
                                                s, nullptr);
 }
 

@@ -1119,15 +1119,25 @@ int launch(const void* A, const int32_t* tiles, int64_t capacity, const void* co
   return check_launch(kGateUp ? "gemm_mfma_kernel<gate_up>" : "gemm_mfma_kernel<down>");
 }
 
-// Row tiles of `bm` rows that n_rows rows over n_experts experts make, expected
-// under even routing (an expert's rows about normal, with their mean as
-// variance); exact for one expert.
-double expected_row_tiles(int64_t n_rows, int n_experts, int bm) {
-  if (n_experts == 1) return (double)ceil_div(n_rows, bm);
-  const double r = (double)n_rows / n_experts, sd = std::sqrt(std::max(r, 1.0));
+// Row tiles of `bm` rows that a load makes: expected under even routing (an
+// expert's rows about normal, with their mean as variance); under a skewed one
+// (the last tile of nearly every expert nearly empty: routers biased by Zipf
+// weights of exponents 0.4 to 4 over 8 to 128 experts gave rows / bm + 0.1 to 0.85
+// per expert); and the most that any routing makes, the list's capacity. The
+// same number where the host knows every expert's rows.
+struct RowTileCount {
+  double even, skewed, most;
+};
+RowTileCount count_row_tiles(const RowCounts& rows, int bm) {
+  const double exact = (double)rows.exact * (double)ceil_div(rows.exact_rows, bm);
+  if (rows.experts == 0) return {exact, exact, exact};
+  const double r = (double)rows.rows / rows.experts, sd = std::sqrt(std::max(r, 1.0));
   double tiles = 0.0;
   for (int64_t j = 0; j * bm < r + 8.0 * sd; ++j) tiles += 0.5 * std::erfc(((double)(j * bm) - r) / (sd * 1.41421356));
-  return n_experts * tiles;
+  const int64_t most = std::min(rows.rows, (rows.rows + (int64_t)rows.experts * (bm - 1)) / bm);
+  const double even = std::min(rows.experts * tiles, (double)most);
+  const double skewed = std::min(std::max(even, (double)rows.rows / bm + 0.8 * rows.experts), (double)most);
+  return {exact + even, exact + skewed, exact + (double)most};
 }
 
 // Which tiles a GEMM takes on a list of 128- or 256-row tiles: the list's own
@@ -1139,15 +1149,19 @@ enum class Tiles { kList, kHalves, kNarrow, kNarrowHalves, kNarrowMid };
 // A GEMM of few tiles takes rounds of its compute units times a tile's K steps,
 // however few the tiles of the last round: 1.4 us a step of a 256 x 256 tile,
 // 1.07 of 128 x 256, 0.83 of 64 x 256, 0.71 of 128 x 128, 0.55 of 64 x 128
-// (measured; the small tiles pay more per flop). Taken where
-// this promises a tenth; only within kFewRounds rounds of the list's own tiles,
-// past which the shares are even and the memory system decides. 256-row tiles of
-// kSplitMinTileSteps steps keep their kernel, which splits its last round.
+// (measured; the small tiles pay more per flop). The others are taken where
+// this promises a tenth under even routing and loses no more than a twentieth up
+// to a skewed one, since a few row tiles more can cost a whole round of the
+// smaller tiles (D 4096, F 14336, 8 experts, top-2, 256 tokens, 128-row list: a
+// layer 559 us against 609 evenly routed, and 670 against 601 skewed); only within
+// kFewRounds rounds of the list's own tiles, past which the shares are even and
+// the memory system decides. A last round that the 256-row down GEMM splits
+// along K (SplitWalk) counts the share of a round that its slices take and their
+// reduction.
 // Measured, us, a down GEMM of the list's tiles / the ones taken:
 // - 8 experts, top-2, D 1000, F 2664, 130 to 375 rows an expert 50 / 31 to 58 /
 //   33, and 9 of 500 rows 59 / 50 (halves); D 512, F 1024, 130 to 768 rows 23 / 14
-//   to 26 / 15 (gate/up 17 / 13 to 19 / 14.5); D 4096, F 14336, 64 rows (128-row
-//   list) 241 / 191;
+//   to 26 / 15 (gate/up 17 / 13 to 19 / 14.5);
 // - 16 experts, top-4, D 704, F 576, 64 to 512 rows 12 / 10 to 21 / 17 (gate/up
 //   21 / 17.5 at 130 to 256); D 2048, F 1408, 64 rows 27 / 20, 130 37 / 29 (halves),
 //   256 (a third more row tiles than places in a round) 42 / 44 if taken;
@@ -1158,26 +1172,43 @@ struct Pick {
   Tiles tiles;
   double us_per_step;  // rounds times a step's time
 };
-Pick pick_tiles(int64_t n_rows, int n_experts, int block_m, int64_t k, int64_t n, bool gate_up) {
-  const double cu = cu_count(), step = block_m == kMfmaBigBM ? 1.4 : block_m == kMfmaMid2BM ? 1.07 : 0.83;
+Pick pick_tiles(const RowCounts& rows, int block_m, int64_t k, int64_t n, bool gate_up) {
+  const bool big = block_m == kMfmaBigBM;
+  const double cu = cu_count(), step = big ? 1.4 : block_m == kMfmaMid2BM ? 1.07 : 0.83;
   const double wide = (double)ceil_div(n, gate_up ? 128 : 256), narrow = (double)ceil_div(n, gate_up ? 64 : 128);
-  const double least = (double)n_rows / block_m * wide;  // (bounds the sum below)
+  const double least = (double)rows.total() / block_m * wide;  // (bounds the counting below)
   if (block_m < kMfmaMidBM || least > kFewRounds * cu) return {Tiles::kList, std::ceil(least / cu) * step};
-  const double row_tiles = expected_row_tiles(n_rows, n_experts, block_m), rounds = std::ceil(row_tiles * wide / cu);
-  const Pick own{Tiles::kList, rounds * step};
-  if (row_tiles * wide > kFewRounds * cu || (block_m == kMfmaBigBM && splits_tail(k))) return own;
-  // 128-row halves of a 256-row tile: one without a second half still takes its
-  // place in the walk
-  const double halves = block_m == kMfmaBigBM ? 2.0 * row_tiles : row_tiles;
-  const double t_wide = block_m == kMfmaBigBM ? std::ceil(halves * wide / cu) * 1.07 : own.us_per_step;
-  const double t_narrow = std::ceil(halves * narrow / cu) * (block_m == kMfmaMidBM ? 0.55 : 0.71);
-  if (t_narrow <= t_wide && t_narrow < 0.9 * own.us_per_step)
-    return {block_m == kMfmaBigBM    ? Tiles::kNarrowHalves
-            : block_m == kMfmaMid2BM ? Tiles::kNarrow
-                                     : Tiles::kNarrowMid,
-            t_narrow};
-  if (t_wide < 0.9 * own.us_per_step) return {Tiles::kHalves, t_wide};
-  return own;
+  const RowTileCount count = count_row_tiles(rows, block_m);
+  // times by the number of row tiles; 128-row halves of a 256-row tile: one
+  // without a second half still takes its place in the walk
+  const double halves = big ? 2.0 : 1.0, narrow_step = block_m == kMfmaMidBM ? 0.55 : 0.71;
+  const bool split = big && !gate_up && splits_tail(k);
+  auto own = [&](double row_tiles) {
+    if (split) {
+      const int64_t tiles = std::llround(row_tiles * wide), g = std::min<int64_t>(std::llround(count.most * wide), cu);
+      const int64_t left = g > 0 ? tiles % g : 0;
+      const int64_t slices = left > 0 && 2 * left <= g ? std::min<int64_t>(g / left, k_steps(k) / kSplitMinSteps) : 1;
+      if (slices >= 2) return ((double)(tiles / g) + 1.0 / (double)slices) * step + kSplitReduceUs / k_steps(k);
+    }
+    return std::ceil(row_tiles * wide / cu) * step;
+  };
+  auto wide_halves = [&](double row_tiles) { return std::ceil(halves * row_tiles * wide / cu) * 1.07; };
+  auto narrow_tiles = [&](double row_tiles) { return std::ceil(halves * row_tiles * narrow / cu) * narrow_step; };
+  const double t_own = own(count.even);
+  if (count.even * wide > kFewRounds * cu) return {Tiles::kList, t_own};
+  auto gains = [&](auto time) {
+    if (!(time(count.even) < 0.9 * t_own)) return false;
+    const double by = std::max(1.0, (count.skewed - count.even) / 64.0);
+    for (double r = std::floor(count.even) + 1.0; r <= count.skewed; r += by)
+      if (time(r) > 1.05 * own(r)) return false;
+    return true;
+  };
+  const double t_wide = wide_halves(count.even), t_narrow = narrow_tiles(count.even);
+  const bool take_wide = big && gains(wide_halves);
+  if ((!take_wide || t_narrow <= t_wide) && gains(narrow_tiles))
+    return {big ? Tiles::kNarrowHalves : block_m == kMfmaMid2BM ? Tiles::kNarrow : Tiles::kNarrowMid, t_narrow};
+  if (take_wide) return {Tiles::kHalves, t_wide};
+  return {Tiles::kList, t_own};
 }
 
 template <bool kGateUp, bool kGather = false>
@@ -1195,10 +1226,10 @@ int launch_picked(Tiles pick, const void* A, const int32_t* tiles, int64_t capac
 
 template <bool kPacked>
 int gate_up_dispatch(const void* x_perm, const int32_t* tiles, int64_t capacity, const void* const* w_gate,
-                     const void* const* w_up, int64_t n_rows, int n_experts, int64_t dim, int64_t dim_ffn,
+                     const void* const* w_up, const RowCounts& rows, int64_t dim, int64_t dim_ffn,
                      int block_m, void* h, hipStream_t s, const GemmWorkspace& ws) {
   if constexpr (!kPacked) {
-    const Tiles pick = pick_tiles(n_rows, n_experts, block_m, dim, dim_ffn, true).tiles;
+    const Tiles pick = pick_tiles(rows, block_m, dim, dim_ffn, true).tiles;
     if (pick != Tiles::kList)
       return launch_picked<true>(pick, x_perm, tiles, capacity, w_gate, w_up, nullptr, dim, dim_ffn, h, s);
   }
@@ -1214,10 +1245,10 @@ int gate_up_dispatch(const void* x_perm, const int32_t* tiles, int64_t capacity,
 
 template <bool kPacked>
 int down_dispatch(const void* h, const int32_t* tiles, int64_t capacity, const void* const* w_down,
-                  const void* sorted_w, int64_t n_rows, int n_experts, int64_t dim_ffn, int64_t dim, int block_m,
+                  const void* sorted_w, const RowCounts& rows, int64_t dim_ffn, int64_t dim, int block_m,
                   void* y, hipStream_t s, const GemmWorkspace& ws) {
   if constexpr (!kPacked) {
-    const Tiles pick = pick_tiles(n_rows, n_experts, block_m, dim_ffn, dim, false).tiles;
+    const Tiles pick = pick_tiles(rows, block_m, dim_ffn, dim, false).tiles;
     if (pick != Tiles::kList)
       return launch_picked<false>(pick, h, tiles, capacity, w_down, nullptr, sorted_w, dim_ffn, dim, y, s);
   }
@@ -1251,9 +1282,9 @@ bool mfma_gate_up_supported(int64_t dim, int64_t dim_ffn, int block_m, const voi
 // 238, 185 and 131, 120, 219; D 1536, F 4096, 1280 rows 48, 51, 34 and 28, 33, 71.
 int dense_gemm_block_m(int64_t n_rows, int64_t k, int64_t n, bool gate_up) {
   int best = kMfmaBigBM;
-  double least = pick_tiles(n_rows, 1, best, k, n, gate_up).us_per_step;
+  double least = pick_tiles({n_rows, 1}, best, k, n, gate_up).us_per_step;
   for (int bm : {kMfmaMid2BM, kMfmaMidBM}) {
-    const double t = pick_tiles(n_rows, 1, bm, k, n, gate_up).us_per_step;
+    const double t = pick_tiles({n_rows, 1}, bm, k, n, gate_up).us_per_step;
     if (t < 0.95 * least) best = bm, least = t;
   }
   return best;
@@ -1276,30 +1307,30 @@ namespace ragged {
 #endif
 
 int launch_mfma_gate_up(const void* x_perm, const int32_t* tiles, int64_t capacity, const void* const* w_gate,
-                        const void* const* w_up, int64_t n_rows, int n_experts, int64_t dim, int64_t dim_ffn, int block_m,
+                        const void* const* w_up, const RowCounts& rows, int64_t dim, int64_t dim_ffn, int block_m,
                         bool packed, void* h, hipStream_t s, const GemmWorkspace& ws) {
 #if ASTRAI_MOE_RAGGED_K
   if (packed) return fail(ASTRAI_MOE_EINVAL, "gemm_gate_up: packed weights need whole K steps");
 #else
   if (dim % kBK != 0)
-    return ragged::launch_mfma_gate_up(x_perm, tiles, capacity, w_gate, w_up, n_rows, n_experts, dim, dim_ffn, block_m, packed,
+    return ragged::launch_mfma_gate_up(x_perm, tiles, capacity, w_gate, w_up, rows, dim, dim_ffn, block_m, packed,
                                        h, s, ws);
 #endif
-  return packed ? gate_up_dispatch<!kRagged>(x_perm, tiles, capacity, w_gate, w_gate, n_rows, n_experts, dim, dim_ffn, block_m, h, s, ws)
-                : gate_up_dispatch<false>(x_perm, tiles, capacity, w_gate, w_up, n_rows, n_experts, dim, dim_ffn, block_m, h, s, ws);
+  return packed ? gate_up_dispatch<!kRagged>(x_perm, tiles, capacity, w_gate, w_gate, rows, dim, dim_ffn, block_m, h, s, ws)
+                : gate_up_dispatch<false>(x_perm, tiles, capacity, w_gate, w_up, rows, dim, dim_ffn, block_m, h, s, ws);
 }
 
 int launch_mfma_down(const void* h, const int32_t* tiles, int64_t capacity, const void* const* w_down,
-                     const void* sorted_w, int64_t n_rows, int n_experts, int64_t dim_ffn, int64_t dim, int block_m,
+                     const void* sorted_w, const RowCounts& rows, int64_t dim_ffn, int64_t dim, int block_m,
                      bool packed, void* y, hipStream_t s, const GemmWorkspace& ws) {
 #if ASTRAI_MOE_RAGGED_K
   if (packed) return fail(ASTRAI_MOE_EINVAL, "gemm_down: packed weights need whole K steps");
 #else
   if (dim_ffn % kBK != 0)
-    return ragged::launch_mfma_down(h, tiles, capacity, w_down, sorted_w, n_rows, n_experts, dim_ffn, dim, block_m, packed, y, s, ws);
+    return ragged::launch_mfma_down(h, tiles, capacity, w_down, sorted_w, rows, dim_ffn, dim, block_m, packed, y, s, ws);
 #endif
-  return packed ? down_dispatch<!kRagged>(h, tiles, capacity, w_down, sorted_w, n_rows, n_experts, dim_ffn, dim, block_m, y, s, ws)
-                : down_dispatch<false>(h, tiles, capacity, w_down, sorted_w, n_rows, n_experts, dim_ffn, dim, block_m, y, s, ws);
+  return packed ? down_dispatch<!kRagged>(h, tiles, capacity, w_down, sorted_w, rows, dim_ffn, dim, block_m, y, s, ws)
+                : down_dispatch<false>(h, tiles, capacity, w_down, sorted_w, rows, dim_ffn, dim, block_m, y, s, ws);
 }
 
 int launch_mfma_gate_up_save(const void* x_perm, const int32_t* tiles, int64_t capacity, const void* const* w_gate,
@@ -1325,15 +1356,15 @@ int launch_mfma_down_save(const void* h, const int32_t* tiles, int64_t capacity,
 }
 
 int launch_mfma_gate_up_gather(const void* x, const int32_t* sorted_token, const int32_t* tiles, int64_t capacity,
-                               const void* const* w_gate, const void* const* w_up, int64_t n_rows, int n_experts,
+                               const void* const* w_gate, const void* const* w_up, const RowCounts& rows,
                                int64_t dim, int64_t dim_ffn, int block_m, void* h, hipStream_t s,
                                const GemmWorkspace& ws) {
 #if !ASTRAI_MOE_RAGGED_K
   if (dim % kBK != 0)
-    return ragged::launch_mfma_gate_up_gather(x, sorted_token, tiles, capacity, w_gate, w_up, n_rows, n_experts, dim,
+    return ragged::launch_mfma_gate_up_gather(x, sorted_token, tiles, capacity, w_gate, w_up, rows, dim,
                                               dim_ffn, block_m, h, s, ws);
 #endif
-  const Tiles pick = pick_tiles(n_rows, n_experts, block_m, dim, dim_ffn, true).tiles;
+  const Tiles pick = pick_tiles(rows, block_m, dim, dim_ffn, true).tiles;
   if (pick != Tiles::kList)
     return launch_picked<true, true>(pick, x, tiles, capacity, w_gate, w_up, nullptr, dim, dim_ffn, h, s, sorted_token);
   if (block_m == kMfmaBigBM)

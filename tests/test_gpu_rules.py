@@ -1,0 +1,39 @@
+"""Which kernels a layer's GEMMs run on where the rules' lines lie: the rules
+see a load's sizes only, so a choice has to hold for skewed routers too."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+from torch.profiler import ProfilerActivity, profile
+
+from test_gpu_backward import _random_layer
+
+pytestmark = pytest.mark.gpu
+
+
+def _gemms(run):
+    """Names of the GEMM kernels that ``run`` launches, in order."""
+    run()
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA, ProfilerActivity.CPU]) as p:
+        run()
+        torch.cuda.synchronize()
+    names = [(e.time_range.start, torch._C._demangle(e.name)) for e in p.events() if "gemm_" in e.name and "kernel" in e.name]
+    return [n for _, n in sorted(names)]
+
+
+@pytest.mark.parametrize("n_tok,n_exp,top_k,n_shared,dim,dim_ffn,up,down", [
+    # 8 row tiles of 128 rows if even, 9 if not: 32 columns of 128 fill one round exactly or take two
+    (256, 8, 2, 0, 4096, 128, "gemm_mfma_kernel", "TileCfg<128, 256"),
+    # one round of long 256-row tiles that is not split along K (more than half a round): narrower tiles
+    (640, 8, 2, 0, 1000, 4096, "gemm_stream_kernel", "TileCfg<128, 128"),
+    (640, 8, 2, 0, 1000, 4040, "gemm_stream_kernel", "TileCfg<128, 128"),
+    # a short last round of them that is
+    (8192, 8, 2, 0, 1000, 4040, "gemm_stream_kernel", "gemm_stream_kernel"),
+])
+def test_tiles(gpu, n_tok, n_exp, top_k, n_shared, dim, dim_ffn, up, down):
+    layer = _random_layer(gpu, dim, dim_ffn, n_exp, n_shared, top_k, torch.bfloat16, seed=1).requires_grad_(False)
+    x = torch.randn(1, n_tok, dim, device=gpu).to(torch.bfloat16)
+    first, second = _gemms(lambda: layer(x))[:2]
+    assert up in first and down in second, (first, second)
