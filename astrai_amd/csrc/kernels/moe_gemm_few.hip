@@ -319,7 +319,7 @@ int launch_few_cfg(const void* A, const RowTiles<kDense>& tiles, int64_t capacit
 
 // Experts that meet one of n_rows rows, expected under even routing.
 double live_experts(int64_t n_rows, int n_experts) {
-  return n_experts * (1.0 - std::pow(1.0 - 1.0 / n_experts, (double)n_rows));
+  return n_experts > 0 ? n_experts * (1.0 - std::pow(1.0 - 1.0 / n_experts, (double)n_rows)) : 0.0;
 }
 
 // Share of the compute-unit time that `tiles` equal tiles fill, a partial last
@@ -330,8 +330,8 @@ double fill(double tiles) {
 }
 
 // Limits of few_rows (below), which has the figures.
-constexpr int kFewRowsPerExpert = 24, kFewDenseRows = 128, kFewLongSteps = 12;
-constexpr double kFewMaxFill = 0.9;
+constexpr int kFewRowsPerExpert = 8, kFewExactRows = 64, kFewSmallRows = 24, kFewDenseRows = 128, kFewLongSteps = 12;
+constexpr double kFewMaxFill = 0.88, kFewMaxFillLong = 0.86, kFewLongRounds = 3.0;
 
 // Tiles of 64 activation rows where most experts, or more than two runs of 32
 // of one expert, have more than 32 rows (MLP of D 4096, F 14336: 96 rows 197 ->
@@ -348,7 +348,7 @@ template <bool kGateUp, bool kGather, bool kPacked, bool kDense>
 int launch_few_tiles(const void* A, const RowTiles<kDense>& tiles, int64_t capacity, const void* const* W0, const void* const* W1,
                const void* row_w, const RowCounts& load, int64_t K, int64_t N, void* C, hipStream_t s,
                const int32_t* row_src) {
-  if (load.total() > (load.dense() ? 2 * FewCfg<32, 32>::BM : (int64_t)kFewRowsPerExpert * (load.experts + load.exact)))
+  if (load.total() > (load.dense() ? 2 * FewCfg<32, 32>::BM : (int64_t)kFewSmallRows * (load.experts + load.exact)))
     return launch_few_cfg<FewCfg<64, 32>, kGateUp, kGather, kPacked, kDense>(A, tiles, capacity, W0, W1, row_w, K, N, C, s,
                                                                      row_src);
   if (load.dense() && load.total() <= FewCfg<32, 16>::BM &&
@@ -367,35 +367,51 @@ int launch_few(const void* A, const int32_t* tiles, int64_t capacity, const void
 
 }  // namespace
 
-// Where these kernels replace the 256-column tiles of moe_gemm_mfma.hip:
-// - up to kFewRowsPerExpert rows per expert (above, experts of more than 32 rows
-//   read their weights in two runs), or kFewDenseRows of one expert, whose rows
-//   are known, where the other kernel's last round of tiles would leave more
-//   than a tenth of its compute-unit time idle;
-// - up to twice as many where its tiles occupy at most half the compute units
-//   and are long, kFewLongSteps K steps or more (16 experts, top-4 and a shared
-//   one, D 704, F 576, 9 and 11 steps, 160 tokens: 47.9 / 49.8).
+// Where these kernels replace the 256-column tiles of moe_gemm_mfma.hip. An
+// expert of more than 32 rows reads its weights once for each run, so the lines
+// lie where a skewed router, of which the host sees nothing, loses nothing
+// either (a Zipf bias of exponent 1.44 below; us per layer or MLP without and
+// with, replayed from a graph):
+// - up to kFewRowsPerExpert routed rows per expert, where the other kernel's
+//   last round of tiles would leave more than kFewMaxFill of its compute-unit
+//   time idle (kFewMaxFillLong past kFewLongRounds rounds, of which one more
+//   costs less). 8 experts, top-2, D 4096, F 14336: 1 token 264 / 165, 8 532 /
+//   495; past the line, 33 tokens 539 / 520, skewed 555 / 522, but 48 538 / 590
+//   skewed, 80 553 / 673 and 96 552 / 711. 64 experts, top-6, D 2048, F 1408: 1
+//   token 74 / 60, 32 (2.6 rounds, 0.87) 229 / 217; 128 experts, top-8, D 4096, F
+//   1536, 33 tokens (5.2 rounds, 0.87) 797 / 813, skewed 298 / 311. Shared
+//   experts run along with up to two runs of rows each (kFewExactRows; 128
+//   experts and a shared one, 256 tokens 908 / 961, skewed 615 / 742);
+// - small layers, whose tiles occupy at most a quarter of the compute units and
+//   whose weights the caches hold: below kFewSmallRows rows per expert, and twice
+//   as many where they occupy an eighth in kFewLongSteps K steps or more. 8
+//   experts, top-2, D 1000, F 2664, 64 tokens 73 / 53, 192 77 / 68, skewed 76 / 59
+//   and 77 / 75; D 512, F 4096, 64 66 / 43, 192 72 / 55; a quarter, D 2048, F 8192:
+//   64 212 / 178, skewed 189 / 145; past the line 192 skewed 219 / 262;
+// - one expert, whose rows are known, up to kFewDenseRows of them by the first
+//   rule, and twice as many where its tiles occupy at most half the compute units
+//   in kFewLongSteps K steps or more. D 4096, F 14336: 1 row 201 / 81, 24 217 /
+//   90, 64 214 / 133, 128 235 / 156, 256 (the down GEMM; its gate/up GEMM has 448
+//   tiles) 255 / 191; D 2048, F 5632: 24 66 / 28, 128 72 / 43, 256 73 / 44.
 // The same for tiles of 32, 64 and 128 rows, so that these give the same bits;
 // lists of 256-row tiles keep their kernels, whose bits the training forward
-// shares. Measured, us per layer or MLP without and with (replayed from a
-// graph, three sets of weights in turn):
-// - 8 experts, top-2, D 4096, F 14336: 1 token 264 / 165, 2 368 / 286, 8 532 /
-//   495, 64 593 / 552, 96 (24 rows per expert) 602 / 590, 128 608 / 716;
-// - 64 experts, top-6, D 2048, F 1408: 1 token 74 / 60, 8 158 / 144, 32 226 /
-//   224, 64 (rounds of 0.92 and 1.0, past the line) 232 / 233;
-// - 8 experts, top-2 and a shared one, D 1000, F 2664, 96 tokens (32 rows per
-//   expert; the down GEMM has 36 tiles) 120 / 97, 160 127 / 109;
-// - MLP, D 4096, F 14336: 1 token 201 / 81, 24 217 / 90, 64 214 / 133, 128 235 /
-//   156, 256 (the down GEMM; its gate/up GEMM has 448 tiles) 255 / 191; D 2048, F
-//   5632: 24 66 / 28, 128 72 / 43, 256 73 / 44.
+// shares.
 bool few_rows(const RowCounts& rows, int block_m, int64_t k, int64_t n, bool gate_up) {
   if (block_m == kMfmaBigBM) return false;
-  const int experts = rows.experts + rows.exact;
-  const int64_t n_rows = rows.total(), most = rows.dense() ? kFewDenseRows : (int64_t)kFewRowsPerExpert * experts;
-  const double cols = (double)ceil_div(n, gate_up ? 128 : 256);
-  if (n_rows <= most) return fill(live_experts(n_rows, experts) * cols) < kFewMaxFill;
-  const double row_tiles = rows.dense() ? (double)ceil_div(n_rows, kMfmaMidBM) : (double)experts;
-  return n_rows <= 2 * most && k_steps(k) >= kFewLongSteps && 2 * row_tiles * cols <= cu_count();
+  const double cols = (double)ceil_div(n, gate_up ? 128 : 256), cu = cu_count();
+  const bool long_steps = k_steps(k) >= kFewLongSteps;
+  if (rows.dense()) {
+    const int64_t n_rows = rows.exact_rows;
+    if (n_rows <= kFewDenseRows) return fill(cols) < kFewMaxFill;
+    return n_rows <= 2 * kFewDenseRows && long_steps && 2.0 * ceil_div(n_rows, kMfmaMidBM) * cols <= cu;
+  }
+  if (rows.rows <= (int64_t)kFewRowsPerExpert * rows.experts && rows.exact_rows <= kFewExactRows) {
+    const double tiles = (live_experts(rows.rows, rows.experts) + rows.exact * ceil_div(rows.exact_rows, kMfmaSmallBM)) * cols;
+    if (fill(tiles) < (tiles <= kFewLongRounds * cu ? kFewMaxFill : kFewMaxFillLong)) return true;
+  }
+  const double tiles = std::max(rows.experts, rows.exact) * cols;
+  const int64_t small = (int64_t)kFewSmallRows * (rows.experts + rows.exact);
+  return (rows.total() < small && 4.0 * tiles <= cu) || (rows.total() <= 2 * small && long_steps && 8.0 * tiles <= cu);
 }
 
 int launch_few_gate_up(const void* x, const int32_t* row_src, const int32_t* tiles, int64_t capacity,

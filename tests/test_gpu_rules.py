@@ -37,3 +37,27 @@ def test_tiles(gpu, n_tok, n_exp, top_k, n_shared, dim, dim_ffn, up, down):
     x = torch.randn(1, n_tok, dim, device=gpu).to(torch.bfloat16)
     first, second = _gemms(lambda: layer(x))[:2]
     assert up in first and down in second, (first, second)
+
+
+FEW, LIST = "gemm_few_kernel", "gemm_mfma_kernel"
+
+
+@pytest.mark.parametrize("n_tok,n_exp,top_k,n_shared,dim,dim_ffn,up,down", [
+    # 8 routed rows per expert and the next (the down GEMM has 128 tiles: half the compute units)
+    (32, 8, 2, 0, 4096, 128, FEW, FEW),
+    (33, 8, 2, 0, 4096, 128, FEW, LIST),
+    (96, 8, 2, 0, 4096, 128, FEW, LIST),
+    # shared experts: two runs of their rows, and three
+    (64, 32, 2, 1, 4096, 128, FEW, FEW),
+    (65, 32, 2, 1, 4096, 128, FEW, LIST),
+    # small layers: a quarter of the compute units, an eighth and many K steps
+    (80, 8, 2, 0, 2048, 128, FEW, FEW),
+    (96, 8, 2, 0, 2048, 768, LIST, LIST),
+    (192, 8, 2, 0, 1024, 768, LIST, FEW),
+    (193, 8, 2, 0, 1024, 768, LIST, LIST),
+])
+def test_few_rows(gpu, n_tok, n_exp, top_k, n_shared, dim, dim_ffn, up, down):
+    layer = _random_layer(gpu, dim, dim_ffn, n_exp, n_shared, top_k, torch.bfloat16, seed=1).requires_grad_(False)
+    x = torch.randn(1, n_tok, dim, device=gpu).to(torch.bfloat16)
+    first, second = _gemms(lambda: layer(x))[:2]
+    assert up in first and down in second, (first, second)
