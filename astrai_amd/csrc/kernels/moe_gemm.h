@@ -175,11 +175,11 @@ int launch_few_gate_up(const void* x, const int32_t* row_src,
                        const int32_t* tiles, int64_t capacity,
                        const void* const* w_gate, const void* const* w_up,
                        const RowCounts& rows, int64_t dim, int64_t dim_ffn,
-                       bool packed, void* h, hipStream_t s);
+                       int block_m, bool packed, void* h, hipStream_t s);
 int launch_few_down(const void* h, const int32_t* tiles, int64_t capacity,
                     const void* const* w_down, const void* sorted_w,
                     const RowCounts& rows, int64_t dim_ffn, int64_t dim,
-                    bool packed, void* y, hipStream_t s);
+                    int block_m, bool packed, void* y, hipStream_t s);
 // Both GEMMs of one dense expert whose GEMMs few_rows both takes, without a
 // tile list.
 int launch_few_dense(const void* x, const void* const* w_gate,

@@ -193,7 +193,7 @@ int launch_gate_up(const void* x_perm, const int32_t* tiles, int64_t tiles_len, 
   if (dtype == ASTRAI_MOE_BF16) {
     const bool mfma = mfma_gate_up_supported(dim, dim_ffn, block_m, x_perm, h);
     if (mfma && few_rows(rows, block_m, dim, dim_ffn, true))
-      return launch_few_gate_up(x_perm, nullptr, tiles, capacity, w_gate, w_up, rows, dim, dim_ffn, packed, h, s);
+      return launch_few_gate_up(x_perm, nullptr, tiles, capacity, w_gate, w_up, rows, dim, dim_ffn, block_m, packed, h, s);
     if (mfma)
       return launch_mfma_gate_up(x_perm, tiles, capacity, w_gate, w_up, rows, dim, dim_ffn, block_m, packed, h, s, ws);
     return launch_generic<bf16_t, true>(x_perm, tiles, capacity, w_gate, w_up, nullptr, dim, dim_ffn, h, s);
@@ -211,7 +211,7 @@ int launch_down(const void* h, const int32_t* tiles, int64_t tiles_len, const vo
   if (dtype == ASTRAI_MOE_BF16) {
     const bool mfma = mfma_down_supported(dim_ffn, dim, block_m, h, y);
     if (mfma && few_rows(rows, block_m, dim_ffn, dim, false))
-      return launch_few_down(h, tiles, capacity, w_down, sorted_w, rows, dim_ffn, dim, packed, y, s);
+      return launch_few_down(h, tiles, capacity, w_down, sorted_w, rows, dim_ffn, dim, block_m, packed, y, s);
     if (mfma)
       return launch_mfma_down(h, tiles, capacity, w_down, sorted_w, rows, dim_ffn, dim, block_m, packed, y, s, ws);
     return launch_generic<bf16_t, false>(h, tiles, capacity, w_down, nullptr, sorted_w, dim_ffn, dim, y, s);
@@ -227,7 +227,7 @@ int launch_gate_up_gather(const void* x, const int32_t* sorted_token, const int3
                           int64_t dim_ffn, int block_m, void* h, const GemmWorkspace& ws, hipStream_t s) {
   const int64_t capacity = tile_capacity(tiles_len);
   if (few_rows(rows, block_m, dim, dim_ffn, true))
-    return launch_few_gate_up(x, sorted_token, tiles, capacity, w_gate, w_up, rows, dim, dim_ffn, false, h, s);
+    return launch_few_gate_up(x, sorted_token, tiles, capacity, w_gate, w_up, rows, dim, dim_ffn, block_m, false, h, s);
   return launch_mfma_gate_up_gather(x, sorted_token, tiles, capacity, w_gate, w_up, rows, dim, dim_ffn, block_m, h, s,
                                     ws);
 }

@@ -24,6 +24,7 @@
 // Measured: an MLP of D 4096, F 14336 over 24 rows 205 -> 100 us (352 MB of
 // weights, 3.5 TB/s), two experts of one token 240 -> 141 us (705 MB, 5.0
 // TB/s; its down GEMM 145 -> 45 us); more at few_rows below.
+#include <algorithm>
 #include <cmath>
 
 #include "mfma_tile.h"
@@ -333,9 +334,12 @@ double fill(double tiles) {
 constexpr int kFewRowsPerExpert = 8, kFewExactRows = 64, kFewSmallRows = 24, kFewDenseRows = 128, kFewLongSteps = 12;
 constexpr double kFewMaxFill = 0.88, kFewMaxFillLong = 0.86, kFewLongRounds = 3.0;
 
-// Tiles of 64 activation rows where most experts, or more than two runs of 32
-// of one expert, have more than 32 rows (MLP of D 4096, F 14336: 96 rows 197 ->
-// 149 us, 64 rows 133 -> 138).
+// Tiles of 64 activation rows on lists of at least that height, where most
+// experts, or more than two runs of 32 of one expert, have more than 32 rows
+// (MLP of D 4096, F 14336: 96 rows 197 -> 149 us, 64 rows 133 -> 138). One
+// expert without a list takes rows of 64 from 65 rows on (80 rows 196 -> 132,
+// 64-row tiles over 32-row ones before; D 2048, F 5632 46 -> 37) unless its
+// 32-row tiles all run at once (D 512, F 1024 9.7 / 10.4).
 //
 // One expert's single run of 32 rows (an MLP decoding) takes tiles of 16 weight
 // rows where those fill the rounds of tiles better: D 4096, F 14336, 24 rows,
@@ -346,9 +350,10 @@ constexpr double kFewMaxFill = 0.88, kFewMaxFillLong = 0.86, kFewLongRounds = 3.
 // -> 560; 64 of D 2048, F 1408, 8 tokens 144 -> 188).
 template <bool kGateUp, bool kGather, bool kPacked, bool kDense>
 int launch_few_tiles(const void* A, const RowTiles<kDense>& tiles, int64_t capacity, const void* const* W0, const void* const* W1,
-               const void* row_w, const RowCounts& load, int64_t K, int64_t N, void* C, hipStream_t s,
+               const void* row_w, const RowCounts& load, int block_m, int64_t K, int64_t N, void* C, hipStream_t s,
                const int32_t* row_src) {
-  if (load.total() > (load.dense() ? 2 * FewCfg<32, 32>::BM : (int64_t)kFewSmallRows * (load.experts + load.exact)))
+  if (block_m >= FewCfg<64, 32>::BM &&
+      load.total() > (load.dense() ? 2 * FewCfg<32, 32>::BM : (int64_t)kFewSmallRows * (load.experts + load.exact)))
     return launch_few_cfg<FewCfg<64, 32>, kGateUp, kGather, kPacked, kDense>(A, tiles, capacity, W0, W1, row_w, K, N, C, s,
                                                                      row_src);
   if (load.dense() && load.total() <= FewCfg<32, 16>::BM &&
@@ -359,9 +364,9 @@ int launch_few_tiles(const void* A, const RowTiles<kDense>& tiles, int64_t capac
 
 template <bool kGateUp, bool kGather, bool kPacked>
 int launch_few(const void* A, const int32_t* tiles, int64_t capacity, const void* const* W0, const void* const* W1,
-               const void* row_w, const RowCounts& load, int64_t K, int64_t N, void* C, hipStream_t s,
+               const void* row_w, const RowCounts& load, int block_m, int64_t K, int64_t N, void* C, hipStream_t s,
                const int32_t* row_src) {
-  return launch_few_tiles<kGateUp, kGather, kPacked>(A, RowTiles<false>{tiles, 0, 0}, capacity, W0, W1, row_w, load, K,
+  return launch_few_tiles<kGateUp, kGather, kPacked>(A, RowTiles<false>{tiles, 0, 0}, capacity, W0, W1, row_w, load, block_m, K,
                                                      N, C, s, row_src);
 }
 
@@ -416,30 +421,33 @@ bool few_rows(const RowCounts& rows, int block_m, int64_t k, int64_t n, bool gat
 
 int launch_few_gate_up(const void* x, const int32_t* row_src, const int32_t* tiles, int64_t capacity,
                        const void* const* w_gate, const void* const* w_up, const RowCounts& rows, int64_t dim,
-                       int64_t dim_ffn, bool packed, void* h, hipStream_t s) {
-  if (packed) return launch_few<true, false, true>(x, tiles, capacity, w_gate, w_gate, nullptr, rows, dim, dim_ffn, h, s, nullptr);
+                       int64_t dim_ffn, int block_m, bool packed, void* h, hipStream_t s) {
+  if (packed) return launch_few<true, false, true>(x, tiles, capacity, w_gate, w_gate, nullptr, rows, block_m, dim, dim_ffn, h, s, nullptr);
   if (row_src != nullptr)
-    return launch_few<true, true, false>(x, tiles, capacity, w_gate, w_up, nullptr, rows, dim, dim_ffn, h, s, row_src);
-  return launch_few<true, false, false>(x, tiles, capacity, w_gate, w_up, nullptr, rows, dim, dim_ffn, h, s, nullptr);
+    return launch_few<true, true, false>(x, tiles, capacity, w_gate, w_up, nullptr, rows, block_m, dim, dim_ffn, h, s, row_src);
+  return launch_few<true, false, false>(x, tiles, capacity, w_gate, w_up, nullptr, rows, block_m, dim, dim_ffn, h, s, nullptr);
 }
 
 int launch_few_down(const void* h, const int32_t* tiles, int64_t capacity, const void* const* w_down,
-                    const void* sorted_w, const RowCounts& rows, int64_t dim_ffn, int64_t dim, bool packed,
+                    const void* sorted_w, const RowCounts& rows, int64_t dim_ffn, int64_t dim, int block_m, bool packed,
                     void* y, hipStream_t s) {
   if (packed)
-    return launch_few<false, false, true>(h, tiles, capacity, w_down, w_down, sorted_w, rows, dim_ffn, dim, y, s, nullptr);
-  return launch_few<false, false, false>(h, tiles, capacity, w_down, w_down, sorted_w, rows, dim_ffn, dim, y, s, nullptr);
+    return launch_few<false, false, true>(h, tiles, capacity, w_down, w_down, sorted_w, rows, block_m, dim_ffn, dim, y, s, nullptr);
+  return launch_few<false, false, false>(h, tiles, capacity, w_down, w_down, sorted_w, rows, block_m, dim_ffn, dim, y, s, nullptr);
 }
 
 int launch_few_dense(const void* x, const void* const* w_gate, const void* const* w_up, const void* const* w_down,
                      int64_t n_rows, int64_t dim, int64_t dim_ffn, int block_m, void* h, void* out, hipStream_t s) {
+  using Low = FewCfg<32, 32>;
+  if (n_rows > 2 * Low::BM && ceil_div(n_rows, Low::BM) * ceil_div(dim_ffn, Low::BN / 2) > cu_count())
+    block_m = std::max(block_m, FewCfg<64, 32>::BM);
   const RowTiles<true> rows{nullptr, (int)n_rows, block_m};
   const RowCounts load(n_rows, 1);
   const int64_t n_tiles = ceil_div(n_rows, block_m);
-  if (int rc = launch_few_tiles<true, false, false>(x, rows, n_tiles, w_gate, w_up, nullptr, load, dim, dim_ffn, h,
+  if (int rc = launch_few_tiles<true, false, false>(x, rows, n_tiles, w_gate, w_up, nullptr, load, block_m, dim, dim_ffn, h,
                                                     s, nullptr))
     return rc;
-  return launch_few_tiles<false, false, false>(h, rows, n_tiles, w_down, nullptr, nullptr, load, dim_ffn, dim, out,
+  return launch_few_tiles<false, false, false>(h, rows, n_tiles, w_down, nullptr, nullptr, load, block_m, dim_ffn, dim, out,
                                                s, nullptr);
 }
 

@@ -7,6 +7,7 @@ import pytest
 import torch
 from torch.profiler import ProfilerActivity, profile
 
+from astrai_amd.extension import ops
 from test_gpu_backward import _random_layer
 
 pytestmark = pytest.mark.gpu
@@ -61,3 +62,17 @@ def test_few_rows(gpu, n_tok, n_exp, top_k, n_shared, dim, dim_ffn, up, down):
     x = torch.randn(1, n_tok, dim, device=gpu).to(torch.bfloat16)
     first, second = _gemms(lambda: layer(x))[:2]
     assert up in first and down in second, (first, second)
+
+
+@pytest.mark.parametrize("n_tok,dim_ffn,listed,rows", [
+    (64, 4096, False, 32), (65, 4096, False, 64), (95, 4096, False, 64), (96, 4096, False, 64), (95, 1024, False, 32),
+    (95, 4096, True, 32), (96, 4096, True, 64),
+])
+def test_few_row_tiles_fit_the_list(gpu, n_tok, dim_ffn, listed, rows):
+    # one expert: 64-row tiles only over row tiles of that height, which a list of 65 to 95 rows has not
+    ws = [(torch.randn(*s, device=gpu) * 0.02).bfloat16() for s in ((dim_ffn, 512), (dim_ffn, 512), (512, dim_ffn))]
+    tables = [ops.expert_weight_table([w], tuple(w.shape)) for w in ws]
+    x = torch.randn(n_tok, 512, device=gpu).bfloat16()
+    tiles = ops.dense_tiles(n_tok, ops.dense_block_m(n_tok, 512, dim_ffn, x.dtype), x.device) if listed else None
+    names = _gemms(lambda: ops.moe_dense_mlp(x, *tables, dim_ffn, tiles=tiles))
+    assert len(names) == 2 and all(f"FewCfg<{rows}, 32>" in n for n in names), names
