@@ -27,11 +27,14 @@ struct Sizes {
 // Byte offsets of the workspace's parts, 256-byte aligned.
 struct Plan {
   int experts, slots, block_m;
+  bool packed_up, packed_down;  // the GEMM reads the packed copies
   int64_t rows, tiles_len;
   bool gather, gather_ragged, gather_f32;
   int64_t topk_idx, topk_w, chunk_hist, chunk_base, offsets, sorted_token, sorted_w, token_pos, tiles, x_perm, h, y,
       gemm_ws, gemm_ws_bytes, bytes;
 };
+
+RowCounts row_counts(const Sizes& z) { return {z.n_tokens * z.top_k, z.n_experts, z.n_shared, z.n_tokens}; }
 
 int check_sizes(const Sizes& z) {
   ASTRAI_REQUIRE(z.dtype == ASTRAI_MOE_BF16 || z.dtype == ASTRAI_MOE_F32, "forward: unsupported dtype %d", z.dtype);
@@ -56,13 +59,18 @@ Plan make_plan(const Sizes& z) {
   p.rows = T * p.slots;
   p.block_m = astrai_moe_select_block_m(T, z.n_experts, z.top_k, z.dim, z.dim_ffn, z.dtype);
   p.tiles_len = astrai_moe_tile_list_len(T, p.experts, p.slots, p.block_m);
+  // Few rows read the live weights: the same bits, and their tiles of 32 weight
+  // rows stream these better than the copies' blocks of 256 (8 experts, top-2, D
+  // 4096, F 14336, 8 tokens 538 / 502 us a layer, 32 545 / 500).
+  p.packed_up = z.packed && !few_rows(row_counts(z), p.block_m, z.dim, z.dim_ffn, true);
+  p.packed_down = z.packed && !few_rows(row_counts(z), p.block_m, z.dim_ffn, z.dim, false);
   // the bf16 gate/up GEMM reads the token rows itself where its kernels do
   // (32-bit row offsets: x under 4 GiB)
-  p.gather = z.dtype == ASTRAI_MOE_BF16 && !z.packed && mfma_shape_supported(z.dim, z.dim_ffn) && z.dim % 64 == 0 &&
+  p.gather = z.dtype == ASTRAI_MOE_BF16 && !p.packed_up && mfma_shape_supported(z.dim, z.dim_ffn) && z.dim % 64 == 0 &&
              z.dim_ffn % 64 == 0 && T * z.dim * 2 < (1ll << 32);
   // (other dims: where x is aligned, below; 1500 tokens of D 1000, F 2664 with a
   // shared expert 162 us a layer with copied rows, 149 without)
-  p.gather_ragged = z.dtype == ASTRAI_MOE_BF16 && !z.packed && mfma_shape_supported(z.dim, z.dim_ffn) && !p.gather &&
+  p.gather_ragged = z.dtype == ASTRAI_MOE_BF16 && !p.packed_up && mfma_shape_supported(z.dim, z.dim_ffn) && !p.gather &&
                     T * z.dim * 2 < (1ll << 32);
   p.gather_f32 = z.dtype == ASTRAI_MOE_F32 && T * z.dim * 4 < (1ll << 32) &&
                  mfma_f32_supported(z.dim, z.dim_ffn, true, p.block_m, nullptr, nullptr, nullptr);
@@ -154,7 +162,7 @@ extern "C" int astrai_moe_forward(const void* x, const void* logits, const void*
                             i32(p.chunk_base), stream);
   }
   if (rc) return rc;
-  const RowCounts rows(n_tokens * top_k, n_experts, n_shared, n_tokens);
+  const RowCounts rows = row_counts(z);
   const GemmWorkspace ws{gws, p.gemm_ws_bytes};
   if (gather)
     rc = launch_gate_up_gather(x, sorted_token, tiles, p.tiles_len, w_gate, w_up, rows, dim, dim_ffn, p.block_m, h, ws,
@@ -163,11 +171,11 @@ extern "C" int astrai_moe_forward(const void* x, const void* logits, const void*
     rc = launch_mfma_f32_gate_up(x, tiles, (p.tiles_len - ASTRAI_MOE_TILE_HEADER) / ASTRAI_MOE_TILE_STRIDE, w_gate, w_up,
                                  p.rows, p.experts, dim, dim_ffn, h, nullptr, s, sorted_token);
   else
-    rc = launch_gate_up(x_perm, tiles, p.tiles_len, z.packed ? packed_gate_up : w_gate, z.packed ? packed_gate_up : w_up,
-                        dtype, rows, dim, dim_ffn, p.block_m, z.packed, h, ws, s);
+    rc = launch_gate_up(x_perm, tiles, p.tiles_len, p.packed_up ? packed_gate_up : w_gate,
+                        p.packed_up ? packed_gate_up : w_up, dtype, rows, dim, dim_ffn, p.block_m, p.packed_up, h, ws, s);
   if (rc) return rc;
-  rc = launch_down(h, tiles, p.tiles_len, z.packed ? packed_down : w_down, sorted_w, dtype, rows, dim_ffn, dim, p.block_m,
-                   z.packed, y, ws, s);
+  rc = launch_down(h, tiles, p.tiles_len, p.packed_down ? packed_down : w_down, sorted_w, dtype, rows, dim_ffn, dim,
+                   p.block_m, p.packed_down, y, ws, s);
   if (rc) return rc;
   const int64_t size = dtype == ASTRAI_MOE_BF16 ? 2 : 4;
   const void* shared = n_shared > 0 ? static_cast<const char*>(y) + n_tokens * top_k * dim * size : nullptr;

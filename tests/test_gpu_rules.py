@@ -76,3 +76,12 @@ def test_few_row_tiles_fit_the_list(gpu, n_tok, dim_ffn, listed, rows):
     tiles = ops.dense_tiles(n_tok, ops.dense_block_m(n_tok, 512, dim_ffn, x.dtype), x.device) if listed else None
     names = _gemms(lambda: ops.moe_dense_mlp(x, *tables, dim_ffn, tiles=tiles))
     assert len(names) == 2 and all(f"FewCfg<{rows}, 32>" in n for n in names), names
+
+
+def test_few_rows_of_a_packed_layer_read_the_live_weights(gpu):
+    layer = _random_layer(gpu, 512, 1024, 8, 1, 2, torch.bfloat16, seed=1).requires_grad_(False)
+    layer.pack_weights = True
+    x = torch.randn(1, 8, 512, device=gpu).to(torch.bfloat16)
+    first, second = _gemms(lambda: layer(x))[:2]
+    # gemm_few_kernel<..., gate/up, gather, packed, dense>
+    assert "true, true, false, false>" in first and "false, false, false, false>" in second, (first, second)
