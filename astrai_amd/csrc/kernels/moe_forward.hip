@@ -169,7 +169,7 @@ extern "C" int astrai_moe_forward(const void* x, const void* logits, const void*
                                s);
   else if (gather_f32)
     rc = launch_mfma_f32_gate_up(x, tiles, (p.tiles_len - ASTRAI_MOE_TILE_HEADER) / ASTRAI_MOE_TILE_STRIDE, w_gate, w_up,
-                                 p.rows, p.experts, dim, dim_ffn, h, nullptr, s, sorted_token);
+                                 rows, dim, dim_ffn, h, nullptr, s, sorted_token);
   else
     rc = launch_gate_up(x_perm, tiles, p.tiles_len, p.packed_up ? packed_gate_up : w_gate,
                         p.packed_up ? packed_gate_up : w_up, dtype, rows, dim, dim_ffn, p.block_m, p.packed_up, h, ws, s);

@@ -4,6 +4,9 @@
 
 #include "moe_common.h"
 
+#include <algorithm>
+#include <cmath>
+
 namespace astrai_moe {
 
 // Row-tile heights of the bf16 matrix-core kernels. The large tile serves
@@ -81,6 +84,27 @@ struct RowCounts {
   int64_t total() const { return rows + exact * exact_rows; }
   bool dense() const { return experts == 0 && exact == 1; }
 };
+
+// Row tiles of `bm` rows that a load makes: expected under even routing (an
+// expert's rows about normal, with their mean as variance); under a skewed one
+// (the last tile of nearly every expert nearly empty: routers biased by Zipf
+// weights of exponents 0.4 to 4 over 8 to 128 experts gave rows / bm + 0.1 to 0.85
+// per expert); and the most that any routing makes, the list's capacity. The
+// same number where the host knows every expert's rows.
+struct RowTileCount {
+  double even, skewed, most;
+};
+inline RowTileCount count_row_tiles(const RowCounts& rows, int bm) {
+  const double exact = (double)rows.exact * (double)ceil_div(rows.exact_rows, bm);
+  if (rows.experts == 0) return {exact, exact, exact};
+  const double r = (double)rows.rows / rows.experts, sd = std::sqrt(std::max(r, 1.0));
+  double tiles = 0.0;
+  for (int64_t j = 0; j * bm < r + 8.0 * sd; ++j) tiles += 0.5 * std::erfc(((double)(j * bm) - r) / (sd * 1.41421356));
+  const int64_t most = std::min(rows.rows, (rows.rows + (int64_t)rows.experts * (bm - 1)) / bm);
+  const double even = std::min(rows.experts * tiles, (double)most);
+  const double skewed = std::min(std::max(even, (double)rows.rows / bm + 0.8 * rows.experts), (double)most);
+  return {exact + even, exact + skewed, exact + (double)most};
+}
 
 // `packed`: the weight tables point at packed copies written by launch_pack
 // (bf16, 256-row tiles of K / 64 contiguous 32 KB blocks in staged order).
@@ -218,15 +242,13 @@ bool mfma_f32_supported(int64_t k, int64_t n, bool gate_up, int block_m,
                         const void* a, const void* c, const void* s0);
 int launch_mfma_f32_gate_up(const void* x_perm, const int32_t* tiles,
                             int64_t capacity, const void* const* w_gate,
-                            const void* const* w_up, int64_t n_rows,
-                            int n_experts, int64_t dim, int64_t dim_ffn,
-                            void* h, void* gu, hipStream_t s,
-                            const int32_t* row_src = nullptr);
+                            const void* const* w_up, const RowCounts& rows,
+                            int64_t dim, int64_t dim_ffn, void* h, void* gu,
+                            hipStream_t s, const int32_t* row_src = nullptr);
 int launch_mfma_f32_down(const void* h, const int32_t* tiles, int64_t capacity,
                          const void* const* w_down, const void* sorted_w,
-                         int64_t n_rows, int n_experts, int64_t dim_ffn,
-                         int64_t dim, void* y, void* y_unweighted,
-                         hipStream_t s);
+                         const RowCounts& rows, int64_t dim_ffn, int64_t dim,
+                         void* y, void* y_unweighted, hipStream_t s);
 
 // fp32 backward on the matrix cores (moe_gemm_mfma_f32_bwd.hip): the dgrad
 // GEMMs over 64-row tile lists with K a multiple of 32 and N of 4, wgrad with

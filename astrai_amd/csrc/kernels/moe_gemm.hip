@@ -199,8 +199,7 @@ int launch_gate_up(const void* x_perm, const int32_t* tiles, int64_t tiles_len, 
     return launch_generic<bf16_t, true>(x_perm, tiles, capacity, w_gate, w_up, nullptr, dim, dim_ffn, h, s);
   }
   if (mfma_f32_supported(dim, dim_ffn, true, block_m, x_perm, h, nullptr))
-    return launch_mfma_f32_gate_up(x_perm, tiles, capacity, w_gate, w_up, rows.total(), rows.experts + rows.exact, dim,
-                                   dim_ffn, h, nullptr, s);
+    return launch_mfma_f32_gate_up(x_perm, tiles, capacity, w_gate, w_up, rows, dim, dim_ffn, h, nullptr, s);
   return launch_generic<float, true>(x_perm, tiles, capacity, w_gate, w_up, nullptr, dim, dim_ffn, h, s);
 }
 
@@ -217,8 +216,7 @@ int launch_down(const void* h, const int32_t* tiles, int64_t tiles_len, const vo
     return launch_generic<bf16_t, false>(h, tiles, capacity, w_down, nullptr, sorted_w, dim_ffn, dim, y, s);
   }
   if (mfma_f32_supported(dim_ffn, dim, false, block_m, h, y, nullptr))
-    return launch_mfma_f32_down(h, tiles, capacity, w_down, sorted_w, rows.total(), rows.experts + rows.exact, dim_ffn,
-                                dim, y, nullptr, s);
+    return launch_mfma_f32_down(h, tiles, capacity, w_down, sorted_w, rows, dim_ffn, dim, y, nullptr, s);
   return launch_generic<float, false>(h, tiles, capacity, w_down, nullptr, sorted_w, dim_ffn, dim, y, s);
 }
 
@@ -421,7 +419,7 @@ extern "C" int astrai_moe_gemm_gate_up_train(const void* x_perm, const int32_t* 
     return launch_generic<bf16_t, true, true>(x_perm, tiles, capacity, w_gate, w_up, nullptr, dim, dim_ffn, h, s,
                                               gu);
   if (mfma_f32_supported(dim, dim_ffn, true, block_m, x_perm, h, gu))
-    return launch_mfma_f32_gate_up(x_perm, tiles, capacity, w_gate, w_up, n_rows, n_experts, dim, dim_ffn, h, gu, s);
+    return launch_mfma_f32_gate_up(x_perm, tiles, capacity, w_gate, w_up, {n_rows, n_experts}, dim, dim_ffn, h, gu, s);
   return launch_generic<float, true, true>(x_perm, tiles, capacity, w_gate, w_up, nullptr, dim, dim_ffn, h, s, gu);
 }
 
@@ -449,7 +447,7 @@ extern "C" int astrai_moe_gemm_down_train(const void* h, const int32_t* tiles, i
     return launch_generic<bf16_t, false, true>(h, tiles, capacity, w_down, nullptr, sorted_w, dim_ffn, dim, y, s,
                                                y_unweighted);
   if (mfma_f32_supported(dim_ffn, dim, false, block_m, h, y, y_unweighted))
-    return launch_mfma_f32_down(h, tiles, capacity, w_down, sorted_w, n_rows, n_experts, dim_ffn, dim, y,
+    return launch_mfma_f32_down(h, tiles, capacity, w_down, sorted_w, {n_rows, n_experts}, dim_ffn, dim, y,
                                 y_unweighted, s);
   return launch_generic<float, false, true>(h, tiles, capacity, w_down, nullptr, sorted_w, dim_ffn, dim, y, s,
                                             y_unweighted);

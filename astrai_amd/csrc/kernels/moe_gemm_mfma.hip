@@ -1119,27 +1119,6 @@ int launch(const void* A, const int32_t* tiles, int64_t capacity, const void* co
   return check_launch(kGateUp ? "gemm_mfma_kernel<gate_up>" : "gemm_mfma_kernel<down>");
 }
 
-// Row tiles of `bm` rows that a load makes: expected under even routing (an
-// expert's rows about normal, with their mean as variance); under a skewed one
-// (the last tile of nearly every expert nearly empty: routers biased by Zipf
-// weights of exponents 0.4 to 4 over 8 to 128 experts gave rows / bm + 0.1 to 0.85
-// per expert); and the most that any routing makes, the list's capacity. The
-// same number where the host knows every expert's rows.
-struct RowTileCount {
-  double even, skewed, most;
-};
-RowTileCount count_row_tiles(const RowCounts& rows, int bm) {
-  const double exact = (double)rows.exact * (double)ceil_div(rows.exact_rows, bm);
-  if (rows.experts == 0) return {exact, exact, exact};
-  const double r = (double)rows.rows / rows.experts, sd = std::sqrt(std::max(r, 1.0));
-  double tiles = 0.0;
-  for (int64_t j = 0; j * bm < r + 8.0 * sd; ++j) tiles += 0.5 * std::erfc(((double)(j * bm) - r) / (sd * 1.41421356));
-  const int64_t most = std::min(rows.rows, (rows.rows + (int64_t)rows.experts * (bm - 1)) / bm);
-  const double even = std::min(rows.experts * tiles, (double)most);
-  const double skewed = std::min(std::max(even, (double)rows.rows / bm + 0.8 * rows.experts), (double)most);
-  return {exact + even, exact + skewed, exact + (double)most};
-}
-
 // Which tiles a GEMM takes on a list of 128- or 256-row tiles: the list's own
 // with 256 columns (gate/up: 128 of each), or, where those leave compute units
 // idle, 128 rows by 128 columns, and on a 256-row list also 128 by 256.

@@ -21,13 +21,12 @@
 // BN = 64 weight rows per column tile (gate/up: 32 gate rows then the same 32
 // up rows), 4 waves of 32 x 32, three 16 KB stages in flight, so a compute
 // unit holds three workgroups and a wave waiting at its barrier leaves the
-// matrix core to the other two. The down GEMM takes BN = 32, four workgroups
-// per compute unit (us with 64 / 32 columns at D 512, F 1024, 8 experts, top-2:
-// 64 tokens 21.6 / 14.2, 1024 37.8 / 31.7, 2048 56.5 / 51.1; D 1024, F 2048,
-// 2048 tokens 182 / 175), and the gate/up GEMM (16 gate rows and 16 up rows)
-// where 64-wide column tiles would leave most workgroup slots empty (D 512, 64
-// tokens with a shared expert 21.4 / 18.1; with more tiles than that it is the
-// slower one, 2048 tokens 130 / 136). Bound by the matrix cores: busy for 79 %
+// matrix core to the other two. BN = 32, four workgroups per compute unit, for
+// the down GEMM where its rounds come out better (narrow_down) and for the
+// gate/up GEMM (16 gate rows and 16 up rows) where 64-wide column tiles would
+// leave most workgroup slots empty (D 512, 64 tokens with a shared expert 21.4 /
+// 18.1 us; with more tiles than that it is the slower one, 2048 tokens 130 /
+// 136). Bound by the matrix cores: busy for 79 %
 // of 2.15 GHz at D 1024, F 2048, 2048 tokens (107 of 157 TFLOP/s). The launch is
 // persistent, round r of workgroup b taking logical tile r * G + b: with
 // several workgroups per compute unit, the XCD-contiguous order of the bf16
@@ -274,28 +273,46 @@ int launch_f32_bn(const void* A, const int32_t* tiles, int64_t capacity, const v
   return check_launch(kGateUp ? "gemm_f32_mfma_kernel<gate_up>" : "gemm_f32_mfma_kernel<down>");
 }
 
-template <bool kGateUp, bool kSave>
-int launch_f32(const void* A, const int32_t* tiles, int64_t capacity, const void* const* W0, const void* const* W1,
-               const void* row_w, int64_t n_rows, int n_experts, int64_t K, int64_t N, void* C, void* S0,
-               hipStream_t s, const int32_t* row_src = nullptr) {
+// 32 weight rows (16 gate, 16 up) when 64-row tiles, estimated from the rows and
+// the experts' partial last tiles, would not give every compute unit two.
+bool narrow_gate_up(const RowCounts& rows, int64_t n) {
+  const int64_t row_tiles = ceil_div(rows.total(), kF32BM) + (rows.experts + rows.exact) / 2;
+  return row_tiles * (n / 32) < 2ll * cu_count();
+}
+
+// 32 weight rows for the down GEMM where they end sooner. A compute unit takes
+// some 6 us and then, at K 1024, 16.2 for each of its tiles of 64 columns and 8.75
+// for each of 32: narrow tiles pay 8 % more per flop and gain where its share of
+// the tiles rounds up by half a tile and not by a whole one. Measured, us with 64 / 32 columns, 8 experts, top-2: D
+// 512, F 1024 64 tokens 21.2 / 13.8, 1024 37.3 / 30.8, 4096 83.7 / 78.3, 8192 146.4
+// / 146.1; D 2048, F 4096 1024 tokens 321 / 305, 2048 577 / 592, 8192 2118 / 2260;
+// D 4096, F 4096 128 tokens 149 / 152, 8192 4265 / 4601.
+bool narrow_down(const RowCounts& rows, int64_t n) {
+  if (n % 64 != 0) return true;
+  const double cu = cu_count(), cols = (double)(n / 64);
+  constexpr double kMost = 7.0;  // tiles per compute unit from which the rule never gives the narrow ones
+  if ((double)rows.total() / kF32BM * cols > kMost * cu) return false;
+  const double share = count_row_tiles(rows, kF32BM).even * cols / cu;
+  return 8.75 * std::ceil(2.0 * share) < 16.2 * std::ceil(share);
+}
+
+template <bool kSave, bool kGather>
+int launch_f32_gate_up(const void* x, const int32_t* tiles, int64_t capacity, const void* const* W0,
+                       const void* const* W1, const RowCounts& rows, int64_t K, int64_t N, void* C, void* S0,
+                       hipStream_t s, const int32_t* row_src) {
   if (capacity == 0) return ASTRAI_MOE_OK;
-  if constexpr (!kGateUp) {
-    (void)n_rows, (void)n_experts, (void)row_src;
-    return launch_f32_bn<32, false, kSave>(A, tiles, capacity, W0, W1, row_w, K, N, C, S0, s);
-  } else {
-    // 32 weight rows (16 gate, 16 up) when 64-row tiles, estimated from the
-    // rows and the experts' partial last tiles, would not give every compute
-    // unit two
-    const int64_t row_tiles = ceil_div(n_rows, kF32BM) + n_experts / 2;
-    const bool narrow = row_tiles * (N / 32) < 2ll * cu_count();
-    if (row_src != nullptr) {
-      if constexpr (!kSave)
-        return narrow ? launch_f32_bn<32, true, false, true>(A, tiles, capacity, W0, W1, row_w, K, N, C, S0, s, row_src)
-                      : launch_f32_bn<64, true, false, true>(A, tiles, capacity, W0, W1, row_w, K, N, C, S0, s, row_src);
-    }
-    if (narrow) return launch_f32_bn<32, true, kSave>(A, tiles, capacity, W0, W1, row_w, K, N, C, S0, s);
-    return launch_f32_bn<64, true, kSave>(A, tiles, capacity, W0, W1, row_w, K, N, C, S0, s);
-  }
+  if (narrow_gate_up(rows, N))
+    return launch_f32_bn<32, true, kSave, kGather>(x, tiles, capacity, W0, W1, nullptr, K, N, C, S0, s, row_src);
+  return launch_f32_bn<64, true, kSave, kGather>(x, tiles, capacity, W0, W1, nullptr, K, N, C, S0, s, row_src);
+}
+
+template <bool kSave>
+int launch_f32_down(const void* h, const int32_t* tiles, int64_t capacity, const void* const* W, const void* row_w,
+                    const RowCounts& rows, int64_t K, int64_t N, void* C, void* S0, hipStream_t s) {
+  if (capacity == 0) return ASTRAI_MOE_OK;
+  if (narrow_down(rows, N))
+    return launch_f32_bn<32, false, kSave>(h, tiles, capacity, W, nullptr, row_w, K, N, C, S0, s);
+  return launch_f32_bn<64, false, kSave>(h, tiles, capacity, W, nullptr, row_w, K, N, C, S0, s);
 }
 
 }  // namespace
@@ -308,23 +325,23 @@ bool mfma_f32_supported(int64_t k, int64_t n, bool gate_up, int block_m, const v
 }
 
 int launch_mfma_f32_gate_up(const void* x_perm, const int32_t* tiles, int64_t capacity, const void* const* w_gate,
-                            const void* const* w_up, int64_t n_rows, int n_experts, int64_t dim, int64_t dim_ffn,
-                            void* h, void* gu, hipStream_t s, const int32_t* row_src) {
+                            const void* const* w_up, const RowCounts& rows, int64_t dim, int64_t dim_ffn, void* h,
+                            void* gu, hipStream_t s, const int32_t* row_src) {
   if (gu != nullptr)
-    return launch_f32<true, true>(x_perm, tiles, capacity, w_gate, w_up, nullptr, n_rows, n_experts, dim, dim_ffn,
-                                  h, gu, s);
-  return launch_f32<true, false>(x_perm, tiles, capacity, w_gate, w_up, nullptr, n_rows, n_experts, dim, dim_ffn, h,
-                                 nullptr, s, row_src);
+    return launch_f32_gate_up<true, false>(x_perm, tiles, capacity, w_gate, w_up, rows, dim, dim_ffn, h, gu, s, nullptr);
+  if (row_src != nullptr)
+    return launch_f32_gate_up<false, true>(x_perm, tiles, capacity, w_gate, w_up, rows, dim, dim_ffn, h, nullptr, s,
+                                           row_src);
+  return launch_f32_gate_up<false, false>(x_perm, tiles, capacity, w_gate, w_up, rows, dim, dim_ffn, h, nullptr, s,
+                                          nullptr);
 }
 
 int launch_mfma_f32_down(const void* h, const int32_t* tiles, int64_t capacity, const void* const* w_down,
-                         const void* sorted_w, int64_t n_rows, int n_experts, int64_t dim_ffn, int64_t dim, void* y,
+                         const void* sorted_w, const RowCounts& rows, int64_t dim_ffn, int64_t dim, void* y,
                          void* y_unweighted, hipStream_t s) {
   if (y_unweighted != nullptr)
-    return launch_f32<false, true>(h, tiles, capacity, w_down, nullptr, sorted_w, n_rows, n_experts, dim_ffn, dim, y,
-                                   y_unweighted, s);
-  return launch_f32<false, false>(h, tiles, capacity, w_down, nullptr, sorted_w, n_rows, n_experts, dim_ffn, dim, y,
-                                  nullptr, s);
+    return launch_f32_down<true>(h, tiles, capacity, w_down, sorted_w, rows, dim_ffn, dim, y, y_unweighted, s);
+  return launch_f32_down<false>(h, tiles, capacity, w_down, sorted_w, rows, dim_ffn, dim, y, nullptr, s);
 }
 
 }  // namespace astrai_moe

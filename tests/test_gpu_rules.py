@@ -9,6 +9,7 @@ from torch.profiler import ProfilerActivity, profile
 
 from astrai_amd.extension import ops
 from test_gpu_backward import _random_layer
+from test_gpu_layer import check_layer
 
 pytestmark = pytest.mark.gpu
 
@@ -85,3 +86,17 @@ def test_few_rows_of_a_packed_layer_read_the_live_weights(gpu):
     first, second = _gemms(lambda: layer(x))[:2]
     # gemm_few_kernel<..., gate/up, gather, packed, dense>
     assert "true, true, false, false>" in first and "false, false, false, false>" in second, (first, second)
+
+
+@pytest.mark.parametrize("n_tok,dim,n_shared,cols", [
+    (1024, 512, 0, 32),  # 36 row tiles x 8: a compute unit's share is 1.1 of 64 columns, 2.3 of 32
+    (128, 4096, 0, 64),  # 8 x 64: 2 or 4
+    (2048, 2048, 1, 64),  # past the shares that can gain
+    (1500, 96, 1, 32),  # columns no multiple of 64
+])
+def test_fp32_down_columns(gpu, n_tok, dim, n_shared, cols):
+    layer = _random_layer(gpu, dim, 160, 8, n_shared, 2, torch.float32, seed=1).requires_grad_(False)
+    x = torch.randn(1, n_tok, dim, device=gpu)
+    first, second = _gemms(lambda: layer(x))[:2]
+    assert f"gemm_f32_mfma_kernel<{cols}, false" in second, second
+    check_layer(layer, x, f"d{dim}_t{n_tok}_s{n_shared}")
