@@ -89,11 +89,9 @@ Plan make_plan(const Sizes& z) {
   p.sorted_w = part(p.rows * size);
   p.token_pos = part(p.rows * 4);
   p.tiles = part(p.tiles_len * 4);
-  // (such an x, or an fp32 one, off the 16-byte grid is copied after all: it
-  // needs the place)
-  p.x_perm = p.gather ? 0 : part(p.rows * z.dim * size);
   p.h = part(p.rows * z.dim_ffn * size);
   p.y = part(p.rows * z.dim * size);
+  p.x_perm = p.y;  // copied rows are read by the gate/up GEMM, before the down GEMM writes y
   // the 256-row GEMMs' scheduling block, and partial sums where the down
   // GEMM's tiles are long enough to be split
   if (p.block_m == kMfmaBigBM) p.gemm_ws_bytes = gemm_workspace_bytes(splits_tail(z.dim_ffn));

@@ -34,6 +34,14 @@ def test_shared_experts_of_another_width(gpu):
     check_layer(layer, x, "narrow shared expert")
 
 
+def test_copied_rows_need_no_place_of_their_own():
+    # fp32 and ragged layers (whose unaligned x is copied), packed ones: h, y and some lists
+    size = loader.library().astrai_moe_forward_workspace_bytes
+    for dim, dim_ffn, dtype, packed in ((512, 1024, 0, 0), (1000, 2664, 1, 0), (512, 1024, 1, 1)):
+        rows, item = 4096 * 3, 4 if dtype == 0 else 2
+        assert size(4096, 8, 2, 1, dim, dim_ffn, dtype, packed) < rows * ((dim + dim_ffn) * item + 100) + (1 << 20)
+
+
 def test_arguments_are_checked_on_the_host():
     lib = loader.library()
     size = lib.astrai_moe_forward_workspace_bytes
