@@ -316,8 +316,8 @@ class DeepSeekMoE(nn.Module):
         dim_ffn = st.routed[1][0].shape[0]
         packed_tables = self._packed_tables(x.dtype, st)
         packed = packed_tables is not None
-        if packed:
-            tg, td = packed_tables
+        if packed:  # (the routed experts' copies, those of the shared ones come behind)
+            tg, td = (ops.weight_table_slice(t, 0, len(st.routed[0])) for t in packed_tables)
             tu = tg
         else:
             tg, tu, td = st.tables[0]

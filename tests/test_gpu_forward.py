@@ -42,6 +42,21 @@ def test_copied_rows_need_no_place_of_their_own():
         assert size(4096, 8, 2, 1, dim, dim_ffn, dtype, packed) < rows * ((dim + dim_ffn) * item + 100) + (1 << 20)
 
 
+@pytest.mark.gpu
+def test_separate_calls_of_a_packed_layer_with_shared_experts(gpu):
+    # the packed tables hold the shared experts' copies too; the separate calls take the routed ones
+    layer = _random_layer(gpu, 256, 512, 4, 2, 2, torch.bfloat16, seed=5).requires_grad_(False)
+    x = torch.randn(1, 300, 256, device=gpu).to(torch.bfloat16)
+    st = layer._current(x.dtype, x.device)
+
+    def apart():
+        return layer._routed_forward(x[0], st, layer._shared_forward(x[0], st))
+
+    live = apart()
+    layer.pack_weights = True
+    assert torch.equal(apart(), live)
+
+
 def test_arguments_are_checked_on_the_host():
     lib = loader.library()
     size = lib.astrai_moe_forward_workspace_bytes
