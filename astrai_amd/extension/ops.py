@@ -533,6 +533,24 @@ def layer_forward_supported(n_experts: int, n_shared: int, top_k: int) -> bool:
     return n_experts + n_shared <= MAX_EXPERTS and top_k + n_shared <= MAX_TOPK
 
 
+# Most bytes of h that the shared experts' rows may add to a forward in one
+# call. Run by themselves they give that memory back before the routed experts
+# take theirs; joined, they hold it next to it, for a gain that shrinks as the
+# GEMMs grow: D 4096, F 14336, 8 experts, top-2 and a shared one, 512 tokens (15
+# MB) 981 -> 797 us a layer, 2048 (59 MB) 1905 -> 1814, 4096 (117 MB) 3233 -> 3217,
+# 16384 (470 MB) 11602 -> 11552; with four shared experts 1024 tokens (117 MB)
+# 2761 -> 2007, 4096 (470 MB) 6136 -> 6040.
+SHARED_ROWS_BYTES = 128 << 20
+
+
+def layer_forward_pays(n_tokens: int, n_shared: int, top_k: int, dim_ffn: int, itemsize: int) -> bool:
+    """Whether this many tokens go through ``moe_layer_forward`` with their
+    shared experts (``SHARED_ROWS_BYTES``; the joint permutation's rows are
+    counted in 31 bits)."""
+    return (n_tokens * n_shared * dim_ffn * itemsize <= SHARED_ROWS_BYTES
+            and n_tokens * (top_k + n_shared) < 1 << 31)
+
+
 def moe_layer_forward(x: torch.Tensor, logits: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor,
                       w_down: torch.Tensor, n_shared: int, dim_ffn: int, top_k: int,
                       packed: tuple[torch.Tensor, torch.Tensor] | None = None) -> torch.Tensor:

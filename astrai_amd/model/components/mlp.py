@@ -289,10 +289,12 @@ class DeepSeekMoE(nn.Module):
         if torch.is_grad_enabled() and (x_flat.requires_grad or router_w.requires_grad
                                         or any(map(_requires_grad, st.flat))):
             return self._forward_autograd(x_flat, st).view(bsz, seq_len, dim)
-        if x_flat.shape[0] and self._joint(st):
+        n_tokens, dim_ffn = x_flat.shape[0], st.routed[1][0].shape[0]
+        if n_tokens and self._joint(st) and ops.layer_forward_pays(
+                n_tokens, len(st.shared[0]), self.n_activated_experts, dim_ffn, x_flat.element_size()):
             packed = self._packed_tables(x_flat.dtype, st) if self.pack_weights else None
-            out = ops.moe_layer_forward(x_flat, self.router(x_flat), *st.joint, len(st.shared[0]),
-                                        st.routed[1][0].shape[0], self.n_activated_experts, packed)
+            out = ops.moe_layer_forward(x_flat, self.router(x_flat), *st.joint, len(st.shared[0]), dim_ffn,
+                                        self.n_activated_experts, packed)
         else:
             out = self._routed_forward(x_flat, st, self._shared_forward(x_flat, st))
         return out.view(bsz, seq_len, dim)

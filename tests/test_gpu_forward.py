@@ -57,6 +57,41 @@ def test_separate_calls_of_a_packed_layer_with_shared_experts(gpu):
     assert torch.equal(apart(), live)
 
 
+def _peak(run):
+    run()  # allocations that stay
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    run()
+    return torch.cuda.max_memory_allocated() - before
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("pack", [False, True])
+@pytest.mark.parametrize("n_tok,joint", [(4096, True), (20000, False)])
+def test_shared_experts_memory_is_bounded(gpu, n_tok, joint, pack):
+    # two shared experts of F 2048: 32 MB of h at 4096 tokens, 156 at 20000, past
+    # the line where they run by themselves before the routed experts
+    layer = _random_layer(gpu, 256, 2048, 4, 2, 1, torch.bfloat16, seed=5).requires_grad_(False)
+    layer.pack_weights = pack
+    x = torch.randn(1, n_tok, 256, device=gpu).to(torch.bfloat16)
+    assert ops.layer_forward_pays(n_tok, 2, 1, 2048, 2) == joint
+    st = layer._current(x.dtype, x.device)
+
+    def apart():
+        return layer._routed_forward(x[0], st, layer._shared_forward(x[0], st))
+
+    extra = _peak(lambda: layer(x)) - _peak(apart)
+    assert extra <= (ops.SHARED_ROWS_BYTES if joint else 1 << 20), extra
+    assert torch.allclose(layer(x)[0].float(), apart().float(), rtol=2e-2, atol=2e-2)
+    check_layer(layer, x[:, :256], "first tokens")
+
+
+def test_one_call_takes_the_rows_that_fit_31_bits():
+    assert ops.layer_forward_pays((1 << 31) // 3 - 1, 1, 2, 0, 2) and not ops.layer_forward_pays((1 << 31) // 3 + 1, 1, 2, 0, 2)
+
+
 def test_arguments_are_checked_on_the_host():
     lib = loader.library()
     size = lib.astrai_moe_forward_workspace_bytes
