@@ -135,6 +135,9 @@ class RouteWeights(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dw, *_):
         logits, topk_idx = ctx.saved_tensors
+        if torch.is_grad_enabled():  # create_graph: the operators, whose gradient has one of its own
+            w = routing_weights(logits, topk_idx, logits.dtype)
+            return torch.autograd.grad(w, logits, dw, create_graph=True)[0], None
         return ops.moe_route_grad(logits, topk_idx, dw.contiguous()), None
 
 
@@ -183,7 +186,8 @@ def routing_weights(logits: Tensor, topk_idx: Tensor, dtype: torch.dtype) -> Ten
     """The renormalised top-k weights as differentiable torch ops
     (mlp.py:84-87) in ``dtype``, evaluated at the route kernel's indices, with
     autograd's path back to the logits: for logits of another dtype than the
-    activations (autocast), where ``RouteWeights``' weights would have theirs."""
+    activations (autocast), where ``RouteWeights``' weights would have theirs,
+    and for derivatives of its gradient."""
     probs = torch.softmax(logits.float(), dim=-1).to(dtype)
     w = probs.gather(1, topk_idx.long())
     return w / w.sum(dim=-1, keepdim=True)

@@ -8,6 +8,7 @@ import pytest
 import torch
 
 from astrai_amd.extension import loader, ops
+from astrai_amd.model.components.autograd import RouteWeights, routing_weights
 from test_gpu_backward import _random_layer
 
 
@@ -42,6 +43,37 @@ def test_layer_under_autocast_still_trains(gpu):
     out.sum().backward()
     assert out.dtype == torch.float32 and torch.isfinite(x.grad).all()
     assert layer.router.weight.grad is not None and torch.isfinite(layer.router.weight.grad).all()
+
+
+def _route_on_cpu(logits, top_k):
+    probs = torch.softmax(logits.float(), -1).to(logits.dtype)
+    w, idx = probs.topk(top_k, -1)
+    return ops.RouteResult(idx.int(), w / w.sum(-1, keepdim=True), torch.zeros(1, logits.shape[1], dtype=torch.int32))
+
+
+def test_second_derivatives_reach_the_logits(monkeypatch):
+    # create_graph: the logits' gradient is itself differentiable, as torch's operators make it
+    monkeypatch.setattr(ops, "moe_route", _route_on_cpu)
+    logits = torch.randn(5, 6, generator=torch.Generator().manual_seed(1), dtype=torch.float32).requires_grad_(True)
+    c = torch.randn(5, 2, generator=torch.Generator().manual_seed(2))
+
+    def second(weights):
+        (g,) = torch.autograd.grad((weights * c).sum(), logits, create_graph=True)
+        return g, torch.autograd.grad(g.square().sum(), logits)[0]
+
+    topk_w, topk_idx, _ = RouteWeights.apply(logits, 2)
+    got = second(topk_w)
+    want = second(routing_weights(logits, topk_idx, logits.dtype))
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.gpu
+def test_gradient_penalty_reaches_the_router(gpu):
+    layer = _random_layer(gpu, 64, 96, 4, 0, 2, torch.float32, seed=1)
+    x = torch.randn(1, 40, 64, device=gpu)
+    (g,) = torch.autograd.grad(layer(x).square().sum(), layer.router.weight, create_graph=True)
+    g.square().sum().backward()
+    assert torch.isfinite(layer.router.weight.grad).all() and layer.router.weight.grad.abs().max() > 0
 
 
 def test_arguments_are_checked_on_the_host():
