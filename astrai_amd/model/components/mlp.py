@@ -274,8 +274,9 @@ class DeepSeekMoE(nn.Module):
     def _joint(self, st: _ExpertState) -> bool:
         """Whether routed and shared experts run in one forward call
         (``ops.moe_layer_forward``)."""
-        return st.joint is not None and ops.layer_forward_supported(len(st.routed[0]), len(st.shared[0]),
-                                                                    self.n_activated_experts)
+        n_shared = len(st.shared[0])
+        return (st.joint is not None and n_shared == self.n_shared_experts
+                and ops.layer_forward_supported(len(st.routed[0]), n_shared, self.n_activated_experts))
 
     # -- forward ----------------------------------------------------------------
     def forward(self, x: Tensor) -> Tensor:

@@ -34,6 +34,20 @@ def test_shared_experts_of_another_width(gpu):
     check_layer(layer, x, "narrow shared expert")
 
 
+@pytest.mark.gpu
+def test_shared_experts_switched_off(gpu):
+    # n_shared_experts decides, as in training and in the reference (mlp.py:75-76), not the modules there are
+    layer = _random_layer(gpu, 128, 192, 4, 1, 2, torch.bfloat16, seed=7).requires_grad_(False)
+    x = torch.randn(1, 50, 128, device=gpu).to(torch.bfloat16)
+    with_shared = layer(x)
+    layer.n_shared_experts = 0
+    out = layer(x)
+    assert not torch.equal(out, with_shared)
+    assert torch.equal(out[0], layer._routed_forward(x[0], layer._current(x.dtype, x.device)))
+    layer.n_shared_experts = 1
+    assert torch.equal(layer(x), with_shared)
+
+
 def test_copied_rows_need_no_place_of_their_own():
     # fp32 and ragged layers (whose unaligned x is copied), packed ones: h, y and some lists
     size = loader.library().astrai_moe_forward_workspace_bytes
