@@ -601,6 +601,15 @@ def train_block_m(dim: int, dim_ffn: int, dtype: torch.dtype) -> int:
     return TRAIN_BLOCK_M if backward_on_matrix_cores(dim, dim_ffn, dtype) else 64
 
 
+def _train_height(tiles: torch.Tensor, dim: int, dim_ffn: int, dtype: torch.dtype) -> int:
+    """The height at which a training GEMM walks ``tiles``: ``train_block_m``'s,
+    or 64 where the list was built so and the general kernels take it (dims that
+    are no multiples of 64)."""
+    if getattr(tiles, "_astrai_block_m", None) == 64 and (dim % 64 != 0 or dim_ffn % 64 != 0):
+        return 64
+    return train_block_m(dim, dim_ffn, dtype)
+
+
 def _lib_call(name: str, *args) -> None:
     _check(getattr(loader.library(), name)(*args), name)
 
@@ -613,7 +622,7 @@ def moe_gemm_gate_up_train(x_perm: torch.Tensor, tiles: torch.Tensor, w_gate: to
     _require_gpu(x_perm, "x_perm", 2)
     code = _dtype_code(x_perm, "x_perm")
     n_rows, dim = x_perm.shape
-    bm = train_block_m(dim, dim_ffn, x_perm.dtype)
+    bm = _train_height(tiles, dim, dim_ffn, x_perm.dtype)
     _check_tiles(tiles, bm, x_perm, "moe_gemm_gate_up_train")
     _require_table(w_gate, "w_gate", n_experts, x_perm)
     _require_table(w_up, "w_up", n_experts, x_perm)
@@ -650,7 +659,7 @@ def moe_gemm_down_train(h: torch.Tensor, tiles: torch.Tensor, w_down: torch.Tens
     n_rows, dim_ffn = h.shape
     if sorted_w.numel() != n_rows or sorted_w.dtype != h.dtype:
         raise ValueError("sorted_w must hold one weight of h's dtype per row")
-    bm = train_block_m(dim, dim_ffn, h.dtype)
+    bm = _train_height(tiles, dim, dim_ffn, h.dtype)
     _check_tiles(tiles, bm, h, "moe_gemm_down_train")
     _require_table(w_down, "w_down", n_experts, h)
     y, y_unw = (torch.empty(n_rows, dim, dtype=h.dtype, device=h.device) for _ in range(2))
@@ -703,7 +712,7 @@ def moe_gemm_dgrad_down(dy: torch.Tensor, tiles: torch.Tensor, w_down: torch.Ten
     code = _dtype_code(dy, "dy")
     n_rows, dim = dy.shape
     dim_ffn = gu.shape[1] // 2
-    bm = train_block_m(dim, dim_ffn, dy.dtype)
+    bm = _train_height(tiles, dim, dim_ffn, dy.dtype)
     _check_tiles(tiles, bm, dy, "moe_gemm_dgrad_down")
     _require_table(w_down, "w_down", n_experts, dy)
     dg, du = (torch.empty(n_rows, dim_ffn, dtype=dy.dtype, device=dy.device) for _ in range(2))
@@ -721,7 +730,7 @@ def moe_gemm_dgrad_gate_up(dg: torch.Tensor, du: torch.Tensor, tiles: torch.Tens
     _require_gpu(dg, "dg", 2)
     code = _dtype_code(dg, "dg")
     n_rows, dim_ffn = dg.shape
-    bm = train_block_m(dim, dim_ffn, dg.dtype)
+    bm = _train_height(tiles, dim, dim_ffn, dg.dtype)
     _check_tiles(tiles, bm, dg, "moe_gemm_dgrad_gate_up")
     _require_table(w_gate, "w_gate", n_experts, dg)
     _require_table(w_up, "w_up", n_experts, dg)

@@ -55,6 +55,29 @@ def test_unaligned_rows_still_run(gpu):
     check_layer(layer, x, "unaligned")
 
 
+def test_training_on_a_64_row_list(gpu):
+    # the general kernels' lists, which such dims trained on before the matrix cores took them
+    dim, dim_ffn, e = 72, 120, 4
+    x = torch.randn(130, dim, device=gpu).to(torch.bfloat16)
+    route = ops.moe_route(torch.randn(130, e, device=gpu).to(torch.bfloat16), 2)
+    ws = [[(torch.randn(*s, device=gpu) * 0.1).bfloat16() for _ in range(e)]
+          for s in ((dim_ffn, dim), (dim_ffn, dim), (dim, dim_ffn))]
+    tg, tu, td = (ops.expert_weight_table(w, tuple(w[0].shape)) for w in ws)
+
+    def step(block_m):
+        perm = ops.moe_permute(route, x, e, block_m)
+        h, gu = ops.moe_gemm_gate_up_train(perm.x_perm, perm.tiles, tg, tu, e, dim_ffn)
+        y, y_unw = ops.moe_gemm_down_train(h, perm.tiles, td, perm.sorted_w, e, dim)
+        dg, du = ops.moe_gemm_dgrad_down(y, perm.tiles, td, gu, e)
+        return h, gu, y, y_unw, dg, du, ops.moe_gemm_dgrad_gate_up(dg, du, perm.tiles, tg, tu, e, dim)
+
+    for got, want in zip(step(64), step(256)):
+        # values rounded to bf16 at the same points, up to three in a chain; fp32 sums in another order
+        torch.testing.assert_close(got, want, rtol=3e-2, atol=3e-2 * want.abs().max().item())
+    with pytest.raises(ValueError, match="block_m"):
+        step(128)
+
+
 @pytest.mark.parametrize("dim,dim_ffn", [(72, 328), (1000, 424), (2056, 136)])
 @pytest.mark.parametrize("n_tok", [1, 32, 33, 300, 1400])
 def test_gathered_rows_are_the_copied_ones(gpu, n_tok, dim, dim_ffn):
