@@ -151,8 +151,7 @@ extern "C" int astrai_moe_forward(const void* x, const void* logits, const void*
   // tokens its many workgroups.)
   if (n_tokens <= ASTRAI_MOE_CHUNK_TOKENS && x_perm == nullptr) {
     const RouteList list{sorted_token, sorted_w, token_pos, tiles,
-                         (p.tiles_len - ASTRAI_MOE_TILE_HEADER) / ASTRAI_MOE_TILE_STRIDE, p.block_m,
-                         dim >= kGroupTilesMinDim};
+                         (p.tiles_len - ASTRAI_MOE_TILE_HEADER) / ASTRAI_MOE_TILE_STRIDE, p.block_m};
     rc = launch_route_list(logits, dtype, n_tokens, n_experts, top_k, n_shared, list, s);
   } else if ((rc = launch_route(logits, dtype, n_tokens, n_experts, top_k, n_shared, topk_idx, topk_w, hist, s)) == 0) {
     rc = astrai_moe_permute(topk_idx, topk_w, hist, x, dtype, n_tokens, p.experts, p.slots, dim, p.block_m,

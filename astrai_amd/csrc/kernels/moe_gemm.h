@@ -277,8 +277,8 @@ int launch_route(const void* logits, int dtype, int64_t n_tokens,
                  void* topk_w, int32_t* chunk_hist, hipStream_t s);
 
 // The same for at most ASTRAI_MOE_CHUNK_TOKENS tokens, straight to what
-// astrai_moe_permute writes of the decisions (tiles of block_m >= 32 rows, the
-// grouped order's header where `group`); neither x_perm nor expert offsets.
+// astrai_moe_permute writes of the decisions (tiles of block_m >= 32 rows, so one
+// for every expert that has any); neither x_perm nor expert offsets.
 struct RouteList {
   int32_t* sorted_token;
   void* sorted_w;
@@ -286,7 +286,6 @@ struct RouteList {
   int32_t* tiles;
   int64_t tile_capacity;
   int block_m;
-  bool group;
 };
 int launch_route_list(const void* logits, int dtype, int64_t n_tokens,
                       int n_experts, int top_k, int n_shared,

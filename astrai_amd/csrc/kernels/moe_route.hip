@@ -113,7 +113,7 @@ __device__ void write_chunk_list(const uint32_t* mask, int* base, const int* s_e
     out.tiles[0] = n_tiles;
     out.tiles[1] = out.block_m;
     out.tiles[2] = (int32_t)out.tile_capacity;
-    out.tiles[3] = out.group ? 0 : n_tiles;  // no expert has a whole group of tiles
+    out.tiles[3] = 0;  // no expert has a whole group of tiles
   }
   __syncthreads();
   if (tid < n_tokens * slots) {
@@ -310,7 +310,7 @@ int launch_route_list(const void* logits, int dtype, int64_t n_tokens, int n_exp
                       const RouteList& list, hipStream_t s) {
   if (n_tokens > ASTRAI_MOE_CHUNK_TOKENS || n_experts + n_shared > ASTRAI_MOE_MAX_EXPERTS ||
       top_k + n_shared > ASTRAI_MOE_MAX_TOPK || list.block_m < ASTRAI_MOE_CHUNK_TOKENS)
-    return fail(ASTRAI_MOE_EINVAL, "route: more than one chunk of tokens, or too many experts or slots");
+    return fail(ASTRAI_MOE_EINVAL, "route: more than one chunk of tokens, too many experts or slots, or short tiles");
   if (dtype == ASTRAI_MOE_BF16)
     return dispatch_route<bf16_t>(logits, n_tokens, n_experts, top_k, n_shared, nullptr, nullptr, nullptr, &list, s);
   return dispatch_route<float>(logits, n_tokens, n_experts, top_k, n_shared, nullptr, nullptr, nullptr, &list, s);

@@ -139,3 +139,13 @@ def test_one_chunk_is_routed_and_listed_by_one_kernel(gpu, n_tok, n_exp, top_k, 
     st = layer._current(dtype, x.device)
     for _ in range(2):
         assert torch.equal(layer(x)[0], layer._routed_forward(x[0], st))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n_tok", [5, 32])
+def test_one_chunk_of_long_rows(gpu, n_tok):
+    # rows of 3072, whose permutation lists whole groups of tiles first: one chunk has none
+    layer = _random_layer(gpu, 3072, 64, 8, 0, 2, torch.bfloat16, seed=n_tok).requires_grad_(False)
+    x = torch.randn(1, n_tok, 3072, device=gpu).to(torch.bfloat16)
+    assert torch.equal(layer(x)[0], layer._routed_forward(x[0], layer._current(x.dtype, x.device)))
+    check_layer(layer, x, f"t{n_tok}")
