@@ -266,8 +266,8 @@ int launch_mfma_f32_dgrad_in(const void* d, const int32_t* tiles,
                              int64_t n, const void* add, void* dx,
                              hipStream_t s);
 int launch_mfma_f32_wgrad(const void* a, const void* b, const int32_t* offsets,
-                          int n_experts, int64_t m, int64_t n, void* dw,
-                          hipStream_t s);
+                          int64_t n_rows, int n_experts, int64_t m, int64_t n,
+                          void* dw, hipStream_t s);
 
 // Routing with n_shared always-chosen experts behind the n_experts routed ones
 // (moe_route.hip): topk_idx, topk_w [n_tokens, top_k + n_shared], chunk_hist

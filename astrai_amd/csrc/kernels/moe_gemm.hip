@@ -539,6 +539,6 @@ extern "C" int astrai_moe_gemm_wgrad(const void* a, const void* b, const int32_t
       aligned16_ptr(dw))
     return launch_wgrad(a, b, expert_offsets, n_experts, m, n, dw, s);
   if (dtype == ASTRAI_MOE_F32 && mfma_f32_wgrad_supported(m, n, a, b, dw))
-    return launch_mfma_f32_wgrad(a, b, expert_offsets, n_experts, m, n, dw, s);
+    return launch_mfma_f32_wgrad(a, b, expert_offsets, n_rows, n_experts, m, n, dw, s);
   return launch_generic_wgrad(dtype, a, b, expert_offsets, n_experts, m, n, dw, s);
 }

@@ -30,6 +30,7 @@
 // second operand's lane l % 16. Over q = 0..3 a lane thus holds four
 // consecutive columns per r: one 16-byte store each.
 #include <climits>
+#include <cmath>
 
 #include "mfma_tile.h"
 
@@ -213,33 +214,37 @@ __global__ __launch_bounds__(256) void gemm_f32_dgrad_kernel(const float* __rest
 }
 
 // ---------------------------------------------------------------------------
-// wgrad: dw[e] [M, N] = a[rows_e]^T . b[rows_e] for every expert with rows,
-// 64 x 64 tiles, 4 waves of 32 x 32, K = the expert's rows in steps of 32 (rows
-// past the expert's last read zeros); three 16 KB stages, three workgroups per
-// CU, persistent over (expert, M tile, N tile).
+// wgrad: dw[e] [M, N] = a[rows_e]^T . b[rows_e] for every expert with rows, 4
+// waves of WT x WT, K = the expert's rows in steps of 32 (rows past the expert's
+// last read zeros), persistent over (expert, M tile, N tile). WT = 32: 64 x 64
+// tiles, three 16 KB stages, three workgroups per CU; WT = 64: 128 x 128 tiles,
+// three 32 KB stages, one.
 //
-// Operand reads: for MFMA step s of a 16-K half, lane (g = l / 16, c = l % 16)
-// reads K-row 4 g + s, columns 2 c and 2 c + 1 of its wave's 32 (8 bytes; a
-// 16-lane group covers 128 contiguous bytes). Value q feeds the MFMAs of block
-// q, whose local column c is column 2 c + q. Output (b as the first operand):
-// element r of blocks (qa, qb) is row 2 c + qa, column 2 (4 g + r) + qb, so a
-// lane holds 8 consecutive columns per row.
+// Operand reads, Q = WT / 16: for MFMA step s of a 16-K half, lane (g = l / 16, c
+// = l % 16) reads K-row 4 g + s, columns Q c .. Q c + Q - 1 of its wave's WT (a
+// 16-lane group covers 4 WT contiguous bytes). Value q feeds the MFMAs of block
+// q, whose local column c is column Q c + q. Output (b as the first operand):
+// element r of blocks (qa, qb) is row Q c + qa, column Q (4 g + r) + qb, so a lane
+// holds 4 Q consecutive columns per row. The same sums in the same order for both.
 //
-// Bound by the matrix cores once enough tiles are in flight: 128 x 128 tiles
-// with one 4-wave workgroup per CU left them waiting on every barrier, and gave
-// one shared expert of D 512, F 1024 32 workgroups. 1024 tokens over 8 experts
-// of that size, top-2: 74 -> 28 us a GEMM, the shared expert's 29 -> 23.
+// Bound by the matrix cores once enough tiles are in flight. The large tiles do
+// twice the flops per byte, but their one workgroup per CU waits on every barrier
+// (wide_wgrad has the line): 1024 tokens over 8 experts of D 512, F 1024, top-2,
+// large to small 74 -> 28 us a GEMM, one shared expert's (32 large tiles) 29 -> 23.
 // ---------------------------------------------------------------------------
+template <int WT>
 __global__ __launch_bounds__(256) void gemm_f32_wgrad_kernel(const float* __restrict__ a,
                                                             const float* __restrict__ b,
                                                             const int32_t* __restrict__ offsets, int n_experts,
                                                             int M, int N, int n_tiles_m, int n_tiles_n,
                                                             float* __restrict__ dw) {
-  typedef float f32x2_t __attribute__((ext_vector_type(2)));
-  constexpr int OP_BYTES = kF32K * 256;  // 32 K-rows x 64 columns, per operand
+  constexpr int Q = WT / 16, TILE = 2 * WT, ROW = TILE * 4;  // ROW: bytes of a staged K-row
+  typedef float vq_t __attribute__((ext_vector_type(Q)));
+  constexpr int OP_BYTES = kF32K * ROW;  // per operand
+  constexpr int OPS = OP_BYTES / 1024 / 4;  // DMA ops per operand and wave
   constexpr int STAGE = 2 * OP_BYTES;
   constexpr int S = kF32Stages;
-  constexpr int DPW = 4;  // 2 ops per operand and wave
+  constexpr int DPW = 2 * OPS;
   __shared__ __attribute__((aligned(1024))) char smem[S * STAGE];
 
   const int per_e = n_tiles_m * n_tiles_n;
@@ -251,8 +256,8 @@ __global__ __launch_bounds__(256) void gemm_f32_wgrad_kernel(const float* __rest
 
   const int c = lane & 15;
   const int g = lane >> 4;
-  f32x2_t fa[2][4], fb[2][4];
-  f32x4_t acc[2][2];
+  vq_t fa[2][4], fb[2][4];
+  f32x4_t acc[Q][Q];
 
   for (int logical = (int)blockIdx.x; logical < total; logical += (int)gridDim.x) {
     const int e = logical / per_e;
@@ -264,16 +269,16 @@ __global__ __launch_bounds__(256) void gemm_f32_wgrad_kernel(const float* __rest
     const int KT = (rows + kF32K - 1) / kF32K;
     const char* a_base = reinterpret_cast<const char*>(a + (int64_t)r0 * M);
     const char* b_base = reinterpret_cast<const char*>(b + (int64_t)r0 * N);
-    const uint32_t acol0 = (uint32_t)mt * 256u, bcol0 = (uint32_t)nt * 256u;
+    const uint32_t acol0 = (uint32_t)mt * ROW, bcol0 = (uint32_t)nt * ROW;
 
     auto issue_stage = [&](int kstep, int buf) {
       char* sa = smem + buf * STAGE;
       char* sb = sa + OP_BYTES;
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const int o = wave * 2 + i;
-        dma_mn_f32<64>(a_base, kstep * kF32K, rows, m4, acol0, m4, lane, o, sa + o * 1024);
-        dma_mn_f32<64>(b_base, kstep * kF32K, rows, n4, bcol0, n4, lane, o, sb + o * 1024);
+      for (int i = 0; i < OPS; ++i) {
+        const int o = wave * OPS + i;
+        dma_mn_f32<TILE>(a_base, kstep * kF32K, rows, m4, acol0, m4, lane, o, sa + o * 1024);
+        dma_mn_f32<TILE>(b_base, kstep * kF32K, rows, n4, bcol0, n4, lane, o, sb + o * 1024);
       }
     };
     auto read_frags = [&](int buf, int kh, int slot) {
@@ -282,17 +287,17 @@ __global__ __launch_bounds__(256) void gemm_f32_wgrad_kernel(const float* __rest
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
         const int krow = kh * 16 + 4 * g + s;
-        fa[slot][s] = *reinterpret_cast<const f32x2_t*>(sa + krow * 256 + wm * 128 + c * 8);
-        fb[slot][s] = *reinterpret_cast<const f32x2_t*>(sb + krow * 256 + wn * 128 + c * 8);
+        fa[slot][s] = *reinterpret_cast<const vq_t*>(sa + krow * ROW + wm * (ROW / 2) + c * (4 * Q));
+        fb[slot][s] = *reinterpret_cast<const vq_t*>(sb + krow * ROW + wn * (ROW / 2) + c * (4 * Q));
       }
     };
     auto mfmas = [&](int slot) {
 #pragma unroll
       for (int s = 0; s < 4; ++s)
 #pragma unroll
-        for (int qa = 0; qa < 2; ++qa)
+        for (int qa = 0; qa < Q; ++qa)
 #pragma unroll
-          for (int qb = 0; qb < 2; ++qb)
+          for (int qb = 0; qb < Q; ++qb)
             acc[qa][qb] =
                 __builtin_amdgcn_mfma_f32_16x16x4f32(fb[slot][s][qb], fa[slot][s][qa], acc[qa][qb], 0, 0, 0);
     };
@@ -301,9 +306,9 @@ __global__ __launch_bounds__(256) void gemm_f32_wgrad_kernel(const float* __rest
     for (int s = 0; s < S; ++s)
       if (s < KT) issue_stage(s, s);
 #pragma unroll
-    for (int qa = 0; qa < 2; ++qa)
+    for (int qa = 0; qa < Q; ++qa)
 #pragma unroll
-      for (int qb = 0; qb < 2; ++qb) acc[qa][qb] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+      for (int qb = 0; qb < Q; ++qb) acc[qa][qb] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
     wait_groups<DPW, S - 1>(min(S - 1, KT - 1));  // step 0 landed
     lds_barrier();
     read_frags(0, 0, 0);
@@ -327,18 +332,20 @@ __global__ __launch_bounds__(256) void gemm_f32_wgrad_kernel(const float* __rest
     mfmas(0);
     mfmas(1);
 
-    // ---- epilogue: rows 2 c + qa, columns 8 g .. + 7 of the wave's 32 x 32 ----
+    // ---- epilogue: rows Q c + qa, columns 4 Q g .. + 4 Q - 1 of the wave's WT x WT ----
 #pragma unroll
-    for (int qa = 0; qa < 2; ++qa) {
-      const int m = mt * 64 + wm * 32 + 2 * c + qa;
+    for (int qa = 0; qa < Q; ++qa) {
+      const int m = mt * TILE + wm * WT + Q * c + qa;
       if (m >= M) continue;
       float* out = dw + ((int64_t)e * M + m) * N;
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int n = nt * 64 + wn * 32 + 8 * g + 4 * h;
-        if (n < N)  // N % 4 == 0
-          *reinterpret_cast<f32x4_t*>(out + n) = f32x4_t{acc[qa][0][2 * h], acc[qa][1][2 * h], acc[qa][0][2 * h + 1],
-                                                         acc[qa][1][2 * h + 1]};
+      for (int h = 0; h < Q; ++h) {
+        const int n = nt * TILE + wn * WT + 4 * Q * g + 4 * h;
+        if (n >= N) continue;  // N % 4 == 0
+        f32x4_t v;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = acc[qa][(4 * h + i) % Q][(4 * h + i) / Q];
+        *reinterpret_cast<f32x4_t*>(out + n) = v;
       }
     }
     lds_barrier();  // every wave is done with the stage buffers before the next tile's DMA
@@ -358,6 +365,19 @@ int launch_f32_dgrad(const void* a, const int32_t* tiles, int64_t capacity, cons
                      static_cast<const float*>(a), tiles, w, static_cast<const float*>(e0), (int)k, (int)n,
                      (int)n_tiles_n, (int)capacity, static_cast<float*>(c0), static_cast<float*>(c1));
   return check_launch(name);
+}
+
+// Whether wgrad takes 128 x 128 tiles. With r rows per expert, a compute unit
+// takes 5 us and 0.0675 r for each of them, 1 us and 0.0724 r for four of 64 x 64
+// (after some 5 us either way): the large ones gain from about 1000 rows on where
+// they fill their rounds. Measured, us, 128 x 128 / 64 x 64: 8 experts, dW 2048 x
+// 1024, 256 rows each 94 / 82, 1024 299 / 301, 2048 576 / 593, 8192 2228 / 2354; one
+// expert, 4096 x 4096, 8192 rows 2222 / 2347; 2048 x 1024 (half a round) 555 / 332.
+bool wide_wgrad(int64_t n_rows, int n_experts, int64_t m, int64_t n) {
+  const double r = (double)n_rows / n_experts;
+  const double share = (double)(n_experts * ceil_div(m, 128) * ceil_div(n, 128)) / cu_count();
+  const double share64 = (double)(n_experts * ceil_div(m, 64) * ceil_div(n, 64)) / cu_count();
+  return std::ceil(share) * (5.0 + 0.0675 * r) < std::ceil(share64) / 4.0 * (1.0 + 0.0724 * r);
 }
 
 }  // namespace
@@ -389,16 +409,18 @@ int launch_mfma_f32_dgrad_in(const void* d, const int32_t* tiles, int64_t capaci
                                            "gemm_f32_dgrad_kernel<dgrad_in>");
 }
 
-int launch_mfma_f32_wgrad(const void* a, const void* b, const int32_t* offsets, int n_experts, int64_t m, int64_t n,
-                          void* dw, hipStream_t s) {
-  const int64_t n_tiles_m = ceil_div(m, 64), n_tiles_n = ceil_div(n, 64);
+int launch_mfma_f32_wgrad(const void* a, const void* b, const int32_t* offsets, int64_t n_rows, int n_experts,
+                          int64_t m, int64_t n, void* dw, hipStream_t s) {
+  const bool wide = wide_wgrad(n_rows, n_experts, m, n);
+  const int64_t tile = wide ? 128 : 64, n_tiles_m = ceil_div(m, tile), n_tiles_n = ceil_div(n, tile);
   const int64_t total = (int64_t)n_experts * n_tiles_m * n_tiles_n;
   if (total >= (1ll << 31))
     return fail(ASTRAI_MOE_EINVAL, "gemm_wgrad: %lld tiles exceed the tile-index range", (long long)total);
-  const int64_t grid = std::min<int64_t>(total, 3ll * cu_count());  // three 48 KB workgroups per CU
-  hipLaunchKernelGGL(gemm_f32_wgrad_kernel, dim3((unsigned)grid), dim3(256), 0, s, static_cast<const float*>(a),
-                     static_cast<const float*>(b), offsets, n_experts, (int)m, (int)n, (int)n_tiles_m,
-                     (int)n_tiles_n, static_cast<float*>(dw));
+  // one 96 KB workgroup per CU or three of 48 KB
+  const int64_t grid = std::min<int64_t>(total, (wide ? 1ll : 3ll) * cu_count());
+  hipLaunchKernelGGL(wide ? gemm_f32_wgrad_kernel<64> : gemm_f32_wgrad_kernel<32>, dim3((unsigned)grid), dim3(256), 0,
+                     s, static_cast<const float*>(a), static_cast<const float*>(b), offsets, n_experts, (int)m, (int)n,
+                     (int)n_tiles_m, (int)n_tiles_n, static_cast<float*>(dw));
   return check_launch("gemm_f32_wgrad_kernel");
 }
 

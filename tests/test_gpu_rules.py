@@ -100,3 +100,25 @@ def test_fp32_down_columns(gpu, n_tok, dim, n_shared, cols):
     first, second = _gemms(lambda: layer(x))[:2]
     assert f"gemm_f32_mfma_kernel<{cols}, false" in second, second
     check_layer(layer, x, f"d{dim}_t{n_tok}_s{n_shared}")
+
+
+@pytest.mark.parametrize("rows,m,n,wt", [
+    ([2000, 0, 2100, 1901], 1024, 1024, 64),  # 256 tiles of 128 x 128: one round
+    ([500, 0, 600, 401], 1024, 1024, 32),  # the same of fewer rows
+    ([2000, 0, 2100, 1901], 1024, 512, 32),  # half a round
+    ([1301, 1, 1500, 2000], 1020, 996, 64),  # partial tiles and K steps
+])
+def test_fp32_weight_gradient_tiles(gpu, rows, m, n, wt):
+    g = torch.Generator(device=gpu).manual_seed(m + n)
+    a = torch.randn(sum(rows), m, generator=g, device=gpu)
+    b = torch.randn(sum(rows), n, generator=g, device=gpu)
+    first = [sum(rows[:i]) for i in range(len(rows) + 1)]
+    offsets = torch.tensor(first, dtype=torch.int32, device=gpu)
+    names = _gemms(lambda: ops.moe_gemm_wgrad(a, b, offsets, len(rows)))
+    assert [f"gemm_f32_wgrad_kernel<{wt}>" in k for k in names] == [True], names
+    dw = ops.moe_gemm_wgrad(a, b, offsets, len(rows))
+    for e, (i, j) in enumerate(zip(first, first[1:])):
+        if j > i:
+            want = a[i:j].double().t() @ b[i:j].double()
+            # at most 2100 products of N(0, 1) values in fp32: error of about 1e-7 of sqrt(2100) each
+            assert (dw[e] - want).abs().max().item() < 2e-6 * (j - i) ** 0.5 * 10
