@@ -9,21 +9,23 @@
 // of one token at 1.6 TB/s (145 us). Here a column tile is 32 weight rows
 // (down) or 16 gate and 16 up rows, eight times as many workgroups, and the
 // four waves of a workgroup share a tile by taking every fourth 64-K step of
-// it: each wave streams its steps through an LDS ring of its own (four stages
-// of 32 activation and 32 weight rows by 128 bytes, DMA'd and swizzled as in
-// moe_gemm_mfma.hip), with no barrier in the K loop and across tile ends.
-// Then the waves' fp32 sums meet in LDS, summed in wave order, one barrier per
-// tile (the LDS they meet in alternates between two halves).
+// it: each wave streams its steps through an LDS ring of its own, DMA'd and
+// swizzled as in moe_gemm_mfma.hip, with no barrier in the K loop and across
+// tile ends. Three sizes of a stage (activation by weight rows of 128 bytes):
+// 32 x 32, four stages; 32 x 16, six; 64 x 32, three. Then the waves' fp32 sums
+// meet in LDS, summed in wave order, 32 rows at a time: one barrier for each 32,
+// the place they meet in alternating between two halves, or two barriers and one
+// place for the 64 x 32 stages, whose rings leave no room for more.
 //
 // Persistent, workgroup b taking tiles b, b + G, ...: consecutive workgroups
-// read consecutive weight rows of one expert. The steps of a tile start at a
-// place that depends on its expert and columns (see gemm_mfma_kernel), never
-// on the row tile's height, and each tile is walked in runs of 32 rows, so
-// results are the same for every height and for packed and gathered operands.
+// read consecutive weight rows of one expert. A row tile is walked in runs of
+// the stage's rows. The K order of a column tile's sums, which step each wave
+// starts at and the order of the waves, depends only on the expert and the column
+// tile (see gemm_mfma_kernel), so results are the same for every row tile height
+// and run, for packed and gathered operands.
 //
-// Measured: an MLP of D 4096, F 14336 over 24 rows 205 -> 100 us (352 MB of
-// weights, 3.5 TB/s), two experts of one token 240 -> 141 us (705 MB, 5.0
-// TB/s; its down GEMM 145 -> 45 us); more at few_rows below.
+// Measured at few_rows below; an MLP of D 4096, F 14336 over 24 rows streams its
+// 352 MB of weights at 4.4 TB/s (205 -> 80 us).
 #include <algorithm>
 #include <cmath>
 

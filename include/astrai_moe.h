@@ -384,8 +384,9 @@ int astrai_moe_forward(const void* x, const void* logits,
 
 /*
  * One dense expert over n_rows rows in one call (MLP.forward, mlp.py:22-25):
- * astrai_moe_dense_tiles and the grouped GEMMs with one-entry weight tables,
- * the same values; few rows without the list.
+ * astrai_moe_dense_tiles and the grouped GEMMs with one-entry weight tables, a
+ * list of its own height for each (the same values up to the order of a GEMM's
+ * fp32 sums); few rows without the list.
  *   x, out     [n_rows, dim] dtype
  *   workspace  astrai_moe_dense_forward_workspace_bytes(...) bytes for the
  *              same sizes, 256-byte aligned, nothing to initialise; calls

@@ -42,6 +42,23 @@ def test_layer(gpu, n_tok, n_exp, top_k, n_shared):
     assert torch.equal(layer(x), live)  # packed copies: the same bits
 
 
+@pytest.mark.parametrize("n_tok", [1200, 2000, 4400])
+def test_one_call_where_the_down_list_is_shorter(gpu, n_tok):
+    # listed on 256-row tiles; in one call the down GEMM has a list of 128 or 64 rows, or (4400) splits
+    # the last round of 256-row ones as well: the same sums in an order of their own at most
+    dim, dim_ffn = 4096, 14336
+    torch.manual_seed(n_tok)
+    ws = [(torch.randn(*s, device=gpu) * 0.02).bfloat16() for s in ((dim_ffn, dim), (dim_ffn, dim), (dim, dim_ffn))]
+    tables = [ops.expert_weight_table([w], tuple(w.shape)) for w in ws]
+    x = torch.randn(n_tok, dim, device=gpu).bfloat16()
+    assert ops.dense_block_m(n_tok, dim, dim_ffn, x.dtype) == 256
+    listed = ops.moe_dense_mlp(x, *tables, dim_ffn, tiles=ops.dense_tiles(n_tok, 256, x.device))
+    got = ops.moe_dense_mlp(x, *tables, dim_ffn)
+    torch.testing.assert_close(got, listed, rtol=2e-2, atol=2e-3)
+    want = R.expert_mlp(x[-300:], R.ExpertWeights(*ws))
+    torch.testing.assert_close(got[-300:], want, rtol=2e-2, atol=2e-2)
+
+
 @pytest.mark.parametrize("dim,dim_ffn", [(64, 64), (72, 328), (512, 1408), (1536, 4096)])
 @pytest.mark.parametrize("n_tok", [0, 1, 32, 33, 64, 65, 95, 96, 128, 129, 256, 257, 900])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
