@@ -12,13 +12,15 @@ Prints one JSON line:
   roofline        the dominant kernel (grouped gate/up GEMM): algorithmic
                   FLOPs (or bytes) per launch / its average launch time,
                   measured with HIP events on the launch stream around each
-                  launch in an instrumented pass of the layer forward; for a
+                  launch in a pass of the separate entry points; for a
                   launch under 0.2 ms, whose events would add the gaps around
                   it, around back-to-back launches of the same call on the
                   same inputs replayed from one HIP graph instead (longer
                   GEMMs run back to back at a lower clock than in the layer:
                   up to 30 % slower at 0.5 ms)
-  kernels_ms      average time of every stage
+  kernels_ms      average time of every stage in that pass (the layer's one
+                  call runs the same kernels, but an fp32 layer's gathers
+                  the token rows that the separate calls copy)
   cpu_baseline    the reference path (the oracle's torch restatement of
                   mlp.py:64-100) on the host CPU, on a bounded token sample of
                   the same layer, with every host core the process may use
@@ -361,15 +363,12 @@ def main():
         t_wall = time.perf_counter() - t_wall
         ms_per_step = start.elapsed_time(end) / args.steps
 
-        # the same kernels through their own entry points, each between events
+        # the separate entry points (no shared experts in these workloads), each between events
         x_rows = x.view(-1, w.dim)
         state = layer._current(x.dtype, x.device)
-        packed = layer._packed_tables(x.dtype, state)
-        tables = (packed[0], *packed) if packed is not None else state.tables[0]
         with StageTimer(ops) as timer:
             for _ in range(args.steps):
-                ops.moe_routed_forward(x_rows, layer.router(x_rows), *tables, w.dim_ffn, w.top_k,
-                                       packed=packed is not None)
+                layer._routed_forward(x_rows, state)
             torch.cuda.synchronize()
         stage_ms = timer.avg_ms()
 
@@ -442,14 +441,14 @@ def main():
     t_gu, t_dn = stage_ms["moe_gemm_gate_up"] / 1e3, stage_ms["moe_gemm_down"] / 1e3
     gemm_tflops = (flops_gate_up + flops_down) / (t_gu + t_dn) / 1e12
     t_roof = t_gu  # the dominant kernel's average launch duration
-    timing = f"HIP events on the launch stream around each of its {args.steps} launches in the layer forward"
+    timing = f"HIP events on the launch stream around each of its {args.steps} launches through the separate entry points"
     if t_gu < 2e-4 and "moe_gemm_gate_up" in timer.last_call:
         with torch.inference_mode():
             b2b_ms, n_b2b = back_to_back_ms(timer.last_call["moe_gemm_gate_up"], t_gu * 1e3)
         t_roof = b2b_ms / 1e3
         timing = (f"HIP events on the replay stream around {n_b2b} back-to-back launches of the layer's gate/up "
-                  f"call replayed from one HIP graph (median of 3; events around each launch in the layer "
-                  f"forward: {t_gu * 1e3:.4f} ms)")
+                  f"call replayed from one HIP graph (median of 3; events around each launch "
+                  f"through the separate entry points: {t_gu * 1e3:.4f} ms)")
     n_active = int((counts > 0).sum().item())
     weight_bytes = n_active * 3.0 * w.dim * w.dim_ffn * s
     # permutation: the index outputs (routing entries and chunk histograms
