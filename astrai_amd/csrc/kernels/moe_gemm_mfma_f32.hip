@@ -194,26 +194,30 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(
     lds_barrier();
     read_frags(0, 0, 0);
     int buf = 0;
-    // (the last step stands behind the loop: with it inside, the compiler waited
-    // for the next step's fragment reads before each step's second half)
-    for (int kt = 0; kt + 1 < KT; ++kt) {
+    // (the saving kernels' last step stands behind the loop: 0.5 to 1 % faster
+    // there, 1 to 3 % slower in the others)
+    for (int kt = 0; kt < (kSave ? KT - 1 : KT); ++kt) {
       read_frags(buf, 1, 1);
       mfmas(0);
       const int nbuf = (buf + 1 == S) ? 0 : buf + 1;
-      wait_groups<DPW, S - 2>(min(S - 2, KT - 2 - kt));
-      __builtin_amdgcn_sched_barrier(0);
-      lds_barrier();  // step kt + 1 landed; every wave is done reading buffer `buf`
-      __builtin_amdgcn_sched_barrier(0);
-      read_frags(nbuf, 0, 0);
-      __builtin_amdgcn_sched_barrier(0);
-      if (kt + S < KT) issue_stage(kt + S, buf);
-      __builtin_amdgcn_sched_barrier(0);
+      if (kSave || kt + 1 < KT) {
+        wait_groups<DPW, S - 2>(min(S - 2, KT - 2 - kt));
+        __builtin_amdgcn_sched_barrier(0);
+        lds_barrier();  // step kt + 1 landed; every wave is done reading buffer `buf`
+        __builtin_amdgcn_sched_barrier(0);
+        read_frags(nbuf, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        if (kt + S < KT) issue_stage(kt + S, buf);
+        __builtin_amdgcn_sched_barrier(0);
+      }
       mfmas(1);
       buf = nbuf;
     }
-    read_frags(buf, 1, 1);
-    mfmas(0);
-    mfmas(1);
+    if constexpr (kSave) {
+      read_frags(buf, 1, 1);
+      mfmas(0);
+      mfmas(1);
+    }
 
     // ---- epilogue: 16 contiguous bytes per lane and tile ----
 #pragma unroll

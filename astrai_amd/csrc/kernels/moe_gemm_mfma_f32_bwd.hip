@@ -153,26 +153,23 @@ __global__ __launch_bounds__(256) void gemm_f32_dgrad_kernel(const float* __rest
     lds_barrier();
     read_frags(0, 0, 0);
     int buf = 0;
-    // (the last step stands behind the loop: with it inside, the compiler waited
-    // for the next step's fragment reads before each step's second half)
-    for (int kt = 0; kt + 1 < KT; ++kt) {
+    for (int kt = 0; kt < KT; ++kt) {
       read_frags(buf, 1, 1);
       mfmas(0);
       const int nbuf = (buf + 1 == S) ? 0 : buf + 1;
-      wait_groups<DPW, S - 2>(min(S - 2, KT - 2 - kt));
-      __builtin_amdgcn_sched_barrier(0);
-      lds_barrier();  // step kt + 1 landed; every wave is done reading buffer `buf`
-      __builtin_amdgcn_sched_barrier(0);
-      read_frags(nbuf, 0, 0);
-      __builtin_amdgcn_sched_barrier(0);
-      if (kt + S < KT) issue_stage(kt + S, buf);
-      __builtin_amdgcn_sched_barrier(0);
+      if (kt + 1 < KT) {
+        wait_groups<DPW, S - 2>(min(S - 2, KT - 2 - kt));
+        __builtin_amdgcn_sched_barrier(0);
+        lds_barrier();  // step kt + 1 landed; every wave is done reading buffer `buf`
+        __builtin_amdgcn_sched_barrier(0);
+        read_frags(nbuf, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        if (kt + S < KT) issue_stage(kt + S, buf);
+        __builtin_amdgcn_sched_barrier(0);
+      }
       mfmas(1);
       buf = nbuf;
     }
-    read_frags(buf, 1, 1);
-    mfmas(0);
-    mfmas(1);
 
     // ---- epilogue: row wave * 16 + c, columns 16 g + 4 r .. + 3 ----
     const int rr = wave * 16 + c;
