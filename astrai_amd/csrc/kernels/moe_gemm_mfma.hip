@@ -1053,9 +1053,10 @@ using MidCfg = TileCfg<kMfmaMidBM, 256, 3, 2, 4, 8>;
 // the down epilogue's per-wave 16-row slices stay small), three 48 KB stages
 // in flight: 144 KB of stages + 10 KB of epilogue slices.
 using Mid2Cfg = TileCfg<kMfmaMid2BM, 256, 3, 1, 8, 8>;
-// Few tiles: 128 x 128 outputs, 8 waves of 64 x 32, four 32 KB stages. LDS
-// bandwidth bounds a step (96 KB of fragments read and 32 KB written for 0.21 us
-// of MFMA), but twice as many compute units work on a GEMM as with 256 columns.
+// Few tiles: 128 x 128 outputs, 8 waves of 64 x 32, four 32 KB stages. A step
+// moves 96 KB of fragments out of LDS and 32 KB into it, 0.43 us at 128 bytes a
+// clock, for 0.21 us of MFMA (0.71 measured, without bank conflicts), but twice as
+// many compute units work on a GEMM as with 256 columns.
 using NarrowCfg = TileCfg<kMfmaMid2BM, 128, 4, 2, 4, 8>;
 // The same of 64-row lists: 64 x 128 outputs, 4 waves of 64 x 32, three stages.
 using NarrowMidCfg = TileCfg<kMfmaMidBM, 128, 3, 1, 4, 8>;

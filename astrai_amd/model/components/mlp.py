@@ -164,8 +164,9 @@ class DeepSeekMoE(nn.Module):
         # Opt-in, inference only: keep a packed copy of the experts' weights
         # in the order the GEMMs stage it (ops.moe_pack_*), rebuilt when a
         # weight moves or changes (its version counter), for bf16 shapes the
-        # packed GEMMs take. Same results; doubles the weights' memory for about 1 % less GEMM time (3 % on the down GEMM of
-        # decode-sized loads), so it is off by default.
+        # packed GEMMs take (few rows read the live weights). Same results;
+        # doubles the weights' memory for about 1 % less GEMM time (3 % on the
+        # down GEMM of decode-sized loads), so it is off by default.
         self.pack_weights = False
         self._packed: tuple | None = None
 
@@ -247,8 +248,9 @@ class DeepSeekMoE(nn.Module):
         this forward reads the live weights. The copies are rebuilt whenever a
         weight's storage or version counter changes (the shared experts' are
         packed with the routed ones where both run in one forward call); the
-        cache holds a view of each source weight so that its storage (and address) cannot be
-        reused by another tensor while the copy made from it is in use."""
+        cache holds a view of each source weight so that its storage (and
+        address) cannot be reused by another tensor while the copy made from it
+        is in use."""
         if not self.uses_packed_weights(dtype):
             return None
         g, u, d = map(list.__add__, st.routed, st.shared) if self._joint(st) else st.routed
