@@ -94,7 +94,8 @@ Plan make_plan(const Sizes& z) {
   p.x_perm = p.y;  // copied rows are read by the gate/up GEMM, before the down GEMM writes y
   // the 256-row GEMMs' scheduling block, and partial sums where the down
   // GEMM's tiles are long enough to be split
-  if (p.block_m == kMfmaBigBM) p.gemm_ws_bytes = gemm_workspace_bytes(splits_tail(z.dim_ffn));
+  if (p.block_m == kMfmaBigBM)
+    p.gemm_ws_bytes = gemm_workspace_bytes(down_splits(row_counts(z), p.block_m, z.dim_ffn, z.dim, p.packed_down));
   p.gemm_ws = part(p.gemm_ws_bytes);
   p.bytes = at;
   return p;
@@ -223,7 +224,7 @@ DensePlan dense_plan(int64_t n_rows, int64_t dim, int64_t dim_ffn, int dtype) {
   p.tiles_down = p.len_down > 0 ? part(p.len_down * 4) : p.tiles;
   p.h = part(n_rows * dim_ffn * (dtype == ASTRAI_MOE_BF16 ? 2 : 4));
   if (p.block_m == kMfmaBigBM || p.block_m_down == kMfmaBigBM)
-    p.gemm_ws_bytes = gemm_workspace_bytes(p.block_m_down == kMfmaBigBM && splits_tail(dim_ffn));
+    p.gemm_ws_bytes = gemm_workspace_bytes(down_splits({n_rows, 1}, p.block_m_down, dim_ffn, dim, false));
   p.gemm_ws = part(p.gemm_ws_bytes);
   return p;
 }

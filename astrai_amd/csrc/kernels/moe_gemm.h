@@ -85,6 +85,10 @@ struct RowCounts {
   bool dense() const { return experts == 0 && exact == 1; }
 };
 
+// Whether a down GEMM takes whole 256-row tiles and splits its last round of them
+// (its workspace then holds the partial sums).
+bool down_splits(const RowCounts& rows, int block_m, int64_t k, int64_t n, bool packed);
+
 // Row tiles of `bm` rows that a load makes: expected under even routing (an
 // expert's rows about normal, with their mean as variance); under a skewed one
 // (the last tile of nearly every expert nearly empty: routers biased by Zipf

@@ -1270,6 +1270,11 @@ int dense_gemm_block_m(int64_t n_rows, int64_t k, int64_t n, bool gate_up) {
   return best;
 }
 
+bool down_splits(const RowCounts& rows, int block_m, int64_t k, int64_t n, bool packed) {
+  return block_m == kMfmaBigBM && splits_tail(k) &&
+         (packed || pick_tiles(rows, block_m, k, n, false).tiles == Tiles::kList);
+}
+
 int64_t gemm_workspace_bytes(bool down) {
   return kSchedBytes + (down ? (int64_t)cu_count() * (int64_t)sizeof(float) * kSplitUnitFloats : 0);
 }

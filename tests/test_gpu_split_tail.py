@@ -16,10 +16,14 @@ SIZES = [(4024, False), (4032, False), (4040, True), (4088, True), (4096, True)]
 
 @pytest.mark.parametrize("dim_ffn,split", SIZES)
 def test_workspaces_hold_the_partial_sums(dim_ffn, split):
-    lib, t, dim = loader.library(), 2048, 1000
+    lib, t, dim = loader.library(), 8192, 1000
     sums = lib.astrai_moe_gemm_workspace_bytes(1) - lib.astrai_moe_gemm_workspace_bytes(0)
+    rows = 2 * t * (dim + dim_ffn) * 2  # h and y
     layer = lib.astrai_moe_forward_workspace_bytes(t, 8, 2, 0, dim, dim_ffn, 1, 0)
-    assert (layer > sums) == split, layer
+    assert (layer > rows + sums) == split, layer
+    # few tiles, which are halved and not split: none
+    assert lib.astrai_moe_forward_workspace_bytes(640, 8, 2, 0, dim, dim_ffn, 1, 0) < sums
+    assert lib.astrai_moe_dense_forward_workspace_bytes(1024, 4096, dim_ffn, 1) < sums
     x = torch.empty(0, dtype=torch.bfloat16)
     assert (ops._workspace(x, dim, dim_ffn, 256, down=True)[1] > sums) == split
 
