@@ -135,15 +135,16 @@ extern "C" int astrai_moe_forward(const void* x, const void* logits, const void*
                  (long long)dim_ffn);
   ASTRAI_REQUIRE(workspace_bytes >= p.bytes, "forward: workspace holds %lld bytes, needs %lld",
                  (long long)workspace_bytes, (long long)p.bytes);
-  ASTRAI_REQUIRE(!p.gather || reinterpret_cast<uintptr_t>(x) % 16 == 0,
+  // (a layer with packed copies copies such rows, whichever weights its GEMMs read)
+  const bool x_aligned = reinterpret_cast<uintptr_t>(x) % 16 == 0;
+  ASTRAI_REQUIRE(!p.gather || z.packed || x_aligned,
                  "forward: unsupported alignment (x must start on a 16-byte boundary)");
   char* const base = static_cast<char*>(workspace);
   auto i32 = [&](int64_t off) { return reinterpret_cast<int32_t*>(base + off); };
   int32_t *topk_idx = i32(p.topk_idx), *hist = i32(p.chunk_hist), *sorted_token = i32(p.sorted_token),
           *token_pos = i32(p.token_pos), *tiles = i32(p.tiles);
   void *topk_w = base + p.topk_w, *sorted_w = base + p.sorted_w, *h = base + p.h, *y = base + p.y;
-  const bool x_aligned = reinterpret_cast<uintptr_t>(x) % 16 == 0;
-  const bool gather = p.gather || (p.gather_ragged && x_aligned), gather_f32 = p.gather_f32 && x_aligned;
+  const bool gather = (p.gather || p.gather_ragged) && x_aligned, gather_f32 = p.gather_f32 && x_aligned;
   void* const x_perm = gather || gather_f32 ? nullptr : base + p.x_perm;
   void* const gws = p.gemm_ws_bytes > 0 ? base + p.gemm_ws : nullptr;
   hipStream_t s = static_cast<hipStream_t>(stream);

@@ -71,6 +71,18 @@ def test_separate_calls_of_a_packed_layer_with_shared_experts(gpu):
     assert torch.equal(apart(), live)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("n_tok", [5, 40, 700])
+def test_packed_layers_take_unaligned_rows(gpu, n_tok):
+    # copied, also where few rows read the live weights: the bits of the aligned rows
+    layer = _random_layer(gpu, 256, 512, 4, 1, 2, torch.bfloat16, seed=n_tok).requires_grad_(False)
+    layer.pack_weights = True
+    flat = torch.randn(4 + n_tok * 256, device=gpu).to(torch.bfloat16)
+    x = flat[4:].view(1, n_tok, 256)
+    assert x.data_ptr() % 16 == 8
+    assert torch.equal(layer(x), layer(x.clone()))
+
+
 def _peak(run):
     run()  # allocations that stay
     torch.cuda.synchronize()
