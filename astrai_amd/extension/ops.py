@@ -557,7 +557,8 @@ def moe_layer_forward(x: torch.Tensor, logits: torch.Tensor, w_gate: torch.Tenso
     """The layer's output for ``x [T, D]`` and its router logits (mlp.py:71-100)
     in one call of the library. The pointer tables hold the routed experts and
     then the ``n_shared`` shared ones; ``packed``: tables (gate/up, down) of
-    their packed copies, read in place of the weights."""
+    their packed copies, read in place of the weights except by GEMMs of few
+    rows (the same bits)."""
     _require_gpu(x, "x", 2)
     _require_gpu(logits, "logits", 2)
     code = _dtype_code(x, "x")

@@ -359,7 +359,8 @@ int astrai_moe_combine(const void* y, const int32_t* token_pos, const void* row_
  *   w_gate, w_up, w_down  device arrays of n_experts + n_shared pointers, the
  *            routed experts' first ([dim_ffn, dim], [dim_ffn, dim], [dim, dim_ffn])
  *   packed_gate_up, packed_down  tables of packed copies of the same experts
- *            (astrai_moe_pack_*), read in place of the weights, or NULL
+ *            (astrai_moe_pack_*), read in place of the weights, or NULL; GEMMs
+ *            of few rows read the weights all the same (the same bits)
  *   workspace  astrai_moe_forward_workspace_bytes(...) bytes for the same
  *            sizes, 256-byte aligned, nothing to initialise; calls sharing one
  *            must not overlap
